@@ -202,6 +202,68 @@ struct TableQueryUnit {
   }
 };
 
+// The table's row of a position; a negative position (the sine is negated, reference rope_correction.py:36-42)
+// is kept as the complement of its row.
+__device__ __forceinline__ int table_row(const RopeDev& rope, long long pos) {
+  const long long a = pos < 0 ? -pos : pos;
+  const int row = (int)(a > rope.max_pos - 1 ? rope.max_pos - 1 : a);
+  return pos < 0 ? ~row : row;
+}
+// Cosines and sines of eight pairs, loaded ahead of their use, and the rotation of a rotary pair of pieces
+// in place by them: fp32 products and sums, each rounded by itself, one rounding to the element type.
+struct TableTurn {
+  float4 c[2], s[2];
+  __device__ __forceinline__ void load(const float* entry, int half) {
+    c[0] = *(const float4*)entry;
+    c[1] = *(const float4*)(entry + 4);
+    s[0] = *(const float4*)(entry + half);
+    s[1] = *(const float4*)(entry + half + 4);
+  }
+  template <typename E>
+  __device__ __forceinline__ void apply(bool back, va_u32x4& xa, va_u32x4& xb) const {
+    using S = typename E::storage;
+    const float ct[8] = {c[0].x, c[0].y, c[0].z, c[0].w, c[1].x, c[1].y, c[1].z, c[1].w};
+    const float st[8] = {s[0].x, s[0].y, s[0].z, s[0].w, s[1].x, s[1].y, s[1].z, s[1].w};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      float y1[2], y2[2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const float x1 = E::load(__builtin_bit_cast(S, (uint16_t)(xa[w] >> (16 * b))));
+        const float x2 = E::load(__builtin_bit_cast(S, (uint16_t)(xb[w] >> (16 * b))));
+        const float sn = back ? -st[2 * w + b] : st[2 * w + b];
+        y1[b] = mul_rounded(ct[2 * w + b], x1) - mul_rounded(sn, x2);
+        y2[b] = mul_rounded(ct[2 * w + b], x2) + mul_rounded(sn, x1);
+      }
+      xa[w] = Mma<E>::pack(y1[0], y1[1]);
+      xb[w] = Mma<E>::pack(y2[0], y2[1]);
+    }
+  }
+};
+
+// mRoPE rotation of a rotary pair of pieces in place; `cs`: their eight cos|sin entries, cast to the element
+// type and packed (cosine in the low half).  The arithmetic is rope_pair's: every product and the sum are
+// rounded to the element type.
+template <typename E>
+__device__ __forceinline__ void rotate_packed(const va_u32x4 (&cs)[2], va_u32x4& xa, va_u32x4& xb) {
+  using S = typename E::storage;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    float y1[2], y2[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const uint32_t e = cs[w / 2][2 * (w % 2) + b];
+      const float c = E::load(__builtin_bit_cast(S, (uint16_t)e)), sn = E::load(__builtin_bit_cast(S, (uint16_t)(e >> 16)));
+      const float x1 = E::load(__builtin_bit_cast(S, (uint16_t)(xa[w] >> (16 * b))));
+      const float x2 = E::load(__builtin_bit_cast(S, (uint16_t)(xb[w] >> (16 * b))));
+      y1[b] = round_through<E>(mul_rounded(x1, c)) + round_through<E>(mul_rounded(-x2, sn));
+      y2[b] = round_through<E>(mul_rounded(x2, c)) + round_through<E>(mul_rounded(x1, sn));
+    }
+    xa[w] = Mma<E>::pack(y1[0], y1[1]);  // the last rounding
+    xb[w] = Mma<E>::pack(y2[0], y2[1]);
+  }
+}
+
 // Wait until the matrix pipe has written the results of the products issued from assembly
 // (run32_acc) into the accumulators `o`, before anything but another product touches them.  A
 // 32x32x16 product runs for 8 passes of 4 clocks and its result needs 3 more wait states to reach

@@ -29,6 +29,8 @@
 // ring buffers that are not yet in use.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "va_internal.h"
 #include "va_launch.h"
 #include "va_mfma_common.h"
@@ -56,7 +58,6 @@ struct WideShape {
   static constexpr int kLoadsPerWave = 2 * kLoadsPerKind / kWideWaves;
   static constexpr int kTileBytes = kWideTokens * kRowBytes;  // a K (or V) tile
   static constexpr int kBufferBytes = 2 * kTileBytes;
-  static constexpr int kLdsBytes = kWideBuffers * kBufferBytes;  // 128 KB at D = 256
   // 32-row blocks per wave.  Two blocks halve the LDS bytes read per flop, but the state of a row
   // (D fp32 accumulators + D 16-bit query elements) then fills the register file at D = 256:
   // 64 rows need 256 + 128 of the 512 registers before any operand is staged, and the compiler
@@ -64,13 +65,18 @@ struct WideShape {
   static constexpr int kBlocks = kD == 256 ? 1 : 2;
   static constexpr int kWaveRows = 32 * kBlocks;
   static constexpr int kTileRows = kWideWaves * kWaveRows;  // MFMA rows per workgroup
-  static_assert(128 * kRowBytes == 2 * kBufferBytes, "one row block of every wave fills two ring buffers");
+  // The cosines and sines of an mRoPE tile (at most one row per MFMA row, kD / 2 entries of four bytes)
+  // lie behind the tiles requested during the set-up: at D = 256 in the rest of the ring (128 KB in all),
+  // at smaller head dims past its end.
+  static constexpr int kTurnBytes = kTileRows * (kD / 2) * 4;
+  static constexpr int kRingBytes = kWideBuffers * kBufferBytes, kSetupBytes = kWideAhead * kBufferBytes + kTurnBytes;
+  static constexpr int kLdsBytes = kRingBytes > kSetupBytes ? kRingBytes : kSetupBytes;
 };
 
-template <int kD>
-__device__ __forceinline__ int wide_swz(int r) {
-  if constexpr (kD >= 128) return r & 15;
-  return (r >> 1) & 7;
+// Word of the cos|sin entry (row iq, pair dim) in LDS: rows of `half` words, their 16-byte pieces swizzled
+// by the row so that the rows a wave reads side by side spread over the banks.
+__device__ __forceinline__ int turn_word(int iq, int pair, int half) {
+  return iq * half + 4 * ((pair >> 2) ^ (iq & min(7, (half >> 2) - 1))) + (pair & 3);
 }
 
 // Ring buffer of a tile (tile numbers are never negative: the unsigned remainder is one instruction
@@ -121,7 +127,15 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     const unsigned block = turn / (g * a.num_kv_heads), within = turn % (g * a.num_kv_heads);
     where = ItemHead{(int)((block * g + within % g) * 8u + die), (int)(within / g)};
   }
-  const int item_begin = a.wide_slots[where.item], item_end = a.wide_slots[where.item + 1];
+  // The plan is read through the constant address space: scalar loads, all words of an item or a link in one
+  // trip (as ordinary loads they go out one after the other, each waiting for the one before it)
+  using PlanWords = const __attribute__((address_space(4))) int32_t*;
+  // mRoPE: threads per pair dim when cosines and sines are taken, the rows of a tile rounded up to a power of two
+  int turn_lanes = 1;
+  while (turn_lanes < Sh::kTileRows / (a.num_q_heads / a.num_kv_heads)) turn_lanes <<= 1;
+  const int turn_iq = threadIdx.x & (turn_lanes - 1);
+  const PlanWords slots_of = (PlanWords)a.wide_slots + where.item;
+  const int item_begin = slots_of[0], item_end = slots_of[1];
   const int hk = where.head;
   const int G = a.num_q_heads / a.num_kv_heads;
   const int tid = threadIdx.x;
@@ -194,11 +208,24 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
   const uint32_t lds_base = lds_address(lds);
 
   for (int item_index = item_begin; item_index < item_end; ++item_index) {
-  const int32_t* item = a.items + (long long)item_index * VA_ITEM_WORDS;
+  const PlanWords item = (PlanWords)a.items + (long long)item_index * VA_ITEM_WORDS;
   const int n_q = item[VA_I_N_Q];
   if (n_q == 0) continue;  // padding item
   const int part_base = item[VA_I_PART_BASE];
   const bool wave_active = (kWaveRows * wave) / G < n_q;  // the wave owns real rows
+  // This lane's query rows: the links of an item serve the same output rows, so the first one tells them.
+  // Rows past the tile repeat its last row.
+  const S* q_row[kB];
+  {
+    const PlanWords link0 = item + VA_I_LINK0;
+#pragma unroll
+    for (int b = 0; b < kB; ++b) {
+      const int at = link0[VA_L_QREF] + min(row_iq[b], n_q - 1);
+      const long long src_row = a.sub_worker[(link0[VA_L_FLAGS] & VA_LINK_INDIRECT) ? a.qrefs[at] : at];
+      const int g = row0 + 32 * b - row_iq[b] * G;
+      q_row[b] = (const S*)a.q + src_row * a.q_row_stride + (long long)(hk * G + g) * kD + 8 * h;
+    }
+  }
 
   float m_ref[kB], m_tile[kB], l_run[kB];  // reference maximum (log2 units), last tile maximum, row sum
   float raise_above[kB];                    // m_ref + kWideRaise: what a tile's maximum is tested against
@@ -215,8 +242,11 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
       for (int r = 0; r < 16; ++r) o[b][t][r] = 0.f;
   }
 
-  for (int li = 0; li < item[VA_I_N_LINKS]; ++li) {
-    const int32_t* link = a.links + (long long)(item[VA_I_LINK_BEGIN] + li) * VA_LINK_WORDS;
+  const int wave_half = wave & 1;
+  const bool table = a.rope.mode == VA_ROPE_TABLE;
+  const int n_links = item[VA_I_N_LINKS];
+  PlanWords link = (PlanWords)a.links + (long long)item[VA_I_LINK_BEGIN] * VA_LINK_WORDS;
+  for (int li = 0; li < n_links; ++li, link += VA_LINK_WORDS) {
     const int lflags = link[VA_L_FLAGS];
     const int qref = link[VA_L_QREF];
     const int kv_begin = link[VA_L_KV_BEGIN];
@@ -245,7 +275,6 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     // the visible range, and page tables with pages under 16 tokens or slot lists, look every
     // row up per lane instead (rows past the range re-read the last visible token; their scores
     // are masked).
-    const int wave_half = wave & 1;
     const char* wave_pool = (const char*)(wave_is_v ? vp : kp);
     const char* wave_plain = wave_pool - kLoadBias;  // base of plain loads: the per-lane offsets carry the bias
     const uint32_t wave_lds = __builtin_amdgcn_readfirstlane(lds_address(lds)) + (wave_is_v ? Sh::kTileBytes : 0) +
@@ -260,8 +289,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     };
     auto half_row = [&](int i) __attribute__((always_inline)) {
       const int t = tok_begin + i * kWideTokens + 16 * wave_half;
-      const int page = ((const __attribute__((address_space(4))) int32_t*)a.kv_indices)[kv_begin + (t >> p_shift)];
-      return half_offset(page, t);
+      return half_offset(((PlanWords)a.kv_indices)[kv_begin + (t >> p_shift)], t);
     };
     auto tile_is_plain = [&](int i) __attribute__((always_inline)) {
       return uniform_pages && tok_begin + (i + 1) * kWideTokens - 1 <= t_last;
@@ -281,104 +309,152 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
         }
       }
     };
-    auto issue_now = [&](int i) __attribute__((always_inline)) { issue(i, tile_is_plain(i) ? half_row(i) : 0); };
+    // The pool row of the tile a ring step requests is looked up a whole step earlier (a scalar load whose
+    // result is not touched before the next step): its latency never shows.
+    auto row_of = [&](int tile) __attribute__((always_inline)) {
+      return (tile < n_tiles && tile_is_plain(tile)) ? half_row(tile) : 0ull;
+    };
 
-    // ---- set-up: first two tiles on their way, then the query tile (staged in buffers 2 and 3) ----
-    __syncthreads();  // every wave is done with the previous link's buffers
+    // ---- set-up: the first two tiles on their way, the query rows rotated for this link ----
+    // Every lane loads its own rows in operand order and rotates them in registers: a rotary pair
+    // (dim d, dim d + half) is the same element of operands s and s + half / 16 of one lane, so nothing is
+    // exchanged between lanes (staged through LDS the tile took two barriers and 13 300 cycles a link at D = 256
+    // with the table, 21 200 under mRoPE; 11 900 and 13 300 like this).  What bounds it now is the L1's rate
+    // for 64 KB of query pieces at 16 bytes a row and the table entries.  Positions, query rows and the page
+    // numbers of the first tiles are requested together, ahead of the barrier; the tiles and the table entries,
+    // which need them, behind it.
+    va_u32x4 qf[kB][kSteps];  // B operands: row of block b, dims [16s + 8h, +8)
+    uint32_t* turns = (uint32_t*)(lds + kWideAhead * Sh::kBufferBytes);
+    const int half = a.rope.half, half_steps = a.rope.rotary_dim % 32 == 0 ? a.rope.rotary_dim / 32 : -1;
+    const bool in_turn = half_steps > 0 && (half_steps == kSteps / 2 || half_steps == kSteps / 4 || half_steps == kSteps / 8);
+    auto subrow_of = [&](int iq) __attribute__((always_inline)) {
+      const int at = qref + min(iq, n_q - 1);
+      return (lflags & VA_LINK_INDIRECT) ? a.qrefs[at] : at;
+    };
+    long long pos[kB < 3 ? 3 : kB];  // table: the positions of the lane's rows; mRoPE: that of row turn_iq, three axes
+    if (table) {
+#pragma unroll
+      for (int b = 0; b < kB; ++b) pos[b] = a.sub_loc[subrow_of(row_iq[b])];
+    } else {
+      const Pos3 p = load_pos(a.sub_loc, a.sub_loc_axis_stride, subrow_of(turn_iq));
+      pos[0] = p.t;
+      pos[1] = p.h;
+      pos[2] = p.w;
+    }
+#pragma unroll
+    for (int b = 0; b < kB; ++b)
+#pragma unroll
+      for (int s = 0; s < kSteps; ++s) qf[b][s] = *(const va_u32x4*)(q_row[b] + 16 * s);
+    unsigned long long first_rows[kWideAhead];
+#pragma unroll
+    for (int i = 0; i < kWideAhead; ++i) first_rows[i] = row_of(i);
+    // (the positions are waited for before the tiles are requested: later they would have to wait for the tiles)
+    if (table) {
+#pragma unroll
+      for (int b = 0; b < kB; ++b) asm volatile("" : "+v"(pos[b]));
+    } else {
+      asm volatile("" : "+v"(pos[0]), "+v"(pos[1]), "+v"(pos[2]));
+    }
+    ring_barrier<kAnyInFlight>();  // every wave has read the previous link's last tile
 #pragma unroll
     for (int i = 0; i < kWideAhead; ++i)
-      if (i < n_tiles) issue_now(i);
-    va_u32x4* q_stage = (va_u32x4*)(lds + kWideAhead * Sh::kBufferBytes);
-    va_u32x4 qf[kB][kSteps];  // B operands: row of block b, dims [16s + 8h, +8)
+      if (i < n_tiles) issue(i, first_rows[i]);
+    if (!table && in_turn) {
+      // mRoPE: the cosines and sines of the tile's positions, each taken once and shared by the G query
+      // heads of a row (an entry is cos | sin in the element type, as the rotation rounds them).  A thread
+      // keeps to one row; the lanes of a wave work on few pair dims, so that the long argument reduction
+      // of the fast turning ones stays out of most waves.
+      const float axes[3] = {(float)pos[0], (float)pos[1], (float)pos[2]};
+      const int first = tid / turn_lanes, step = kWideThreads / turn_lanes;
+      if (turn_iq < n_q) {
+        constexpr int kBatch = 8;  // frequencies requested together
+#pragma unroll 1
+        for (int pair0 = first; pair0 < half; pair0 += kBatch * step) {
+          float freq[kBatch];
 #pragma unroll
-    for (int pass = 0; pass < kB; ++pass) {
-      if (a.rope.mode == VA_ROPE_TABLE) {
-        // Every thread stages one unit (two pieces) of kIts rows.  The sub-row numbers are fetched
-        // for all rows at once, source rows and positions, then pieces and table entries, for
-        // kBatch rows at once: a row's chain of dependent loads (sub-row -> source row and position
-        // -> query pieces and cos|sin entries) is paid once per batch, not once per row (row by row
-        // this set-up was an eighth of the kernel on long views of many blocks).
-        constexpr int kUnits = kChunks / 2, kRowStep = kWideThreads / kUnits, kIts = 128 / kRowStep;
-        constexpr int kBatch = kIts < 4 ? kIts : 4;
-        static_assert(kWideThreads % kUnits == 0 && 128 % kRowStep == 0 && kIts % kBatch == 0, "staging pattern");
-        const int x = tid % kUnits, rl0 = tid / kUnits;
-        const int pair_units = a.rope.rotary_dim / 16;
-        const bool rotary = x < pair_units;
-        const int c0 = rotary ? x : a.rope.rotary_dim / 8 + 2 * (x - pair_units);
-        const int c1 = rotary ? x + pair_units : c0 + 1;
-        bool live[kIts];
-        int subrow[kIts];
+          for (int x = 0; x < kBatch; ++x) freq[x] = a.rope.inv_freq[min(pair0 + x * step, half - 1)];
 #pragma unroll
-        for (int it = 0; it < kIts; ++it) {
-          const int Rl = rl0 + it * kRowStep;
-          const int R = kWaveRows * (Rl / 32) + 32 * pass + Rl % 32;  // block `pass` of every wave
-          const int iq = R / G;
-          live[it] = iq < n_q;
-          const int iqc = live[it] ? iq : 0;  // rows past the tile stage row 0's numbers and are zeroed below
-          subrow[it] = (lflags & VA_LINK_INDIRECT) ? a.qrefs[qref + iqc] : qref + iqc;
-        }
-#pragma unroll
-        for (int it0 = 0; it0 < kIts; it0 += kBatch) {
-          const S* qh[kBatch];
-          Pos3 pos[kBatch];
-#pragma unroll
-          for (int jj = 0; jj < kBatch; ++jj) {
-            const int Rl = rl0 + (it0 + jj) * kRowStep;
-            const int R = kWaveRows * (Rl / 32) + 32 * pass + Rl % 32;
-            const int iq = R / G, g = R - iq * G;
-            const long long src_row = a.sub_worker[subrow[it0 + jj]];
-            qh[jj] = (const S*)a.q + src_row * a.q_row_stride + (long long)(hk * G + g) * kD;
-            pos[jj] = load_pos(a.sub_loc, a.sub_loc_axis_stride, subrow[it0 + jj]);
+          for (int x = 0; x < kBatch; ++x) {
+            const int pair = pair0 + x * step;
+            float c, sn;
+            mrope_cos_sin(a.rope, axes, freq[x], pair, c, sn);
+            if (pair < half) turns[turn_word(turn_iq, pair, half)] = Mma<E>::pack(c, sn);
           }
-          uint4 p0[kBatch], p1[kBatch];
-          if (rotary) {
-            TableQueryUnit<E> unit[kBatch];
-#pragma unroll
-            for (int jj = 0; jj < kBatch; ++jj) unit[jj].load(a.rope, qh[jj], x, pos[jj]);
-#pragma unroll
-            for (int jj = 0; jj < kBatch; ++jj) unit[jj].finish(a.rope, pos[jj], p0[jj], p1[jj]);
-          } else {
-#pragma unroll
-            for (int jj = 0; jj < kBatch; ++jj) {
-              p0[jj] = *(const uint4*)(qh[jj] + 8 * c0);
-              p1[jj] = *(const uint4*)(qh[jj] + 8 * c1);
-            }
-          }
-#pragma unroll
-          for (int jj = 0; jj < kBatch; ++jj) {
-            const int Rl = rl0 + (it0 + jj) * kRowStep;
-            if (!live[it0 + jj]) p0[jj] = p1[jj] = make_uint4(0, 0, 0, 0);
-            q_stage[Rl * kChunks + (c0 ^ wide_swz<kD>(Rl))] = va_u32x4{p0[jj].x, p0[jj].y, p0[jj].z, p0[jj].w};
-            q_stage[Rl * kChunks + (c1 ^ wide_swz<kD>(Rl))] = va_u32x4{p1[jj].x, p1[jj].y, p1[jj].z, p1[jj].w};
-          }
-        }
-      } else {
-        // mRoPE computes its cosines and sines (no table to wait for): row by row
-        for (int idx = tid; idx < 128 * (kChunks / 2); idx += kWideThreads) {  // two pieces per step
-          const int Rl = idx / (kChunks / 2), x = idx - Rl * (kChunks / 2);
-          const int R = kWaveRows * (Rl / 32) + 32 * pass + Rl % 32;  // block `pass` of every wave
-          const int iq = R / G, g = R - iq * G;
-          int c0 = 2 * x, c1 = 2 * x + 1;
-          uint4 p0 = make_uint4(0, 0, 0, 0), p1 = p0;
-          if (iq < n_q) {
-            const int subrow = (lflags & VA_LINK_INDIRECT) ? a.qrefs[qref + iq] : qref + iq;
-            const long long src_row = a.sub_worker[subrow];
-            const S* qh = (const S*)a.q + src_row * a.q_row_stride + (long long)(hk * G + g) * kD;
-            const Pos3 p = load_pos(a.sub_loc, a.sub_loc_axis_stride, subrow);
-            rotated_query_unit<E>(a.rope, qh, x, p, c0, c1, p0, p1);
-          }
-          q_stage[Rl * kChunks + (c0 ^ wide_swz<kD>(Rl))] = va_u32x4{p0.x, p0.y, p0.z, p0.w};
-          q_stage[Rl * kChunks + (c1 ^ wide_swz<kD>(Rl))] = va_u32x4{p1.x, p1.y, p1.z, p1.w};
         }
       }
       ring_barrier<kAnyInFlight>();
-      {
-        const int Rl = 32 * wave + j;
-#pragma unroll
-        for (int s = 0; s < kSteps; ++s) qf[pass][s] = q_stage[Rl * kChunks + ((2 * s + h) ^ wide_swz<kD>(Rl))];
-      }
-      ring_barrier<kAnyInFlight>();  // staging rows may be overwritten now
     }
+    auto rotate = [&](auto steps) __attribute__((always_inline)) {
+      constexpr int kHalf = decltype(steps)::value;  // operands per rotary half
+      if (table) {
+        // table entries of up to four pairs of operands in flight before the first pair is rotated
+        constexpr int kUnits = kB * kHalf, kAhead = kUnits < 4 ? kUnits : 4;
+        TableTurn turn[kAhead];
+        bool back[kB];
+        const float* entry[kB];
+#pragma unroll
+        for (int b = 0; b < kB; ++b) {
+          const int row = table_row(a.rope, pos[b]);
+          back[b] = row < 0;
+          entry[b] = a.rope.cos_sin + (long long)(back[b] ? ~row : row) * a.rope.rotary_dim + 8 * h;
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) turn[u].load(entry[u / kHalf] + 16 * (u % kHalf), 16 * kHalf);
+#pragma unroll
+        for (int u = 0; u < kUnits; ++u) {
+          const int b = u / kHalf, s = u % kHalf, next = u + kAhead;
+          turn[u % kAhead].template apply<E>(back[b], qf[b][s], qf[b][s + kHalf]);
+          if (next < kUnits) turn[u % kAhead].load(entry[next / kHalf] + 16 * (next % kHalf), 16 * kHalf);
+        }
+      } else {
+#pragma unroll
+        for (int b = 0; b < kB; ++b) {
+          const int iq = min(row_iq[b], n_q - 1);
+#pragma unroll
+          for (int s = 0; s < kHalf; ++s) {
+            va_u32x4 cs[2];
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+              cs[x] = *(const va_u32x4*)(turns + turn_word(iq, 16 * s + 8 * h + 4 * x, 16 * kHalf));
+            rotate_packed<E>(cs, qf[b][s], qf[b][s + kHalf]);
+          }
+        }
+      }
+    };
+    if (wave_active && half_steps != 0) {
+      if (half_steps == kSteps / 2) {
+        rotate(std::integral_constant<int, kSteps / 2>{});
+      } else if (half_steps == kSteps / 4) {
+        rotate(std::integral_constant<int, kSteps / 4>{});
+      } else if (kSteps >= 8 && half_steps == kSteps / 8) {
+        rotate(std::integral_constant<int, (kSteps >= 8 ? kSteps / 8 : 1)>{});
+      } else {
+        // other rotary widths: piece by piece, through a slot per (lane, operand) of the same LDS
+        va_u32x4* mine = (va_u32x4*)turns + tid;
+        auto each = [&](int b, const S* row) __attribute__((always_inline)) {
+          const Pos3 p = load_pos(a.sub_loc, a.sub_loc_axis_stride, subrow_of(row_iq[b]));
+#pragma unroll 1
+          for (int s = 0; s < kSteps; ++s) {
+            const uint4 piece = rotated_query_piece<E>(a.rope, row - 8 * h, 16 * s + 8 * h, p);
+            mine[kWideThreads * s] = va_u32x4{piece.x, piece.y, piece.z, piece.w};
+          }
+        };
+        each(0, q_row[0]);
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) qf[0][s] = mine[kWideThreads * s];
+        if constexpr (kB > 1) {
+          each(kB - 1, q_row[kB - 1]);
+#pragma unroll
+          for (int s = 0; s < kSteps; ++s) qf[kB - 1][s] = mine[kWideThreads * s];
+        }
+      }
+    }
+    // The operands are waited for here: a load the compiler still knows of inside the tile loop would make
+    // it wait for the loop's own requests as well, and drain the ring in every step.
+#pragma unroll
+    for (int b = 0; b < kB; ++b)
+#pragma unroll
+      for (int s = 0; s < kSteps; ++s) asm volatile("" : "+v"(qf[b][s]));
 
     // ---- the tile loop ----
     // Reference maximum.  The softmax runs against a per-row REFERENCE maximum m_ref that is
@@ -404,11 +480,6 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     // needed (its K, for the scores computed one iteration ahead).
     const int n_vis = t_wave > tok_begin ? min(n_tiles, (t_wave - tok_begin + kWideTokens - 1) / kWideTokens) : 0;
     int next_step = 0;
-    // The pool row of the tile a step requests is looked up a whole step earlier (a scalar load whose
-    // result is not touched before the next step): its latency never shows.
-    auto row_of = [&](int tile) __attribute__((always_inline)) {
-      return (tile < n_tiles && tile_is_plain(tile)) ? half_row(tile) : 0ull;
-    };
     unsigned long long row_ahead = row_of(kWideAhead);
     auto ring_step = [&]() __attribute__((always_inline)) {
       const int k = next_step++;
@@ -695,7 +766,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     const int hq = hk * G + g;
     const float inv = l > 0.f ? 1.f / l : 0.f;
     if (part_base < 0) {
-      const int32_t* link0 = a.links + (long long)item[VA_I_LINK_BEGIN] * VA_LINK_WORDS;
+      const PlanWords link0 = item + VA_I_LINK0;
       const int subrow = (link0[VA_L_FLAGS] & VA_LINK_INDIRECT) ? a.qrefs[link0[VA_L_QREF] + iq] : link0[VA_L_QREF] + iq;
       const long long out_row = a.sub_worker[subrow];
       S* orow = (S*)a.out + (out_row * a.num_q_heads + hq) * (long long)kD;
