@@ -403,6 +403,84 @@ __device__ __forceinline__ void load_group_to_lds(const void* base, const uint32
     load_to_lds(base, adjusted_offsets[0], lds_base);
   }
 }
+// Rows scattered over the pool (a 64-bit address per lane): kCount loads behind one saved M0, load u landing
+// 1024 u bytes further on.  `columns`: 128-byte columns of ONE row per lane (the immediate offset moves the
+// LDS address as well, so M0 advances by 1024 - 128); `rows`: another row per load.
+template <int kCount>
+__device__ __forceinline__ void load_columns_to_lds(unsigned long long at, uint32_t lds_base) {
+  static_assert(kCount == 1 || kCount == 2 || kCount == 4, "columns");
+  if constexpr (kCount == 1) {
+    load_to_lds((const void*)at, lds_base);
+  } else {
+    uint32_t saved;
+    if constexpr (kCount == 2) {
+      asm volatile(
+          "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+          "global_load_lds_dwordx4 %1, off\n\t"
+          "s_add_u32 m0, m0, 896\n\ts_nop 0\n\t"
+          "global_load_lds_dwordx4 %1, off offset:128\n\t"
+          "s_mov_b32 m0, %0"
+          : "=&s"(saved)
+          : "v"(at), "s"(lds_base)
+          : "memory", "scc");
+    } else {
+      asm volatile(
+          "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+          "global_load_lds_dwordx4 %1, off\n\t"
+          "s_add_u32 m0, m0, 896\n\ts_nop 0\n\t"
+          "global_load_lds_dwordx4 %1, off offset:128\n\t"
+          "s_add_u32 m0, m0, 896\n\ts_nop 0\n\t"
+          "global_load_lds_dwordx4 %1, off offset:256\n\t"
+          "s_add_u32 m0, m0, 896\n\ts_nop 0\n\t"
+          "global_load_lds_dwordx4 %1, off offset:384\n\t"
+          "s_mov_b32 m0, %0"
+          : "=&s"(saved)
+          : "v"(at), "s"(lds_base)
+          : "memory", "scc");
+    }
+  }
+}
+template <int kCount>
+__device__ __forceinline__ void load_rows_to_lds(const unsigned long long* at, uint32_t lds_base) {
+  static_assert(kCount == 2 || kCount == 4, "rows");
+  uint32_t saved;
+  if constexpr (kCount == 2) {
+    asm volatile(
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, off\n\t"
+        "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\t"
+        "global_load_lds_dwordx4 %2, off\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(at[0]), "v"(at[1]), "s"(lds_base)
+        : "memory", "scc");
+  } else {
+    asm volatile(
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %5\n\ts_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, off\n\t"
+        "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\t"
+        "global_load_lds_dwordx4 %2, off\n\t"
+        "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\t"
+        "global_load_lds_dwordx4 %3, off\n\t"
+        "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\t"
+        "global_load_lds_dwordx4 %4, off\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "s"(lds_base)
+        : "memory", "scc");
+  }
+}
+// One word per lane, pool side -> LDS: lane l's four bytes land at lds_base + 4 l.
+__device__ __forceinline__ void load_word_to_lds(const void* src, uint32_t lds_base) {
+  uint32_t saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+      "global_load_lds_dword %1, off\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(saved)
+      : "v"(src), "s"(lds_base)
+      : "memory");
+}
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }

@@ -70,7 +70,9 @@ struct WideShape {
   // at smaller head dims past its end.
   static constexpr int kTurnBytes = kTileRows * (kD / 2) * 4;
   static constexpr int kRingBytes = kWideBuffers * kBufferBytes, kSetupBytes = kWideAhead * kBufferBytes + kTurnBytes;
-  static constexpr int kLdsBytes = kRingBytes > kSetupBytes ? kRingBytes : kSetupBytes;
+  // Scattered rows: the index entries of eight tiles, for every wave its own (va_mfma_wide: gather)
+  static constexpr int kIndexOffset = kRingBytes > kSetupBytes ? kRingBytes : kSetupBytes;
+  static constexpr int kLdsBytes = kIndexOffset + kWideWaves * 2 * kWave * 4;
 };
 
 // Word of the cos|sin entry (row iq, pair dim) in LDS: rows of `half` words, their 16-byte pieces swizzled
@@ -105,7 +107,8 @@ __device__ __forceinline__ float half_wave_max(float x) {
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
-template <typename E, int kD>
+// kGather: every token of the launch has an index entry of its own (slot lists, pages of 1, 2, 4 or 8 tokens).
+template <typename E, int kD, bool kGather>
 __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArgs a) {
   using S = typename E::storage;
   using Sh = WideShape<kD>;
@@ -255,7 +258,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     const int causal_base = link[VA_L_CAUSAL_BASE];
     const bool slots = lflags & VA_LINK_SLOTS;
     // a 16-token half tile lies inside one page only if the link starts on a 16-token boundary
-    const bool uniform_pages = !slots && pow2_pages && page_fits && P >= 16 && (tok_begin % 16 == 0);
+    const bool uniform_pages = !kGather && !slots && pow2_pages && page_fits && P >= 16 && (tok_begin % 16 == 0);
 
     const int t_stop = min(tok_end, causal_base + n_q);  // tokens any row of the tile sees
     const int t_last = t_stop - 1;
@@ -272,9 +275,13 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     // (w = 2, 3): kL wave-level loads of kRowsPerLoad rows each.  With uniform pages the half lies
     // in one page, so the wave needs ONE scalar page lookup per tile and every load is a
     // wave-uniform base plus a per-lane offset that never changes (ld_off); tiles that reach past
-    // the visible range, and page tables with pages under 16 tokens or slot lists, look every
-    // row up per lane instead (rows past the range re-read the last visible token; their scores
-    // are masked).
+    // the visible range look every row up per lane instead (rows past the range re-read the last
+    // visible token; their scores are masked).
+    // Slot lists and pages under 16 tokens (kGather): looked up by the lanes in front of each request, the
+    // entries cost a trip to memory per tile and drain the ring (6 requests of 60..4096 tokens over slot
+    // lists, 32 q / 8 kv heads of 128 dims: 734 us a layer).  So they travel like the tiles do: one
+    // wave-level load brings a wave's entries of four tiles to LDS, four to eight tiles ahead, and a ring
+    // step reads the entries of the tile the NEXT step requests.
     const char* wave_pool = (const char*)(wave_is_v ? vp : kp);
     const char* wave_plain = wave_pool - kLoadBias;  // base of plain loads: the per-lane offsets carry the bias
     const uint32_t wave_lds = __builtin_amdgcn_readfirstlane(lds_address(lds)) + (wave_is_v ? Sh::kTileBytes : 0) +
@@ -293,6 +300,56 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     };
     auto tile_is_plain = [&](int i) __attribute__((always_inline)) {
       return uniform_pages && tok_begin + (i + 1) * kWideTokens - 1 <= t_last;
+    };
+    // gather: entries of tiles 4 group .. 4 group + 3, this wave's half; lane -> (tile, token)
+    const int g_shift = slots ? 0 : p_shift, g_mask = slots ? 0 : P - 1;
+    const uint32_t wave_index_lds = __builtin_amdgcn_readfirstlane(lds_address(lds)) + Sh::kIndexOffset + wave * (2 * kWave * 4);
+    const int32_t* wave_index = (const int32_t*)(lds + Sh::kIndexOffset + wave * (2 * kWave * 4));
+    auto gather_token = [&](int i, int row) __attribute__((always_inline)) {
+      return min(tok_begin + i * kWideTokens + 16 * wave_half + row, t_last);
+    };
+    auto request_entries = [&](int group) __attribute__((always_inline)) {
+      const int t = gather_token(4 * group + lane / 16, lane % 16);
+      load_word_to_lds(a.kv_indices + kv_begin + (t >> g_shift), wave_index_lds + (group & 1) * (kWave * 4));
+    };
+    // The rows of a wave's requests: lane % 8 and 8 + lane % 8 for every 128-byte column of K, another row per
+    // request of V (ld_row).
+    constexpr int kVBases = kD == 256 ? 2 : 1;  // the swizzle of V's pieces repeats every 1 or 2 requests
+    const unsigned long long gather_base[2] = {(unsigned long long)(wave_pool + 16 * ld_piece(0)),
+                                               (unsigned long long)(wave_pool + 16 * ld_piece(wave_is_v ? kVBases - 1 : kColumns))};
+    auto gather_row = [&](int x) __attribute__((always_inline)) { return wave_is_v ? ld_row(x) : 8 * (x & 1) + lane % 8; };
+    auto read_slots = [&](int i, int (&slot)[kL], auto entry_of) __attribute__((always_inline)) {
+      auto one = [&](int x) __attribute__((always_inline)) {
+        const int row = gather_row(x);
+        slot[x] = (entry_of(i, row) << g_shift) + (gather_token(i, row) & g_mask);
+      };
+      one(0);
+      one(1);
+      if (wave_is_v)
+#pragma unroll
+        for (int x = 2; x < kL; ++x) one(x);
+    };
+    auto entry_in_lds = [&](int i, int row) __attribute__((always_inline)) { return wave_index[(i & 7) * 16 + row]; };
+    auto entry_in_memory = [&](int i, int row) __attribute__((always_inline)) {
+      return a.kv_indices[kv_begin + (gather_token(i, row) >> g_shift)];
+    };
+    auto issue_gather = [&](int i, const int (&slot)[kL]) __attribute__((always_inline)) {
+      const uint32_t dst = wave_lds + ring_slot(i) * Sh::kBufferBytes;
+      auto at = [&](int x, int base) __attribute__((always_inline)) {
+        return (unsigned long long)(uint32_t)slot[x] * (uint32_t)row_bytes + gather_base[base];
+      };
+      if (wave_is_v) {
+#pragma unroll
+        for (int u = 0; u < kL; u += kLoadGroup) {
+          unsigned long long rows[kLoadGroup];
+#pragma unroll
+          for (int x = 0; x < kLoadGroup; ++x) rows[x] = at(u + x, (u + x) % kVBases);
+          load_rows_to_lds<kLoadGroup>(rows, dst + u * 1024);
+        }
+      } else {
+        load_columns_to_lds<kColumns>(at(0, 0), dst);
+        load_columns_to_lds<kColumns>(at(1, 1), dst + kColumns * 1024);
+      }
     };
     auto issue = [&](int i, unsigned long long row) __attribute__((always_inline)) {
       const uint32_t dst = wave_lds + ring_slot(i) * Sh::kBufferBytes;
@@ -348,6 +405,11 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     unsigned long long first_rows[kWideAhead];
 #pragma unroll
     for (int i = 0; i < kWideAhead; ++i) first_rows[i] = row_of(i);
+    int first_slots[kWideAhead][kL];
+    if (kGather && n_tiles > 0) {
+#pragma unroll
+      for (int i = 0; i < kWideAhead; ++i) read_slots(i, first_slots[i], entry_in_memory);
+    }
     // (the positions are waited for before the tiles are requested: later they would have to wait for the tiles)
     if (table) {
 #pragma unroll
@@ -356,9 +418,15 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
       asm volatile("" : "+v"(pos[0]), "+v"(pos[1]), "+v"(pos[2]));
     }
     ring_barrier<kAnyInFlight>();  // every wave has read the previous link's last tile
+    if (kGather && n_tiles > 0) {
+      request_entries(0);
 #pragma unroll
-    for (int i = 0; i < kWideAhead; ++i)
-      if (i < n_tiles) issue(i, first_rows[i]);
+      for (int i = 0; i < kWideAhead; ++i) issue_gather(i, first_slots[i]);  // (past the range: the last visible token)
+    } else {
+#pragma unroll
+      for (int i = 0; i < kWideAhead; ++i)
+        if (i < n_tiles) issue(i, first_rows[i]);
+    }
     if (!table && in_turn) {
       // mRoPE: the cosines and sines of the tile's positions, each taken once and shared by the G query
       // heads of a row (an entry is cos | sin in the element type, as the rotation rounds them).  A thread
@@ -481,6 +549,9 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     const int n_vis = t_wave > tok_begin ? min(n_tiles, (t_wave - tok_begin + kWideTokens - 1) / kWideTokens) : 0;
     int next_step = 0;
     unsigned long long row_ahead = row_of(kWideAhead);
+    int slots_ahead[kL];  // gather: the same for scattered rows, read from LDS a step earlier
+#pragma unroll
+    for (int u = 0; u < kL; ++u) slots_ahead[u] = 0;
     auto ring_step = [&]() __attribute__((always_inline)) {
       const int k = next_step++;
       const bool refill = k + kWideAhead < n_tiles;
@@ -494,7 +565,17 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
       } else {
         ring_barrier<0>();
       }
-      if (refill) issue(k + kWideAhead, row);
+      if constexpr (kGather) {
+        if (k % 4 == 0) request_entries(k / 4 + 1);
+        if (refill) {
+          int slot[kL];
+          read_slots(k + kWideAhead, slot, entry_in_lds);
+          issue_gather(k + kWideAhead, slot);
+        }
+        read_slots(k + 1 + kWideAhead, slots_ahead, entry_in_lds);
+      } else if (refill) {
+        issue(k + kWideAhead, row);
+      }
     };
 
     // The same step for the steady part of a link (uniform pages; the requested tile and the one
@@ -524,6 +605,21 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
       }
       row_ahead = half_offset(page + zero, t);
     };
+    // The steady step of scattered rows (tiles past the range repeat the last visible token: only a next tile to
+    // request must exist).  Entries requested in step 4m are complete behind the barrier of step 4m + 1, the
+    // first of them is read there.
+    auto ring_step_gather = [&]() __attribute__((always_inline)) {
+      const int k = next_step++;
+      if (k % 4 == 0) request_entries(k / 4 + 1);
+      if (!wave_is_v) {
+        issue_gather(k + kWideAhead, slots_ahead);
+        ring_barrier<kWideAhead * kL>();
+      } else {
+        ring_barrier<(kWideAhead - 1) * kL>();
+        issue_gather(k + kWideAhead, slots_ahead);
+      }
+      read_slots(k + 1 + kWideAhead, slots_ahead, entry_in_lds);
+    };
     // iterations [1, i_steady_end) may take it: tiles i + 1 + kWideAhead and i + 2 + kWideAhead are plain,
     // tile i is unmasked for every row of the wave and a next tile exists
     int i_steady_end = 0;
@@ -531,6 +627,9 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
       const int plain_tiles = (t_last + 1 - tok_begin) / kWideTokens;  // tiles 0 .. plain_tiles - 1 are plain
       const int unmasked_tiles = t_wave_min > tok_begin ? (t_wave_min - tok_begin) / kWideTokens : 0;
       i_steady_end = min(min(plain_tiles - 2 - kWideAhead, unmasked_tiles), n_vis - 1);
+    } else if (kGather && P < 16) {
+      const int unmasked_tiles = t_wave_min > tok_begin ? (t_wave_min - tok_begin) / kWideTokens : 0;
+      i_steady_end = min(min(n_tiles - 1 - kWideAhead, unmasked_tiles), n_vis - 1);
     }
 
     // Scores of two tiles: the exponentials of one are taken in place while the products of the next
@@ -703,16 +802,30 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     while (i < n_vis) {
       bool raise = false;
       if (i >= 1 && i < i_steady_end) {
-        // steady part
-        do {
-          ring_step_steady();
-          raise = steady_test();
-          if (raise) break;
-          tile_body(i, sc, sc_next);
+        if constexpr (kGather) {
+          // (written without a break in the middle: with one the compiler keeps the accumulators of before
+          // and after the products side by side, copies one to the other every tile and spills)
+          do {
+            ring_step_gather();
+            raise = steady_test();
+            if (!raise) {
+              tile_body(i, sc, sc_next);
 #pragma unroll
-          for (int b = 0; b < kB; ++b) sc[b] = sc_next[b];
-          ++i;
-        } while (i < i_steady_end);
+              for (int b = 0; b < kB; ++b) sc[b] = sc_next[b];
+              ++i;
+            }
+          } while (!raise && i < i_steady_end);
+        } else {
+          do {
+            ring_step_steady();
+            raise = steady_test();
+            if (raise) break;
+            tile_body(i, sc, sc_next);
+#pragma unroll
+            for (int b = 0; b < kB; ++b) sc[b] = sc_next[b];
+            ++i;
+          } while (i < i_steady_end);
+        }
         early_max_valid = true;  // (a next tile exists throughout the steady part)
         if (!raise) continue;
       } else {
@@ -799,31 +912,35 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
   }  // items of the slot
 }
 
-template <typename E, int kD>
+template <typename E, int kD, bool kGather>
 static int launch_wide_one(const AttnArgs& a, int n_items, hipStream_t stream) {
   constexpr int bytes = WideShape<kD>::kLdsBytes;
   static bool configured = false;  // raising the limit is idempotent; a race only repeats the call
   if (!configured) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_mfma_wide_kernel<E, kD>),
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_mfma_wide_kernel<E, kD, kGather>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e != hipSuccess) return va_fail(VA_ERR_HIP, "raising the LDS limit: %s", hipGetErrorString(e));
     configured = true;
   }
   const dim3 grid((unsigned)n_items * (unsigned)a.num_kv_heads), block(kWideThreads);
-  hipLaunchKernelGGL((attn_mfma_wide_kernel<E, kD>), grid, block, bytes, stream, a);
+  hipLaunchKernelGGL((attn_mfma_wide_kernel<E, kD, kGather>), grid, block, bytes, stream, a);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? VA_OK : va_fail(VA_ERR_HIP, "wide attention launch: %s", hipGetErrorString(e));
 }
 
 template <typename E>
 static int launch_wide_typed(const AttnArgs& a, int n_items, hipStream_t stream) {
+  // Pages of at least 16 tokens take one lookup per half tile, smaller ones (a slot list has pages of one) an
+  // entry per token; the choice hangs on the page size alone, so that a recorded launch keeps its kernel.
+  // (Other page sizes, and slot lists beside larger pages, go through the first kernel's per-lane lookups.)
+  const bool gather = a.page_size < 16 && (a.page_size & (a.page_size - 1)) == 0;
   switch (a.head_dim) {
     case 64:
-      return launch_wide_one<E, 64>(a, n_items, stream);
+      return gather ? launch_wide_one<E, 64, true>(a, n_items, stream) : launch_wide_one<E, 64, false>(a, n_items, stream);
     case 128:
-      return launch_wide_one<E, 128>(a, n_items, stream);
+      return gather ? launch_wide_one<E, 128, true>(a, n_items, stream) : launch_wide_one<E, 128, false>(a, n_items, stream);
     case 256:
-      return launch_wide_one<E, 256>(a, n_items, stream);
+      return gather ? launch_wide_one<E, 256, true>(a, n_items, stream) : launch_wide_one<E, 256, false>(a, n_items, stream);
     default:
       return va_fail(VA_ERR_ARG, "matrix-core path supports head_dim 64, 128, 256");
   }
