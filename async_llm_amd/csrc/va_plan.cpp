@@ -946,7 +946,7 @@ static int write_plan(const Built& b, const VaSubRequests* subs, const VaShape* 
   off += cap_rows;
   // The waves of a merge workgroup split a row's states, so rows of many states (long views cut
   // into many chunks) get more waves; when the rows are many (split prefill tiles: thousands of
-  // rows of a few states each) one wave per row keeps more rows in flight.  A fixed plan decides
+  // rows of a few states each) a workgroup takes a whole row (word 1).  A fixed plan decides
   // from its capacity, a packed one from its counts: either way the word is part of the header the
   // launches are derived from.  Measured on one MI355X: 17 states per row take 9.9 / 14.7 / 20.6 us
   // with 4 / 8 / 16 waves, 72 per row 16.4 / 12.0 / 9.5 us.

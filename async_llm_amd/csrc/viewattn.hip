@@ -453,9 +453,7 @@ __global__ __launch_bounds__(kGenThreads) void attn_generic_kernel(AttnArgs a) {
 // for latency: wave w folds partials w, w + kMergeWaves, ... of the row, eight per round (the last
 // round exactly what is left) with all their loads in flight together, and the running states meet
 // in LDS.  Lane l owns dims l, l + 64, ...
-// Four waves for a decode batch (few rows, up to dozens of partial states each); one wave when the
-// rows are many (split prefill tiles: thousands of rows of a few states each), where four times as
-// many rows in flight per CU count for more than the parallel fold.
+// For a decode batch: few rows, up to dozens of partial states each.
 template <typename E, int kMergeWaves>
 __global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(MergeArgs a) {
   using S = typename E::storage;
@@ -549,6 +547,91 @@ __global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(MergeArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// merge of many rows of few states (split prefill tiles): one workgroup per row
+// ---------------------------------------------------------------------------
+// The states of a row lie as [heads * dims] floats each, so a thread takes four consecutive floats of every
+// 1024 and the workgroup reads whole states, two at a time with all their loads in flight; rows that an item
+// has written itself leave at once.  (As one workgroup per (row, head) such a launch was bound by the rate
+// at which workgroups start: 7571 rows of 32 heads, most of them written directly, took 53 us.)
+template <typename E>
+__global__ __launch_bounds__(256) void merge_rows_kernel(MergeArgs a) {
+  using S = typename E::storage;
+  typedef const __attribute__((address_space(4))) int32_t* Words;
+  const long long row = blockIdx.x;
+  const int flags = ((Words)a.row_flags)[row];
+  if (flags & VA_ROW_DIRECT) return;
+  const int width = a.num_q_heads * a.head_dim, d_shift = __builtin_ctz(a.head_dim);  // (head dims are powers of two)
+  S* out = (S*)a.out + row * (long long)width;
+  float* lse = a.lse ? a.lse + row * a.num_q_heads : nullptr;
+  if (flags & VA_ROW_EMPTY) {
+    for (int i = threadIdx.x; i < width; i += 256) out[i] = E::store(0.f);
+    if (lse)
+      for (int i = threadIdx.x; i < a.num_q_heads; i += 256) lse[i] = -INFINITY;
+    return;
+  }
+  const int begin = ((Words)a.row_indptr)[row], end = ((Words)a.row_indptr)[row + 1];
+  constexpr int kRuns = 4;  // runs of 1024 floats per pass
+  for (int base = 4 * threadIdx.x; base < width; base += kRuns * 1024) {
+    int at[kRuns];
+    float m[kRuns], l[kRuns];
+    float4 v[kRuns];
+#pragma unroll
+    for (int k = 0; k < kRuns; ++k) {
+      at[k] = min(base + 1024 * k, width - 4);  // (runs past the end repeat the last one; not stored)
+      m[k] = kNegBig;
+      l[k] = 0.f;
+      v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    auto fold = [&](int i, auto n_tag) __attribute__((always_inline)) {
+      constexpr int n = decltype(n_tag)::value;
+      float2 ml[n][kRuns];
+      float4 x[n][kRuns];
+#pragma unroll
+      for (int u = 0; u < n; ++u) {
+        const long long state = (long long)((Words)a.row_ids)[i + u] * a.num_q_heads;
+#pragma unroll
+        for (int k = 0; k < kRuns; ++k) {
+          ml[u][k] = *(const float2*)(a.part_ml + 2 * (state + (at[k] >> d_shift)));
+          x[u][k] = *(const float4*)(a.part_acc + (state << d_shift) + at[k]);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < n; ++u)
+#pragma unroll
+        for (int k = 0; k < kRuns; ++k) {
+          const float m_new = fmaxf(m[k], ml[u][k].x);
+          const float sa = exp2f(m[k] - m_new), sb = exp2f(ml[u][k].x - m_new);
+          l[k] = l[k] * sa + ml[u][k].y * sb;
+          v[k].x = v[k].x * sa + x[u][k].x * sb;
+          v[k].y = v[k].y * sa + x[u][k].y * sb;
+          v[k].z = v[k].z * sa + x[u][k].z * sb;
+          v[k].w = v[k].w * sa + x[u][k].w * sb;
+          m[k] = m_new;
+        }
+    };
+    int i = begin;
+    for (; i + 2 <= end; i += 2) fold(i, std::integral_constant<int, 2>{});
+    if (i < end) fold(i, std::integral_constant<int, 1>{});
+#pragma unroll
+    for (int k = 0; k < kRuns; ++k) {
+      if (base + 1024 * k >= width) continue;
+      const bool any = l[k] > 0.f;
+      S y[4] = {E::store(any ? v[k].x / l[k] : 0.f), E::store(any ? v[k].y / l[k] : 0.f),
+                E::store(any ? v[k].z / l[k] : 0.f), E::store(any ? v[k].w / l[k] : 0.f)};
+      if constexpr (sizeof(S) == 2) {
+        *(uint2*)(out + at[k]) = *(const uint2*)y;
+      } else {
+        *(float4*)(out + at[k]) = *(const float4*)y;
+      }
+      if (lse && (at[k] & (a.head_dim - 1)) == 0) {
+        const float lse2 = any ? m[k] + log2f(l[k]) : -INFINITY;
+        lse[at[k] >> d_shift] = a.lse_base2 ? lse2 : lse2 * kLn2;
+      }
+    }
+  }
+}
+
 template <typename E>
 int launch_generic(const AttnArgs& a, int n_items, hipStream_t stream) {
   const dim3 grid((unsigned)n_items * (unsigned)a.num_kv_heads), block(kGenThreads);
@@ -573,13 +656,13 @@ int launch_generic(const AttnArgs& a, int n_items, hipStream_t stream) {
   return check_hip(hipGetLastError(), "attention launch");
 }
 
-// `waves`: waves per (row, q head) workgroup, chosen by the planner (plan header).
+// `waves`: waves per (row, q head) workgroup, chosen by the planner (plan header); 1: one workgroup per row.
 template <typename E>
 int launch_merge(const MergeArgs& a, int n_rows, int waves, hipStream_t stream) {
   const dim3 grid((unsigned)n_rows, (unsigned)a.num_q_heads);
   switch (waves) {
     case 1:
-      hipLaunchKernelGGL((merge_kernel<E, 1>), grid, dim3(64), 0, stream, a);
+      hipLaunchKernelGGL((merge_rows_kernel<E>), dim3((unsigned)n_rows), dim3(256), 0, stream, a);
       break;
     case 4:
       hipLaunchKernelGGL((merge_kernel<E, 4>), grid, dim3(256), 0, stream, a);
