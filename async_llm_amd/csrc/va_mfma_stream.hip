@@ -55,7 +55,11 @@ struct StreamShape {
   static constexpr int kPvWaves = kD >= 128 ? 4 : 2;         // waves that own a slice of the head dim
   static constexpr int kDimsPerWave = kD / kPvWaves;
   static constexpr int kRun = kDimsPerWave / 16;             // contiguous dims a lane reads per V token
-  static constexpr int kLdsBytes = kBuffers * 2 * kTileUnits * 16;
+  static constexpr int kRingBytes = kBuffers * 2 * kTileUnits * 16;
+  // Behind the ring, for every wave its own: the index entries of eight tiles (two wave-level loads), see `gather`.
+  static constexpr int kIndexBytes = 2 * kWave * 4;
+  static constexpr int lds_bytes(bool gather) { return kRingBytes + (gather ? kStreamWaves * kIndexBytes : 0); }
+  static_assert(kBuffers <= 4, "the entries of a tile are read four tiles after they were requested");
   static_assert(kLoadsPerWave >= 1 && kRun >= 2 && kRun <= 4, "unsupported head_dim");
 };
 
@@ -77,7 +81,8 @@ __device__ __forceinline__ float max_over_contraction_groups(float x) {
   return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
-template <typename E, int kD>
+// kGather: pages hold less than a tile (1, 2, 4 or 8 tokens; a slot list has pages of one).
+template <typename E, int kD, bool kGather>
 __global__ __launch_bounds__(kStreamThreads, StreamShape<kD>::kMinBlocks) void attn_stream_kernel(AttnArgs a) {
   using S = typename E::storage;
   using Sh = StreamShape<kD>;
@@ -127,8 +132,8 @@ __global__ __launch_bounds__(kStreamThreads, StreamShape<kD>::kMinBlocks) void a
   int ld_row[Sh::kLoadsPerWave], ld_byte[Sh::kLoadsPerWave];
 #pragma unroll
   for (int u = 0; u < Sh::kLoadsPerWave; ++u) {
-    const int q = (wave * Sh::kLoadsPerWave + u) % Sh::kLoadsPerKind;
-    ld_row[u] = q * Sh::kRowsPerLoad + lane / kChunks;
+    // (a wave's loads are consecutive ones of one kind)
+    ld_row[u] = (wave * Sh::kLoadsPerWave) % Sh::kLoadsPerKind * Sh::kRowsPerLoad + lane / kChunks + u * Sh::kRowsPerLoad;
     ld_byte[u] = 16 * ((lane % kChunks) ^ swz<kD>(ld_row[u]));
   }
   // LDS byte offsets (within a tile) of what this lane reads.  The swizzle only touches the low
@@ -180,7 +185,7 @@ __global__ __launch_bounds__(kStreamThreads, StreamShape<kD>::kMinBlocks) void a
     // no other query tile reads these rows: they are requested as lines to evict first
     const bool read_once = lflags & VA_LINK_ONCE;
     // a 16-token tile lies inside one page: one wave-uniform page read per tile
-    const bool uniform_pages = !slots && pow2_pages && P >= 16 && (tok_begin % 16 == 0);
+    const bool uniform_pages = !kGather && !slots && pow2_pages && P >= 16 && (tok_begin % 16 == 0);
 
     const int t_stop = min(tok_end, causal_base + n_q);        // tokens any row of the tile sees
     const int t_row = min(tok_end, causal_base + row_iq + 1);  // tokens this lane's row sees
@@ -195,7 +200,31 @@ __global__ __launch_bounds__(kStreamThreads, StreamShape<kD>::kMinBlocks) void a
     auto page_of = [&](int i) __attribute__((always_inline)) {
       return ((const __attribute__((address_space(4))) int32_t*)a.kv_indices)[kv_begin + ((tok_begin + i * kStreamTok) >> p_shift)];
     };
-    auto issue = [&](int i, auto uniform_tag, auto once_tag, int page) __attribute__((always_inline)) {
+    // kGather.  Looked up by the lanes in front of each request, the entries cost a trip to memory per tile and
+    // the compiler's wait for it drained the ring (32 requests of 100..8000 token slots, 32 q / 8 kv heads of 128
+    // dims, bf16: 124.7 us a layer; 92.7 us = 5.7 TB/s this way).  So they travel like the tiles do: one wave-level load brings a
+    // wave's entries of four tiles to LDS, five to eight tiles ahead of their requests, and an iteration reads
+    // those of the tile it requests beside its K.
+    const int g_shift = slots ? 0 : p_shift, g_mask = slots ? 0 : P - 1;
+    auto token_of = [&](int i, int row) __attribute__((always_inline)) { return min(tok_begin + i * kStreamTok + row, t_last); };
+    auto entry_of = [&](int t) __attribute__((always_inline)) {
+      return a.kv_indices + kv_begin + (t >> g_shift);
+    };
+    auto slot_of = [&](int entry, int t) __attribute__((always_inline)) {
+      return (entry << g_shift) + (t & g_mask);
+    };
+    const uint32_t index_lds =
+        __builtin_amdgcn_readfirstlane(lds_address(ring)) + Sh::kRingBytes + (uint32_t)wave * Sh::kIndexBytes;
+    const int32_t* index = (const int32_t*)(lds + Sh::kRingBytes + wave * Sh::kIndexBytes);
+    auto request_entries = [&](int group) __attribute__((always_inline)) {  // of tiles 4 group .. 4 group + 3
+      load_word_to_lds(entry_of(token_of(4 * group + lane / kStreamTok, lane % kStreamTok)),
+                       index_lds + (uint32_t)(group & 1) * (kWave * 4));
+    };
+    struct Slots {
+      int row[Sh::kLoadsPerWave];
+    };
+    auto issue = [&](int i, auto uniform_tag, auto once_tag, int page, const Slots& rows) __attribute__((always_inline)) {
+      const int (&slot)[Sh::kLoadsPerWave] = rows.row;
       constexpr bool kUniform = decltype(uniform_tag)::value;
       constexpr bool kOnce = decltype(once_tag)::value;
       const int t0 = tok_begin + i * kStreamTok;
@@ -214,6 +243,8 @@ __global__ __launch_bounds__(kStreamThreads, StreamShape<kD>::kMinBlocks) void a
         const char* src;
         if constexpr (kUniform) {
           src = (const char*)(is_v ? vp : kp) + base_byte + (uint32_t)(r * row_bytes + ld_byte[u]);
+        } else if constexpr (kGather) {
+          src = (const char*)(is_v ? vp : kp) + (unsigned long long)(uint32_t)slot[u] * (uint32_t)row_bytes + ld_byte[u];
         } else {
           src = (const char*)(is_v ? vp : kp) + kv_slot(a.kv_indices, kv_begin, t0 + r, P, slots) * row_bytes +
                 ld_byte[u];
@@ -229,15 +260,32 @@ __global__ __launch_bounds__(kStreamThreads, StreamShape<kD>::kMinBlocks) void a
 
     // ---- set-up: first tiles on their way, then the query tile ----
     __syncthreads();  // every wave is done with the previous link's buffers
+    Slots first[kBuffers];  // gather: rows of the first tiles, looked up in one trip
+#pragma unroll
+    for (int i = 0; i < kBuffers; ++i)
+#pragma unroll
+      for (int u = 0; u < Sh::kLoadsPerWave; ++u) first[i].row[u] = 0;
     auto first_tiles = [&](auto uniform_tag, auto once_tag) __attribute__((always_inline)) {
+      if (kGather && n_tiles > 0) {
+#pragma unroll
+        for (int i = 0; i < kBuffers; ++i)
+#pragma unroll
+          for (int u = 0; u < Sh::kLoadsPerWave; ++u) first[i].row[u] = *entry_of(token_of(i, ld_row[u]));
+        request_entries(0);
+        request_entries(1);
+#pragma unroll
+        for (int i = 0; i < kBuffers; ++i)
+#pragma unroll
+          for (int u = 0; u < Sh::kLoadsPerWave; ++u) first[i].row[u] = slot_of(first[i].row[u], token_of(i, ld_row[u]));
+      }
 #pragma unroll
       for (int i = 0; i < kBuffers - 1; ++i)
-        if (i < n_tiles) issue(i, uniform_tag, once_tag, decltype(uniform_tag)::value ? page_of(i) : 0);
+        if (i < n_tiles) issue(i, uniform_tag, once_tag, decltype(uniform_tag)::value ? page_of(i) : 0, first[i]);
     };
     // (one instance of the requests and of the tile loop per page-table kind and per cache policy,
     // so that none carries the others' branches)
     auto per_kind = [&](auto&& body) __attribute__((always_inline)) {
-      if (uniform_pages) {
+      if (!kGather && uniform_pages) {
         if (read_once) {
           body(std::true_type{}, std::true_type{});
         } else {
@@ -289,18 +337,27 @@ __global__ __launch_bounds__(kStreamThreads, StreamShape<kD>::kMinBlocks) void a
 
     // ---- the tile loop ----
     auto stream = [&](auto uniform_tag, auto once_tag) __attribute__((always_inline)) {
-    if (kBuffers - 1 < n_tiles) issue(kBuffers - 1, uniform_tag, once_tag, decltype(uniform_tag)::value ? page_of(kBuffers - 1) : 0);
+    if (kBuffers - 1 < n_tiles)
+      issue(kBuffers - 1, uniform_tag, once_tag, decltype(uniform_tag)::value ? page_of(kBuffers - 1) : 0, first[kBuffers - 1]);
     for (int i = 0; i < n_tiles; ++i) {
       // This wave's loads of tile i have landed once at most the loads of the tiles requested
       // after it are outstanding; the barrier then covers the other waves' loads.
       if (i + kBuffers - 1 < n_tiles) {
-        ring_barrier<(kBuffers - 1) * Sh::kLoadsPerWave>();
+        if (kGather && (i & 3) != 0 && (i & 3) < kBuffers) {
+          ring_barrier<(kBuffers - 1) * Sh::kLoadsPerWave + 1>();  // (and the entries requested between them)
+        } else {
+          ring_barrier<(kBuffers - 1) * Sh::kLoadsPerWave>();
+        }
       } else {
         ring_barrier<0>();
       }
 
       const bool refill = i + kBuffers < n_tiles;
       int next_page = 0;
+      Slots next_rows;  // gather: index entries, then rows, of the tile requested at the end of this iteration
+#pragma unroll
+      for (int u = 0; u < Sh::kLoadsPerWave; ++u)
+        next_rows.row[u] = kGather ? index[((i + kBuffers) & 7) * kStreamTok + ld_row[u]] : 0;
       const int t0 = tok_begin + i * kStreamTok;
       const char* kt = lds + (i % kBuffers) * kBufferBytes;
       const char* vt = kt + kTileUnits * 16;
@@ -373,7 +430,13 @@ __global__ __launch_bounds__(kStreamThreads, StreamShape<kD>::kMinBlocks) void a
       // refill this tile's buffer once every wave has consumed it
       if (refill) {
         ring_barrier<kAnyInFlight>();
-        issue(i + kBuffers, uniform_tag, once_tag, next_page);
+        if constexpr (kGather) {
+          if (i % 4 == 0) request_entries(i / 4 + 2);  // (over those of tiles i .. i + 3, whose rows are known by now)
+#pragma unroll
+          for (int u = 0; u < Sh::kLoadsPerWave; ++u)
+            next_rows.row[u] = slot_of(next_rows.row[u], token_of(i + kBuffers, ld_row[u]));
+        }
+        issue(i + kBuffers, uniform_tag, once_tag, next_page, next_rows);
       }
     }
     };
@@ -425,32 +488,38 @@ __global__ __launch_bounds__(kStreamThreads, StreamShape<kD>::kMinBlocks) void a
   }
 }
 
-template <typename E, int kD>
+template <typename E, int kD, bool kGather>
 static int launch_stream_one(const AttnArgs& a, int n_items, hipStream_t stream) {
   const dim3 grid((unsigned)n_items * (unsigned)a.num_kv_heads), block(kStreamThreads);
-  if constexpr (StreamShape<kD>::kLdsBytes > 64 * 1024) {  // (deeper rings than the default need the limit raised)
+  constexpr int bytes = StreamShape<kD>::lds_bytes(kGather);
+  if constexpr (bytes > 64 * 1024) {  // (deeper rings than the default need the limit raised)
     static bool configured = false;  // raising the limit is idempotent; a race only repeats the call
     if (!configured) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_stream_kernel<E, kD>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, StreamShape<kD>::kLdsBytes);
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_stream_kernel<E, kD, kGather>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
       if (e != hipSuccess) return va_fail(VA_ERR_HIP, "raising the LDS limit: %s", hipGetErrorString(e));
       configured = true;
     }
   }
-  hipLaunchKernelGGL((attn_stream_kernel<E, kD>), grid, block, StreamShape<kD>::kLdsBytes, stream, a);
+  hipLaunchKernelGGL((attn_stream_kernel<E, kD, kGather>), grid, block, bytes, stream, a);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? VA_OK : va_fail(VA_ERR_HIP, "streaming attention launch: %s", hipGetErrorString(e));
 }
 
 template <typename E>
 static int launch_stream_typed(const AttnArgs& a, int n_items, hipStream_t stream) {
+  // Pages of at least 16 tokens take one scalar lookup per tile, smaller ones an entry per token.  The choice hangs
+  // on the page size alone, so that a recorded launch keeps its kernel; in one kernel, the registers of the second
+  // kind spilled into the first at head_dim 256.  (Other page sizes, and slot lists beside larger pages, go through
+  // the first kernel's per-lane lookups.)
+  const bool gather = a.page_size < kStreamTok && (a.page_size & (a.page_size - 1)) == 0;
   switch (a.head_dim) {
     case 64:
-      return launch_stream_one<E, 64>(a, n_items, stream);
+      return gather ? launch_stream_one<E, 64, true>(a, n_items, stream) : launch_stream_one<E, 64, false>(a, n_items, stream);
     case 128:
-      return launch_stream_one<E, 128>(a, n_items, stream);
+      return gather ? launch_stream_one<E, 128, true>(a, n_items, stream) : launch_stream_one<E, 128, false>(a, n_items, stream);
     case 256:
-      return launch_stream_one<E, 256>(a, n_items, stream);
+      return gather ? launch_stream_one<E, 256, true>(a, n_items, stream) : launch_stream_one<E, 256, false>(a, n_items, stream);
     default:
       return va_fail(VA_ERR_ARG, "matrix-core path supports head_dim 64, 128, 256");
   }
