@@ -151,12 +151,7 @@ class ViewAttnBackend(BaseAttnBackend):
         sub_worker_host = np.arange(n_rows, dtype=np.int64)
         subs = self._subs(qo, kv, lens, flags, chain, sub_worker_host)
         counts = native.VaPlanCounts()
-        scratch = op._plan_scratch
-        rc = native.lib.va_plan_build(subs, op._shape, op.plan_params, scratch.ctypes.data, scratch.size, counts)
-        if rc == native.VA_ERR_CAPACITY and counts.plan_words > scratch.size:
-            scratch = op._plan_scratch = np.empty(2 * counts.plan_words, dtype=np.int32)
-            rc = native.lib.va_plan_build(subs, op._shape, op.plan_params, scratch.ctypes.data, scratch.size, counts)
-        native.check(rc)
+        scratch = op._plan_into_scratch(subs, counts)
         host = torch.empty(counts.plan_words, dtype=torch.int32, pin_memory=True)
         host.numpy()[:] = scratch[: counts.plan_words]
         blob = host.to(self.device, non_blocking=True)

@@ -98,10 +98,32 @@ inline int32_t visible_end(int32_t len, int32_t nq, bool causal, int32_t b) {
   return causal ? std::min(len, len - nq + b) : len;
 }
 
+// How finely the walks of chains may be cut (tokens; `gran` below is 64).  The cost of a wide tile's set-up in
+// walked tokens decides what a cut is worth; the floors keep the pieces of small launches worth their
+// launch.  The fine cuts are the rule: a chunk of 333 tokens over four blocks (16 q / 4 kv heads of 256 dims) used
+// 44 % of the machine under floors of 1024 tokens, whose longest slot walked 1700 tokens where an even share is
+// 620.  Measured, kernels of one layer, coarse -> fine: that chunk 81 -> 72 us; 4 chunks of 300..1500
+// tokens at 32 q / 8 kv heads of 128 dims 654 -> 604 us; plain prefill of 6 requests, whose launch of narrow tiles was
+// ONE row walking 1363 tokens, 433 -> 364 us; two chunks of 60 tokens 102 -> 54 us.
+// Charging a set-up: at head_dim 256, where a tile is 128 rows, 640 and 384 tokens differ by under 4 % either way;
+// at 64 and 128 (256 rows, twice the work per token) 384 is the better by up to 15 % (drawn chunk batches).
+// Finer cuts leave more partial states, so the coarse ones remain for callers whose scratch holds no more.
+struct Cuts {
+  bool fine = true;
+  int32_t seg_cost(int head_dim) const { return fine && head_dim <= 128 ? 384 : 640; }
+  int32_t part(int head_dim) const { return !fine ? 512 : head_dim <= 128 ? 256 : 384; }  // a part of a walk, side by side with others
+  int32_t group_floor() const { return fine ? 128 : 1024; }  // walk of a group of wide slots
+  int32_t least_piece(int64_t group_budget) const {          // of a wide tile: an eighth of the share, within limits
+    return fine ? (int32_t)std::min<int64_t>(384, std::max<int64_t>(64, group_budget / 8)) : 384;
+  }
+  int32_t narrow_floor() const { return fine ? 128 : 1024; }
+  int32_t narrow_least() const { return fine ? 64 : 384; }
+};
+
 // `cap`, when given, bounds the number of entries a die may receive in each class, so that a plan
 // whose real items fit the capacity still fits it after the per-die padding.
 int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* params, Built& out,
-          const VaPlanCapacity* cap = nullptr) {
+          const VaPlanCapacity* cap = nullptr, const Cuts& cuts_of_chains = Cuts()) {
   int rc = check_subs(s, shape);
   if (rc) return rc;
   const int kernel = resolve_kernel(shape, params);
@@ -277,22 +299,20 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
 
   // contributions per output row decide direct-vs-partial
   std::vector<int32_t> row_count(s->n_rows, 0);
-  struct Pending {
-    int32_t item;
-    std::vector<int32_t> rows;  // output row per tile row
-  };
-  std::vector<Pending> pend;
+  std::vector<int32_t> item_rows;  // output row per tile row, item after item
 
   int32_t next_unit = 0;
-  auto emit = [&](int32_t n_q, const std::vector<Link>& links, std::vector<int32_t>&& rows, int32_t unit = -1,
-                  int32_t slot = -1) {
+  // row_of(i): output row of tile row i
+  auto emit = [&](int32_t n_q, const std::vector<Link>& links, auto&& row_of, int32_t unit = -1, int32_t slot = -1) {
     int32_t tokens = 0;
     for (auto& l : links) tokens += l.tok_end - l.tok_begin;
     Item it{(int32_t)out.links.size(), (int32_t)links.size(), n_q, -1, tokens, n_q > q_tile ? 1 : 0,
             unit >= 0 ? unit : next_unit++, n_q > q_tile ? slot : -1};
     out.links.insert(out.links.end(), links.begin(), links.end());
-    for (int32_t r : rows) ++row_count[r];
-    pend.push_back(Pending{(int32_t)out.items.size(), std::move(rows)});
+    for (int32_t i = 0; i < n_q; ++i) {
+      item_rows.push_back(row_of(i));
+      ++row_count[item_rows.back()];
+    }
     out.items.push_back(it);
   };
 
@@ -324,9 +344,8 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     }
     auto emit_range = [&](size_t ti, int32_t t0, int32_t t1, int32_t unit = -1) {
       const size_t a = tiles[ti].first, b = tiles[ti].second;
-      std::vector<int32_t> rows;
-      for (size_t r = a; r < b; ++r) rows.push_back((int32_t)s->sub_worker[gr.subrows[r]]);
-      emit((int32_t)(b - a), {Link{s->kv_indptr[rep], t0, t1, tile_qref[ti], VA_NO_CAUSAL, lflags}}, std::move(rows), unit);
+      emit((int32_t)(b - a), {Link{s->kv_indptr[rep], t0, t1, tile_qref[ti], VA_NO_CAUSAL, lflags}},
+           [&](int32_t i) { return (int32_t)s->sub_worker[gr.subrows[a + i]]; }, unit);
     };
     auto chunk_len = [&](int32_t chunk) {
       const int32_t n_chunks = (len + chunk - 1) / chunk;
@@ -367,9 +386,9 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   // A piece of a wide tile stages its query tile once per segment of the view it walks (the query is
   // rotated for every block anew), which costs about as much as walking `seg_cost` tokens: the packing
   // charges every (piece, segment) to the room it fills.  A remainder that would cost less than
-  // `min_piece` stays with the piece before it.
-  const int32_t seg_cost = 10 * gran;
-  const int32_t min_piece = 6 * gran;
+  // `min_piece` (below) stays with the piece before it.
+  const int32_t seg_cost = cuts_of_chains.seg_cost(shape->head_dim);
+  const int32_t narrow_least = cuts_of_chains.narrow_least();
   if (chain_tiles > 0 && chain_tiles < 4 * slots_wanted) {
     // The budget cuts the walks of the NARROW chain tiles only (wide tiles are packed in bundles by
     // budgets of their own, below), so it is their tokens that size it: a narrow tile of t tokens
@@ -379,7 +398,7 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     // into hundreds of pieces.)
     const int64_t want = std::max<int64_t>(1, std::min<int64_t>(target, slots_wanted));
     const int64_t narrow_chain_tokens = chain_tokens - wide_chain_tokens;
-    chain_budget = std::max<int64_t>((narrow_chain_tokens + want - 1) / want, 16 * gran);
+    chain_budget = std::max<int64_t>((narrow_chain_tokens + want - 1) / want, cuts_of_chains.narrow_floor());
   }
   // cuts inside a segment keep to multiples of 16 tokens where the kernels profit (pages of 16
   // tokens or more: a piece that starts on such a boundary is fetched with uniform loads)
@@ -433,7 +452,7 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
       pos += align_cuts ? round_up(vis, 16) : vis;  // every member starts at a multiple of 16: so do all cuts within it
     }
     if (pos == 0) return bd;
-    bd.f = (int32_t)std::max<int64_t>(1, std::min<int64_t>(lanes / m, pos / (8 * gran)));
+    bd.f = (int32_t)std::max<int64_t>(1, std::min<int64_t>(lanes / m, pos / cuts_of_chains.part(shape->head_dim)));
     bd.part = bd.f == 1 ? (int32_t)pos : round_up((pos + bd.f - 1) / bd.f, 16);
     for (int32_t g = 0; g < bd.f; ++g)
       for (int32_t o : bd.off) {
@@ -471,7 +490,8 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   // to be opened, so that a group closed early (less than min_piece of its room left) or run over (a
   // bundle's short remainder kept with the piece before it) is made up for by the groups after it,
   // and their number never exceeds the number wanted.
-  const int64_t group_budget = pack ? std::max<int64_t>((wide_walk + groups_wanted - 1) / groups_wanted, 16 * gran) : 0;
+  const int64_t group_budget = pack ? std::max<int64_t>((wide_walk + groups_wanted - 1) / groups_wanted, cuts_of_chains.group_floor()) : 0;
+  const int32_t min_piece = cuts_of_chains.least_piece(group_budget);
   int64_t groups_left = pack ? std::max<int64_t>(1, (wide_walk + group_budget - 1) / group_budget) : 0;
   // What is still to be placed, set-ups included: every segment of every bundle, and one more for
   // every group boundary (it falls inside some segment, which is then staged on both sides).  An
@@ -525,13 +545,13 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   };
 
   // Cut a narrow tile's walk (links in walking order) into budgets of `slot_room` tokens, one item a
-  // piece; a remainder of less than min_piece stays with the piece before it.
+  // piece; a remainder of less than narrow_least stays with the piece before it.
   auto cut_walk = [&](const std::vector<Link>& walk, auto&& close) {
     int32_t room = slot_room;
     int64_t left = 0;  // tokens of the walk not yet in a piece
     for (auto& l : walk) left += l.tok_end - l.tok_begin;
     auto fit_room = [&]() {
-      if (left > room && left - room < min_piece) room = (int32_t)left;
+      if (left > room && left - room < narrow_least) room = (int32_t)left;
     };
     fit_room();
     std::vector<Link> cur;
@@ -545,7 +565,7 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
         int32_t take = std::min(room, l.tok_end - l.tok_begin);
         if (aligned && take < l.tok_end - l.tok_begin) take = take / 16 * 16;  // l.tok_begin is a multiple of 16: segments start at 0, cuts keep it so
         if (take <= 0) {  // no room left to go on here: the piece ends
-          if (!cur.empty() && left < min_piece) {  // ... unless what is left is too little for a piece of its own
+          if (!cur.empty() && left < narrow_least) {  // ... unless what is left is too little for a piece of its own
             room = (int32_t)left;
             continue;
           }
@@ -561,7 +581,7 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
         left -= take;
         room -= take;
         if (room <= 0 && left > 0) {
-          if (left < min_piece) {  // too little for a piece of its own: it stays with this one
+          if (left < narrow_least) {  // too little for a piece of its own: it stays with this one
             room = (int32_t)left;
             continue;
           }
@@ -578,8 +598,9 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     const int32_t nq = s->qo_indptr[ch[0] + 1] - s->qo_indptr[ch[0]];
     cut_tiles(nq, tiles);
     // the links of tile rows [a, b), clipped to walk positions [lo, hi) of a bundle (all of them without one)
-    auto tile_links = [&](int32_t a, int32_t b, const Bundle* bd, int64_t lo, int64_t hi) {
-      std::vector<Link> links;
+    std::vector<Link> links;
+    auto tile_links = [&](int32_t a, int32_t b, const Bundle* bd, int64_t lo, int64_t hi) -> const std::vector<Link>& {
+      links.clear();
       size_t k = 0;
       for (int32_t m : ch) {
         const bool causal = s->flags[m] & VA_SUB_CAUSAL;
@@ -598,10 +619,8 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
       }
       return links;
     };
-    auto tile_rows = [&](int32_t a, int32_t b) {
-      std::vector<int32_t> rows;
-      for (int32_t r = a; r < b; ++r) rows.push_back((int32_t)s->sub_worker[s->qo_indptr[ch[0]] + r]);
-      return rows;
+    auto tile_rows = [&](int32_t a) {
+      return [rows = s->sub_worker + s->qo_indptr[ch[0]] + a](int32_t i) { return (int32_t)rows[i]; };
     };
     if (pack) {
       bundles_of(ch, nq, bundles);
@@ -610,8 +629,8 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
           for (int32_t g = 0; g < bd.f; ++g)
             for (int32_t j = 0; j < bd.m; ++j) {
               const int32_t a = tiles[bd.first + j].first, b = tiles[bd.first + j].second;
-              const std::vector<Link> links = tile_links(a, b, &bd, (int64_t)g * bd.part + x0, (int64_t)g * bd.part + x1);
-              if (!links.empty()) emit(b - a, links, tile_rows(a, b), -1, group * lanes + g * bd.m + j);
+              tile_links(a, b, &bd, (int64_t)g * bd.part + x0, (int64_t)g * bd.part + x1);
+              if (!links.empty()) emit(b - a, links, tile_rows(a), -1, group * lanes + g * bd.m + j);
             }
         });
       }
@@ -619,37 +638,47 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     for (auto& tl : tiles) {
       const int32_t a = tl.first, b = tl.second;
       if (pack && b - a > q_tile) continue;  // packed above
-      const std::vector<Link> all = tile_links(a, b, nullptr, 0, 0);
+      const std::vector<Link>& all = tile_links(a, b, nullptr, 0, 0);
       if (all.empty()) continue;
       if (!pack) {
-        emit(b - a, all, tile_rows(a, b));
+        emit(b - a, all, tile_rows(a));
         continue;
       }
-      cut_walk(all, [&](const std::vector<Link>& cur) { emit(b - a, cur, tile_rows(a, b)); });
+      cut_walk(all, [&](const std::vector<Link>& cur) { emit(b - a, cur, tile_rows(a)); });
     }
   }
 
   // ---- partial slots and the per-row merge lists ----
-  std::vector<std::vector<int32_t>> parts_of_row(s->n_rows);
-  for (auto& p : pend) {
-    bool direct = true;
-    for (int32_t r : p.rows) direct = direct && row_count[r] == 1;
-    Item& it = out.items[p.item];
-    if (direct) {
-      it.part_base = -1;
-    } else {
-      it.part_base = out.n_partials;
-      for (size_t i = 0; i < p.rows.size(); ++i) parts_of_row[p.rows[i]].push_back(out.n_partials + (int32_t)i);
-      out.n_partials += (int32_t)p.rows.size();
-    }
-  }
+  // (an item whose rows no other item serves writes them itself; the states of the others are numbered item
+  // after item, and a row's list holds its own in that order)
   out.row_indptr.assign(s->n_rows + 1, 0);
   out.row_flags.assign(s->n_rows, 0);
+  {
+    const int32_t* rows = item_rows.data();
+    for (Item& it : out.items) {
+      const bool direct = std::all_of(rows, rows + it.n_q, [&](int32_t r) { return row_count[r] == 1; });
+      if (!direct) {
+        it.part_base = out.n_partials;
+        out.n_partials += it.n_q;
+        for (int32_t i = 0; i < it.n_q; ++i) ++out.row_indptr[rows[i] + 1];
+      }
+      rows += it.n_q;
+    }
+  }
   for (int32_t r = 0; r < s->n_rows; ++r) {
-    out.row_indptr[r + 1] = out.row_indptr[r] + (int32_t)parts_of_row[r].size();
-    out.row_ids.insert(out.row_ids.end(), parts_of_row[r].begin(), parts_of_row[r].end());
     if (row_count[r] == 0) out.row_flags[r] = VA_ROW_EMPTY;
-    else if (parts_of_row[r].empty()) out.row_flags[r] = VA_ROW_DIRECT;
+    else if (out.row_indptr[r + 1] == 0) out.row_flags[r] = VA_ROW_DIRECT;
+    out.row_indptr[r + 1] += out.row_indptr[r];
+  }
+  out.row_ids.resize(out.n_partials);
+  {
+    std::vector<int32_t> next(out.row_indptr.begin(), out.row_indptr.end() - 1);
+    const int32_t* rows = item_rows.data();
+    for (const Item& it : out.items) {
+      if (it.part_base >= 0)
+        for (int32_t i = 0; i < it.n_q; ++i) out.row_ids[next[rows[i]]++] = it.part_base + i;
+      rows += it.n_q;
+    }
   }
 
   // Launch order.  Wide items first (their own launch), then narrow ones.  The hardware hands
@@ -823,11 +852,26 @@ void fill_counts(const Built& b, const VaSubRequests* s, const VaShape* shape, V
 
 }  // namespace
 
+// The plan of fine cuts, unless only that of coarse ones leaves room in `workspace_bytes` (<= 0: no limit).
+static int build_within(const VaSubRequests* subs, const VaShape* shape, const VaPlanParams* params,
+                        int64_t workspace_bytes, Built& out) {
+  const int rc = build(subs, shape, params, out);
+  auto fits = [&](const Built& plan) {
+    return va_workspace_bytes_for(plan.n_partials, shape->num_q_heads, shape->head_dim) <= workspace_bytes;
+  };
+  if (rc || workspace_bytes <= 0 || fits(out)) return rc;
+  Built coarse;
+  Cuts cuts;
+  cuts.fine = false;
+  if (build(subs, shape, params, coarse, nullptr, cuts) == VA_OK && fits(coarse)) out = std::move(coarse);
+  return VA_OK;
+}
+
 extern "C" int va_plan_count(const VaSubRequests* subs, const VaShape* shape, const VaPlanParams* params,
                              VaPlanCounts* counts) {
   if (!counts) return va_fail(VA_ERR_ARG, "null counts");
   Built b;
-  int rc = build(subs, shape, params, b);
+  int rc = build_within(subs, shape, params, VA_STATIC_SCRATCH_BYTES, b);
   if (rc) return rc;
   fill_counts(b, subs, shape, counts);
   return VA_OK;
@@ -966,9 +1010,15 @@ static int write_plan(const Built& b, const VaSubRequests* subs, const VaShape* 
 
 extern "C" int va_plan_build(const VaSubRequests* subs, const VaShape* shape, const VaPlanParams* params,
                              int32_t* plan_host, int64_t plan_capacity_words, VaPlanCounts* counts) {
+  return va_plan_build_within(subs, shape, params, VA_STATIC_SCRATCH_BYTES, plan_host, plan_capacity_words, counts);
+}
+
+extern "C" int va_plan_build_within(const VaSubRequests* subs, const VaShape* shape, const VaPlanParams* params,
+                                    int64_t workspace_bytes, int32_t* plan_host, int64_t plan_capacity_words,
+                                    VaPlanCounts* counts) {
   if (!plan_host) return va_fail(VA_ERR_ARG, "null plan buffer");
   Built b;
-  int rc = build(subs, shape, params, b);
+  const int rc = build_within(subs, shape, params, workspace_bytes, b);
   if (rc) return rc;
   return write_plan(b, subs, shape, nullptr, plan_host, plan_capacity_words, counts);
 }

@@ -33,6 +33,7 @@ EXPORTED_SYMBOLS = (
     "va_store_kv_rope",
     "va_plan_count",
     "va_plan_build",
+    "va_plan_build_within",
     "va_copy_shift_kv",
     "va_plan_capacity",
     "va_plan_fixed_words",
@@ -155,6 +156,9 @@ def _load() -> C.CDLL:
     lib.va_plan_build.restype = C.c_int
     lib.va_plan_build.argtypes = [C.POINTER(VaSubRequests), C.POINTER(VaShape), C.POINTER(VaPlanParams),
                                   vp, i64, C.POINTER(VaPlanCounts)]
+    lib.va_plan_build_within.restype = C.c_int
+    lib.va_plan_build_within.argtypes = [C.POINTER(VaSubRequests), C.POINTER(VaShape), C.POINTER(VaPlanParams),
+                                         i64, vp, i64, C.POINTER(VaPlanCounts)]
     lib.va_attention.restype = C.c_int
     lib.va_attention.argtypes = [vp, i64, vp, vp, i64, vp, vp, vp, vp, vp, i64, vp, vp, i32, vp, i64,
                                  C.POINTER(VaShape), C.POINTER(VaRope), vp]

@@ -277,6 +277,19 @@ class SharedCacheAttention:
     # ------------------------------------------------------------------
     # planning
     # ------------------------------------------------------------------
+    def _plan_into_scratch(self, subs, counts) -> np.ndarray:
+        """Plan into the op's host scratch (grown on demand), within the workspace once that is fixed."""
+        limit = self._workspace.numel() if self._workspace_prepared and self._workspace is not None else 0
+        scratch = self._plan_scratch
+        rc = native.lib.va_plan_build_within(subs, self._shape, self.plan_params, limit, scratch.ctypes.data,
+                                             scratch.size, counts)
+        if rc == native.VA_ERR_CAPACITY and counts.plan_words > scratch.size:
+            scratch = self._plan_scratch = np.empty(2 * counts.plan_words, dtype=np.int32)
+            rc = native.lib.va_plan_build_within(subs, self._shape, self.plan_params, limit, scratch.ctypes.data,
+                                                 scratch.size, counts)
+        native.check(rc)
+        return scratch
+
     def _build_launch(self, qo_indptr, kv_indptr, kv_indices_host, seq_lens, flags, chain, sub_worker_host,
                       n_rows: int, kv_indices_dev: torch.Tensor, refs: list) -> LaunchPlan:
         """Run the native work decomposition over the planned tables and upload
@@ -293,13 +306,7 @@ class SharedCacheAttention:
         # one pass of the planner: build into a scratch that is normally large enough, then copy
         # the blob to pinned staging of its exact size
         counts = native.VaPlanCounts()
-        scratch = self._plan_scratch
-        rc = native.lib.va_plan_build(subs, self._shape, self.plan_params, scratch.ctypes.data, scratch.size, counts)
-        if rc == native.VA_ERR_CAPACITY and counts.plan_words > scratch.size:
-            scratch = self._plan_scratch = np.empty(2 * counts.plan_words, dtype=np.int32)
-            rc = native.lib.va_plan_build(subs, self._shape, self.plan_params, scratch.ctypes.data, scratch.size,
-                                          counts)
-        native.check(rc)
+        scratch = self._plan_into_scratch(subs, counts)
         pin = self.device.type == "cuda"
         host = torch.empty(counts.plan_words, dtype=torch.int32, pin_memory=pin)
         host.numpy()[:] = scratch[: counts.plan_words]

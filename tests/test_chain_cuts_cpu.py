@@ -1,0 +1,74 @@
+"""Cutting the walks of prefill tiles: every pair is covered whatever the size, and a caller whose workspace is
+fixed gets the coarse cuts where only their partial states fit."""
+
+import numpy as np
+import pytest
+
+from async_llm_amd import native
+
+from .test_native_abi_cpu import H, build_plan, check_coverage, decode_plan
+
+
+def _tables(requests, page):
+    """requests: (new tokens, own prefix, context lengths) -> tables of chained sub-requests."""
+    qo, kvp, kvi, lens, flags, chain, sw, n_rows = [0], [0], [], [], [], [], [], 0
+    for r, (new, prefix, segments) in enumerate(requests):
+        rows = list(range(n_rows, n_rows + new))
+        n_rows += new
+        for length, causal in [(n, 0) for n in segments] + [(prefix + new, 1)]:
+            kvi += list(range(len(kvi), len(kvi) - (-length // page)))
+            kvp.append(len(kvi)), lens.append(length), flags.append(causal), chain.append(r)
+            sw += rows
+            qo.append(len(sw))
+    return qo, kvp, kvi, lens, flags, chain, sw, n_rows
+
+
+@pytest.mark.parametrize("heads", [(16, 4, 256), (32, 8, 128), (8, 2, 128), (64, 16, 64)])
+@pytest.mark.parametrize("page", [1, 16])
+@pytest.mark.parametrize("requests", [
+    [(1, 1362, [])],  # one row over a walk of its own
+    [(65, 700, [])],  # a wide tile and one row behind it
+    [(33, 0, [1])],
+    [(5, 127, [129]), (40, 64, [1, 63]), (130, 0, [257])],
+    [(70, 3, [400, 17, 900])],
+])
+def test_small_chains_are_covered_once(heads, page, requests):
+    tables = _tables(requests, page)
+    rc, blob, _ = build_plan(*tables, heads=heads, page=page, dtype=native.VA_BF16, kernel=native.VA_KERNEL_MFMA)
+    assert rc == 0
+    qo, kvp, _, lens, flags, _, sw, n_rows = tables
+    check_coverage(blob, qo, kvp, lens, flags, sw, n_rows)
+
+
+def test_walk_of_one_row_is_cut_into_short_pieces():
+    rc, blob, counts = build_plan(*_tables([(1, 1362, [])], 1), heads=(32, 8, 128), page=1, dtype=native.VA_BF16,
+                                  kernel=native.VA_KERNEL_MFMA)
+    assert rc == 0
+    tokens = [int(it[4]) for it in decode_plan(blob)[1] if it[2] > 0]
+    assert sum(tokens) == 1363 and max(tokens) <= 256
+
+
+def _plan_within(tables, limit):
+    qo, kvp, kvi, lens, flags, chain, sw, n_rows = tables
+    i32 = [np.asarray(a, dtype=np.int32) for a in (qo, kvp, kvi, lens, flags, chain)]
+    rows = np.asarray(sw, dtype=np.int64)
+    subs = native.VaSubRequests(len(lens), len(sw), n_rows, *(a.ctypes.data for a in i32), rows.ctypes.data)
+    shape = native.VaShape(16, 4, 256, 16, native.VA_BF16)
+    blob, counts = np.empty(1 << 18, dtype=np.int32), native.VaPlanCounts()
+    rc = native.lib.va_plan_build_within(subs, shape, native.VaPlanParams(native.VA_KERNEL_MFMA, 0, 0, 0, 0), limit,
+                                         blob.ctypes.data, blob.size, counts)
+    assert rc == 0
+    header = blob[: native.PLAN_HEADER_WORDS]
+    assert header[H["N_PARTIALS"]] == counts.n_partials
+    check_coverage(blob[: counts.plan_words], qo, kvp, lens, flags, sw, n_rows)
+    return counts.workspace_bytes
+
+
+def test_fixed_workspace_gets_coarse_cuts_only_where_they_help():
+    tables = _tables([(58, 40, [700, 300])], 16)
+    fine = _plan_within(tables, 0)
+    coarse = _plan_within(tables, fine - 1)
+    assert coarse < fine
+    assert _plan_within(tables, fine) == fine and _plan_within(tables, coarse) == coarse
+    if coarse:
+        assert _plan_within(tables, coarse - 1) == fine  # neither fits: the caller is told what the plan needs
