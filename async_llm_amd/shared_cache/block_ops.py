@@ -37,6 +37,18 @@ def token_slots(block: CacheBlock) -> np.ndarray:
     return grid.reshape(-1)[: block.num_tokens]
 
 
+def slots_meet(a: np.ndarray, b: np.ndarray) -> bool:
+    """Whether two non-empty slot lists share a slot.  Slots of one pool lie in a range not much larger than
+    the pool, where marking ``a``'s and looking ``b``'s up takes 25 us for 7000 slots against 200 for a sort.
+    The marks stay under 64 MB (of which only the touched pages cost); wider ranges are sorted."""
+    low, high = int(min(a.min(), b.min())), int(max(a.max(), b.max()))
+    if high - low >= 1 << 26:
+        return bool(np.intersect1d(a, b).size)
+    marked = np.zeros(high - low + 1, dtype=bool)
+    marked[a - low] = True
+    return bool(marked[b - low].any())
+
+
 class BlockKVOps:
     """``merge_blocks`` / ``append_block`` over a paged pool.
 
@@ -155,7 +167,7 @@ class BlockKVOps:
         target = token_slots(destination)[destination_start: destination_start + n]
         assert target.size == n, "destination block is too short for the copied run"
         # the kernel scatters while it gathers: a slot read by one token and written by another would race
-        if np.intersect1d(source, target).size:
+        if slots_meet(source, target):
             raise ValueError("source and destination slots of a block copy overlap")
         self._launch(source, target, int(position_shift))
 
