@@ -511,30 +511,28 @@ __global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(MergeArgs a) {
     i0 += 2 * kMergeWaves;
   }
   if (mine & 1) fold(i0, std::integral_constant<int, 1>{});
-  if constexpr (kMergeWaves > 1) {
-    // fold the waves' states: wave 0 collects
-    __shared__ float s_ml[kMergeWaves][2];
-    __shared__ float s_av[kMergeWaves][4][64];
-    if (wave > 0) {
-      if (lane == 0) {
-        s_ml[wave][0] = mm;
-        s_ml[wave][1] = ll;
-      }
-#pragma unroll
-      for (int k = 0; k < 4; ++k) s_av[wave][k][lane] = av[k];
+  // fold the waves' states: wave 0 collects
+  __shared__ float s_ml[kMergeWaves][2];
+  __shared__ float s_av[kMergeWaves][4][64];
+  if (wave > 0) {
+    if (lane == 0) {
+      s_ml[wave][0] = mm;
+      s_ml[wave][1] = ll;
     }
-    __syncthreads();
-    if (wave > 0) return;
 #pragma unroll
-    for (int w = 1; w < kMergeWaves; ++w) {
-      const float mw = s_ml[w][0], lw = s_ml[w][1];
-      const float m_new = fmaxf(mm, mw);
-      const float sa = exp2f(mm - m_new), sb = exp2f(mw - m_new);
-      ll = ll * sa + lw * sb;
+    for (int k = 0; k < 4; ++k) s_av[wave][k][lane] = av[k];
+  }
+  __syncthreads();
+  if (wave > 0) return;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) av[k] = av[k] * sa + s_av[w][k][lane] * sb;
-      mm = m_new;
-    }
+  for (int w = 1; w < kMergeWaves; ++w) {
+    const float mw = s_ml[w][0], lw = s_ml[w][1];
+    const float m_new = fmaxf(mm, mw);
+    const float sa = exp2f(mm - m_new), sb = exp2f(mw - m_new);
+    ll = ll * sa + lw * sb;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) av[k] = av[k] * sa + s_av[w][k][lane] * sb;
+    mm = m_new;
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
