@@ -75,16 +75,28 @@ __device__ __forceinline__ Pos3 load_pos(const int64_t* pos, int64_t axis_stride
 __device__ __forceinline__ float mul_rounded(float a, float b);
 
 // sin and cos of an angle, both from one argument reduction: the nearest multiple of pi / 2 is taken off in
-// double precision (pi / 2 as a sum of two doubles: the remainder is exact to far below an fp32 ulp for any
-// position a table could hold), Taylor polynomials on [-pi/4, pi/4] whose first omitted terms are under half
-// an fp32 ulp.  No branch and some 35 instructions, where the library's sinf and cosf with their general
-// reduction take five times as long -- which was most of what rotating an mRoPE query tile cost (64 rows of
-// 64 pairs: 19 300 -> 7 000 cycles).
+// double precision (pi / 2 as a sum of two doubles: the remainder is exact to far below an fp32 ulp), Taylor
+// polynomials on [-pi/4, pi/4] whose first omitted terms are under half an fp32 ulp.  No branch that a real
+// position takes and some 35 instructions, where the library's sinf and cosf with their general reduction take
+// five times as long -- which was most of what rotating an mRoPE query tile cost (64 rows of 64 pairs:
+// 19 300 -> 7 000 cycles).  Error against 64 bits over positions to 2^50 and 64 frequencies: at most 1.56 ulp and
+// 1.49e-8 rms, the library's functions 1.56 ulp and 1.61e-8.
+// From 2^50 on the quotient no longer comes out to the unit: the multiple taken off first is up to
+// 2^(e - 53) units away from the nearest one (e: the angle's exponent), and what is left is reduced once
+// more.  An angle within 64 bits (any int64 position, frequencies up to 1) leaves 2^11 units then, and
+// an error of 2^-41 in them.
 __device__ __forceinline__ void sin_cos(float x, float& s, float& c) {
   const double k = rint((double)x * 0.63661977236758134308);
-  const double near = fma(-k, 1.57079632679489655800, (double)x);
-  const float r = (float)fma(-k, 6.12323399573676603587e-17, near), z = r * r;
-  const int quadrant = (int)(k - 4.0 * floor(0.25 * k));
+  double near = fma(-k, 1.57079632679489655800, (double)x), units = k;
+  if (fabsf(x) > 0x1p50f) {
+    near = fma(-k, 6.12323399573676603587e-17, near);
+    const double more = rint(near * 0.63661977236758134308);
+    near = fma(-more, 1.57079632679489655800, near);
+    units = more;
+  }
+  const float r = (float)fma(-units, 6.12323399573676603587e-17, near), z = r * r;
+  int quadrant = (int)(k - 4.0 * floor(0.25 * k));
+  if (fabsf(x) > 0x1p50f) quadrant += (int)units;
   const float sp = fmaf(z, fmaf(z, fmaf(z, fmaf(z, -2.50521084e-8f, 2.75573192e-6f), -1.98412698e-4f), 8.33333333e-3f), -1.66666667e-1f);
   const float cp = fmaf(z, fmaf(z, fmaf(z, fmaf(z, -2.75573192e-7f, 2.48015873e-5f), -1.38888889e-3f), 4.16666667e-2f), -0.5f);
   const float sr = fmaf(r * z, sp, r), cr = fmaf(z, cp, 1.f);
