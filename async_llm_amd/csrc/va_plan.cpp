@@ -990,12 +990,13 @@ static int write_plan(const Built& b, const VaSubRequests* subs, const VaShape* 
   off += cap_rows;
   // The waves of a merge workgroup split a row's states, so rows of many states (long views cut
   // into many chunks) get more waves; when the rows are many (split prefill tiles: thousands of
-  // rows of a few states each) a workgroup takes a whole row (word 1).  A fixed plan decides
+  // rows of a few states each) a workgroup takes a whole row (word 1) and the long rows among them are
+  // found and merged head by head.  A fixed plan decides
   // from its capacity, a packed one from its counts: either way the word is part of the header the
   // launches are derived from.  Measured on one MI355X: 17 states per row take 9.9 / 14.7 / 20.6 us
   // with 4 / 8 / 16 waves, 72 per row 16.4 / 12.0 / 9.5 us.
-  // A workgroup a row pays from about 8192 (row, head) pairs: 7571 rows of 32 heads 53 -> 13 us; at 17 rows of 32 heads
-  // and 23 states the launch would cost 17 us more, between 512 and 8192 pairs prefill does not care (1 %).
+  // A workgroup a row pays from about 8192 (row, head) pairs: 7571 rows of 32 heads 53 -> 13 us; between 512 and 8192
+  // pairs prefill does not care (1 %), and rows of a few dozen states want their waves from the start.
   {
     const int64_t rows = std::max<int64_t>(1, cap ? cap_rows : subs->n_rows);
     const int64_t per_row = (cap ? cap_row_parts : c.n_row_parts) / rows;

@@ -4,6 +4,7 @@
 
 #include <type_traits>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -460,20 +461,10 @@ __global__ __launch_bounds__(kGenThreads) void attn_generic_kernel(AttnArgs a) {
 // in LDS.  Lane l owns dims l, l + 64, ...
 // For a decode batch: few rows, up to dozens of partial states each.
 template <typename E, int kMergeWaves>
-__global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(MergeArgs a) {
+__device__ __forceinline__ void merge_row_head(const MergeArgs& a, long long row, int hq, int begin, int end) {
   using S = typename E::storage;
-  const long long row = blockIdx.x;
-  const int hq = blockIdx.y;
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  const int flags = a.row_flags[row];
-  if (flags & VA_ROW_DIRECT) return;
   S* o = (S*)a.out + (row * a.num_q_heads + hq) * (long long)a.head_dim;
-  if (flags & VA_ROW_EMPTY) {
-    for (int d = threadIdx.x; d < a.head_dim; d += 64 * kMergeWaves) o[d] = E::store(0.f);
-    if (threadIdx.x == 0 && a.lse) a.lse[row * a.num_q_heads + hq] = -INFINITY;
-    return;
-  }
-  const int b = a.row_indptr[row], e = a.row_indptr[row + 1];
   const int n_d = (a.head_dim + 63) / 64;  // dims per lane: d = lane + 64*k (at most 4 for D = 256)
   float mm = kNegBig, ll = 0.f;
   float av[4] = {0.f, 0.f, 0.f, 0.f};
@@ -504,8 +495,8 @@ __global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(MergeArgs a) {
   };
   // this wave's partials, eight per round; the last round takes exactly what is left (a split
   // prefill row has two or three states: a padded round of eight would quadruple its loads)
-  int i0 = b + wave;
-  int mine = i0 < e ? (e - i0 + kMergeWaves - 1) / kMergeWaves : 0;
+  int i0 = begin + wave;
+  int mine = i0 < end ? (end - i0 + kMergeWaves - 1) / kMergeWaves : 0;
   for (; mine >= 8; mine -= 8, i0 += 8 * kMergeWaves) fold(i0, std::integral_constant<int, 8>{});
   if (mine & 4) {
     fold(i0, std::integral_constant<int, 4>{});
@@ -550,18 +541,66 @@ __global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(MergeArgs a) {
   }
 }
 
+template <typename E, int kMergeWaves>
+__global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(MergeArgs a) {
+  using S = typename E::storage;
+  const long long row = blockIdx.x;
+  const int hq = blockIdx.y;
+  const int flags = a.row_flags[row];
+  if (flags & VA_ROW_DIRECT) return;
+  if (flags & VA_ROW_EMPTY) {
+    S* o = (S*)a.out + (row * a.num_q_heads + hq) * (long long)a.head_dim;
+    for (int d = threadIdx.x; d < a.head_dim; d += 64 * kMergeWaves) o[d] = E::store(0.f);
+    if (threadIdx.x == 0 && a.lse) a.lse[row * a.num_q_heads + hq] = -INFINITY;
+    return;
+  }
+  merge_row_head<E, kMergeWaves>(a, row, hq, a.row_indptr[row], a.row_indptr[row + 1]);
+}
+
 // ---------------------------------------------------------------------------
-// merge of many rows of few states (split prefill tiles): one workgroup per row
+// merge of many rows (split prefill tiles): one workgroup per row of few states
 // ---------------------------------------------------------------------------
 // The states of a row lie as [heads * dims] floats each, so a thread takes four consecutive floats of every
 // 1024 and the workgroup reads whole states, two at a time with all their loads in flight; rows that an item
 // has written itself leave at once.  (As one workgroup per (row, head) such a launch was bound by the rate
 // at which workgroups start: 7571 rows of 32 heads, most of them written directly, took 53 us.)
+// Rows of more than kFewStates states (decode rows beside prefill chunks, a recorded plan of room for many rows with a
+// few long ones) would be a chain of a trip to memory per pair of states here.  They are left to `finders`
+// workgroups per head at the front of the launch: each looks through every finders-th row and merges its head of the
+// long ones with four waves, eight states per round and wave.  At 16 heads of 256 dims, every row by itself ->
+// long rows found: 8 decode rows of 16 k..32 k tokens beside a chunk of 512 rows 52.0 -> 15.5 us, 48 beside 4 chunks
+// 28.1 -> 17.9, a recorded plan of 512 rows with 4 long ones 97.1 -> 21.3 (the same launches with one wave per (row,
+// head): 38.7, 28.2, 106.3).  Looking costs 0.4 to 0.8 us where no row is long.
+constexpr int kFewStates = 8;
 template <typename E>
-__global__ __launch_bounds__(256) void merge_rows_kernel(MergeArgs a) {
+__device__ void merge_long_rows(const MergeArgs& a, int n_rows, int finders, int finder, int hq) {
+  __shared__ unsigned long long found[4];
+  for (int base = finder; base < n_rows; base += 256 * finders) {
+    const long long mine = base + (long long)threadIdx.x * finders;
+    const bool is_long = mine < n_rows && a.row_indptr[mine + 1] - a.row_indptr[mine] > kFewStates;
+    const unsigned long long in_wave = __ballot(is_long);
+    if (threadIdx.x % 64 == 0) found[threadIdx.x / 64] = in_wave;
+    __syncthreads();
+    for (int w = 0; w < 4; ++w) {
+      for (unsigned long long left = found[w]; left; left &= left - 1) {
+        const long long row = base + (64ll * w + __builtin_ctzll(left)) * finders;
+        merge_row_head<E, 4>(a, row, hq, a.row_indptr[row], a.row_indptr[row + 1]);
+        __syncthreads();  // the states of the waves have been read
+      }
+    }
+    __syncthreads();
+  }
+}
+
+template <typename E>
+__global__ __launch_bounds__(256, 4) void merge_rows_kernel(MergeArgs a, int n_rows, int finders) {
   using S = typename E::storage;
   typedef const __attribute__((address_space(4))) int32_t* Words;
-  const long long row = blockIdx.x;
+  if (blockIdx.x < (unsigned)(finders * a.num_q_heads)) {
+    merge_long_rows<E>(a, n_rows, finders, blockIdx.x / a.num_q_heads, blockIdx.x % a.num_q_heads);
+    return;
+  }
+  const long long row = blockIdx.x - finders * a.num_q_heads;
   const int flags = ((Words)a.row_flags)[row];
   if (flags & VA_ROW_DIRECT) return;
   const int width = a.num_q_heads * a.head_dim, d_shift = __builtin_ctz(a.head_dim);  // (head dims are powers of two)
@@ -574,6 +613,7 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(MergeArgs a) {
     return;
   }
   const int begin = ((Words)a.row_indptr)[row], end = ((Words)a.row_indptr)[row + 1];
+  if (end - begin > kFewStates) return;  // a finder's
   constexpr int kRuns = 4;  // runs of 1024 floats per pass
   for (int base = 4 * threadIdx.x; base < width; base += kRuns * 1024) {
     int at[kRuns];
@@ -663,9 +703,13 @@ int launch_generic(const AttnArgs& a, int n_items, hipStream_t stream) {
 template <typename E>
 int launch_merge(const MergeArgs& a, int n_rows, int waves, hipStream_t stream) {
   const dim3 grid((unsigned)n_rows, (unsigned)a.num_q_heads);
+  // Finders of long rows: up to 64 a head, that a batch of decode rows spreads over them; at most four workgroups a
+  // compute unit in all, and sixteen rows to look through each, that they start in a microsecond or less.
+  const int finders = std::max(1, std::min({64, 1024 / a.num_q_heads, n_rows / 16}));
   switch (waves) {
     case 1:
-      hipLaunchKernelGGL((merge_rows_kernel<E>), dim3((unsigned)n_rows), dim3(256), 0, stream, a);
+      hipLaunchKernelGGL((merge_rows_kernel<E>), dim3((unsigned)(n_rows + finders * a.num_q_heads)), dim3(256), 0,
+                         stream, a, n_rows, finders);
       break;
     case 4:
       hipLaunchKernelGGL((merge_kernel<E, 4>), grid, dim3(256), 0, stream, a);

@@ -1,6 +1,7 @@
 """Merge of many rows (8192 (row, head) pairs and more): one workgroup per row, four floats a thread of every 1024 of
 a row's [heads * dims] states.  Row widths below, at and past a pass of 4096 floats, and no multiple of 1024; rows
-of several states, rows an item writes itself and (a fixed plan) rows nobody serves."""
+of several states, rows of so many that they are found and merged head by head, rows an item writes itself and (a
+fixed plan) rows nobody serves."""
 
 from types import SimpleNamespace
 
@@ -9,10 +10,12 @@ import torch
 
 from async_llm_amd.shared_cache import CacheBlock, PrefillSpec, WorkerGroup
 from async_llm_amd.shared_cache.attention_graph import SharedPrefillAttentionBuffers
+from tests.test_native_abi_cpu import H
 from tests.util import assert_close, make_op_and_pool, oracle_prefill, prefill_inputs, run_decode_parity, run_prefill_parity
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda")
+OFF_ROW_INDPTR, MERGE_WORD = H["OFF_ROW_INDPTR"], H["MERGE_WAVES"]
 
 
 def setup(dtype, heads, new, lengths, seed=3):
@@ -63,6 +66,33 @@ def test_many_decode_rows(dtype, heads, workers):
     fresh = SimpleNamespace(alloc_pages=lambda n: torch.arange(8 + workers, 8 + workers + n, dtype=torch.int32) * page)
     *_, meta = run_decode_parity(op, cpu_pool, dev_pool, group, fresh, 1e6, gen)
     assert workers * heads[0] >= 8192 and meta.launch.counts.n_partials > 0
+
+
+@pytest.mark.parametrize("dtype,heads,workers,blocks_of", [
+    (torch.bfloat16, (16, 4, 64), 530, lambda w: 1 + w % 13),              # long rows (over eight states) all along
+    (torch.float32, (32, 8, 128), 260, lambda w: 30 if w in (0, 259) else 1),  # first and last row, several rounds
+    (torch.bfloat16, (64, 16, 64), 4200, lambda w: 9 if w > 4180 else 1),  # past the first 256 rows of a finder
+])
+def test_few_long_rows_among_many(dtype, heads, workers, blocks_of):
+    page = 16
+    total = sum(blocks_of(w) for w in range(workers))
+    op, cpu_pool, dev_pool, gen = make_op_and_pool(DEV, dtype, heads, page, total + workers, 1e6, seed=7, max_pos=512)
+    at, views = 0, []
+    for w in range(workers):
+        view = []
+        for i in range(blocks_of(w)):
+            b = CacheBlock(DEV, page)
+            b.grow_pages(torch.tensor([at * page]), 1 + (w + i) % 15)
+            at += 1
+            view.append(b)
+        views.append(view)
+    group = WorkerGroup(cache_structure=views, write_to=[v[-1] for v in views])
+    fresh = SimpleNamespace(alloc_pages=lambda n: torch.arange(total, total + n, dtype=torch.int32) * page)
+    *_, meta = run_decode_parity(op, cpu_pool, dev_pool, group, fresh, 1e6, gen)
+    header = meta.launch.header
+    assert header[MERGE_WORD] == 1  # the kernel under test
+    indptr = meta.launch.blob[header[OFF_ROW_INDPTR]:][:workers + 1].cpu()
+    assert torch.equal((indptr[1:] - indptr[:-1]) > 8, torch.tensor([blocks_of(w) > 8 for w in range(workers)]))
 
 
 def test_rows_nobody_serves_come_back_empty():
