@@ -592,7 +592,10 @@ __device__ void merge_long_rows(const MergeArgs& a, int n_rows, int finders, int
   }
 }
 
-template <typename E>
+// kRuns: runs of 1024 floats a pass takes, no more than a row has: the runs of a narrower row would all repeat its
+// last piece, loads and exponentials included.  2517 rows of 1024 floats 14.3 us with four runs, 8.1 with one (a wave
+// per (row, head): 11.9), of 2048 floats 14.6 -> 12.1, of 512 floats 9.7 -> 6.2, 1200 fp32 rows of 1024 11.9 -> 6.5.
+template <typename E, int kRuns>
 __global__ __launch_bounds__(256, 4) void merge_rows_kernel(MergeArgs a, int n_rows, int finders) {
   using S = typename E::storage;
   typedef const __attribute__((address_space(4))) int32_t* Words;
@@ -614,7 +617,7 @@ __global__ __launch_bounds__(256, 4) void merge_rows_kernel(MergeArgs a, int n_r
   }
   const int begin = ((Words)a.row_indptr)[row], end = ((Words)a.row_indptr)[row + 1];
   if (end - begin > kFewStates) return;  // a finder's
-  constexpr int kRuns = 4;  // runs of 1024 floats per pass
+  constexpr int kAtOnce = kRuns == 4 ? 2 : 4;  // states in flight together
   for (int base = 4 * threadIdx.x; base < width; base += kRuns * 1024) {
     int at[kRuns];
     float m[kRuns], l[kRuns];
@@ -654,7 +657,11 @@ __global__ __launch_bounds__(256, 4) void merge_rows_kernel(MergeArgs a, int n_r
         }
     };
     int i = begin;
-    for (; i + 2 <= end; i += 2) fold(i, std::integral_constant<int, 2>{});
+    for (; i + kAtOnce <= end; i += kAtOnce) fold(i, std::integral_constant<int, kAtOnce>{});
+    if (kAtOnce > 2 && i + 2 <= end) {
+      fold(i, std::integral_constant<int, 2>{});
+      i += 2;
+    }
     if (i < end) fold(i, std::integral_constant<int, 1>{});
 #pragma unroll
     for (int k = 0; k < kRuns; ++k) {
@@ -707,10 +714,18 @@ int launch_merge(const MergeArgs& a, int n_rows, int waves, hipStream_t stream) 
   // compute unit in all, and sixteen rows to look through each, that they start in a microsecond or less.
   const int finders = std::max(1, std::min({64, 1024 / a.num_q_heads, n_rows / 16}));
   switch (waves) {
-    case 1:
-      hipLaunchKernelGGL((merge_rows_kernel<E>), dim3((unsigned)(n_rows + finders * a.num_q_heads)), dim3(256), 0,
-                         stream, a, n_rows, finders);
+    case 1: {
+      const dim3 blocks((unsigned)(n_rows + finders * a.num_q_heads)), threads(256);
+      const int width = a.num_q_heads * a.head_dim;
+      if (width <= 1024) {
+        hipLaunchKernelGGL((merge_rows_kernel<E, 1>), blocks, threads, 0, stream, a, n_rows, finders);
+      } else if (width <= 2048) {
+        hipLaunchKernelGGL((merge_rows_kernel<E, 2>), blocks, threads, 0, stream, a, n_rows, finders);
+      } else {
+        hipLaunchKernelGGL((merge_rows_kernel<E, 4>), blocks, threads, 0, stream, a, n_rows, finders);
+      }
       break;
+    }
     case 4:
       hipLaunchKernelGGL((merge_kernel<E, 4>), grid, dim3(256), 0, stream, a);
       break;

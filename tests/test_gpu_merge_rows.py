@@ -1,7 +1,7 @@
 """Merge of many rows (8192 (row, head) pairs and more): one workgroup per row, four floats a thread of every 1024 of
-a row's [heads * dims] states.  Row widths below, at and past a pass of 4096 floats, and no multiple of 1024; rows
-of several states, rows of so many that they are found and merged head by head, rows an item writes itself and (a
-fixed plan) rows nobody serves."""
+a row's [heads * dims] states, one, two or four runs of 1024 a pass.  Row widths at and past each of these, and no
+multiple of 1024; rows of several states, rows of so many that they are found and merged head by head, rows an item
+writes itself and (a fixed plan) rows nobody serves."""
 
 from types import SimpleNamespace
 
@@ -38,6 +38,7 @@ def setup(dtype, heads, new, lengths, seed=3):
 
 @pytest.mark.parametrize("dtype,heads,new", [
     (torch.bfloat16, (16, 4, 64), (513, 3)),     # 1024 floats a row
+    (torch.float16, (16, 4, 128), (500, 40)),    # 2048
     (torch.float16, (32, 8, 128), (200, 60)),    # 4096
     (torch.bfloat16, (24, 6, 256), (345,)),      # 6144: a second, half-filled pass
 ])
