@@ -713,6 +713,9 @@ int launch_merge(const MergeArgs& a, int n_rows, int waves, hipStream_t stream) 
   // Finders of long rows: up to 64 a head, that a batch of decode rows spreads over them; at most four workgroups a
   // compute unit in all, and sixteen rows to look through each, that they start in a microsecond or less.
   const int finders = std::max(1, std::min({64, 1024 / a.num_q_heads, n_rows / 16}));
+  // The row kernel moves four elements at a time; buffers of a caller's that are only aligned to an element (with
+  // the vector-ALU kernel nothing else asks for more) go element by element.
+  if (waves == 1 && ((uintptr_t)a.out % (4 * sizeof(typename E::storage)) || (uintptr_t)a.part_acc % 16)) waves = 4;
   switch (waves) {
     case 1: {
       const dim3 blocks((unsigned)(n_rows + finders * a.num_q_heads)), threads(256);

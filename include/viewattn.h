@@ -299,6 +299,9 @@ VA_API int va_copy_shift_kv(void* k_pool_dev, void* v_pool_dev, int64_t pool_row
  * plan_dev / kv_indices_dev / sub_worker_dev are device copies of the host
  * tables the plan was built from.  Rows no sub-request serves get out = 0 and
  * lse = -inf.  workspace_dev must hold counts.workspace_bytes.
+ * Alignment: pool rows start on 16-byte boundaries; with the matrix-core kernels
+ * (16-bit types) so do q rows, out and workspace_dev, with the vector-ALU kernel
+ * these need the alignment of an element only.
  */
 VA_API int va_attention(const void* q_dev, int64_t q_row_stride, const void* k_pool_dev,
                  const void* v_pool_dev, int64_t pool_row_stride, const int32_t* plan_dev,

@@ -96,6 +96,31 @@ def test_few_long_rows_among_many(dtype, heads, workers, blocks_of):
     assert torch.equal((indptr[1:] - indptr[:-1]) > 8, torch.tensor([blocks_of(w) > 8 for w in range(workers)]))
 
 
+@pytest.mark.parametrize("out_offset,workspace_offset", [(1, 0), (0, 1), (3, 2)])
+def test_buffers_aligned_to_an_element(out_offset, workspace_offset):
+    heads, workers, page, dtype = (8, 2, 64), 1030, 16, torch.float32
+    op, cpu_pool, dev_pool, gen = make_op_and_pool(DEV, dtype, heads, page, 2 * workers, 1e6, seed=9, max_pos=512)
+    blocks = []
+    for w in range(workers):
+        blocks.append(CacheBlock(DEV, page))
+        blocks[-1].grow_pages(torch.tensor([w * page]), 1 + w % 15)
+    views = [[blocks[0], b] if w % 2 else [b] for w, b in enumerate(blocks)]
+    group = WorkerGroup(cache_structure=views, write_to=[v[-1] for v in views])
+    fresh = SimpleNamespace(alloc_pages=lambda n: torch.arange(workers, workers + n, dtype=torch.int32) * page)
+    *_, meta = run_decode_parity(op, cpu_pool, dev_pool, group, fresh, 1e6, gen)
+    assert meta.launch.header[MERGE_WORD] == 1
+    width = heads[0] * heads[2]
+    q = torch.randn(workers, width, generator=gen).to(DEV)
+    expected = op.attend(q, 0, meta).cpu()
+    out = torch.full((workers * width + 8,), 7.0, device=DEV)
+    used = meta.launch.counts.workspace_bytes
+    room = torch.zeros(used + 64, dtype=torch.uint8, device=DEV)
+    meta.launch.workspace = room[4 * workspace_offset:][:used]
+    op.attend(q, 0, meta, out=out[out_offset:][:workers * width].view(workers, width))
+    assert_close(out[out_offset:][:workers * width].view(workers, width), expected, dtype, "out")
+    assert (out[:out_offset] == 7).all() and (out[out_offset + workers * width:] == 7).all()
+
+
 def test_rows_nobody_serves_come_back_empty():
     heads, new = (32, 8, 128), (130, 20)
     op, cpu_pool, dev_pool, gen, specs = setup(torch.bfloat16, heads, new, (900, 333))
