@@ -852,14 +852,14 @@ void fill_counts(const Built& b, const VaSubRequests* s, const VaShape* shape, V
 
 }  // namespace
 
-// The plan of fine cuts, unless only that of coarse ones leaves room in `workspace_bytes` (<= 0: no limit).
+// The plan of fine cuts, unless only that of coarse ones leaves room in `workspace_bytes` (< 0: no limit).
 static int build_within(const VaSubRequests* subs, const VaShape* shape, const VaPlanParams* params,
                         int64_t workspace_bytes, Built& out) {
   const int rc = build(subs, shape, params, out);
   auto fits = [&](const Built& plan) {
     return va_workspace_bytes_for(plan.n_partials, shape->num_q_heads, shape->head_dim) <= workspace_bytes;
   };
-  if (rc || workspace_bytes <= 0 || fits(out)) return rc;
+  if (rc || workspace_bytes < 0 || fits(out)) return rc;
   Built coarse;
   Cuts cuts;
   cuts.fine = false;

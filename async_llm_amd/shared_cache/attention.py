@@ -279,7 +279,7 @@ class SharedCacheAttention:
     # ------------------------------------------------------------------
     def _plan_into_scratch(self, subs, counts) -> np.ndarray:
         """Plan into the op's host scratch (grown on demand), within the workspace once that is fixed."""
-        limit = self._workspace.numel() if self._workspace_prepared and self._workspace is not None else 0
+        limit = self._workspace.numel() if self._workspace_prepared else -1  # (an arena of no bytes is a limit too)
         scratch = self._plan_scratch
         rc = native.lib.va_plan_build_within(subs, self._shape, self.plan_params, limit, scratch.ctypes.data,
                                              scratch.size, counts)

@@ -198,7 +198,7 @@ VA_API int va_plan_build(const VaSubRequests* subs, const VaShape* shape, const 
                   int32_t* plan_host, int64_t plan_capacity_words, VaPlanCounts* counts);
 
 /*
- * The same for a caller whose workspace is fixed at `workspace_bytes` (<= 0: it is not).  The walks of
+ * The same for a caller whose workspace is fixed at `workspace_bytes` (negative: it is not).  The walks of
  * prefill tiles are cut finely as a rule, which balances small launches at the price of more
  * partial states; a plan whose states would not fit is cut coarsely instead, if those fit.
  * va_plan_build and va_plan_count go by VA_STATIC_SCRATCH_BYTES, the array of va_attention_static.

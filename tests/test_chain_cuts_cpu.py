@@ -64,11 +64,15 @@ def _plan_within(tables, limit):
     return counts.workspace_bytes
 
 
-def test_fixed_workspace_gets_coarse_cuts_only_where_they_help():
-    tables = _tables([(58, 40, [700, 300])], 16)
-    fine = _plan_within(tables, 0)
+@pytest.mark.parametrize("requests,least", [
+    ([(58, 40, [700, 300])], 1),
+    ([(1, 600, [])], 0),  # coarse cuts leave the row whole: no partial state, no workspace
+])
+def test_fixed_workspace_gets_coarse_cuts_only_where_they_help(requests, least):
+    tables = _tables(requests, 16)
+    fine = _plan_within(tables, -1)
     coarse = _plan_within(tables, fine - 1)
-    assert coarse < fine
+    assert least <= coarse < fine and (coarse == 0) == (least == 0)
     assert _plan_within(tables, fine) == fine and _plan_within(tables, coarse) == coarse
     if coarse:
-        assert _plan_within(tables, coarse - 1) == fine  # neither fits: the caller is told what the plan needs
+        assert _plan_within(tables, 0) == _plan_within(tables, coarse - 1) == fine  # neither fits: the caller is told
