@@ -150,16 +150,11 @@ class ViewAttnBackend(BaseAttnBackend):
         n_rows = int(qo[-1])
         sub_worker_host = np.arange(n_rows, dtype=np.int64)
         subs = self._subs(qo, kv, lens, flags, chain, sub_worker_host)
-        counts = native.VaPlanCounts()
-        scratch = op._plan_into_scratch(subs, counts)
-        host = torch.empty(counts.plan_words, dtype=torch.int32, pin_memory=True)
-        host.numpy()[:] = scratch[: counts.plan_words]
-        blob = host.to(self.device, non_blocking=True)
         indices = torch.cat([self.page_table[req.table_idx, : req.device_len] for req in reqs]).to(torch.int32)
         cu_q = torch.from_numpy(qo)
         cu_q_pinned = cu_q.pin_memory()
-        launch = LaunchPlan(host[: native.PLAN_HEADER_WORDS].numpy().copy(), blob, indices, counts,
-                            op._ensure_workspace(counts.workspace_bytes))
+        refs = [cu_q_pinned]
+        launch = op._upload_plan(subs, indices, refs)
         batch.attn_metadata = ViewAttnMetadata(
             cu_seqlens_q_cpu=cu_q, cu_seqlens_k_cpu=torch.from_numpy(kv),
             cu_seqlens_q_gpu=cu_q_pinned.to(self.device, non_blocking=True), indices=indices,
@@ -167,7 +162,7 @@ class ViewAttnBackend(BaseAttnBackend):
             head_dim=op.head_dim, page_size=1, dtype=op.dtype,
             sub_worker=torch.arange(n_rows, dtype=torch.int64, device=self.device),
             sub_loc=torch.zeros(n_rows, dtype=torch.int64, device=self.device), launch=launch,
-            _refs=(host, cu_q_pinned))
+            _refs=tuple(refs))
 
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layer_id: int, batch) -> torch.Tensor:
         """Store the new K/V rows at ``batch.out_loc`` and attend (reference

@@ -54,6 +54,11 @@ class LaunchPlan:
     kv_indices: torch.Tensor  # int32 device
     counts: native.VaPlanCounts
     workspace: Optional[torch.Tensor]
+    # a plan whose partial states do not fit the library's own scratch array: its tables, the pinned copy of ``blob``
+    # (both with room for a second plan) and that second plan, of coarser cuts, once a call has asked for it
+    subs: Optional[native.VaSubRequests] = None
+    staging: Optional[torch.Tensor] = None
+    coarse: Optional["LaunchPlan"] = None
 
 
 @dataclass
@@ -303,17 +308,53 @@ class SharedCacheAttention:
             arrays[0].ctypes.data, arrays[1].ctypes.data, arrays[2].ctypes.data if arrays[2].size else None,
             arrays[3].ctypes.data, arrays[4].ctypes.data, arrays[5].ctypes.data,
             sw.ctypes.data if sw.size else None)
-        # one pass of the planner: build into a scratch that is normally large enough, then copy
-        # the blob to pinned staging of its exact size
+        subs._keepalive = (arrays, sw)
+        return self._upload_plan(subs, kv_indices_dev, refs)
+
+    def _upload_plan(self, subs, kv_indices_dev: torch.Tensor, refs: list) -> LaunchPlan:
+        """One pass of the planner: build into a scratch that is normally large enough, then copy
+        the blob to pinned staging of its exact size (twice that where ``attend`` may need a second plan)."""
         counts = native.VaPlanCounts()
         scratch = self._plan_into_scratch(subs, counts)
-        pin = self.device.type == "cuda"
-        host = torch.empty(counts.plan_words, dtype=torch.int32, pin_memory=pin)
-        host.numpy()[:] = scratch[: counts.plan_words]
-        blob = host.to(self.device, non_blocking=True)
+        words = counts.plan_words
+        roomy = counts.workspace_bytes > native.STATIC_SCRATCH_BYTES
+        host = torch.empty(2 * words if roomy else words, dtype=torch.int32, pin_memory=self.device.type == "cuda")
+        host.numpy()[:words] = scratch[:words]
+        if roomy:
+            blob = torch.empty(2 * words, dtype=torch.int32, device=self.device)
+            blob[:words].copy_(host[:words], non_blocking=True)
+        else:
+            blob = host.to(self.device, non_blocking=True)
         refs.extend((host, blob))
         header = host[: native.PLAN_HEADER_WORDS].numpy().copy()
-        return LaunchPlan(header, blob, kv_indices_dev, counts, self._ensure_workspace(counts.workspace_bytes))
+        launch = LaunchPlan(header, blob, kv_indices_dev, counts, self._ensure_workspace(counts.workspace_bytes))
+        if roomy:
+            launch.subs, launch.staging = subs, host
+        return launch
+
+    def _within_static_scratch(self, launch: LaunchPlan) -> LaunchPlan:
+        """The launch as ``va_attention_static`` can run it.  Plans are cut as finely as a workspace that
+        grows allows; where their states exceed the library's array and those of coarser cuts fit, the tables are
+        planned once more, behind the first plan (nothing is allocated on the device).  The copy is waited for,
+        so that later calls may come from any stream; under capture it is recorded with the launch instead."""
+        if launch.subs is None:
+            return launch
+        at, capturing = launch.counts.plan_words, torch.cuda.is_current_stream_capturing()
+        if launch.coarse is None or capturing:
+            counts, words = native.VaPlanCounts(), np.empty(at, dtype=np.int32)
+            rc = native.lib.va_plan_build_within(launch.subs, self._shape, self.plan_params, native.STATIC_SCRATCH_BYTES,
+                                                 words.ctypes.data, at, counts)
+            if rc != 0 or counts.workspace_bytes > native.STATIC_SCRATCH_BYTES:
+                return launch  # refused by the call, with the bytes it needs
+            n = counts.plan_words
+            launch.staging.numpy()[at: at + n] = words[:n]
+            blob = launch.blob[at: at + n]
+            blob.copy_(launch.staging[at: at + n], non_blocking=capturing)
+            coarse = LaunchPlan(words[: native.PLAN_HEADER_WORDS], blob, launch.kv_indices, counts, None)
+            if capturing:
+                return coarse
+            launch.coarse = coarse
+        return launch.coarse
 
     def _walk_decode(self, group, new_page_for_block, new_token_slots):
         """Sub-requests of one decode step: per worker one paged sub-request per
@@ -703,6 +744,8 @@ class SharedCacheAttention:
         native.require_device(q, "q")
         launch = meta.launch
         assert launch is not None, "metadata carries no launch plan"
+        if static_scratch:
+            launch = self._within_static_scratch(launch)
         W, Hq, D = meta.num_workers, self.num_qo_heads, self.head_dim
         q2 = q.reshape(q.shape[0], Hq * D)
         if q2.stride(-1) != 1:

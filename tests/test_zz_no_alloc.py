@@ -2,12 +2,15 @@
 the same plan, the same kernels, the partial states in the library's own per-GPU array instead
 of a caller's workspace.  Results must be identical bit for bit, on two calls in a row of which
 the second is smaller (the array keeps the first call's contents), and a plan whose partial
-states exceed the array must be refused with a clear error."""
+states exceed the array must be refused with a clear error -- but for one that exceeds it by its
+fine cuts only, which the call plans anew with coarse ones."""
 
 import pytest
 import torch
 
 from async_llm_amd import native, workloads
+from async_llm_amd.shared_cache import CacheBlock, PrefillSpec
+from tests.util import assert_close, make_op_and_pool, run_prefill_parity
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda")
@@ -62,3 +65,50 @@ def test_static_scratch_refuses_a_plan_that_does_not_fit():
         op.attend(wl.q, 0, meta, out=out, static_scratch=True)
     op.attend(wl.q, 0, meta, out=out)  # the workspace path takes it
     torch.cuda.synchronize()
+
+
+def _cut_finely(heads, new, context):
+    """A prefill whose fine cuts leave too many partial states for the array, and its coarse ones not."""
+    page, total = 16, -(-new // 16) + -(-context // 16)
+    op, cpu_pool, dev_pool, gen = make_op_and_pool(DEV, torch.bfloat16, heads, page, total, 1e6, seed=new, scale=0.5)
+    blocks = []
+    if context:
+        blocks.append(CacheBlock(DEV, page))
+        blocks[0].grow_pages(torch.arange(-(-context // page)) * page, context)
+    specs = [PrefillSpec(blocks, torch.arange(-(-context // page), total, dtype=torch.int32) * page, new)]
+    *_, meta = run_prefill_parity(op, cpu_pool, dev_pool, specs, 1e6, gen, scale=0.5)
+    assert meta.launch.counts.workspace_bytes > native.STATIC_SCRATCH_BYTES
+    q = torch.randn(new, heads[0] * heads[2], generator=gen).to(op.dtype).to(DEV)
+    return op, meta, q, op.attend(q, 0, meta, return_lse=True)
+
+
+@pytest.mark.parametrize("heads,new,context", [((32, 8, 128), 1500, 0), ((16, 4, 256), 800, 1000)])
+def test_static_scratch_takes_what_coarser_cuts_fit(heads, new, context):
+    op, meta, q, (want, want_lse) = _cut_finely(heads, new, context)
+    out, lse = torch.full_like(want, float("nan")), torch.full_like(want_lse, float("nan"))
+    for _ in range(2):
+        op.attend(q, 0, meta, return_lse=True, out=out, lse=lse, static_scratch=True)
+        assert_close(out, want.float(), op.dtype, "out")
+        assert_close(lse, want_lse, op.dtype, "lse")
+        out.fill_(float("nan"))
+        lse.fill_(float("nan"))
+    again = op.attend(q, 0, meta)  # the first plan is untouched
+    assert torch.equal(again, want)
+
+
+def test_static_scratch_takes_them_under_capture():
+    op, meta, q, (want, want_lse) = _cut_finely((32, 8, 128), 1000, 500)
+    out, lse = torch.empty_like(want), torch.empty_like(want_lse)
+    other = op.attend(q, 0, meta)  # (loads the kernels)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        op.attend(q, 0, meta, return_lse=True, out=out, lse=lse, static_scratch=True)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        lse.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_close(out, want.float(), op.dtype, "out")
+        assert_close(lse, want_lse, op.dtype, "lse")
+        assert torch.equal(op.attend(q, 0, meta), other)
