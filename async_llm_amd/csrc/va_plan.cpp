@@ -1117,8 +1117,15 @@ extern "C" int va_plan_build_fixed(const VaSubRequests* subs, const VaShape* sha
   if (!plan_host || !cap) return va_fail(VA_ERR_ARG, "null plan buffer or capacity");
   if (cap->max_items % kXcds || cap->max_wide_items % kXcds || cap->max_items < 0 || cap->max_wide_items < 0)
     return va_fail(VA_ERR_ARG, "capacity: item counts must be non-negative multiples of 8");
-  Built b;
-  int rc = build(subs, shape, params, b, cap);
-  if (rc) return rc;
-  return write_plan(b, subs, shape, cap, plan_host, plan_capacity_words, counts);
+  // (a capacity of the caller's own may hold the plan of coarse cuts only)
+  int rc = VA_OK;
+  for (const bool fine : {true, false}) {
+    Built b;
+    Cuts cuts;
+    cuts.fine = fine;
+    rc = build(subs, shape, params, b, cap, cuts);
+    if (rc == VA_OK) rc = write_plan(b, subs, shape, cap, plan_host, plan_capacity_words, counts);
+    if (rc != VA_ERR_CAPACITY || plan_capacity_words < va_plan_fixed_words(cap)) break;
+  }
+  return rc;
 }

@@ -65,6 +65,20 @@ def test_fixed_plans_share_one_header_and_cover_every_pair_once(prefill, kernel,
     assert all(np.array_equal(h, headers[0]) for h in headers)
 
 
+def test_a_capacity_of_coarse_cuts_takes_a_plan_of_coarse_cuts():
+    # one row over 601 tokens of its own: whole under coarse cuts, several pieces and their states under fine ones
+    tables = [0, 1], [0, 38], list(range(38)), [601], [native.VA_SUB_CAUSAL], [0], [0], 1
+    own = native.VaPlanCapacity(8, 0, 1, 0, 0, 0, 1)  # items, wide items, links, query references, states, row parts, rows
+    rc, blob, counts, _ = fixed_plan(tables, None, heads=(16, 4, 256), page=16, kernel=native.VA_KERNEL_MFMA, capacity=own)
+    assert rc == 0, native.lib.va_last_error()
+    check_coverage(blob, *tables[:2], *tables[3:5], tables[6], tables[7], fixed=True)
+    roomy = native.VaPlanLimits(0, 0, 1, 1, 1, 1)
+    rc, blob, *_ = fixed_plan(tables, roomy, heads=(16, 4, 256), page=16, kernel=native.VA_KERNEL_MFMA)
+    assert rc == 0 and sum(1 for item in decode_plan(blob)[1] if item[2] > 0) > 1
+    own.max_rows = 0
+    assert fixed_plan(tables, None, heads=(16, 4, 256), page=16, capacity=own)[0] == native.VA_ERR_CAPACITY
+
+
 @pytest.mark.parametrize("heads", [(16, 4, 256), (4, 2, 64), (8, 8, 128), (4, 1, 64)])
 def test_capacity_holds_chains_packed_in_bundles(heads):
     """Prefill chunks of a few wide tiles over views of several thousand tokens: the planner packs
