@@ -15,14 +15,15 @@ pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda")
 
 
-@pytest.mark.parametrize("heads", [(16, 4, 64), (8, 2, 128), (16, 4, 256)])
+@pytest.mark.parametrize("dtype,heads", [(torch.bfloat16, (16, 4, 64)), (torch.bfloat16, (8, 2, 128)),
+                                         (torch.bfloat16, (16, 4, 256)), (torch.float16, (16, 4, 256))])
 @pytest.mark.parametrize("page", [1, 2, 8, 24])
-def test_walks_around_the_index_ring_periods(page, heads):
+def test_walks_around_the_index_ring_periods(page, dtype, heads):
     lengths = (1, 15, 16, 17, 31, 32, 33, 47, 49, 63, 64, 65, 79, 81, 112, 127, 128, 129, 144, 191, 193, 255, 257, 1000)
     print(f"page {page} heads {heads}", flush=True)
     total = sum(-(-k // page) for k in lengths)
-    op, cpu_pool, dev_pool, gen = make_op_and_pool(DEV, torch.bfloat16, heads, page, total + 2 * len(lengths), 1e6,
-                                                   seed=page, scale=0.5, max_pos=4096)
+    op, cpu_pool, dev_pool, gen = make_op_and_pool(DEV, dtype, heads, page, total + 2 * len(lengths), 1e6, seed=page,
+                                                   scale=0.5, kernel="mfma", max_pos=4096)
     order = torch.randperm(total + 2 * len(lengths), generator=gen).to(torch.int32) * page
     blocks, at = [], 0
     for k in lengths:
@@ -39,4 +40,5 @@ def test_walks_around_the_index_ring_periods(page, heads):
     spare = iter(order[at:].split(1))
     allocator = SimpleNamespace(alloc_pages=lambda n: torch.cat([next(spare) for _ in range(n)]))
     group = WorkerGroup(cache_structure=views, write_to=targets)
-    run_decode_parity(op, cpu_pool, dev_pool, group, allocator, 1e6, gen)
+    *_, meta = run_decode_parity(op, cpu_pool, dev_pool, group, allocator, 1e6, gen)
+    assert meta.launch.counts.n_wide_items == 0 < meta.launch.counts.n_items  # the streaming kernel's

@@ -18,16 +18,20 @@ def widths(d):
 
 
 @pytest.mark.parametrize("mrope", [False, True])
-@pytest.mark.parametrize("heads", [(4, 4, 64), (16, 2, 64), (3, 1, 128), (8, 2, 128), (4, 4, 256), (16, 4, 256)])
-def test_wide_tiles_rotate_every_width(heads, mrope):
+@pytest.mark.parametrize("dtype,heads", [
+    (torch.bfloat16, (4, 4, 64)), (torch.float16, (16, 2, 64)), (torch.bfloat16, (16, 1, 128)),
+    (torch.float16, (8, 2, 128)), (torch.bfloat16, (8, 2, 128)), (torch.float16, (4, 4, 256)),
+    (torch.bfloat16, (16, 4, 256)), (torch.float16, (16, 1, 256)),
+])
+def test_wide_tiles_rotate_every_width(dtype, heads, mrope):
     d, page = heads[2], 16
     for rotary in widths(d):
         if mrope and rotary == 0:
             continue
-        print(f"rotary {rotary} heads {heads} mrope {mrope}", flush=True)
+        print(f"rotary {rotary} heads {heads} mrope {mrope} {dtype}", flush=True)
         section = (rotary // 2 - 2 * (rotary // 6), rotary // 6, rotary // 6) if mrope else None
-        op, cpu_pool, dev_pool, gen = make_op_and_pool(DEV, torch.bfloat16, heads, page, 40, 1e6, rotary_dim=rotary,
-                                                       mrope_section=section, seed=rotary, scale=0.5, max_pos=1024)
+        op, cpu_pool, dev_pool, gen = make_op_and_pool(DEV, dtype, heads, page, 40, 1e6, rotary_dim=rotary, mrope_section=section,
+                                                       seed=rotary, scale=0.5, kernel="mfma", max_pos=1024)
         context = []
         for first, length in ((0, 75), (5, 32)):
             b = CacheBlock(DEV, page)
@@ -41,4 +45,5 @@ def test_wide_tiles_rotate_every_width(heads, mrope):
             p = torch.arange(new)
             rel = torch.stack([p // 9, p // 3, p % 5]) if mrope and w != 1 else None
             specs.append(PrefillSpec(context[:2 - w % 2], pages, new, prefix, 50000 + prefix if mrope else prefix, rel))
-        run_prefill_parity(op, cpu_pool, dev_pool, specs, 1e6, gen, scale=0.5)
+        *_, meta = run_prefill_parity(op, cpu_pool, dev_pool, specs, 1e6, gen, scale=0.5)
+        assert meta.launch.counts.n_wide_items > 0
