@@ -203,8 +203,8 @@ __global__ __launch_bounds__(kStreamThreads, StreamShape<kD>::kMinBlocks) void a
     // kGather.  Looked up by the lanes in front of each request, the entries cost a trip to memory per tile and
     // the compiler's wait for it drained the ring (32 requests of 100..8000 token slots, 32 q / 8 kv heads of 128
     // dims, bf16: 124.7 us a layer; 92.7 us = 5.7 TB/s this way).  So they travel like the tiles do: one wave-level load brings a
-    // wave's entries of four tiles to LDS, five to eight tiles ahead of their requests, and an iteration reads
-    // those of the tile it requests beside its K.
+    // wave's entries of four tiles to LDS, 8 - kBuffers to 11 - kBuffers iterations ahead of their requests, and an
+    // iteration reads those of the tile it requests beside its K.
     const int g_shift = slots ? 0 : p_shift, g_mask = slots ? 0 : P - 1;
     auto token_of = [&](int i, int row) __attribute__((always_inline)) { return min(tok_begin + i * kStreamTok + row, t_last); };
     auto entry_of = [&](int t) __attribute__((always_inline)) {
@@ -260,7 +260,10 @@ __global__ __launch_bounds__(kStreamThreads, StreamShape<kD>::kMinBlocks) void a
 
     // ---- set-up: first tiles on their way, then the query tile ----
     __syncthreads();  // every wave is done with the previous link's buffers
-    Slots first[kBuffers];  // gather: rows of the first tiles, looked up in one trip
+    // gather: rows of the first tiles.  All their entries are requested together, but the compiler turns those of a
+    // later tile into rows behind the requests of the tiles before it, and waits for these with them; at 256 dims
+    // the set-up also spills 36 bytes a lane (the tile loop does not)
+    Slots first[kBuffers];
 #pragma unroll
     for (int i = 0; i < kBuffers; ++i)
 #pragma unroll

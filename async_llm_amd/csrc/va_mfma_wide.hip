@@ -22,11 +22,12 @@
 // under the exponentials of tile i (each taken of scale * score - reference, formed in fp32 right
 // in front of it), the products of tile i under the maxima of tile i + 1.  Interior tiles of a link
 // take a branch-free ring step, in a loop of their own.
-// V tiles and the staged query tile keep whole rows in LDS, unpadded and swizzled (piece c of row r
-// at position c ^ swz(r)); K tiles land in fragment order (8-token x 128-byte blocks, see the load
-// pattern in the kernel), so that the K reads of a tile share one address register.  The query tile
-// is rotated by all 256 threads, one row block of every wave (128 rows) at a time, into the two
-// ring buffers that are not yet in use.
+// V tiles keep whole rows in LDS, unpadded and swizzled (piece c of row r at position c ^ swz(r)); K
+// tiles land in fragment order (8-token x 128-byte blocks, see the load pattern in the kernel), so
+// that the K reads of a tile share one address register.  The query never goes through LDS: every
+// lane loads its own rows in operand order and rotates them in registers, once per link.  Only the
+// cosines and sines of an mRoPE tile pass through the ring buffers that are not yet in use (past the
+// end of the ring at head dims under 256), and the pieces of rotary widths that no operand fits.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -280,8 +281,8 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     // Slot lists and pages under 16 tokens (kGather): looked up by the lanes in front of each request, the
     // entries cost a trip to memory per tile and drain the ring (6 requests of 60..4096 tokens over slot
     // lists, 32 q / 8 kv heads of 128 dims: 734 us a layer).  So they travel like the tiles do: one
-    // wave-level load brings a wave's entries of four tiles to LDS, four to eight tiles ahead, and a ring
-    // step reads the entries of the tile the NEXT step requests.
+    // wave-level load brings a wave's entries of four tiles to LDS, two to five ring steps ahead of their
+    // requests, and a ring step reads the entries of the tile the NEXT step requests.
     const char* wave_pool = (const char*)(wave_is_v ? vp : kp);
     const char* wave_plain = wave_pool - kLoadBias;  // base of plain loads: the per-lane offsets carry the bias
     const uint32_t wave_lds = __builtin_amdgcn_readfirstlane(lds_address(lds)) + (wave_is_v ? Sh::kTileBytes : 0) +
@@ -379,7 +380,9 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     // with the table, 21 200 under mRoPE; 11 900 and 13 300 like this).  What bounds it now is the L1's rate
     // for 64 KB of query pieces at 16 bytes a row and the table entries.  Positions, query rows and the page
     // numbers of the first tiles are requested together, ahead of the barrier; the tiles and the table entries,
-    // which need them, behind it.
+    // which need them, behind it.  (Not so the index entries of scattered rows: those of V rows past the first
+    // two are a case of the V waves' own, and the compiler waits for each of them, and for the query rows
+    // before it, in turn.)
     va_u32x4 qf[kB][kSteps];  // B operands: row of block b, dims [16s + 8h, +8)
     uint32_t* turns = (uint32_t*)(lds + kWideAhead * Sh::kBufferBytes);
     const int half = a.rope.half, half_steps = a.rope.rotary_dim % 32 == 0 ? a.rope.rotary_dim / 32 : -1;
@@ -430,8 +433,8 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     if (!table && in_turn) {
       // mRoPE: the cosines and sines of the tile's positions, each taken once and shared by the G query
       // heads of a row (an entry is cos | sin in the element type, as the rotation rounds them).  A thread
-      // keeps to one row; the lanes of a wave work on few pair dims, so that the long argument reduction
-      // of the fast turning ones stays out of most waves.
+      // keeps to one row, so that its positions are loaded once, and the lanes of a wave to few pair dims, so
+      // that their frequencies are a broadcast.
       const float axes[3] = {(float)pos[0], (float)pos[1], (float)pos[2]};
       const int first = tid / turn_lanes, step = kWideThreads / turn_lanes;
       if (turn_iq < n_q) {

@@ -102,9 +102,9 @@ inline int32_t visible_end(int32_t len, int32_t nq, bool causal, int32_t b) {
 // walked tokens decides what a cut is worth; the floors keep the pieces of small launches worth their
 // launch.  The fine cuts are the rule: a chunk of 333 tokens over four blocks (16 q / 4 kv heads of 256 dims) used
 // 44 % of the machine under floors of 1024 tokens, whose longest slot walked 1700 tokens where an even share is
-// 620.  Measured, kernels of one layer, coarse -> fine: that chunk 81 -> 72 us; 4 chunks of 300..1500
-// tokens at 32 q / 8 kv heads of 128 dims 654 -> 604 us; plain prefill of 6 requests, whose launch of narrow tiles was
-// ONE row walking 1363 tokens, 433 -> 364 us; two chunks of 60 tokens 102 -> 54 us.
+// 620.  Measured, attention and merge of one layer, coarse -> fine: that chunk 79 -> 69 us; 4 chunks of 300..1500
+// tokens at 32 q / 8 kv heads of 128 dims 720 -> 704 us; plain prefill of 6 requests, whose launch of narrow tiles was
+// ONE row walking 1363 tokens, 454 -> 404 us; two chunks of 60 tokens over 2100 tokens each 51 -> 41 us.
 // Charging a set-up: at head_dim 256, where a tile is 128 rows, 640 and 384 tokens differ by under 4 % either way;
 // at 64 and 128 (256 rows, twice the work per token) 384 is the better by up to 15 % (drawn chunk batches).
 // Finer cuts leave more partial states, so the coarse ones remain for callers whose scratch holds no more.
