@@ -487,9 +487,9 @@ __device__ __forceinline__ void merge_row_head(const MergeArgs& a, long long row
     for (int u = 0; u < n; ++u) {
       const float m_new = fmaxf(mm, mp[u]);
       const float sa = exp2f(mm - m_new), sb = exp2f(mp[u] - m_new);
-      ll = ll * sa + lp[u] * sb;
+      ll = fmaf(ll, sa, lp[u] * sb);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) av[k] = av[k] * sa + ap[u][k] * sb;
+      for (int k = 0; k < 4; ++k) av[k] = fmaf(ap[u][k], sb, av[k] * sa);
       mm = m_new;
     }
   };
@@ -525,9 +525,9 @@ __device__ __forceinline__ void merge_row_head(const MergeArgs& a, long long row
     const float mw = s_ml[w][0], lw = s_ml[w][1];
     const float m_new = fmaxf(mm, mw);
     const float sa = exp2f(mm - m_new), sb = exp2f(mw - m_new);
-    ll = ll * sa + lw * sb;
+    ll = fmaf(ll, sa, lw * sb);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) av[k] = av[k] * sa + s_av[w][k][lane] * sb;
+    for (int k = 0; k < 4; ++k) av[k] = fmaf(av[k], sa, s_av[w][k][lane] * sb);
     mm = m_new;
   }
 #pragma unroll
