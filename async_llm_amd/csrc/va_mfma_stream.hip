@@ -59,7 +59,6 @@ struct StreamShape {
   // Behind the ring, for every wave its own: the index entries of eight tiles (two wave-level loads), see `gather`.
   static constexpr int kIndexBytes = 2 * kWave * 4;
   static constexpr int lds_bytes(bool gather) { return kRingBytes + (gather ? kStreamWaves * kIndexBytes : 0); }
-  static_assert(kBuffers <= 4, "the entries of a tile are read four tiles after they were requested");
   static_assert(kLoadsPerWave >= 1 && kRun >= 2 && kRun <= 4, "unsupported head_dim");
 };
 
@@ -86,6 +85,7 @@ template <typename E, int kD, bool kGather>
 __global__ __launch_bounds__(kStreamThreads, StreamShape<kD>::kMinBlocks) void attn_stream_kernel(AttnArgs a) {
   using S = typename E::storage;
   using Sh = StreamShape<kD>;
+  static_assert(!kGather || Sh::kBuffers <= 4, "the entries of a tile are read four iterations after they were requested");
   constexpr int kChunks = Sh::kChunks, kSteps = Sh::kSteps, kTileUnits = Sh::kTileUnits, kBuffers = Sh::kBuffers;
   constexpr int kRun = Sh::kRun;
 
@@ -509,20 +509,28 @@ static int launch_stream_one(const AttnArgs& a, int n_items, hipStream_t stream)
   return e == hipSuccess ? VA_OK : va_fail(VA_ERR_HIP, "streaming attention launch: %s", hipGetErrorString(e));
 }
 
-template <typename E>
-static int launch_stream_typed(const AttnArgs& a, int n_items, hipStream_t stream) {
+template <typename E, int kD>
+static int launch_stream_dim(const AttnArgs& a, int n_items, hipStream_t stream) {
   // Pages of at least 16 tokens take one scalar lookup per tile, smaller ones an entry per token.  The choice hangs
   // on the page size alone, so that a recorded launch keeps its kernel; in one kernel, the registers of the second
-  // kind spilled into the first at head_dim 256.  (Other page sizes, and slot lists beside larger pages, go through
-  // the first kernel's per-lane lookups.)
-  const bool gather = a.page_size < kStreamTok && (a.page_size & (a.page_size - 1)) == 0;
+  // kind spilled into the first at head_dim 256.  (Other page sizes, slot lists beside larger pages, and rings
+  // built deeper than the index entries allow go through the first kernel's per-lane lookups.)
+  if constexpr (StreamShape<kD>::kBuffers <= 4) {
+    if (a.page_size < kStreamTok && (a.page_size & (a.page_size - 1)) == 0)
+      return launch_stream_one<E, kD, true>(a, n_items, stream);
+  }
+  return launch_stream_one<E, kD, false>(a, n_items, stream);
+}
+
+template <typename E>
+static int launch_stream_typed(const AttnArgs& a, int n_items, hipStream_t stream) {
   switch (a.head_dim) {
     case 64:
-      return gather ? launch_stream_one<E, 64, true>(a, n_items, stream) : launch_stream_one<E, 64, false>(a, n_items, stream);
+      return launch_stream_dim<E, 64>(a, n_items, stream);
     case 128:
-      return gather ? launch_stream_one<E, 128, true>(a, n_items, stream) : launch_stream_one<E, 128, false>(a, n_items, stream);
+      return launch_stream_dim<E, 128>(a, n_items, stream);
     case 256:
-      return gather ? launch_stream_one<E, 256, true>(a, n_items, stream) : launch_stream_one<E, 256, false>(a, n_items, stream);
+      return launch_stream_dim<E, 256>(a, n_items, stream);
     default:
       return va_fail(VA_ERR_ARG, "matrix-core path supports head_dim 64, 128, 256");
   }
