@@ -73,7 +73,7 @@ struct WideShape {
   static constexpr int kRingBytes = kWideBuffers * kBufferBytes, kSetupBytes = kWideAhead * kBufferBytes + kTurnBytes;
   // Scattered rows: the index entries of eight tiles, for every wave its own (va_mfma_wide: gather)
   static constexpr int kIndexOffset = kRingBytes > kSetupBytes ? kRingBytes : kSetupBytes;
-  static constexpr int kLdsBytes = kIndexOffset + kWideWaves * 2 * kWave * 4;
+  static constexpr int lds_bytes(bool gather) { return kIndexOffset + (gather ? kWideWaves * 2 * kWave * 4 : 0); }
 };
 
 // Word of the cos|sin entry (row iq, pair dim) in LDS: rows of `half` words, their 16-byte pieces swizzled
@@ -113,6 +113,7 @@ template <typename E, int kD, bool kGather>
 __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArgs a) {
   using S = typename E::storage;
   using Sh = WideShape<kD>;
+  static_assert(!kGather || kWideAhead <= 2, "the entries of a tile are read a step after their request, behind its wait");
   constexpr int kChunks = Sh::kChunks, kSteps = Sh::kSteps, kDimTiles = Sh::kDimTiles;
   constexpr int kRowBytes = Sh::kRowBytes, kL = Sh::kLoadsPerWave, kB = Sh::kBlocks, kWaveRows = Sh::kWaveRows;
 
@@ -917,7 +918,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
 
 template <typename E, int kD, bool kGather>
 static int launch_wide_one(const AttnArgs& a, int n_items, hipStream_t stream) {
-  constexpr int bytes = WideShape<kD>::kLdsBytes;
+  constexpr int bytes = WideShape<kD>::lds_bytes(kGather);
   static bool configured = false;  // raising the limit is idempotent; a race only repeats the call
   if (!configured) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_mfma_wide_kernel<E, kD, kGather>),
@@ -931,19 +932,28 @@ static int launch_wide_one(const AttnArgs& a, int n_items, hipStream_t stream) {
   return e == hipSuccess ? VA_OK : va_fail(VA_ERR_HIP, "wide attention launch: %s", hipGetErrorString(e));
 }
 
-template <typename E>
-static int launch_wide_typed(const AttnArgs& a, int n_items, hipStream_t stream) {
+template <typename E, int kD>
+static int launch_wide_dim(const AttnArgs& a, int n_items, hipStream_t stream) {
   // Pages of at least 16 tokens take one lookup per half tile, smaller ones (a slot list has pages of one) an
   // entry per token; the choice hangs on the page size alone, so that a recorded launch keeps its kernel.
-  // (Other page sizes, and slot lists beside larger pages, go through the first kernel's per-lane lookups.)
-  const bool gather = a.page_size < 16 && (a.page_size & (a.page_size - 1)) == 0;
+  // (Other page sizes, slot lists beside larger pages, and rings built deeper than the index entries allow go
+  // through the first kernel's per-lane lookups.)
+  if constexpr (kWideAhead <= 2) {
+    if (a.page_size < 16 && (a.page_size & (a.page_size - 1)) == 0)
+      return launch_wide_one<E, kD, true>(a, n_items, stream);
+  }
+  return launch_wide_one<E, kD, false>(a, n_items, stream);
+}
+
+template <typename E>
+static int launch_wide_typed(const AttnArgs& a, int n_items, hipStream_t stream) {
   switch (a.head_dim) {
     case 64:
-      return gather ? launch_wide_one<E, 64, true>(a, n_items, stream) : launch_wide_one<E, 64, false>(a, n_items, stream);
+      return launch_wide_dim<E, 64>(a, n_items, stream);
     case 128:
-      return gather ? launch_wide_one<E, 128, true>(a, n_items, stream) : launch_wide_one<E, 128, false>(a, n_items, stream);
+      return launch_wide_dim<E, 128>(a, n_items, stream);
     case 256:
-      return gather ? launch_wide_one<E, 256, true>(a, n_items, stream) : launch_wide_one<E, 256, false>(a, n_items, stream);
+      return launch_wide_dim<E, 256>(a, n_items, stream);
     default:
       return va_fail(VA_ERR_ARG, "matrix-core path supports head_dim 64, 128, 256");
   }

@@ -13,6 +13,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs hipcc")
 @pytest.mark.parametrize("source,flags,scattered", [
+    ("va_mfma_wide.hip", [], True),
+    ("va_mfma_wide.hip", ["-DVA_WIDE_BUFFERS=5"], False),
     ("va_mfma_stream.hip", ["-DVA_STREAM_BUFFERS_256=4", "-DVA_STREAM_BLOCKS_256=2"], True),
     ("va_mfma_stream.hip", ["-DVA_STREAM_BUFFERS_256=5", "-DVA_STREAM_BLOCKS_256=2"], False),
 ])
