@@ -568,9 +568,9 @@ __global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(MergeArgs a) {
 // few long ones) would be a chain of a trip to memory per pair of states here.  They are left to `finders`
 // workgroups per head at the front of the launch: each looks through every finders-th row and merges its head of the
 // long ones with four waves, eight states per round and wave.  At 16 heads of 256 dims, every row by itself ->
-// long rows found: 8 decode rows of 16 k..32 k tokens beside a chunk of 512 rows 52.0 -> 15.5 us, 48 beside 4 chunks
-// 28.1 -> 17.9, a recorded plan of 512 rows with 4 long ones 97.1 -> 21.3 (the same launches with one wave per (row,
-// head): 38.7, 28.2, 106.3).  Looking costs 0.4 to 0.8 us where no row is long.
+// long rows found: 8 decode rows of 16 k..32 k tokens beside a chunk of 512 rows 52.4 -> 16.2 us, 48 beside 4 chunks
+// 29.4 -> 18.4, a recorded plan of 512 rows with 4 long ones 97.7 -> 20.9 (the same launches with one wave per (row,
+// head): 40.0, 29.7, 105.4).  Looking costs 0.3 to 0.9 us where no row is long.
 constexpr int kFewStates = 8;
 template <typename E>
 __device__ void merge_long_rows(const MergeArgs& a, int n_rows, int finders, int finder, int hq) {
