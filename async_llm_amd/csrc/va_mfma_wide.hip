@@ -276,9 +276,9 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     // Loads of a tile.  Wave w fetches one 16-token half of the K tile (w = 0, 1) or of the V tile
     // (w = 2, 3): kL wave-level loads of kRowsPerLoad rows each.  With uniform pages the half lies
     // in one page, so the wave needs ONE scalar page lookup per tile and every load is a
-    // wave-uniform base plus a per-lane offset that never changes (ld_off); tiles that reach past
-    // the visible range look every row up per lane instead (rows past the range re-read the last
-    // visible token; their scores are masked).
+    // wave-uniform base plus a per-lane offset that never changes (ld_off); in tiles that reach past
+    // the visible range rows past it re-read the last visible token (their scores are masked).  Links
+    // of other page tables look every row up per lane.
     // Slot lists and pages under 16 tokens (kGather): looked up by the lanes in front of each request, the
     // entries cost a trip to memory per tile and drain the ring (6 requests of 60..4096 tokens over slot
     // lists, 32 q / 8 kv heads of 128 dims: 734 us a layer).  So they travel like the tiles do: one
@@ -296,8 +296,9 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     auto half_offset = [&](int page, int t) __attribute__((always_inline)) {
       return (unsigned long long)(uint32_t)page * page_bytes + (uint32_t)(t & (P - 1)) * (uint32_t)row_bytes;
     };
+    // (past the visible range: that of the last visible token)
     auto half_row = [&](int i) __attribute__((always_inline)) {
-      const int t = tok_begin + i * kWideTokens + 16 * wave_half;
+      const int t = min(tok_begin + i * kWideTokens + 16 * wave_half, t_last);
       return half_offset(((PlanWords)a.kv_indices)[kv_begin + (t >> p_shift)], t);
     };
     auto tile_is_plain = [&](int i) __attribute__((always_inline)) {
@@ -358,6 +359,15 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
       if (tile_is_plain(i)) {
         const char* base = wave_plain + row;
         issue_plain(base, dst);
+      } else if (uniform_pages) {
+        // The last tile of a link: its visible rows lie in the page of the half's first token all the same, rows
+        // past them repeat the last visible one.  (Looked up row by row, each request waited for an entry and
+        // with it for the whole ring: 4 ragged requests of 300..1500 tokens over up to six blocks, 32 q / 8 kv
+        // heads of 128 dims, two layers 1318 -> 1299 us; 8 of 2048 over eight blocks, 256 dims, 10860 -> 10813.)
+        const int left = max(0, t_last - (tok_begin + i * kWideTokens + 16 * wave_half));
+#pragma unroll
+        for (int u = 0; u < kL; ++u)
+          load_to_lds(wave_pool + row, (uint32_t)(min(ld_row(u), left) * row_bytes + 16 * ld_piece(u)), dst + u * 1024);
       } else {
         const int t0 = tok_begin + i * kWideTokens + 16 * wave_half;
 #pragma unroll
@@ -371,7 +381,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
     // The pool row of the tile a ring step requests is looked up a whole step earlier (a scalar load whose
     // result is not touched before the next step): its latency never shows.
     auto row_of = [&](int tile) __attribute__((always_inline)) {
-      return (tile < n_tiles && tile_is_plain(tile)) ? half_row(tile) : 0ull;
+      return (uniform_pages && tile < n_tiles) ? half_row(tile) : 0ull;
     };
 
     // ---- set-up: the first two tiles on their way, the query rows rotated for this link ----
