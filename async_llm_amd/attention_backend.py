@@ -151,18 +151,15 @@ class ViewAttnBackend(BaseAttnBackend):
         sub_worker_host = np.arange(n_rows, dtype=np.int64)
         subs = self._subs(qo, kv, lens, flags, chain, sub_worker_host)
         indices = torch.cat([self.page_table[req.table_idx, : req.device_len] for req in reqs]).to(torch.int32)
-        cu_q = torch.from_numpy(qo)
-        cu_q_pinned = cu_q.pin_memory()
-        refs = [cu_q_pinned]
-        launch = op._upload_plan(subs, indices, refs)
+        refs: list = []
+        launch, (cu_q_dev, sub_worker, sub_loc) = op._upload_plan(
+            subs, indices, refs, (qo, sub_worker_host, np.zeros(n_rows, dtype=np.int64)))
         batch.attn_metadata = ViewAttnMetadata(
-            cu_seqlens_q_cpu=cu_q, cu_seqlens_k_cpu=torch.from_numpy(kv),
-            cu_seqlens_q_gpu=cu_q_pinned.to(self.device, non_blocking=True), indices=indices,
+            cu_seqlens_q_cpu=torch.from_numpy(qo), cu_seqlens_k_cpu=torch.from_numpy(kv),
+            cu_seqlens_q_gpu=cu_q_dev, indices=indices,
             seq_lens_cpu=torch.from_numpy(lens), num_qo_heads=op.num_qo_heads, num_kv_heads=op.num_kv_heads,
             head_dim=op.head_dim, page_size=1, dtype=op.dtype,
-            sub_worker=torch.arange(n_rows, dtype=torch.int64, device=self.device),
-            sub_loc=torch.zeros(n_rows, dtype=torch.int64, device=self.device), launch=launch,
-            _refs=tuple(refs))
+            sub_worker=sub_worker, sub_loc=sub_loc, launch=launch, _refs=tuple(refs))
 
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layer_id: int, batch) -> torch.Tensor:
         """Store the new K/V rows at ``batch.out_loc`` and attend (reference

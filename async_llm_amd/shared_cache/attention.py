@@ -33,7 +33,7 @@ import numpy as np
 import torch
 
 from .. import native
-from .attention_metadata import page_numbers_array, upload_page_indices
+from .attention_metadata import join_page_indices, page_numbers_array
 from .rope_correction import rope_rows
 
 
@@ -296,11 +296,12 @@ class SharedCacheAttention:
         return scratch
 
     def _build_launch(self, qo_indptr, kv_indptr, kv_indices_host, seq_lens, flags, chain, sub_worker_host,
-                      n_rows: int, kv_indices_dev: torch.Tensor, refs: list) -> LaunchPlan:
-        """Run the native work decomposition over the planned tables and upload
-        the resulting plan blob."""
-        arrays = [np.ascontiguousarray(a, dtype=np.int32) for a in (qo_indptr, kv_indptr, kv_indices_host,
-                                                                    seq_lens, flags, chain)]
+                      n_rows: int, tables: Sequence, refs: list):
+        """Run the native work decomposition over the planned tables and upload the resulting plan blob
+        together with ``kv_indices`` and ``tables`` (int64 arrays); returns the launch and the device tables."""
+        kv_indices = np.ascontiguousarray(kv_indices_host, dtype=np.int32)
+        arrays = [np.ascontiguousarray(a, dtype=np.int32) for a in (qo_indptr, kv_indptr, seq_lens, flags, chain)]
+        arrays.insert(2, kv_indices)
         sw = np.ascontiguousarray(sub_worker_host, dtype=np.int64)
         n_sub = len(arrays[3])
         subs = native.VaSubRequests(
@@ -309,28 +310,50 @@ class SharedCacheAttention:
             arrays[3].ctypes.data, arrays[4].ctypes.data, arrays[5].ctypes.data,
             sw.ctypes.data if sw.size else None)
         subs._keepalive = (arrays, sw)
-        return self._upload_plan(subs, kv_indices_dev, refs)
+        launch, (dev_indices, *dev_tables) = self._upload_plan(subs, None, refs, (kv_indices, *tables))
+        launch.kv_indices = dev_indices
+        return launch, dev_tables
 
-    def _upload_plan(self, subs, kv_indices_dev: torch.Tensor, refs: list) -> LaunchPlan:
-        """One pass of the planner: build into a scratch that is normally large enough, then copy
-        the blob to pinned staging of its exact size (twice that where ``attend`` may need a second plan)."""
+    def _upload_plan(self, subs, kv_indices_dev: Optional[torch.Tensor], refs: list, tables: Sequence):
+        """One pass of the planner: build into a scratch that is normally large enough, then copy the blob
+        and ``tables`` (int32 or int64), each on a 256-byte boundary, to one pinned staging tensor and from there
+        in one transfer (apart, each of three to seven tables cost a pinned allocation and a copy command).  Plans that ``attend`` may need a second time get a
+        tensor of their own, with room for both.  Returns the launch and the device copies of ``tables``."""
         counts = native.VaPlanCounts()
         scratch = self._plan_into_scratch(subs, counts)
         words = counts.plan_words
         roomy = counts.workspace_bytes > native.STATIC_SCRATCH_BYTES
-        host = torch.empty(2 * words if roomy else words, dtype=torch.int32, pin_memory=self.device.type == "cuda")
-        host.numpy()[:words] = scratch[:words]
+        pinned = self.device.type == "cuda"
+        blob = None
         if roomy:
+            host = torch.empty(2 * words, dtype=torch.int32, pin_memory=pinned)
+            host.numpy()[:words] = scratch[:words]
             blob = torch.empty(2 * words, dtype=torch.int32, device=self.device)
             blob[:words].copy_(host[:words], non_blocking=True)
-        else:
-            blob = host.to(self.device, non_blocking=True)
-        refs.extend((host, blob))
-        header = host[: native.PLAN_HEADER_WORDS].numpy().copy()
+            refs.extend((host, blob))
+        parts = [*([] if roomy else [scratch[:words]]), *tables]
+        begin, size = [], 0
+        for p in parts:
+            begin.append(size)
+            size += -(-p.nbytes // 256) * 256
+        dev_parts = []
+        if parts:
+            staging = torch.empty(size, dtype=torch.uint8, pin_memory=pinned)
+            raw = staging.numpy()
+            for p, a in zip(parts, begin):
+                raw[a: a + p.nbytes].view(p.dtype)[:] = p.reshape(-1)
+            dev = staging.to(self.device, non_blocking=True)
+            refs.extend((staging, dev))
+            for p, a in zip(parts, begin):
+                part = dev[a: a + p.nbytes].view(torch.int32 if p.dtype == np.int32 else torch.int64)
+                dev_parts.append(part if p.ndim == 1 else part.view(p.shape))
+        if not roomy:
+            blob = dev_parts.pop(0)
+        header = scratch[: native.PLAN_HEADER_WORDS].copy()
         launch = LaunchPlan(header, blob, kv_indices_dev, counts, self._ensure_workspace(counts.workspace_bytes))
         if roomy:
             launch.subs, launch.staging = subs, host
-        return launch
+        return launch, dev_parts
 
     def _within_static_scratch(self, launch: LaunchPlan) -> LaunchPlan:
         """The launch as ``va_attention_static`` can run it.  Plans are cut as finely as a workspace that
@@ -460,18 +483,19 @@ class SharedCacheAttention:
         parts = list(main["pages"])
         if n_aux:
             parts.append(aux["kv"])
-        kv_indices = upload_page_indices(parts, self.device, refs)
-        kv_host = refs[0]
+        kv_host = join_page_indices(parts)
         n_main_entries = int(main["n_pages"].sum())
         main_indptr = np.concatenate(([0], np.cumsum(main["n_pages"])))
 
         main_plan = aux_plan = None
         if n_main:
-            main_plan = dict(indptr=torch.from_numpy(main_indptr.astype(np.int32)), indices=kv_host[:n_main_entries],
+            main_plan = dict(indptr=torch.from_numpy(main_indptr.astype(np.int32)),
+                             indices=torch.from_numpy(kv_host[:n_main_entries]),
                              last_page_len=torch.from_numpy(main["last"].astype(np.int32)),
                              seq_lens=torch.from_numpy(main["len"].astype(np.int32)), page_size=P)
         if n_aux:
-            aux_plan = dict(indptr=torch.arange(n_aux + 1, dtype=torch.int32), indices=kv_host[n_main_entries:],
+            aux_plan = dict(indptr=torch.arange(n_aux + 1, dtype=torch.int32),
+                            indices=torch.from_numpy(kv_host[n_main_entries:]),
                             last_page_len=torch.ones(n_aux, dtype=torch.int32),
                             seq_lens=torch.ones(n_aux, dtype=torch.int32), page_size=1)
 
@@ -480,33 +504,22 @@ class SharedCacheAttention:
         pad_slot = sub_worker * max_segments + np.concatenate([main["slot"], aux["slot"]])
         n_sub = n_main + n_aux
 
-        launch = self._build_launch(
+        launch, (dev_sub_worker, dev_sub_loc, dev_pad) = self._build_launch(
             qo_indptr=np.arange(n_sub + 1),
             kv_indptr=np.concatenate([main_indptr, n_main_entries + 1 + np.arange(n_aux)]),
-            kv_indices_host=kv_host.numpy(),
+            kv_indices_host=kv_host,
             seq_lens=np.concatenate([main["len"], np.ones(n_aux, dtype=np.int64)]),
             flags=np.concatenate([np.zeros(n_main, dtype=np.int32), np.full(n_aux, native.VA_SUB_SLOTS, dtype=np.int32)]),
             chain=np.full(n_sub, -1, dtype=np.int32),
             sub_worker_host=sub_worker,
-            n_rows=W, kv_indices_dev=kv_indices, refs=refs)
+            n_rows=W, tables=(sub_worker, sub_loc, pad_slot), refs=refs)
 
-        dev_sub_worker, dev_sub_loc, dev_pad = self._upload_i64([sub_worker, sub_loc, pad_slot], refs)
         meta = SharedCacheAttnMetadata(
             shared_cache_op=self, sub_worker=dev_sub_worker, sub_loc=dev_sub_loc, pad_slot=dev_pad,
             num_workers=W, max_segments=max_segments, n_main=n_main, n_aux=n_aux,
             main_plan=main_plan, aux_plan=aux_plan, launch=launch)
         meta._plan_refs = tuple(refs)
         return meta
-
-    def _upload_i64(self, rows: Sequence, refs: list) -> List[torch.Tensor]:
-        """One pinned staging tensor and one async copy for several equally long
-        int64 tables; returns the device rows."""
-        host = torch.from_numpy(np.stack([np.asarray(r, dtype=np.int64) for r in rows]))
-        if self.device.type == "cuda":
-            host = host.pin_memory()
-        dev = host.to(self.device, non_blocking=True)
-        refs.extend((host, dev))
-        return [dev[i] for i in range(len(rows))]
 
     def _walk_prefill(self, specs, use_3d: bool):
         """Sub-requests of a batched prefill: per request one non-causal sub-request
@@ -574,51 +587,45 @@ class SharedCacheAttention:
         n_rows = offset
         sub_gather = np.concatenate(ctx["rows"] + own["rows"])
         sub_slot = np.concatenate(ctx["slot"] + own["slot"])
-        sub_loc = torch.cat(ctx["loc"] + own["loc"], dim=1 if use_3d else 0)
+        sub_loc = torch.cat(ctx["loc"] + own["loc"], dim=1 if use_3d else 0).numpy()
         pad_slot = sub_gather * max_segments + sub_slot
         n_ctx_rows = int(sum(ctx["q"]))
 
         refs: List[torch.Tensor] = []
-        kv_indices = upload_page_indices(ctx["pages"] + own["pages"], self.device, refs)
-        kv_host = refs[0]
+        kv_host = join_page_indices(ctx["pages"] + own["pages"])
         n_ctx_entries = sum(ctx["n_pages"])
         ctx_plan = None
         if ctx["q"]:
             ctx_plan = dict(qo_indptr=_cumulative(ctx["q"]), paged_kv_indptr=_cumulative(ctx["n_pages"]),
-                            paged_kv_indices=kv_host[:n_ctx_entries], paged_kv_last_page_len=_i32(ctx["last"]),
-                            seq_lens=_i32(ctx["len"]), max_token_per_sequence=max(ctx["q"]), causal=False,
+                            paged_kv_indices=torch.from_numpy(kv_host[:n_ctx_entries]),
+                            paged_kv_last_page_len=_i32(ctx["last"]), seq_lens=_i32(ctx["len"]),
+                            max_token_per_sequence=max(ctx["q"]), causal=False,
                             page_size=P)
         self_plan = dict(qo_indptr=_cumulative(own["q"]), paged_kv_indptr=_cumulative(own["n_pages"]),
-                         paged_kv_indices=kv_host[n_ctx_entries:], paged_kv_last_page_len=_i32(own["last"]),
-                         seq_lens=_i32(own["len"]), max_token_per_sequence=max(own["q"]), causal=True,
+                         paged_kv_indices=torch.from_numpy(kv_host[n_ctx_entries:]),
+                         paged_kv_last_page_len=_i32(own["last"]), seq_lens=_i32(own["len"]),
+                         max_token_per_sequence=max(own["q"]), causal=True,
                          page_size=P)
 
         n_ctx, n_self = len(ctx["q"]), len(own["q"])
-        launch = self._build_launch(
+        last_rows = np.asarray(last_indices, dtype=np.int64)
+        launch, (dev_sub_worker, dev_sub_loc, dev_pad, dev_last) = self._build_launch(
             qo_indptr=np.cumsum([0] + ctx["q"] + own["q"]),
             kv_indptr=np.cumsum([0] + ctx["n_pages"] + own["n_pages"]),
-            kv_indices_host=kv_host.numpy(),
+            kv_indices_host=kv_host,
             seq_lens=ctx["len"] + own["len"],
             flags=[0] * n_ctx + [native.VA_SUB_CAUSAL] * n_self,
             chain=ctx["chain"] + own["chain"],
             sub_worker_host=sub_gather,
-            n_rows=n_rows, kv_indices_dev=kv_indices, refs=refs)
-
-        def to_dev(t: torch.Tensor) -> torch.Tensor:
-            host = t.contiguous()
-            if self.device.type == "cuda":
-                host = host.pin_memory()
-            dev = host.to(self.device, non_blocking=True)
-            refs.extend((host, dev))
-            return dev
+            n_rows=n_rows, tables=(sub_gather, sub_loc, pad_slot, last_rows), refs=refs)
 
         meta = SharedCacheAttnMetadata(
             shared_cache_op=self,
-            sub_worker=to_dev(torch.from_numpy(sub_gather)),
-            sub_loc=to_dev(sub_loc),
-            pad_slot=to_dev(torch.from_numpy(pad_slot)),
+            sub_worker=dev_sub_worker,
+            sub_loc=dev_sub_loc,
+            pad_slot=dev_pad,
             num_workers=n_rows, max_segments=max_segments, n_ctx_rows=n_ctx_rows,
-            last_indices=to_dev(torch.tensor(last_indices, dtype=torch.int64)),
+            last_indices=dev_last,
             phase="prefill_batch", main_plan=ctx_plan, aux_plan=self_plan, launch=launch)
         meta._plan_refs = tuple(refs)
         return meta
@@ -647,8 +654,7 @@ class SharedCacheAttention:
 
         refs: List[torch.Tensor] = []
         parts = list(main["pages"]) + ([aux["kv"]] if n_aux else []) + ctx["pages"] + own["pages"]
-        kv_indices = upload_page_indices(parts, self.device, refs)
-        kv_host = refs[0]
+        kv_host = join_page_indices(parts)
         kv_counts = main["n_pages"].tolist() + [1] * n_aux + ctx["n_pages"] + own["n_pages"]
 
         dec_worker = np.concatenate([main["worker"], aux["worker"]])
@@ -660,32 +666,24 @@ class SharedCacheAttention:
         if use_3d:
             dec_loc = dec_loc.unsqueeze(0).expand(3, -1)
         sub_worker = np.concatenate([dec_worker, pre_rows])
-        sub_loc = torch.cat([dec_loc, pre_loc], dim=1 if use_3d else 0)
+        sub_loc = torch.cat([dec_loc, pre_loc], dim=1 if use_3d else 0).numpy()
         pad_slot = sub_worker * M + np.concatenate([dec_slot, pre_slot])
 
-        launch = self._build_launch(
+        last_rows = np.concatenate([np.arange(W), np.asarray(last_indices, dtype=np.int64) + W])
+        launch, (dev_sub_worker, dev_sub_loc, dev_pad, dev_last) = self._build_launch(
             qo_indptr=np.cumsum([0] + [1] * (n_main + n_aux) + ctx["q"] + own["q"]),
             kv_indptr=np.cumsum([0] + kv_counts),
-            kv_indices_host=kv_host.numpy(),
+            kv_indices_host=kv_host,
             seq_lens=main["len"].tolist() + [1] * n_aux + ctx["len"] + own["len"],
             flags=[0] * n_main + [native.VA_SUB_SLOTS] * n_aux + [0] * n_ctx + [native.VA_SUB_CAUSAL] * n_self,
             chain=[-1] * (n_main + n_aux) + ctx["chain"] + own["chain"],
             sub_worker_host=sub_worker,
-            n_rows=W + n_new, kv_indices_dev=kv_indices, refs=refs)
+            n_rows=W + n_new, tables=(sub_worker, sub_loc, pad_slot, last_rows), refs=refs)
 
-        def to_dev(t: torch.Tensor) -> torch.Tensor:
-            host = t.contiguous()
-            if self.device.type == "cuda":
-                host = host.pin_memory()
-            dev = host.to(self.device, non_blocking=True)
-            refs.extend((host, dev))
-            return dev
-
-        last = torch.cat([torch.arange(W, dtype=torch.int64), torch.tensor(last_indices, dtype=torch.int64) + W])
         meta = SharedCacheAttnMetadata(
-            shared_cache_op=self, sub_worker=to_dev(torch.from_numpy(sub_worker)), sub_loc=to_dev(sub_loc),
-            pad_slot=to_dev(torch.from_numpy(pad_slot)), num_workers=W + n_new, max_segments=M,
-            n_main=n_main, n_aux=n_aux, n_ctx_rows=int(sum(ctx["q"])), last_indices=to_dev(last),
+            shared_cache_op=self, sub_worker=dev_sub_worker, sub_loc=dev_sub_loc, pad_slot=dev_pad,
+            num_workers=W + n_new, max_segments=M,
+            n_main=n_main, n_aux=n_aux, n_ctx_rows=int(sum(ctx["q"])), last_indices=dev_last,
             phase="mixed", launch=launch)
         meta._plan_refs = tuple(refs)
         return meta

@@ -66,6 +66,11 @@ def page_numbers_array(block, snapshot: Dict[int, np.ndarray], extra_page: Optio
     return cached
 
 
+def join_page_indices(parts) -> np.ndarray:
+    """Per-segment page lists (lists or int arrays) as one int32 table on the host."""
+    return np.concatenate([np.asarray(part, dtype=np.int32) for part in parts] or [np.zeros(0, dtype=np.int32)])
+
+
 def upload_page_indices(parts, device: torch.device, refs: List[torch.Tensor]) -> torch.Tensor:
     """Concatenate per-segment page lists (lists or int arrays) into one int32
     table on ``device``.
