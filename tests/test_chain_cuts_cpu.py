@@ -76,3 +76,48 @@ def test_fixed_workspace_gets_coarse_cuts_only_where_they_help(requests, least):
     assert _plan_within(tables, fine) == fine and _plan_within(tables, coarse) == coarse
     if coarse:
         assert _plan_within(tables, 0) == _plan_within(tables, coarse - 1) == fine  # neither fits: the caller is told
+
+
+def _slot_costs(tables, heads, page, seg):
+    blob, counts = np.empty(1 << 20, dtype=np.int32), native.VaPlanCounts()
+    qo, kvp, kvi, lens, flags, chain, sw, n_rows = tables
+    i32 = [np.asarray(a, dtype=np.int32) for a in (qo, kvp, kvi, lens, flags, chain)]
+    rows = np.asarray(sw, dtype=np.int64)
+    subs = native.VaSubRequests(len(lens), len(sw), n_rows, *(a.ctypes.data for a in i32), rows.ctypes.data)
+    shape = native.VaShape(*heads, page, native.VA_BF16)
+    assert native.lib.va_plan_build_within(subs, shape, native.VaPlanParams(native.VA_KERNEL_MFMA, 0, 0, 0, 0), -1,
+                                           blob.ctypes.data, blob.size, counts) == 0
+    blob = blob[: counts.plan_words]
+    h, items, links, *_ = decode_plan(blob)
+    seen = {}  # (sub-request, row) -> the token ranges its items walk (too many pairs to mark one by one)
+    sub_of = np.searchsorted(qo, np.arange(qo[-1]), side="right") - 1
+    for it in items:
+        for l in links[it[0]: it[0] + it[1]] if it[2] > 0 else ():
+            for i in range(int(it[2])):
+                end = min(int(l[2]), int(l[4]) + i + 1)
+                if end > l[1]:
+                    seen.setdefault(int(l[3]) + i, []).append((int(l[1]), end))
+    for subrow, sub in enumerate(sub_of):
+        last = lens[sub] - (qo[sub + 1] - 1 - subrow if flags[sub] else 0)
+        ranges = sorted(seen[subrow])
+        assert [r[0] for r in ranges] + [last] == [0] + [r[1] for r in ranges], (subrow, ranges)
+    slots = blob[h[H["OFF_WIDE_SLOTS"]]: h[H["OFF_WIDE_SLOTS"]] + h[H["N_WIDE_SLOTS"]] + 1]
+    cost = lambda it: sum(min(int(l[2]), int(l[4]) + int(it[2])) - int(l[1]) + seg
+                          for l in links[it[0]: it[0] + it[1]]) if it[2] > 0 else 0
+    return [sum(cost(it) for it in items[a:b]) for a, b in zip(slots, slots[1:])]
+
+
+@pytest.mark.parametrize("heads,page,seg,requests", [
+    # ragged plain requests: many bundles, every one with a causal end
+    ((32, 8, 128), 1, 384, [(193, 1170, []), (2036, 878, []), (120, 1183, []), (1954, 422, []), (2072, 1665, []),
+                            (1196, 1686, [])]),
+    ((32, 8, 128), 16, 384, [(700, 0, [9000, 31]), (1300, 17, [8000]), (90, 5, [20000])]),
+    # bundles of fewer tiles than lanes, parts side by side, a last narrow tile
+    ((16, 4, 256), 16, 640, [(100, 3, [30000]), (333, 100, [9000, 4097]), (65, 0, [12345]), (512, 1, [777, 16000])]),
+    ((64, 16, 64), 32, 384, [(257, 0, [5000]), (1000, 300, [5000, 200]), (64, 0, [7000])]),
+])
+def test_long_walks_load_the_slots_evenly(heads, page, seg, requests):
+    costs = _slot_costs(_tables(requests, page), heads, page, seg)
+    assert len(costs) <= 256 // heads[1] + 8
+    # one piece may end 1/32 of a slot early and lanes differ by as much before they are dealt out by load
+    assert max(costs) * (256 // heads[1]) <= 1.15 * sum(costs), (max(costs), sum(costs) // (256 // heads[1]))
