@@ -195,7 +195,9 @@ def require_device(t: torch.Tensor, name: str) -> None:
 
 
 def current_stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # (the handle alone: the Stream object around it costs about as much as the rest of a launch's arguments)
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def make_shape(hq: int, hkv: int, d: int, page: int, dtype: torch.dtype) -> VaShape:
