@@ -422,8 +422,6 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     int32_t part = 0;                 // walk positions per part
     std::vector<int32_t> subs;        // the chain members any tile of the bundle sees
     std::vector<int32_t> off;         // walk position of each member's first token
-    std::vector<int32_t> seen;        // tokens of each member tile j sees, at [member * m + j]
-    std::vector<char> same;           // whether all tiles see the same of a member
     std::vector<int32_t> starts;      // positions within a part where some lane starts a member (sorted)
     // What positions [x0, x1) cost the slowest lane of the bundle: its tokens, and a set-up (worth
     // `seg` tokens) for the segment it is in at x0 and for every member that starts inside its range.
@@ -439,23 +437,6 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
       }
       return (x1 - x0) + seg * most;
     }
-    // What positions [x0, x1) of part g cost each of its tiles: the tokens it sees there, and a set-up for every
-    // member.  (Only of the last member, the block the tiles themselves extend, do they see different ends.)
-    void tile_costs(int32_t g, int64_t x0, int64_t x1, int32_t seg, int64_t* cost) const {
-      const int64_t lo = (int64_t)g * part + x0, hi = (int64_t)g * part + x1;
-      auto of = [&](size_t k, int32_t j) -> int64_t {
-        const int64_t n = std::min<int64_t>(hi, off[k] + (int64_t)seen[k * m + j]) - std::max<int64_t>(lo, off[k]);
-        return n > 0 ? n + seg : 0;
-      };
-      int64_t alike = 0;
-      for (size_t k = 0; k < off.size(); ++k)
-        if (same[k] && off[k] < hi) alike += of(k, 0);
-      for (int32_t j = 0; j < m; ++j) {
-        cost[j] = alike;
-        for (size_t k = 0; k < off.size(); ++k)
-          if (!same[k]) cost[j] += of(k, j);
-      }
-    }
   };
   auto make_bundle = [&](const std::vector<int32_t>& ch, int32_t nq, int32_t first, int32_t m) {
     Bundle bd;
@@ -468,9 +449,6 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
       if (vis <= 0) continue;
       bd.subs.push_back(sub);
       bd.off.push_back((int32_t)pos);
-      for (int32_t j = 0; j < m; ++j)
-        bd.seen.push_back(std::max(0, visible_end(s->seq_lens[sub], nq, s->flags[sub] & VA_SUB_CAUSAL, tiles[first + j].second)));
-      bd.same.push_back(bd.seen.back() == bd.seen[bd.seen.size() - m]);
       pos += align_cuts ? round_up(vis, 16) : vis;  // every member starts at a multiple of 16: so do all cuts within it
     }
     if (pos == 0) return bd;
@@ -515,7 +493,6 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   const int64_t group_budget = pack ? std::max<int64_t>((wide_walk + groups_wanted - 1) / groups_wanted, cuts_of_chains.group_floor()) : 0;
   const int32_t min_piece = cuts_of_chains.least_piece(group_budget);
   int64_t groups_left = pack ? std::max<int64_t>(1, (wide_walk + group_budget - 1) / group_budget) : 0;
-  const int32_t n_groups = (int32_t)groups_left;
   // What is still to be placed, set-ups included: every segment of every bundle, and one more for
   // every group boundary (it falls inside some segment, which is then staged on both sides).  An
   // estimate on the high side leaves the LAST group short, one on the low side would leave it long --
@@ -567,131 +544,6 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     }
   };
 
-  // Long walks are packed by what each LANE of a group really walks.  The tiles of a bundle end at different
-  // places of their own block (causal), and a bundle of few tiles leaves lanes without a piece: charged to the
-  // slowest lane, and dealt out by tile number, the ends of four bundles in a group all made the same lane the
-  // longest.  So the pieces of a bundle go to the lanes by load, the longest to the least loaded, and the room of a
-  // group is the smallest for which all bundles fit the groups, found by bisection.  Six plain requests of
-  // 60..4096 tokens, 32 q / 8 kv heads of 128 dims: the longest slot 10 -> 5 % over an even share, wide launch
-  // 349 -> 331 us a layer, merge 13 -> 14.  The bisection takes the host 20 to 70 us, which a launch of short
-  // walks does not give back (333 tokens over 3.7 k of view: wide launch and merge 70.3 -> 68.6 us a layer, but
-  // the pass of four layers 341 -> 360): groups of under 4096 tokens keep the packing above, and so do coarse
-  // cuts, which are what a caller's fixed workspace was found to hold.
-  const bool by_lane = pack && cuts_of_chains.fine && group_budget >= 4096;
-  struct Piece {
-    int32_t bundle;
-    int64_t x0, x1;
-    int32_t group;
-    std::vector<int32_t> lane;  // of part g, tile j at [g * m + j]; -1: the tile sees nothing of this piece
-  };
-  std::vector<Bundle> all_bundles;
-  std::vector<size_t> chain_bundles{0};  // bundles [chain_bundles[c], chain_bundles[c + 1]) belong to chain c
-  std::vector<Piece> pieces;
-  if (by_lane) {
-    std::vector<int64_t> load(lanes), trial(lanes), cost(lanes);
-    int64_t total = 0;
-    for (auto& ch : chains) {
-      const int32_t nq = s->qo_indptr[ch[0] + 1] - s->qo_indptr[ch[0]];
-      cut_tiles(nq, tiles);
-      bundles_of(ch, nq, bundles);
-      for (auto& bd : bundles) {
-        for (int32_t g = 0; g < bd.f; ++g) {
-          bd.tile_costs(g, 0, bd.part, seg_cost, cost.data());
-          total += std::accumulate(cost.begin(), cost.begin() + bd.m, int64_t{0});
-        }
-        all_bundles.push_back(std::move(bd));
-      }
-      chain_bundles.push_back(all_bundles.size());
-    }
-    std::vector<int32_t> by_load(lanes), by_cost(lanes), lane_of(lanes);
-    // Loads of the group's lanes with positions [x0, x1) of a bundle added (trial, lane_of): the longest.
-    // (in the order of the tiles while the lanes differ by little)
-    auto try_piece = [&](const Bundle& bd, int64_t x0, int64_t x1, int64_t room) {
-      const int32_t n = bd.f * bd.m;
-      for (int32_t g = 0; g < bd.f; ++g) bd.tile_costs(g, x0, x1, seg_cost, cost.data() + g * bd.m);
-      // (a handful of lanes: insertion keeps their order and allocates nothing)
-      auto sort_into = [](std::vector<int32_t>& order, int32_t count, auto&& before) {
-        for (int32_t k = 0; k < count; ++k) {
-          int32_t at = k;
-          for (; at > 0 && before(k, order[at - 1]); --at) order[at] = order[at - 1];
-          order[at] = k;
-        }
-      };
-      const auto [low, high] = std::minmax_element(load.begin(), load.end());
-      const bool by_number = *high - *low <= room / 32;
-      sort_into(by_load, lanes, [&](int32_t a, int32_t b) { return !by_number && load[a] < load[b]; });
-      sort_into(by_cost, n, [&](int32_t a, int32_t b) { return !by_number && cost[a] > cost[b]; });
-      trial = load;
-      for (int32_t k = 0; k < n; ++k) {
-        const int32_t e = by_cost[k];
-        lane_of[e] = cost[e] > 0 ? by_load[k] : -1;
-        trial[by_load[k]] += cost[e];
-      }
-      return *std::max_element(trial.begin(), trial.end());
-    };
-    // All bundles, in order, into groups of lanes of at most `room`; the last group takes what is left.
-    // Returns the longest lane.
-    auto pack_all = [&](int64_t room, bool record) {
-      int64_t longest = 0;
-      int32_t group = 0;
-      std::fill(load.begin(), load.end(), 0);
-      for (size_t i = 0; i < all_bundles.size(); ++i) {
-        const Bundle& bd = all_bundles[i];
-        for (int64_t x = 0; x < bd.part;) {
-          int64_t x1 = bd.part;
-          if (group + 1 < n_groups && try_piece(bd, x, x1, room) > room) {
-            // The furthest cut (on a multiple of 16 or of a 64th of the room) that the room pays for (at least what it pays for on the
-            // longest lane with every start counted, at most what it pays for on the shortest without any), and no
-            // piece under min_piece on either side.
-            const auto [low, high] = std::minmax_element(load.begin(), load.end());
-            const int64_t reach = std::min<int64_t>(bd.part, x + room - *low);
-            const int64_t n_starts = 1 + std::count_if(bd.starts.begin(), bd.starts.end(), [&](int32_t p) { return p > x && p < reach; });
-            const int64_t grain = 16 * std::max<int64_t>(1, room / 1024);
-            int64_t fits = std::max<int64_t>(0, (room - *high - seg_cost * n_starts) / grain), over = (reach - x) / grain + 1;
-            while (over - fits > 1) {
-              const int64_t mid = (fits + over) / 2;
-              (try_piece(bd, x, std::min<int64_t>(bd.part, x + grain * mid), room) <= room ? fits : over) = mid;
-            }
-            x1 = std::min<int64_t>(x + grain * fits, (bd.part - min_piece) / 16 * 16);
-            if (x1 - x < min_piece) {
-              const bool fresh = std::all_of(load.begin(), load.end(), [](int64_t l) { return l == 0; });
-              if (!fresh) {  // nothing worth a set-up fits behind what the group holds
-                ++group;
-                std::fill(load.begin(), load.end(), 0);
-                continue;
-              }
-              x1 = bd.part;  // too short to cut
-            }
-          }
-          const int64_t now = try_piece(bd, x, x1, room);
-          longest = std::max(longest, now);
-          load = trial;
-          if (record) pieces.push_back(Piece{(int32_t)i, x, x1, group, std::vector<int32_t>(lane_of.begin(), lane_of.begin() + bd.f * bd.m)});
-          x = x1;
-          if (x < bd.part) {  // (a bundle has one piece in a group: the lanes it leaves idle are for other bundles)
-            ++group;
-            std::fill(load.begin(), load.end(), 0);
-          }
-        }
-      }
-      return longest;
-    };
-    // The room, to 1/128 of an even share: no less than that share, no more than what some packing came to.
-    int64_t lo = total / ((int64_t)n_groups * lanes), best = INT64_MAX, best_room = lo;
-    const int64_t close_enough = std::max<int64_t>(64, lo / 128);
-    for (int64_t room = lo + seg_cost; n_groups > 1 && best - lo > close_enough; room = (lo + best) / 2) {
-      const int64_t longest = pack_all(room, false);
-      if (longest > room) lo = room;
-      if (longest < best) {
-        best = longest;
-        best_room = room;
-      } else if (longest <= room) {
-        break;  // no better than what is known
-      }
-    }
-    pack_all(best_room, true);
-  }
-
   // Cut a narrow tile's walk (links in walking order) into budgets of `slot_room` tokens, one item a
   // piece; a remainder of less than narrow_least stays with the piece before it.
   auto cut_walk = [&](const std::vector<Link>& walk, auto&& close) {
@@ -742,7 +594,6 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     close_piece();
   };
 
-  size_t next_piece = 0;
   for (auto& ch : chains) {
     const int32_t nq = s->qo_indptr[ch[0] + 1] - s->qo_indptr[ch[0]];
     cut_tiles(nq, tiles);
@@ -771,20 +622,7 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     auto tile_rows = [&](int32_t a) {
       return [rows = s->sub_worker + s->qo_indptr[ch[0]] + a](int32_t i) { return (int32_t)rows[i]; };
     };
-    if (by_lane) {
-      const size_t chain_index = &ch - &chains[0];
-      for (; next_piece < pieces.size() && (size_t)pieces[next_piece].bundle < chain_bundles[chain_index + 1]; ++next_piece) {
-        const Piece& p = pieces[next_piece];
-        const Bundle& bd = all_bundles[p.bundle];
-        for (int32_t k = 0; k < bd.f * bd.m; ++k) {
-          if (p.lane[k] < 0) continue;
-          const int64_t at = (int64_t)(k / bd.m) * bd.part;
-          const int32_t a = tiles[bd.first + k % bd.m].first, b = tiles[bd.first + k % bd.m].second;
-          tile_links(a, b, &bd, at + p.x0, at + p.x1);
-          if (!links.empty()) emit(b - a, links, tile_rows(a), -1, p.group * lanes + p.lane[k]);
-        }
-      }
-    } else if (pack) {
+    if (pack) {
       bundles_of(ch, nq, bundles);
       for (auto& bd : bundles) {
         cut_bundle(bd, [&](int64_t x0, int64_t x1, int32_t group) {

@@ -107,17 +107,23 @@ def _slot_costs(tables, heads, page, seg):
     return [sum(cost(it) for it in items[a:b]) for a, b in zip(slots, slots[1:])]
 
 
-@pytest.mark.parametrize("heads,page,seg,requests", [
+@pytest.mark.parametrize("heads,page,seg,requests,bound", [
     # ragged plain requests: many bundles, every one with a causal end
     ((32, 8, 128), 1, 384, [(193, 1170, []), (2036, 878, []), (120, 1183, []), (1954, 422, []), (2072, 1665, []),
-                            (1196, 1686, [])]),
-    ((32, 8, 128), 16, 384, [(700, 0, [9000, 31]), (1300, 17, [8000]), (90, 5, [20000])]),
+                            (1196, 1686, [])], 1.11),
+    ((32, 8, 128), 16, 384, [(700, 0, [9000, 31]), (1300, 17, [8000]), (90, 5, [20000])], 1.055),
     # bundles of fewer tiles than lanes, parts side by side, a last narrow tile
-    ((16, 4, 256), 16, 640, [(100, 3, [30000]), (333, 100, [9000, 4097]), (65, 0, [12345]), (512, 1, [777, 16000])]),
-    ((64, 16, 64), 32, 384, [(257, 0, [5000]), (1000, 300, [5000, 200]), (64, 0, [7000])]),
+    ((16, 4, 256), 16, 640, [(100, 3, [30000]), (333, 100, [9000, 4097]), (65, 0, [12345]), (512, 1, [777, 16000])], 1.18),
+    ((64, 16, 64), 32, 384, [(257, 0, [5000]), (1000, 300, [5000, 200]), (64, 0, [7000])], 1.055),
+    # one request over many blocks, and over one long block
+    ((32, 8, 128), 16, 384, [(581, 0, [1500] * 30)], 1.01),
+    ((32, 8, 128), 16, 384, [(581, 77, [100 + 97 * i for i in range(30)])], 1.023),
+    ((16, 4, 256), 16, 640, [(2048, 0, [32768])], 1.006),
 ])
-def test_long_walks_load_the_slots_evenly(heads, page, seg, requests):
+def test_long_walks_load_the_slots_evenly(heads, page, seg, requests, bound):
+    # The bounds are what cutting every bundle once, at the cost of its slowest lane, comes to (in this order 1.103,
+    # 1.050, 1.176, 1.051, 1.006, 1.021, 1.004): another packing has to be no worse in any of them.  Dealing the
+    # pieces to the lanes by load came to 1.053, 1.068, 1.123, 1.012, 1.016, 1.025, 1.010.
     costs = _slot_costs(_tables(requests, page), heads, page, seg)
     assert len(costs) <= 256 // heads[1] + 8
-    # one piece may end 1/32 of a slot early and lanes differ by as much before they are dealt out by load
-    assert max(costs) * (256 // heads[1]) <= 1.15 * sum(costs), (max(costs), sum(costs) // (256 // heads[1]))
+    assert max(costs) * (256 // heads[1]) <= bound * sum(costs), (max(costs), sum(costs) // (256 // heads[1]))
