@@ -190,7 +190,9 @@ class SharedCacheAttention:
         self._rope_desc: Optional[native.VaRope] = None
         self._workspace: Optional[torch.Tensor] = None
         self._workspace_prepared = False
-        self._plan_scratch = np.empty(1 << 16, dtype=np.int32)  # host scratch of the planner, grown on demand
+        # host scratch of the planner, grown on demand; a plan has it to itself until its words are copied out
+        # (the planner and the transfers run without the interpreter's lock)
+        self._plan_scratch: List[np.ndarray] = []
         self._checked_layers = set()
         if fused_store:
             self._check_pool_layout()
@@ -283,13 +285,18 @@ class SharedCacheAttention:
     # planning
     # ------------------------------------------------------------------
     def _plan_into_scratch(self, subs, counts) -> np.ndarray:
-        """Plan into the op's host scratch (grown on demand), within the workspace once that is fixed."""
+        """Plan into the op's host scratch (grown on demand), within the workspace once that is fixed.  The caller
+        gives the scratch back (``_plan_scratch``) when it has copied the plan; without one at hand, as where another
+        thread is planning, it is a new one."""
         limit = self._workspace.numel() if self._workspace_prepared else -1  # (an arena of no bytes is a limit too)
-        scratch = self._plan_scratch
+        try:
+            scratch = self._plan_scratch.pop()
+        except IndexError:
+            scratch = np.empty(1 << 16, dtype=np.int32)
         rc = native.lib.va_plan_build_within(subs, self._shape, self.plan_params, limit, scratch.ctypes.data,
                                              scratch.size, counts)
         if rc == native.VA_ERR_CAPACITY and counts.plan_words > scratch.size:
-            scratch = self._plan_scratch = np.empty(2 * counts.plan_words, dtype=np.int32)
+            scratch = np.empty(2 * counts.plan_words, dtype=np.int32)
             rc = native.lib.va_plan_build_within(subs, self._shape, self.plan_params, limit, scratch.ctypes.data,
                                                  scratch.size, counts)
         native.check(rc)
@@ -350,6 +357,7 @@ class SharedCacheAttention:
         if not roomy:
             blob = dev_parts.pop(0)
         header = scratch[: native.PLAN_HEADER_WORDS].copy()
+        self._plan_scratch = [scratch]
         launch = LaunchPlan(header, blob, kv_indices_dev, counts, self._ensure_workspace(counts.workspace_bytes))
         if roomy:
             launch.subs, launch.staging = subs, host
