@@ -194,10 +194,16 @@ def require_device(t: torch.Tensor, name: str) -> None:
         )
 
 
+# The current stream's handle by device number, without the Stream object around it (which costs about as much as the
+# rest of a launch's arguments).  torch has no public name for it: builds without this one take the object's.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def current_stream_ptr(device: torch.device) -> int:
-    # (the handle alone: the Stream object around it costs about as much as the rest of a launch's arguments)
+    if _raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
     index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    return _raw_stream(torch.cuda.current_device() if index is None else index)
 
 
 def make_shape(hq: int, hkv: int, d: int, page: int, dtype: torch.dtype) -> VaShape:
