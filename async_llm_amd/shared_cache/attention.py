@@ -324,8 +324,9 @@ class SharedCacheAttention:
     def _upload_plan(self, subs, kv_indices_dev: Optional[torch.Tensor], refs: list, tables: Sequence):
         """One pass of the planner: build into a scratch that is normally large enough, then copy the blob
         and ``tables`` (int32 or int64), each on a 256-byte boundary, to one pinned staging tensor and from there
-        in one transfer (apart, each of three to seven tables cost a pinned allocation and a copy command).  Plans that ``attend`` may need a second time get a
-        tensor of their own, with room for both.  Returns the launch and the device copies of ``tables``."""
+        in one transfer (apart, each of three to seven tables cost a pinned allocation and a copy command).
+        Plans that ``attend`` may need a second time get a tensor of their own, with room for both.  Returns the
+        launch and the device copies of ``tables``."""
         counts = native.VaPlanCounts()
         scratch = self._plan_into_scratch(subs, counts)
         words = counts.plan_words

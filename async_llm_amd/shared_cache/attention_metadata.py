@@ -66,14 +66,14 @@ def page_numbers_array(block, snapshot: Dict[int, np.ndarray], extra_page: Optio
     return cached
 
 
-def join_page_indices(parts) -> np.ndarray:
-    """Per-segment page lists (lists or int arrays) as one int32 table on the host."""
-    return np.concatenate([np.asarray(part, dtype=np.int32) for part in parts] or [np.zeros(0, dtype=np.int32)])
+def join_page_indices(parts, out: Optional[np.ndarray] = None) -> np.ndarray:
+    """Per-segment page lists (lists or int arrays) as one int32 table on the host (``out``, or a new array)."""
+    return np.concatenate([np.asarray(part, dtype=np.int32) for part in parts] or [np.zeros(0, dtype=np.int32)], out=out)
 
 
 def upload_page_indices(parts, device: torch.device, refs: List[torch.Tensor]) -> torch.Tensor:
-    """Concatenate per-segment page lists (lists or int arrays) into one int32
-    table on ``device``.
+    """``join_page_indices`` as a table on ``device``, for a caller with no plan to
+    send beside it (a planned step's table travels with its plan).
 
     The host staging tensor is pinned when the target is a GPU and the copy is
     asynchronous, so both tensors are appended to ``refs`` (host first, device
@@ -81,8 +81,7 @@ def upload_page_indices(parts, device: torch.device, refs: List[torch.Tensor]) -
     """
     total = sum(len(part) for part in parts)
     host = torch.empty(total, dtype=torch.int32, device="cpu", pin_memory=device.type == "cuda")
-    if total:
-        np.concatenate([np.asarray(part, dtype=np.int32) for part in parts], out=host.numpy())
+    join_page_indices(parts, out=host.numpy())
     table = host.to(device, non_blocking=True)
     refs.append(host)
     refs.append(table)
