@@ -649,6 +649,9 @@ __global__ __launch_bounds__(256, 4) void merge_rows_kernel(MergeArgs a, int n_r
           x[u][k] = *(const float4*)(a.part_acc + (state << d_shift) + at[k]);
         }
       }
+      // (Or the scheduler may sink the last loads behind the first state's fold, a second trip: plain prefill of 7571
+      // rows of 32 heads of 128 dims 14.4 us, 13.2 with the barrier, 48 decode rows beside 4 chunks 17.8 and 17.0.)
+      if constexpr (kRuns == 4) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int u = 0; u < n; ++u)
 #pragma unroll
