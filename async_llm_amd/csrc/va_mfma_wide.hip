@@ -363,7 +363,8 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
         // The last tile of a link: its visible rows lie in the page of the half's first token all the same, rows
         // past them repeat the last visible one.  (Looked up row by row, each request waited for an entry and
         // with it for the whole ring: 4 ragged requests of 300..1500 tokens over up to six blocks, 32 q / 8 kv
-        // heads of 128 dims, two layers 1318 -> 1299 us; 8 of 2048 over eight blocks, 256 dims, 10860 -> 10813.)
+        // heads of 128 dims, two layers 1318 -> 1299 us; 8 of 2048 over eight blocks, 256 dims: no more than two
+        // runs differ by.)
         const int left = max(0, t_last - (tok_begin + i * kWideTokens + 16 * wave_half));
 #pragma unroll
         for (int u = 0; u < kL; ++u)

@@ -460,15 +460,17 @@ __global__ __launch_bounds__(kGenThreads) void attn_generic_kernel(AttnArgs a) {
 // round exactly what is left) with all their loads in flight together, and the running states meet
 // in LDS.  Lane l owns dims l, l + 64, ...
 // For a decode batch: few rows, up to dozens of partial states each.
-// What the plan says of a row arrives in one trip of scalar loads (flags, then the list's bounds, then its entries
-// lane by lane were three): 16 heads of 256 dims, 4 rows 6.2 -> 4.6 us, 333 rows 10.4 -> 8.7, 633 rows of 8 heads of
-// 128 dims 7.8 -> 6.0; 8 rows of 32 heads and sixteen waves 4.6 either way.
-using PlanTable = const __attribute__((address_space(4))) int32_t*;  // read only while a launch runs: scalar loads
+// What the plan says of a row comes in scalar loads: flags and bounds of the list in one trip, an entry of the list in
+// front of each state's requests.  (The bounds behind the flags were a trip of their own, and an entry in a vector load
+// was waited for together with the requests of the states before it: a round was a chain of a trip per state.)  16
+// heads of 256 dims, 4 rows 6.2 -> 4.6 us, 333 rows 10.4 -> 8.7, 633 rows of 8 heads of 128 dims 7.8 -> 6.0; 8 rows of
+// 32 heads and sixteen waves 4.6 either way.
+using PlanTable = const __attribute__((address_space(4))) int32_t*;  // read only while a launch runs
 template <typename E, int kMergeWaves>
 __device__ __forceinline__ void merge_row_head(const MergeArgs& a, long long row, int hq, int begin, int end) {
   using S = typename E::storage;
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-  const PlanTable ids = (PlanTable)a.row_ids;  // (the same for a whole wave: scalar loads)
+  const PlanTable ids = (PlanTable)a.row_ids;  // (wave and begin are the same for a whole wave)
   S* o = (S*)a.out + (row * a.num_q_heads + hq) * (long long)a.head_dim;
   const int n_d = (a.head_dim + 63) / 64;  // dims per lane: d = lane + 64*k (at most 4 for D = 256)
   float mm = kNegBig, ll = 0.f;
@@ -575,9 +577,10 @@ __global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(MergeArgs a) {
 // few long ones) would be a chain of a trip to memory per pair of states here.  They are left to `finders`
 // workgroups per head at the front of the launch: each looks through every finders-th row and merges its head of the
 // long ones with four waves, eight states per round and wave.  At 16 heads of 256 dims, every row by itself ->
-// long rows found: 8 decode rows of 16 k..32 k tokens beside a chunk of 512 rows 52.4 -> 16.2 us, 48 beside 4 chunks
-// 29.4 -> 18.4, a recorded plan of 512 rows with 4 long ones 97.7 -> 20.9 (the same launches with one wave per (row,
-// head): 40.0, 29.7, 105.4).  Looking costs 0.3 to 0.9 us where no row is long.
+// long rows found -> their lists read in scalar loads: 8 decode rows of 16 k..32 k tokens beside a chunk of 512 rows
+// 52.4 -> 16.4 -> 12.2 us, 48 beside 4 chunks 29.4 -> 17.1 -> 17.1, a recorded plan of 512 rows with 4 long ones
+// 97.7 -> 20.2 -> 12.4 (the same launches with one wave per (row, head): 40.0, 29.7, 105.4).  Looking costs 0.3 to
+// 0.9 us where no row is long.
 constexpr int kFewStates = 8;
 template <typename E>
 __device__ void merge_long_rows(const MergeArgs& a, int n_rows, int finders, int finder, int hq) {
@@ -650,7 +653,7 @@ __global__ __launch_bounds__(256, 4) void merge_rows_kernel(MergeArgs a, int n_r
         }
       }
       // (Or the scheduler may sink the last loads behind the first state's fold, a second trip: plain prefill of 7571
-      // rows of 32 heads of 128 dims 14.4 us, 13.2 with the barrier, 48 decode rows beside 4 chunks 17.8 and 17.0.)
+      // rows of 32 heads of 128 dims 14.5 us, 13.0 with the barrier, 48 decode rows beside 4 chunks 18.1 and 17.1.)
       if constexpr (kRuns == 4) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int u = 0; u < n; ++u)
