@@ -33,7 +33,10 @@ HOST_FLAGS = ["--offload-arch=gfx950", "--cuda-host-only"]
 # compiler gives every matrix product it selects an accumulator in the accumulation registers; its
 # score products are read by the vector ALU at once and want ordinary registers (the long-lived
 # output accumulators are pinned in accumulation registers by hand).
-SOURCE_DEVICE_FLAGS = {"va_mfma_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# The streaming kernel rescales its accumulators now and then: in accumulation registers it would copy all of them
+# back and forth in every tile.
+SOURCE_DEVICE_FLAGS = {"va_mfma_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+                       "va_mfma_stream.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _run(cmd, verbose):

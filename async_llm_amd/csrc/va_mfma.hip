@@ -3,7 +3,7 @@
 //
 //   * streaming kernel (va_mfma_stream.hip): query tiles of up to 16 MFMA rows (row = tile row
 //     R / G, head R % G with G = q heads per kv head), i.e. decode tiles of 16/G requests that
-//     read the same KV run, and short prefill tiles.  Bound by HBM.
+//     read the same KV run (up to four such tiles a workgroup), and short prefill tiles.  Bound by HBM.
 //   * wide kernel (va_mfma_wide.hip): query tiles of up to 128 MFMA rows for view-conditioned
 //     prefill.  Bound by the matrix pipe.
 // A plan lists its wide items first; each kind gets one launch.

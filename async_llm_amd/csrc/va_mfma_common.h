@@ -312,6 +312,17 @@ __device__ __forceinline__ int ring_barrier_zero() {
 }
 constexpr int kAnyInFlight = 63;  // vmcnt(63): no wait on vector memory at all
 
+// A transposing LDS read (ds_read_b64_tr_b16).  Within every group of 16 lanes, lane s supplies
+// the address of four 16-bit elements E[s][0..3]; lane i receives E[i / 4 + 4 k][i % 4], k = 0..3.
+// With lane s pointed at token T + s / 4, dims c + 4 (s % 4) .. + 3, lane i therefore receives
+// dim c + i of tokens T .. T + 3: four consecutive contraction elements of one row of V^T.
+__device__ __forceinline__ va_u32x2 lds_read_tr16(uint32_t lds_byte_address) {
+  typedef short v4s __attribute__((ext_vector_type(4)));
+  const v4s r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) v4s*)(uintptr_t)lds_byte_address);
+  return __builtin_bit_cast(va_u32x2, r);
+}
+
 // One wave-level pool -> LDS load: lane l's 16 bytes at `src` land at LDS byte address
 // `lds_base + 16 l` (lds_base is wave-uniform and travels in M0).  Written as assembly on purpose:
 // when the compiler sees such a load it makes every later LDS read wait for ALL of them
@@ -329,21 +340,6 @@ __device__ __forceinline__ void load_to_lds(const void* src, uint32_t lds_base) 
       : "v"(src), "s"(lds_base)
       : "memory");
 }
-// The same load marked non-temporal: rows that one workgroup reads once (a block no other query
-// tile shares) are streamed through the caches as lines to evict first, so that they do not push
-// out the rows that several tiles read (a block shared by many views, held in the die's L2).
-// Measured on one MI355X: a pure stream (eight views of 131 072 tokens, nothing shared) 5.74 -> 6.29 TB/s;
-// it is the nt bit that does it, the sc0 / sc1 bits beside it change nothing.
-__device__ __forceinline__ void load_to_lds_once(const void* src, uint32_t lds_base) {
-  uint32_t saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, off nt\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "v"(src), "s"(lds_base)
-      : "memory");
-}
 // The same with a wave-uniform base address and a 32-bit per-lane byte offset (no vector ALU work
 // to form 64-bit addresses).
 __device__ __forceinline__ void load_to_lds(const void* base, uint32_t lane_offset, uint32_t lds_base) {
@@ -356,52 +352,49 @@ __device__ __forceinline__ void load_to_lds(const void* base, uint32_t lane_offs
       : "v"(lane_offset), "s"(base), "s"(lds_base)
       : "memory");
 }
-// Two loads of per-lane addresses behind ONE setting of M0, the second landing 1024 bytes after
-// the first: the instruction's immediate offset is added to the pool address AND to the LDS
-// address, so the caller passes the second address with 1024 taken off.
-__device__ __forceinline__ void load_pair_to_lds(const void* src0, const void* src1_minus_1024, uint32_t lds_base) {
-  uint32_t saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, off\n\t"
-      "global_load_lds_dwordx4 %2, off offset:1024\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "v"(src0), "v"(src1_minus_1024), "s"(lds_base)
-      : "memory");
-}
 // Up to four loads of "uniform base + per-lane offset" behind one setting of M0: load u of a group
 // lands 1024 u bytes further on when its per-lane offset has had 1024 u taken off beforehand
 // (grouped_lane_offset).
+// kOnce marks them non-temporal: rows that one workgroup reads once (a block no other query tile shares) are
+// streamed through the caches as lines to evict first, so that they do not push out the rows that several tiles
+// read (a block shared by many views, held in the die's L2).  Measured on one MI355X: reads that fill LDS and nothing
+// else reach 6.9 TB/s with the bit and 6.1 TB/s without; the sc0 / sc1 bits beside it change nothing.
 __device__ __forceinline__ uint32_t grouped_lane_offset(uint32_t lane_offset, int u) { return lane_offset - 1024u * (u % 4); }
-template <int kCount>
+template <int kCount, bool kOnce = false>
 __device__ __forceinline__ void load_group_to_lds(const void* base, const uint32_t* adjusted_offsets, uint32_t lds_base) {
   static_assert(kCount == 1 || kCount == 2 || kCount == 4, "loads per group");
   uint32_t saved;
+#define VA_FOUR_LOADS(policy)                                                                                         \
+  asm volatile(                                                                                                       \
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %6\n\ts_nop 0\n\t"                                                           \
+      "global_load_lds_dwordx4 %1, %5" policy "\n\t"                                                                  \
+      "global_load_lds_dwordx4 %2, %5 offset:1024" policy "\n\t"                                                      \
+      "global_load_lds_dwordx4 %3, %5 offset:2048" policy "\n\t"                                                      \
+      "global_load_lds_dwordx4 %4, %5 offset:3072" policy "\n\t"                                                      \
+      "s_mov_b32 m0, %0"                                                                                              \
+      : "=&s"(saved)                                                                                                  \
+      : "v"(adjusted_offsets[0]), "v"(adjusted_offsets[1]), "v"(adjusted_offsets[2]), "v"(adjusted_offsets[3]),       \
+        "s"(base), "s"(lds_base)                                                                                      \
+      : "memory")
+#define VA_TWO_LOADS(policy)                                                                                          \
+  asm volatile(                                                                                                       \
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_nop 0\n\t"                                                           \
+      "global_load_lds_dwordx4 %1, %3" policy "\n\t"                                                                  \
+      "global_load_lds_dwordx4 %2, %3 offset:1024" policy "\n\t"                                                      \
+      "s_mov_b32 m0, %0"                                                                                              \
+      : "=&s"(saved)                                                                                                  \
+      : "v"(adjusted_offsets[0]), "v"(adjusted_offsets[1]), "s"(base), "s"(lds_base)                                  \
+      : "memory")
   if constexpr (kCount == 4) {
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %6\n\ts_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, %5\n\t"
-        "global_load_lds_dwordx4 %2, %5 offset:1024\n\t"
-        "global_load_lds_dwordx4 %3, %5 offset:2048\n\t"
-        "global_load_lds_dwordx4 %4, %5 offset:3072\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(saved)
-        : "v"(adjusted_offsets[0]), "v"(adjusted_offsets[1]), "v"(adjusted_offsets[2]), "v"(adjusted_offsets[3]),
-          "s"(base), "s"(lds_base)
-        : "memory");
+    if constexpr (kOnce) VA_FOUR_LOADS(" nt"); else VA_FOUR_LOADS("");
   } else if constexpr (kCount == 2) {
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, %3\n\t"
-        "global_load_lds_dwordx4 %2, %3 offset:1024\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(saved)
-        : "v"(adjusted_offsets[0]), "v"(adjusted_offsets[1]), "s"(base), "s"(lds_base)
-        : "memory");
+    if constexpr (kOnce) VA_TWO_LOADS(" nt"); else VA_TWO_LOADS("");
   } else {
+    static_assert(!kOnce, "single loads carry no cache policy");
     load_to_lds(base, adjusted_offsets[0], lds_base);
   }
+#undef VA_FOUR_LOADS
+#undef VA_TWO_LOADS
 }
 // Rows scattered over the pool (a 64-bit address per lane): kCount loads behind one saved M0, load u landing
 // 1024 u bytes further on.  `columns`: 128-byte columns of ONE row per lane (the immediate offset moves the
@@ -440,35 +433,41 @@ __device__ __forceinline__ void load_columns_to_lds(unsigned long long at, uint3
     }
   }
 }
-template <int kCount>
+template <int kCount, bool kOnce = false>
 __device__ __forceinline__ void load_rows_to_lds(const unsigned long long* at, uint32_t lds_base) {
   static_assert(kCount == 2 || kCount == 4, "rows");
   uint32_t saved;
+#define VA_TWO_ROWS(policy)                                                                                           \
+  asm volatile(                                                                                                       \
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"                                                           \
+      "global_load_lds_dwordx4 %1, off" policy "\n\t"                                                                 \
+      "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\t"                                                                         \
+      "global_load_lds_dwordx4 %2, off" policy "\n\t"                                                                 \
+      "s_mov_b32 m0, %0"                                                                                              \
+      : "=&s"(saved)                                                                                                  \
+      : "v"(at[0]), "v"(at[1]), "s"(lds_base)                                                                         \
+      : "memory", "scc")
+#define VA_FOUR_ROWS(policy)                                                                                          \
+  asm volatile(                                                                                                       \
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %5\n\ts_nop 0\n\t"                                                           \
+      "global_load_lds_dwordx4 %1, off" policy "\n\t"                                                                 \
+      "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\t"                                                                         \
+      "global_load_lds_dwordx4 %2, off" policy "\n\t"                                                                 \
+      "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\t"                                                                         \
+      "global_load_lds_dwordx4 %3, off" policy "\n\t"                                                                 \
+      "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\t"                                                                         \
+      "global_load_lds_dwordx4 %4, off" policy "\n\t"                                                                 \
+      "s_mov_b32 m0, %0"                                                                                              \
+      : "=&s"(saved)                                                                                                  \
+      : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "s"(lds_base)                                                 \
+      : "memory", "scc")
   if constexpr (kCount == 2) {
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, off\n\t"
-        "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\t"
-        "global_load_lds_dwordx4 %2, off\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(saved)
-        : "v"(at[0]), "v"(at[1]), "s"(lds_base)
-        : "memory", "scc");
+    if constexpr (kOnce) VA_TWO_ROWS(" nt"); else VA_TWO_ROWS("");
   } else {
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %5\n\ts_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, off\n\t"
-        "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\t"
-        "global_load_lds_dwordx4 %2, off\n\t"
-        "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\t"
-        "global_load_lds_dwordx4 %3, off\n\t"
-        "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\t"
-        "global_load_lds_dwordx4 %4, off\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(saved)
-        : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "s"(lds_base)
-        : "memory", "scc");
+    if constexpr (kOnce) VA_FOUR_ROWS(" nt"); else VA_FOUR_ROWS("");
   }
+#undef VA_TWO_ROWS
+#undef VA_FOUR_ROWS
 }
 // One word per lane, pool side -> LDS: lane l's four bytes land at lds_base + 4 l.
 __device__ __forceinline__ void load_word_to_lds(const void* src, uint32_t lds_base) {

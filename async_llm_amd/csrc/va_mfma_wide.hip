@@ -91,17 +91,6 @@ __device__ __forceinline__ uint32_t ring_slot(int tile) { return (uint32_t)tile 
 // 128-byte window.
 __device__ __forceinline__ int wide_vswz(int r) { return (r & 3) << 1; }
 
-// A transposing LDS read (ds_read_b64_tr_b16).  Within every group of 16 lanes, lane s supplies
-// the address of four 16-bit elements E[s][0..3]; lane i receives E[i / 4 + 4 k][i % 4], k = 0..3.
-// With lane s pointed at token T + s / 4, dims c + 4 (s % 4) .. + 3, lane i therefore receives
-// dim c + i of tokens T .. T + 3: four consecutive contraction elements of one row of V^T.
-__device__ __forceinline__ va_u32x2 lds_read_tr16(uint32_t lds_byte_address) {
-  typedef short v4s __attribute__((ext_vector_type(4)));
-  const v4s r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (__attribute__((address_space(3))) v4s*)(uintptr_t)lds_byte_address);
-  return __builtin_bit_cast(va_u32x2, r);
-}
-
 // max over the two half-waves (lanes l and l ^ 32) without touching LDS
 __device__ __forceinline__ float half_wave_max(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);

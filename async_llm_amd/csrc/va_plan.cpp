@@ -32,6 +32,8 @@ struct Item {
   int32_t link_begin, n_links, n_q, part_base, tokens, kind;
   int32_t unit;  // items that stream the same K/V chunk share a unit (planner only, not serialised)
   int32_t slot;  // wide items packed into one workgroup share a slot, -1: none (planner only)
+  int32_t together = 1;  // narrow items of its unit that one workgroup serves (planner only)
+  int32_t partners = 0;  // VA_I_PARTNERS
 };
 constexpr int kXcds = 8;  // accelerator dies of an MI355X, each with its own L2; workgroup b runs on die b % 8
 struct Link {
@@ -98,6 +100,22 @@ inline int32_t visible_end(int32_t len, int32_t nq, bool causal, int32_t b) {
   return causal ? std::min(len, len - nq + b) : len;
 }
 
+// Narrow tiles of a run of `tokens` that a workgroup serves together.  Four where the run is long: 64 readers of
+// 8192 tokens beside private blocks (16 q / 4 kv heads of 256 dims) 353 us a layer alone, 322 in pairs, 313 in fours.
+// Four tiles walk at two thirds of the pace of two when memory does not bound them, which a short run beside long ones
+// shows: 48 readers of 512 tokens, 483 us in pairs, 494 in fours.
+int tiles_together(int kernel, int page_size, int64_t tokens) {
+  return kernel != VA_KERNEL_MFMA ? 1 : page_size < 16 || tokens < 4096 ? 2 : VA_TOGETHER;
+}
+
+// Work items wanted per kv head.  The streaming kernel: 512 workgroups, but not so few items that their ends leave the
+// launch uneven.  Attention and merge of a layer under targets of 64 / 128 / 256 / 512 items: 64 requests over a
+// shared prompt 311 / 316 / 329 / 340 us and eight of 131072 tokens 644 / 641 / 651 / 668 (4 kv heads of 256 dims),
+// 32 requests over token slots 98 / 96 / 101 / 115 (8 of 128), 30 requests at 2 kv heads of 128 38.7 / 29.8 / 33.7 / 33.3.
+int default_target(int kernel, int num_kv_heads) {
+  return kernel == VA_KERNEL_MFMA ? std::max(512 / num_kv_heads, num_kv_heads > 8 ? 64 : 128) : std::max(64, 2048 / num_kv_heads);
+}
+
 // How finely the walks of chains may be cut (tokens; `gran` below is 64).  The cost of a wide tile's set-up in
 // walked tokens decides what a cut is worth; the floors keep the pieces of small launches worth their
 // launch.  The fine cuts are the rule: a chunk of 333 tokens over four blocks (16 q / 4 kv heads of 256 dims) used
@@ -159,8 +177,7 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   // group once the groups are known (group_is_wide below); narrow tiles are emitted chunk-major, so the
   // tiles that stream the same chunk run side by side and share it in L2.
   const bool wide_on_request = params && params->wide_tile > 0;
-  const int target = params && params->target_items > 0 ? params->target_items
-                                                        : std::max(64, 2048 / shape->num_kv_heads);
+  const int target = params && params->target_items > 0 ? params->target_items : default_target(kernel, shape->num_kv_heads);
   const int gran = 64;  // chunk boundaries are multiples of this many tokens
 
   // ---- stand-alone sub-requests: batch readers of identical KV lists ----
@@ -260,10 +277,17 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   }
 
   // ---- total tokens -> chunk size for split-KV ----
+  // (walks of a run of `gr`, whose tiles cut_tiles left in `tiles`: narrow tiles walk it together.  A recorded plan
+  // counts every tile: its capacity, and with it the workgroups that find nothing to do, hangs on the items.)
+  auto walks_of = [&](const Group& gr, bool may_be_wide) {
+    const int64_t n = (int64_t)tiles.size(), at_once = tiles_together(kernel, shape->page_size, s->seq_lens[gr.rep]);
+    return may_be_wide || cap ? n : (n + at_once - 1) / at_once;
+  };
   int64_t total_tokens = 0;
   for (auto& gr : groups) {
-    cut_tiles((int64_t)gr.subrows.size(), tiles, group_is_wide[&gr - &groups[0]]);
-    total_tokens += (int64_t)tiles.size() * s->seq_lens[gr.rep];
+    const bool may_be_wide = group_is_wide[&gr - &groups[0]];
+    cut_tiles((int64_t)gr.subrows.size(), tiles, may_be_wide);
+    total_tokens += walks_of(gr, may_be_wide) * s->seq_lens[gr.rep];
   }
   int64_t chain_tiles = 0, chain_tokens = 0, wide_chain_tokens = 0;
   for (auto& ch : chains) {
@@ -281,14 +305,33 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   // below -- so it is sized from their tokens alone: in a mixed batch the prefill chunks' long walks
   // would otherwise triple it, and the decode items would run in two long rounds instead of four short ones)
   int32_t kv_chunk = params && params->kv_chunk > 0 ? round_up(params->kv_chunk, gran) : 0;
+  bool one_round = false;  // the narrow items of the launch all start at once
   if (kv_chunk == 0) {
     const int64_t per_item = (total_tokens + target - 1) / target;
     // No chunk under four granules as a rule (an item's set-up is worth a few hundred tokens) -- unless the
     // launch holds so few tokens that such chunks would leave most of the machine idle: then the time of
     // the launch is the walk of ONE item, a chain of dependent trips to memory, and shorter walks side by
     // side (down to one granule) are what shortens it.
-    const int64_t spread = (total_tokens + (256 / shape->num_kv_heads) - 1) / std::max(1, 256 / shape->num_kv_heads);
-    const int64_t least = std::min<int64_t>(4 * gran, std::max<int64_t>(gran, round_up(spread, gran)));
+    int64_t least = 4 * gran;
+    if (kernel == VA_KERNEL_MFMA && per_item < 8 * gran) {
+      // The shortest chunks of up to eight granules whose items all run at once and leave a quarter of the room: chunks
+      // of 128 / 192 / 256 / 320 tokens, attention and merge of a layer, 4 requests of 2100..4000 tokens (4 kv heads of
+      // 256 dims, 60 / 43 / 35 / 29 items for 64 at once) 18.2 / 15.8 / 16.1 / 17.0 us; 256 / 320 / 384 / 512, 8 of
+      // 1400..4000 (8 of 128 dims, 69 / 60 / 53 / 42 for 64) 21.4 / 19.6 / 20.1 / 19.6.
+      const int64_t at_once = std::max(1, (shape->head_dim == 256 ? 192 : 384) / shape->num_kv_heads);
+      for (least = gran; least < 8 * gran; least += gran) {
+        int64_t n = 0;
+        for (size_t gi = 0; gi < groups.size(); ++gi) {
+          cut_tiles((int64_t)groups[gi].subrows.size(), tiles, group_is_wide[gi]);
+          n += walks_of(groups[gi], group_is_wide[gi]) * ((s->seq_lens[groups[gi].rep] + least - 1) / least);
+        }
+        one_round = n <= at_once;
+        if (one_round) break;
+      }
+    } else if (kernel != VA_KERNEL_MFMA) {
+      const int64_t spread = (total_tokens + (256 / shape->num_kv_heads) - 1) / std::max(1, 256 / shape->num_kv_heads);
+      least = std::min<int64_t>(least, std::max<int64_t>(gran, round_up(spread, gran)));
+    }
     kv_chunk = round_up(std::max<int64_t>(per_item, least), gran);
   }
 
@@ -346,6 +389,7 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
       const size_t a = tiles[ti].first, b = tiles[ti].second;
       emit((int32_t)(b - a), {Link{s->kv_indptr[rep], t0, t1, tile_qref[ti], VA_NO_CAUSAL, lflags}},
            [&](int32_t i) { return (int32_t)s->sub_worker[gr.subrows[a + i]]; }, unit);
+      out.items.back().together = tiles_together(kernel, shape->page_size, len);
     };
     auto chunk_len = [&](int32_t chunk) {
       const int32_t n_chunks = (len + chunk - 1) / chunk;
@@ -354,10 +398,10 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     // narrow tiles: chunk-major; wide tiles: their own (finer) chunking
     const int32_t per = chunk_len(kv_chunk);
     // The last chunk of a run is cut in two: every run then contributes short items, which the
-    // launch order puts last, so the launch does not end on a round of full-length items.
+    // launch order puts last, so the launch does not end on a round of full-length items (not where all run at once).
     std::vector<int32_t> cuts{0};
     for (int32_t t0 = per; t0 < len; t0 += per) cuts.push_back(t0);
-    if (len - cuts.back() >= 4 * gran) cuts.push_back(cuts.back() + round_up((len - cuts.back()) / 2, gran));
+    if (len - cuts.back() >= 4 * gran && !one_round) cuts.push_back(cuts.back() + round_up((len - cuts.back()) / 2, gran));
     cuts.push_back(len);
     for (size_t ci = 0; ci + 1 < cuts.size(); ++ci) {
       if (cuts[ci] >= cuts[ci + 1]) continue;
@@ -709,8 +753,8 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
         units.emplace_back();
       }
       Unit& u = units[at->second];
-      const int64_t cost = it.tokens;  // a tile streams its tokens once whatever its row count
-      u.cost += cost;
+      const int64_t cost = it.tokens;  // a tile streams its tokens once whatever its row count, and so do partners
+      if (u.members.size() % it.together == 0) u.cost += cost;
       u.item_cost = std::max(u.item_cost, cost);
       u.members.push_back(i);
     }
@@ -814,8 +858,15 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
         head.insert(head.end(), rest.begin(), rest.end());
         die_units[d].swap(head);
       }
-      for (int32_t u : die_units[d])
-        die_items[d].insert(die_items[d].end(), units[u].members.begin(), units[u].members.end());
+      for (int32_t u : die_units[d]) {
+        const std::vector<int32_t>& members = units[u].members;
+        for (size_t k = 0; k < members.size(); ++k) {
+          Item& it = out.items[members[k]];
+          const size_t follow = std::min<size_t>(it.together, members.size() - k) - 1;
+          it.partners = kind == 1 ? 0 : k % it.together ? -1 : (int32_t)follow;
+        }
+        die_items[d].insert(die_items[d].end(), members.begin(), members.end());
+      }
       depth = std::max(depth, die_items[d].size());
     }
     const Item padding{0, 0, 0, -1, 0, kind, -1, -1};
@@ -943,6 +994,7 @@ static int write_plan(const Built& b, const VaSubRequests* subs, const VaShape* 
     w[VA_I_PART_BASE] = it.part_base;
     w[VA_I_TOKENS] = it.tokens;
     w[VA_I_KIND] = it.kind;
+    w[VA_I_PARTNERS] = it.partners;
     if (it.n_links > 0) {
       const Link& l = b.links[it.link_begin];
       int32_t* lw = w + VA_I_LINK0;
@@ -1065,8 +1117,7 @@ extern "C" int va_plan_capacity(const VaShape* shape, const VaPlanParams* params
     if (wide_tile <= q_tile) wide_tile = 0;
   }
   const bool wide_groups = params && params->wide_tile > 0 && wide_tile > 0;
-  const int64_t target = params && params->target_items > 0 ? params->target_items
-                                                            : std::max(64, 2048 / shape->num_kv_heads);
+  const int64_t target = params && params->target_items > 0 ? params->target_items : default_target(kernel, shape->num_kv_heads);
   const int64_t subs = lim->max_sub_requests, sub_rows = lim->max_sub_rows;
   const int64_t chains = lim->max_chains, members = lim->max_chain_members, chain_rows = lim->max_chain_rows;
 

@@ -50,9 +50,16 @@ enum {
   VA_I_PART_BASE,  // first partial slot (one per query row), or -1: write `out` directly
   VA_I_TOKENS,     // KV tokens the item walks (scheduling weight)
   VA_I_KIND,       // 1: wide tile (more rows than the streaming kernel's tile)
+  VA_I_PARTNERS,   // narrow tiles that walk the same tokens: the first of up to VA_TOGETHER of them holds how many
+                   // follow at the next turns of its die (8 items apart) and its workgroup serves them all; they hold -1
   VA_I_LINK0 = 8,  // words 8..15: a copy of the item's first link, so that a kernel finds it with the
                    // same load as the item (one level less in the chain of dependent loads at its start)
 };
+
+// narrow tiles of the matrix-core path that one workgroup serves: fewer over scattered rows, whose index entries share
+// the LDS with the query rows
+#define VA_TOGETHER 4
+#define VA_TOGETHER_SCATTERED 2
 
 // link word indices
 enum {
