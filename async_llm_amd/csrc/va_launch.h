@@ -13,7 +13,8 @@ struct AttnArgs {
   const void* k_pool;
   const void* v_pool;
   long long pool_row_stride;  // elements between token slots
-  const int32_t* items;
+  const int32_t* items;         // wide items first
+  const int32_t* narrow_items;  // the narrow ones behind them
   const int32_t* links;
   const int32_t* qrefs;
   const int32_t* kv_indices;
@@ -49,10 +50,11 @@ int make_rope(const VaRope* rope, int head_dim, RopeDev* out);
 
 // Matrix-core attention (launched from va_mfma.hip).
 // `n_wide` leading items are wide tiles (va_mfma_wide.hip: `n_wide_slots` workgroups per kv head, each
-// running the items a.wide_slots gives it), the rest narrow ones (va_mfma_stream.hip).
+// running the items a.wide_slots gives it), the rest narrow ones: in the same launch behind the wide ones, or in
+// one of their own (va_mfma_stream.hip).
 int launch_mfma(const AttnArgs& a, int dtype, int n_items, int n_wide, int n_wide_slots, int q_tile,
                 hipStream_t stream);
-int launch_mfma_wide(const AttnArgs& a, int dtype, int n_slots, hipStream_t stream);
+int launch_mfma_wide(const AttnArgs& a, int dtype, int n_slots, int n_narrow, hipStream_t stream);
 int launch_mfma_stream(const AttnArgs& a, int dtype, int n_items, hipStream_t stream);
 
 }  // namespace va

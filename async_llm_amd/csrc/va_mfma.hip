@@ -6,7 +6,8 @@
 //     read the same KV run (up to four such tiles a workgroup), and short prefill tiles.  Bound by HBM.
 //   * wide kernel (va_mfma_wide.hip): query tiles of up to 128 MFMA rows for view-conditioned
 //     prefill.  Bound by the matrix pipe.
-// A plan lists its wide items first; each kind gets one launch.
+// A plan lists its wide items first.  Where it has both kinds one launch serves them: the streaming workgroups take
+// the CUs that the wide ones leave and, when those are done, all of them.
 #include <hip/hip_runtime.h>
 
 #include "va_internal.h"
@@ -42,11 +43,8 @@ int launch_mfma(const AttnArgs& a_in, int dtype, int n_items, int n_wide, int n_
     return va_fail(VA_ERR_ARG, "matrix-core path needs a 16-byte aligned cos|sin table");
   // the streaming kernel addresses a tile's rows with 32-bit byte offsets from its first row
   if (a.pool_row_stride * 2 * 16 > 0x7fffffffLL) return va_fail(VA_ERR_ARG, "pool rows too far apart");
-  if (n_wide > 0 && n_wide_slots > 0) {
-    const int rc = launch_mfma_wide(a, dtype, n_wide_slots, stream);
-    if (rc) return rc;
-  }
-  a.items += (long long)n_wide * VA_ITEM_WORDS;
+  a.narrow_items = a.items + (long long)n_wide * VA_ITEM_WORDS;
+  if (n_wide > 0 && n_wide_slots > 0) return launch_mfma_wide(a, dtype, n_wide_slots, n_items - n_wide, stream);
   return launch_mfma_stream(a, dtype, n_items - n_wide, stream);
 }
 

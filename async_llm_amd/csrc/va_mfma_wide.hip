@@ -35,6 +35,7 @@
 #include "va_internal.h"
 #include "va_launch.h"
 #include "va_mfma_common.h"
+#include "va_stream_tile.h"
 
 namespace va {
 
@@ -99,7 +100,7 @@ __device__ __forceinline__ float half_wave_max(float x) {
 
 // kGather: every token of the launch has an index entry of its own (slot lists, pages of 1, 2, 4 or 8 tokens).
 template <typename E, int kD, bool kGather>
-__global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArgs a) {
+__device__ __forceinline__ void wide_slot(const AttnArgs& a, unsigned workgroup, unsigned workgroups) {
   using S = typename E::storage;
   using Sh = WideShape<kD>;
   static_assert(!kGather || kWideAhead <= 2, "the entries of a tile are read a step after their request, behind its wait");
@@ -115,7 +116,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
   // K/V rows, so the die's L2 holds one head's stream at a time instead of all of them.
   ItemHead where;
   {
-    const unsigned die = blockIdx.x & 7u, turn = blockIdx.x >> 3, per_die = gridDim.x / (8u * a.num_kv_heads);
+    const unsigned die = workgroup & 7u, turn = workgroup >> 3, per_die = workgroups / (8u * a.num_kv_heads);
     unsigned g = 32;
     while (per_die % g) g >>= 1;
     const unsigned block = turn / (g * a.num_kv_heads), within = turn % (g * a.num_kv_heads);
@@ -922,51 +923,82 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
 }
 
 template <typename E, int kD, bool kGather>
-static int launch_wide_one(const AttnArgs& a, int n_items, hipStream_t stream) {
-  constexpr int bytes = WideShape<kD>::lds_bytes(kGather);
-  static bool configured = false;  // raising the limit is idempotent; a race only repeats the call
+__global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArgs a) {
+  wide_slot<E, kD, kGather>(a, blockIdx.x, gridDim.x);
+}
+
+// Wide and narrow items in one launch: `wide` workgroups of wide slots, then one per narrow item and kv head.  The wide
+// slots are bound by instruction issue and leave the memory idle, the streaming items are bound by memory and need few
+// CUs (one takes in up to 58 GB/s, all 256 share 6.9 TB/s).  The wide slots start first; the planner lets them leave so
+// many CUs that both kinds end together, and when they are done the remaining items have all CUs.  Attention and merge
+// of a layer, two launches and this one: 48 decode rows and 4 chunks of 512 tokens, contexts of 1 k..32 k, 16 q / 4 kv
+// heads of 256 dims 1229 -> 1090 us, 16 rows and 4 chunks of 256 503 -> 457, 24 rows and 4 chunks of 400, 32 q / 8 kv
+// heads of 128 dims 441 -> 373; where the streaming items are a few tail rows it saves their launch (plain prefill of 6
+// requests 0.7 %).  At head dims under 256 a streaming workgroup has a CU to itself here (registers of the wide
+// kind), beside another where no wide items are: all of 48 rows and 3 chunks at 64 dims 1222 -> 1232.
+template <typename E, int kD, bool kGather>
+__global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_joint_kernel(AttnArgs a, unsigned wide) {
+  if (blockIdx.x < wide) {
+    wide_slot<E, kD, kGather>(a, blockIdx.x, wide);
+  } else {
+    stream_block<E, kD, kGather>(a, blockIdx.x - wide);
+  }
+}
+
+template <typename E, int kD, bool kGather>
+static int launch_wide_one(const AttnArgs& a, int n_slots, int n_narrow, hipStream_t stream) {
+  constexpr int wide_bytes = WideShape<kD>::lds_bytes(kGather), narrow_bytes = StreamShape<kD>::lds_bytes(kGather);
+  constexpr int joint_bytes = wide_bytes > narrow_bytes ? wide_bytes : narrow_bytes;
+  static_assert(kWideThreads == kStreamThreads, "one launch serves both kinds");
+  static bool configured = false;  // raising the limits is idempotent; a race only repeats the calls
   if (!configured) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_mfma_wide_kernel<E, kD, kGather>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_mfma_wide_kernel<E, kD, kGather>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, wide_bytes);
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_mfma_joint_kernel<E, kD, kGather>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, joint_bytes);
     if (e != hipSuccess) return va_fail(VA_ERR_HIP, "raising the LDS limit: %s", hipGetErrorString(e));
     configured = true;
   }
-  const dim3 grid((unsigned)n_items * (unsigned)a.num_kv_heads), block(kWideThreads);
-  hipLaunchKernelGGL((attn_mfma_wide_kernel<E, kD, kGather>), grid, block, bytes, stream, a);
+  const unsigned wide = (unsigned)n_slots * (unsigned)a.num_kv_heads, narrow = (unsigned)n_narrow * (unsigned)a.num_kv_heads;
+  if (narrow > 0) {
+    hipLaunchKernelGGL((attn_mfma_joint_kernel<E, kD, kGather>), dim3(wide + narrow), dim3(kWideThreads), joint_bytes, stream, a, wide);
+  } else {
+    hipLaunchKernelGGL((attn_mfma_wide_kernel<E, kD, kGather>), dim3(wide), dim3(kWideThreads), wide_bytes, stream, a);
+  }
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? VA_OK : va_fail(VA_ERR_HIP, "wide attention launch: %s", hipGetErrorString(e));
 }
 
 template <typename E, int kD>
-static int launch_wide_dim(const AttnArgs& a, int n_items, hipStream_t stream) {
+static int launch_wide_dim(const AttnArgs& a, int n_slots, int n_narrow, hipStream_t stream) {
   // Pages of at least 16 tokens take one lookup per half tile, smaller ones (a slot list has pages of one) an
   // entry per token; the choice hangs on the page size alone, so that a recorded launch keeps its kernel.
   // (Other page sizes, slot lists beside larger pages, and rings built deeper than the index entries allow go
   // through the first kernel's per-lane lookups.)
-  if constexpr (kWideAhead <= 2) {
+  if constexpr (kWideAhead <= 2 && StreamShape<kD>::kBuffers <= 4) {
     if (a.page_size < 16 && (a.page_size & (a.page_size - 1)) == 0)
-      return launch_wide_one<E, kD, true>(a, n_items, stream);
+      return launch_wide_one<E, kD, true>(a, n_slots, n_narrow, stream);
   }
-  return launch_wide_one<E, kD, false>(a, n_items, stream);
+  return launch_wide_one<E, kD, false>(a, n_slots, n_narrow, stream);
 }
 
 template <typename E>
-static int launch_wide_typed(const AttnArgs& a, int n_items, hipStream_t stream) {
+static int launch_wide_typed(const AttnArgs& a, int n_slots, int n_narrow, hipStream_t stream) {
   switch (a.head_dim) {
     case 64:
-      return launch_wide_dim<E, 64>(a, n_items, stream);
+      return launch_wide_dim<E, 64>(a, n_slots, n_narrow, stream);
     case 128:
-      return launch_wide_dim<E, 128>(a, n_items, stream);
+      return launch_wide_dim<E, 128>(a, n_slots, n_narrow, stream);
     case 256:
-      return launch_wide_dim<E, 256>(a, n_items, stream);
+      return launch_wide_dim<E, 256>(a, n_slots, n_narrow, stream);
     default:
       return va_fail(VA_ERR_ARG, "matrix-core path supports head_dim 64, 128, 256");
   }
 }
 
-int launch_mfma_wide(const AttnArgs& a, int dtype, int n_items, hipStream_t stream) {
-  if (n_items == 0) return VA_OK;
-  return dtype == VA_BF16 ? launch_wide_typed<BF16>(a, n_items, stream) : launch_wide_typed<F16>(a, n_items, stream);
+int launch_mfma_wide(const AttnArgs& a, int dtype, int n_slots, int n_narrow, hipStream_t stream) {
+  return dtype == VA_BF16 ? launch_wide_typed<BF16>(a, n_slots, n_narrow, stream) : launch_wide_typed<F16>(a, n_slots, n_narrow, stream);
 }
 
 }  // namespace va

@@ -459,7 +459,8 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   // it in the die's L2.  A bundle of m <= lanes / 2 tiles has its walk cut into f = lanes / m parts
   // that run side by side (lane = part * m + tile), so a short chain still fills the group.
   const int64_t want_slots = pack ? std::max<int64_t>(1, std::min<int64_t>(target, slots_wanted)) : 1;
-  const int32_t lanes = (int32_t)std::max<int64_t>(1, want_slots / kXcds);
+  const int32_t all_lanes = (int32_t)std::max<int64_t>(1, want_slots / kXcds);
+  int32_t lanes = all_lanes;
   const int32_t groups_wanted = (int32_t)std::min<int64_t>(want_slots, kXcds);
   struct Bundle {
     int32_t first = 0, m = 0, f = 1;  // tiles [first, first + m) of the chain; f parts side by side
@@ -519,17 +520,48 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   };
   std::vector<Bundle> bundles;
   int64_t wide_walk = 0, wide_cost = 0;  // positions of all bundles; with their set-ups
-  if (pack) {
+  int64_t lane_cost = 0;  // over all lanes that have a part of a bundle
+  auto measure_bundles = [&]() {
+    wide_walk = wide_cost = lane_cost = 0;
     for (auto& ch : chains) {
       const int32_t nq = s->qo_indptr[ch[0] + 1] - s->qo_indptr[ch[0]];
       cut_tiles(nq, tiles);
       bundles_of(ch, nq, bundles);
       for (auto& bd : bundles) {
         wide_walk += bd.part;
-        wide_cost += bd.cost(0, bd.part, seg_cost);
+        const int64_t cost = bd.cost(0, bd.part, seg_cost);
+        wide_cost += cost;
+        lane_cost += cost * bd.m * bd.f;
       }
     }
+  };
+  if (pack && total_tokens > 0 && wide_chain_tokens > 0) {
+    // The launch holds the runs of stand-alone sub-requests as well.  A CU left to those while the wide slots run takes
+    // in twice what it gets when all of them stream (52 against 26 bytes a ns: 256 share what the memory gives), so some
+    // lanes give theirs up: as many as the estimated end of the launch says.  Rates: a wide tile walks a token in 32 ns
+    // where all CUs hold one and in 28 where few do (the clock), what is left to stream behind the wide slots goes out
+    // at 6560 bytes a ns and ends unevenly.  Estimated and measured, us, by lanes (of 8, 16 q / 4 kv heads of 256 dims):
+    // 48 decode rows and 4 chunks of 512, 8 / 7 / 6 / 5 lanes: 1290 / 1160 / 1115 / 1190, 1205 / 1143 / 1093 / 1125
+    // (two launches 1229); 16 rows and 4 chunks of 256: 507 / 471 / 401 / 575, 497 / 472 / 453 / 525 (503);
+    // 40 rows and 3 chunks of 333: 452 / 340 / 342 / 338, 467 / 417 / 396 / 382.
+    const double bytes = 2.0 * (double)total_tokens * shape->num_kv_heads * shape->head_dim * (shape->dtype == VA_F32 ? 4 : 2);
+    double best = 0, all_end = 0;
+    int32_t best_lanes = all_lanes;
+    for (; lanes >= 1; lanes -= std::max(1, all_lanes / 8)) {
+      measure_bundles();
+      const double token_ns = 28.0 + 4.0 * lanes / all_lanes, wide_ns = token_ns * (double)wide_cost / groups_wanted;
+      const double idle_ns = std::max(0.0, 256.0 * wide_ns - token_ns * (double)lane_cost * shape->num_kv_heads);
+      const double rest_ns = std::max(0.0, bytes - std::min(52.0 * idle_ns, 6560.0 * wide_ns)) / 6560.0;
+      const double end = wide_ns + rest_ns + std::min(rest_ns, 40e3);
+      if (lanes == all_lanes) all_end = end;
+      if (lanes == all_lanes || end < 0.98 * best) {
+        best = end;
+        best_lanes = lanes;
+      }
+    }
+    lanes = best < 0.92 * all_end ? best_lanes : all_lanes;  // (an estimate: it has to promise something)
   }
+  if (pack) measure_bundles();
   // The room of a new group is the even share of what is still to be placed over the groups still
   // to be opened, so that a group closed early (less than min_piece of its room left) or run over (a
   // bundle's short remainder kept with the piece before it) is made up for by the groups after it,
