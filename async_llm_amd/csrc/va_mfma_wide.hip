@@ -20,8 +20,8 @@
 //
 // The loop is a hand-ordered software pipeline: the scores of tile i + 1 run on the matrix pipe
 // under the exponentials of tile i (each taken of scale * score - reference, formed in fp32 right
-// in front of it), the products of tile i under the maxima of tile i + 1.  Interior tiles of a link
-// take a branch-free ring step, in a loop of their own.
+// in front of it), the products of tile i under the maxima of tile i + 1 and, at head dims under 256, some of its
+// exponentials.  Interior tiles of a link take a branch-free ring step, in a loop of their own.
 // V tiles keep whole rows in LDS, unpadded and swizzled (piece c of row r at position c ^ swz(r)); K
 // tiles land in fragment order (8-token x 128-byte blocks, see the load pattern in the kernel), so
 // that the K reads of a tile share one address register.  The query never goes through LDS: every
@@ -66,6 +66,14 @@ struct WideShape {
   // spills.  D = 256 therefore runs one block per wave.
   static constexpr int kBlocks = kD == 256 ? 1 : 2;
   static constexpr int kWaveRows = 32 * kBlocks;
+  // Of the sixteen elements a lane has of a row block's tile, those whose exponentials are taken under the P.V products
+  // of the tile before (steady part of a link).  Measured, attention and merge of a layer, 0 / 4 / 6 / 8 elements at 128
+  // dims: 8 x 1500..2048 rows over 8000 tokens (32 q / 8 kv heads, bf16) 2500 / 2052 / 2013 / 2025 us, 4 of 300..1500
+  // over up to six blocks (float16) 600 / 582 / 573 / 573, plain prefill of 6 356 / 332 / 332 / 334; 0 / 4 / 8 / 10
+  // at 64 dims (64 q / 16 kv heads): 4 x 300..1000 over 4000 tokens 324 / 299 / 299 / 294, plain prefill 518 / 441 / 438
+  // / 434.  At 256 dims the P.V products are twice as many per exponential, and full of V reads: 0 / 2 / 4 elements
+  // 9950 / 10160 / 10260 us for 8 x 2048 rows over 41 k tokens.
+  static constexpr int kEarly = kD == 256 ? 0 : kD == 128 ? 6 : 10;
   static constexpr int kTileRows = kWideWaves * kWaveRows;  // MFMA rows per workgroup
   // The cosines and sines of an mRoPE tile (at most one row per MFMA row, kD / 2 entries of four bytes)
   // lie behind the tiles requested during the set-up: at D = 256 in the rest of the ring (128 KB in all),
@@ -550,7 +558,9 @@ __device__ __forceinline__ void wide_slot(const AttnArgs& a, unsigned workgroup,
     // can keep the matrix pipe busy, so the loop body is written as pieces pinned in order with
     // scheduling barriers: while the scores of tile i+1 are computed (matrix pipe), the
     // exponentials of tile i run on the vector ALU; while the products P.V of tile i run, the V
-    // fragments of the next product are transposed.
+    // fragments of the next product are transposed, the maxima of tile i+1 are taken and, at head dims under 256, its
+    // first exponentials (kEarly).  A product takes 32 clocks and its issue four, an exponential with its multiply-add,
+    // sum and half a packing 26: two under each score product, as 128 dims have them, do not fit, one does.
     //
     // Ring.  ring_step(k): wait until tile k has landed for the whole workgroup (one barrier) and
     // request tile k + 2 into the buffer of tile k - 2, which every wave has left by then.  Every
@@ -776,6 +786,114 @@ __device__ __forceinline__ void wide_slot(const AttnArgs& a, unsigned workgroup,
         __builtin_amdgcn_sched_barrier(0);
       }
     };
+    // The same tile in the steady part of a link at head dims under 256, whose two row blocks take twice the
+    // exponentials per product: under the score products alone they do not fit, so the first kEarly elements of a tile
+    // are taken under the P.V products of the tile before (`sum` and `pw` carry them), ahead of the test of its maxima.
+    // Where the test then raises the reference they are dropped and the tile's scores are computed anew.
+    constexpr int kEarly = Sh::kEarly;
+    float sum[kB];
+    uint32_t pw[kB][8];
+    // element r of block b, part [first, end): exponential, the sum and the packing one element behind
+    auto exp_element = [&](auto& of, int b, int r, int first) __attribute__((always_inline)) {
+      of[b][r] = __builtin_amdgcn_exp2f(fmaf(of[b][r], a.scale_log2, -m_ref[b]));
+      if (r > first) sum[b] += of[b][r - 1];
+      if (r % 2 == 0 && r > first) pw[b][r / 2 - 1] = Mma<E>::pack(of[b][r - 2], of[b][r - 1]);
+    };
+    auto exp_finish = [&](auto& of, int b, int end) __attribute__((always_inline)) {
+      sum[b] += of[b][end - 1];
+      pw[b][end / 2 - 1] = Mma<E>::pack(of[b][end - 2], of[b][end - 1]);
+    };
+    auto early_exps = [&](auto& of) __attribute__((always_inline)) {  // (not under anything: the first tile of the part)
+#pragma unroll
+      for (int b = 0; b < kB; ++b) sum[b] = 0.f;
+#pragma unroll
+      for (int r = 0; r < kEarly; ++r)
+#pragma unroll
+        for (int b = 0; b < kB; ++b) exp_element(of, b, r, 0);
+#pragma unroll
+      for (int b = 0; b < kB; ++b) exp_finish(of, b, kEarly);
+    };
+    auto steady_body = [&](int i, auto& cur, auto& nxt) __attribute__((always_inline)) {
+      const uint32_t vt = lds_base + ring_slot(i) * Sh::kBufferBytes + Sh::kTileBytes;
+      const uint32_t vt_even = vt + v_even, vt_odd = vt + v_odd;
+      constexpr int kFrags = 2 * kDimTiles, kVAhead = kFrags < 4 ? kFrags : 4;
+      va_u32x4 vfr[kVAhead];
+      auto read_vfrag = [&](int idx) __attribute__((always_inline)) {
+        const int kk = idx / kDimTiles, t = idx % kDimTiles;
+        const uint32_t at = ((t & 1) ? vt_odd : vt_even) + 128 * (t / 2) + kk * 16 * kRowBytes;
+        const va_u32x2 lo = lds_read_tr16(at), hi = lds_read_tr16(at + 8 * kRowBytes);
+        vfr[idx % kVAhead] = va_u32x4{lo[0], lo[1], hi[0], hi[1]};
+      };
+      // ---- phase A: scores of tile i + 1 under the rest of the exponentials of tile i ----
+      constexpr int kPieces = kB * (16 - kEarly), kLead = 2, kSlots = kB * kSteps;
+      auto piece = [&](int n) __attribute__((always_inline)) { exp_element(cur, n % kB, kEarly + n / kB, kEarly); };
+      read_k(i + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < kLead; ++n) piece(n);  // while the first K fragment is on its way
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int slot = 0; slot < kSlots; ++slot) {
+        const int step = slot / kB, b = slot % kB;
+        nxt[b] = Mma<E>::run32(kf[step % kKRing], qf[b][step], step == 0 ? va_f32x16{} : nxt[b]);
+        if (b == kB - 1 && step + kKRing < kSteps) read_k_fragment(i + 1, step + kKRing);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = kLead; n < kPieces; ++n)
+          if ((n - kLead) * kSlots / (kPieces - kLead) == slot) piece(n);
+        if (slot == kSlots / 2) {
+#pragma unroll
+          for (int idx = 0; idx < kVAhead; ++idx) read_vfrag(idx);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int b = 0; b < kB; ++b) {
+        exp_finish(cur, b, 16);
+        l_run[b] += sum[b];
+        sum[b] = 0.f;
+      }
+      va_u32x4 pf[2][kB];
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int b = 0; b < kB; ++b)
+          pf[kk][b] = va_u32x4{pw[b][4 * kk + 0], pw[b][4 * kk + 1], pw[b][4 * kk + 2], pw[b][4 * kk + 3]};
+      __builtin_amdgcn_sched_barrier(0);
+      // ---- phase B: O^T += V^T . P^T under the first exponentials and the maxima of tile i + 1 (from the third
+      // product on: the scores are written by then).  The maxima come first, the exponentials are taken in place. ----
+      constexpr int kProducts = kB * kFrags, kFirst = 2;
+      // of block b: eight maxima of three, ahead of the exponential of the first element each of them takes in
+      auto max_piece = [&](int b, int e) __attribute__((always_inline)) {
+        early_max[b] = e == 0 ? fmaxf(nxt[b][0], nxt[b][1]) : fmaxf(fmaxf(early_max[b], nxt[b][2 * e]), nxt[b][2 * e + 1]);
+      };
+      constexpr int kMaxes = kB * 8, kExps = kB * kEarly, kUnderB = kMaxes + kExps;
+#pragma unroll
+      for (int product = 0; product < kProducts; ++product) {
+        const int idx = product / kB, b = product % kB, kk = idx / kDimTiles, t = idx % kDimTiles;
+        Mma<E>::run32_acc(vfr[idx % kVAhead], pf[kk][b], o[b][t]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (b == kB - 1 && idx + kVAhead < kFrags) read_vfrag(idx + kVAhead);
+        if (product >= kFirst) {
+#pragma unroll
+          for (int n = 0; n < kUnderB; ++n) {
+            // the maxima of the elements that are exponentiated here go ahead of them, the others behind
+            if (kFirst + n * (kProducts - kFirst) / kUnderB != product) continue;
+            constexpr int kHead = kB * kEarly / 2;
+            if (n < kHead) {
+              max_piece(n % kB, n / kB);
+            } else if (n < kHead + kExps) {
+              exp_element(nxt, (n - kHead) % kB, (n - kHead) / kB, 0);
+            } else {
+              max_piece((n - kExps) % kB, (n - kExps) / kB);
+            }
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int b = 0; b < kB; ++b) exp_finish(nxt, b, kEarly);
+    };
     // The reference of the rows is raised to the maxima of the tile in `cur` (m_tile, log2 units): what was
     // accumulated against the old reference is rescaled; the tile's raw scores stay as they are.
     auto raise_reference = [&](int i, auto& cur) __attribute__((always_inline)) {
@@ -811,58 +929,58 @@ __device__ __forceinline__ void wide_slot(const AttnArgs& a, unsigned workgroup,
     int i = 0;
     while (i < n_vis) {
       bool raise = false;
-      if (i >= 1 && i < i_steady_end) {
-        if constexpr (kGather) {
-          // (written without a break in the middle: with one the compiler keeps the accumulators of before
-          // and after the products side by side, copies one to the other every tile and spills)
-          do {
+      // (a part of one tile is not worth the exponentials and scores that entering and leaving it take)
+      if (i >= 1 && i + (kEarly > 0) < i_steady_end && !steady_test()) {
+        if constexpr (kEarly > 0) early_exps(sc);
+        // (written without a break in the middle: with one the compiler keeps the accumulators of before and after the
+        // products side by side, copies one to the other every tile and spills)
+        do {
+          if constexpr (kGather) {
             ring_step_gather();
-            raise = steady_test();
-            if (!raise) {
-              tile_body(i, sc, sc_next);
-#pragma unroll
-              for (int b = 0; b < kB; ++b) sc[b] = sc_next[b];
-              ++i;
-            }
-          } while (!raise && i < i_steady_end);
-        } else {
-          do {
+          } else {
             ring_step_steady();
-            raise = steady_test();
-            if (raise) break;
+          }
+          if constexpr (kEarly > 0) {
+            steady_body(i, sc, sc_next);
+          } else {
             tile_body(i, sc, sc_next);
+          }
 #pragma unroll
-            for (int b = 0; b < kB; ++b) sc[b] = sc_next[b];
-            ++i;
-          } while (i < i_steady_end);
-        }
+          for (int b = 0; b < kB; ++b) sc[b] = sc_next[b];
+          ++i;
+          raise = steady_test();
+        } while (!raise && i < i_steady_end);
         early_max_valid = true;  // (a next tile exists throughout the steady part)
-        if (!raise) continue;
-      } else {
-        const int t0 = tok_begin + i * kWideTokens;
-        if (i + 1 < n_tiles) ring_step();  // tile i + 1 has landed
-        // mask and find the tile maxima; reg r of a block is token t0 + (r/4)*8 + 4h + r%4 of its row
-        const bool masked = t0 + kWideTokens > t_wave_min;
+        if constexpr (kEarly > 0) {  // the general step wants the scores of its tile as they were
+          read_k(i);
 #pragma unroll
-        for (int b = 0; b < kB; ++b) {
-          if (masked) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-              sc[b][r] = (t0 + (r / 4) * 8 + 4 * h + (r % 4)) < t_row[b] ? sc[b][r] : -INFINITY;
-          }
-          // the tile maximum (raw): from the maxima found under the previous products, or, for a masked or
-          // first tile, from sc
-          float tile_max = early_max[b];
-          if (masked || !early_max_valid) {
-            tile_max = sc[b][0];
-#pragma unroll
-            for (int r = 1; r < 16; ++r) tile_max = fmaxf(tile_max, sc[b][r]);
-          }
-          m_tile[b] = half_wave_max(tile_max) * a.scale_log2;
-          raise = raise || m_tile[b] > raise_above[b];
+          for (int s = 0; s < kSteps; ++s) score_step(i, s, sc);
         }
-        raise = __any(raise);
+        raise = false;  // (it makes the test again)
       }
+      const int t0 = tok_begin + i * kWideTokens;
+      if (i + 1 < n_tiles) ring_step();  // tile i + 1 has landed
+      // mask and find the tile maxima; reg r of a block is token t0 + (r/4)*8 + 4h + r%4 of its row
+      const bool masked = t0 + kWideTokens > t_wave_min;
+#pragma unroll
+      for (int b = 0; b < kB; ++b) {
+        if (masked) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            sc[b][r] = (t0 + (r / 4) * 8 + 4 * h + (r % 4)) < t_row[b] ? sc[b][r] : -INFINITY;
+        }
+        // the tile maximum (raw): from the maxima found under the previous products, or, for a masked or
+        // first tile, from sc
+        float tile_max = early_max[b];
+        if (masked || !early_max_valid) {
+          tile_max = sc[b][0];
+#pragma unroll
+          for (int r = 1; r < 16; ++r) tile_max = fmaxf(tile_max, sc[b][r]);
+        }
+        m_tile[b] = half_wave_max(tile_max) * a.scale_log2;
+        raise = raise || m_tile[b] > raise_above[b];
+      }
+      raise = __any(raise);
       if (raise) raise_reference(i, sc);
       tile_body(i, sc, sc_next);
 #pragma unroll
