@@ -60,6 +60,9 @@ class LaunchPlan:
     staging: Optional[torch.Tensor] = None
     coarse: Optional["LaunchPlan"] = None
 
+    def __post_init__(self) -> None:
+        self.header_ptr = self.header.ctypes.data
+
 
 @dataclass
 class SharedCacheAttnMetadata(BaseAttnMetadata):
@@ -703,42 +706,50 @@ class SharedCacheAttention:
     def store_new_kv(self, k: torch.Tensor, v: torch.Tensor, layer_id: int, batch) -> None:
         """Rotate the new keys to their block-relative positions and write K and
         V rows to ``batch.out_loc`` (negative slots are skipped)."""
-        native.require_device(k, "k")
+        pools = (self.kv_cache.k_cache(layer_id), self.kv_cache.v_cache(layer_id)) if self.fused_store else (None, None)
+        self._store(k, v, layer_id, batch, pools, native.current_stream_ptr(self.device))
+
+    def _store(self, k, v, layer_id: int, batch, pools, stream: int) -> None:
+        if not k.is_cuda:
+            native.require_device(k, "k")
         W = k.shape[0]
         if W == 0:
             return
         Hkv, D = self.num_kv_heads, self.head_dim
         key_pos = batch.positions if batch.mrope_positions is None else batch.mrope_positions
-        key_pos = key_pos.to(device=self.device, dtype=torch.int64)
+        if key_pos.dtype != torch.int64 or key_pos.device != k.device:
+            key_pos = key_pos.to(device=self.device, dtype=torch.int64)
         if not self.fused_store:
             k_rot = self._rope(k.reshape(W, Hkv, D), key_pos)
             self.kv_cache.store_kv(k_rot.view(W, Hkv * D), v.reshape(W, Hkv * D), batch.out_loc, layer_id)
             return
-        axis_stride = 0
-        if key_pos.dim() == 2:
-            key_pos = key_pos.contiguous()
-            axis_stride = key_pos.shape[1]
-        else:
-            key_pos = key_pos.contiguous()
+        key_pos = key_pos.contiguous()
+        axis_stride = key_pos.shape[1] if key_pos.dim() == 2 else 0
         assert key_pos.shape[-1] == W
-        k2 = k.reshape(W, Hkv * D)
-        v2 = v.reshape(W, Hkv * D)
-        if k2.stride(-1) != 1:
-            k2 = k2.contiguous()
-        if v2.stride(-1) != 1:
-            v2 = v2.contiguous()
-        k_pool = self.kv_cache.k_cache(layer_id)
-        v_pool = self.kv_cache.v_cache(layer_id)
+        k2, k_stride = self._rows(k, Hkv)
+        v2, v_stride = self._rows(v, Hkv)
         if layer_id not in self._checked_layers:
             self._check_pool_layout(layer_id)
             self._checked_layers.add(layer_id)
         out_loc = batch.out_loc
-        assert out_loc.dtype in (torch.int32, torch.int64) and out_loc.numel() == W
+        wide_slots = out_loc.dtype == torch.int64
+        assert (wide_slots or out_loc.dtype == torch.int32) and out_loc.numel() == W
         out_loc = out_loc.contiguous()
         native.check(native.lib.va_store_kv_rope(
-            k2.data_ptr(), v2.data_ptr(), k2.stride(0), v2.stride(0), k_pool.data_ptr(), v_pool.data_ptr(),
-            Hkv * D, out_loc.data_ptr(), int(out_loc.dtype == torch.int64), key_pos.data_ptr(), axis_stride,
-            W, self._shape, self._rope_descriptor(), native.current_stream_ptr(self.device)))
+            k2.data_ptr(), v2.data_ptr(), k_stride, v_stride, pools[0].data_ptr(), pools[1].data_ptr(),
+            Hkv * D, out_loc.data_ptr(), wide_slots, key_pos.data_ptr(), axis_stride,
+            W, self._shape, self._rope_descriptor(), stream))
+
+    def _rows(self, x: torch.Tensor, heads: int):
+        """``x`` as ``[rows, heads * head_dim]`` with adjacent elements, and its row stride."""
+        width = heads * self.head_dim
+        if x.dim() != 2 or x.shape[1] != width:
+            x = x.reshape(x.shape[0], width)
+        row, element = x.stride()
+        if element != 1:
+            x = x.contiguous()
+            row = width
+        return x, row
 
     def attend(self, q: torch.Tensor, layer_id: int, meta: SharedCacheAttnMetadata,
                return_lse: bool = False, lse_base2: bool = False, out: Optional[torch.Tensor] = None,
@@ -748,37 +759,42 @@ class SharedCacheAttention:
         ``static_scratch`` (and ``out`` / ``lse`` given) the call goes through
         ``va_attention_static`` and allocates nothing: the partial states live in
         the library's own per-GPU array, which bounds the plan's size."""
-        native.require_device(q, "q")
+        pools = self.kv_cache.k_cache(layer_id), self.kv_cache.v_cache(layer_id)
+        return self._attend(q, meta, pools, native.current_stream_ptr(self.device), return_lse, lse_base2, out, lse,
+                            static_scratch)
+
+    def _attend(self, q, meta, pools, stream: int, return_lse: bool = False, lse_base2: bool = False, out=None, lse=None,
+                static_scratch: bool = False):
+        if not q.is_cuda:
+            native.require_device(q, "q")
         launch = meta.launch
         assert launch is not None, "metadata carries no launch plan"
         if static_scratch:
             launch = self._within_static_scratch(launch)
         W, Hq, D = meta.num_workers, self.num_qo_heads, self.head_dim
-        q2 = q.reshape(q.shape[0], Hq * D)
-        if q2.stride(-1) != 1:
-            q2 = q2.contiguous()
+        q2, q_stride = self._rows(q, Hq)
         assert q2.shape[0] >= W and q2.dtype == self.dtype
         if out is None:
             out = torch.empty((W, Hq * D), dtype=self.dtype, device=self.device)
-        if lse is None and return_lse:
-            lse = torch.empty((W, Hq), dtype=torch.float32, device=self.device)
-        assert out.shape == (W, Hq * D) and out.dtype == self.dtype and out.is_contiguous()
-        assert lse is None or (lse.shape == (W, Hq) and lse.dtype == torch.float32 and lse.is_contiguous())
-        k_pool = self.kv_cache.k_cache(layer_id)
-        v_pool = self.kv_cache.v_cache(layer_id)
+        else:
+            assert out.shape == (W, Hq * D) and out.dtype == self.dtype and out.is_contiguous()
+        if lse is None:
+            lse = torch.empty((W, Hq), dtype=torch.float32, device=self.device) if return_lse else None
+        else:
+            assert lse.shape == (W, Hq) and lse.dtype == torch.float32 and lse.is_contiguous()
         sub_loc = meta.sub_loc
         axis_stride = sub_loc.stride(0) if sub_loc.dim() == 2 else 0
-        head = (q2.data_ptr(), q2.stride(0), k_pool.data_ptr(), v_pool.data_ptr(), self.num_kv_heads * D,
-                launch.blob.data_ptr(), launch.header.ctypes.data, launch.kv_indices.data_ptr(),
+        head = (q2.data_ptr(), q_stride, pools[0].data_ptr(), pools[1].data_ptr(), self.num_kv_heads * D,
+                launch.blob.data_ptr(), launch.header_ptr, launch.kv_indices.data_ptr(),
                 meta.sub_worker.data_ptr(), sub_loc.data_ptr(), axis_stride, out.data_ptr(),
                 None if lse is None else lse.data_ptr(), int(lse_base2))
-        tail = (self._shape, self._rope_descriptor(), native.current_stream_ptr(self.device))
         if static_scratch:
-            native.check(native.lib.va_attention_static(*head, *tail))
+            native.check(native.lib.va_attention_static(*head, self._shape, self._rope_descriptor(), stream))
         else:
             ws = launch.workspace
             native.check(native.lib.va_attention(*head, None if ws is None else ws.data_ptr(),
-                                                 0 if ws is None else ws.numel(), *tail))
+                                                 0 if ws is None else ws.numel(), self._shape, self._rope_descriptor(),
+                                                 stream))
         return (out, lse) if return_lse else out
 
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layer_id: int, batch) -> torch.Tensor:
@@ -788,11 +804,19 @@ class SharedCacheAttention:
         ``[W, Hq*D]`` (reference ``attention.py:624-703``)."""
         meta = batch.attn_metadata
         assert isinstance(meta, SharedCacheAttnMetadata)
-        self.store_new_kv(k, v, layer_id, batch)
-        return self.attend(q, layer_id, meta)
+        return self._forward(q, k, v, layer_id, batch, meta)
+
+    def _forward(self, q, k, v, layer_id: int, batch, meta, *attend_args):
+        if not self.fused_store:
+            self.store_new_kv(k, v, layer_id, batch)
+            return self.attend(q, layer_id, meta, *attend_args)
+        # (the layer's pools and the stream are asked for once: together they cost as much as a launch)
+        pools = self.kv_cache.k_cache(layer_id), self.kv_cache.v_cache(layer_id)
+        stream = native.current_stream_ptr(self.device)
+        self._store(k, v, layer_id, batch, pools, stream)
+        return self._attend(q, meta, pools, stream, *attend_args)
 
     def forward_with_lse(self, q, k, v, layer_id: int, batch, lse_base2: bool = False):
         """``forward`` that also returns the merged logsumexp ``[W, Hq]``."""
         meta = batch.attn_metadata
-        self.store_new_kv(k, v, layer_id, batch)
-        return self.attend(q, layer_id, meta, return_lse=True, lse_base2=lse_base2)
+        return self._forward(q, k, v, layer_id, batch, meta, True, lse_base2)
