@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "va_device.h"
 
 namespace va {
@@ -47,6 +49,18 @@ struct MergeArgs {
 
 // Validate a rotation description and turn it into its device form.
 int make_rope(const VaRope* rope, int head_dim, RopeDev* out);
+
+// Allows `kernel` that much dynamic LDS on the current device (more than 64 KB has to be asked for, on every device
+// that runs the kernel).  `devices`: a bit for each that has it; a race only repeats the call.
+inline hipError_t allow_lds(const void* kernel, int bytes, std::atomic<unsigned long long>& devices) {
+  int device = 0;
+  hipError_t e = hipGetDevice(&device);
+  const unsigned long long bit = device < 64 ? 1ull << device : 0;
+  if (e != hipSuccess || (devices.load(std::memory_order_relaxed) & bit)) return e;
+  e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e == hipSuccess) devices.fetch_or(bit, std::memory_order_relaxed);
+  return e;
+}
 
 // Matrix-core attention (launched from va_mfma.hip).
 // `n_wide` leading items are wide tiles (va_mfma_wide.hip: `n_wide_slots` workgroups per kv head, each

@@ -16,14 +16,10 @@ template <typename E, int kD, bool kGather>
 static int launch_stream_one(const AttnArgs& a, int n_items, hipStream_t stream) {
   const dim3 grid((unsigned)n_items * (unsigned)a.num_kv_heads), block(kStreamThreads);
   constexpr int bytes = StreamShape<kD>::lds_bytes(kGather);
-  if constexpr (bytes > 64 * 1024) {  // (deeper rings than the default need the limit raised)
-    static bool configured = false;  // raising the limit is idempotent; a race only repeats the call
-    if (!configured) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_stream_kernel<E, kD, kGather>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-      if (e != hipSuccess) return va_fail(VA_ERR_HIP, "raising the LDS limit: %s", hipGetErrorString(e));
-      configured = true;
-    }
+  if constexpr (bytes > 64 * 1024) {
+    static std::atomic<unsigned long long> devices{0};
+    const hipError_t e = allow_lds(reinterpret_cast<const void*>(&attn_stream_kernel<E, kD, kGather>), bytes, devices);
+    if (e != hipSuccess) return va_fail(VA_ERR_HIP, "raising the LDS limit: %s", hipGetErrorString(e));
   }
   hipLaunchKernelGGL((attn_stream_kernel<E, kD, kGather>), grid, block, bytes, stream, a);
   const hipError_t e = hipGetLastError();

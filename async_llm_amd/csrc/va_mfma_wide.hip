@@ -1068,17 +1068,12 @@ static int launch_wide_one(const AttnArgs& a, int n_slots, int n_narrow, hipStre
   constexpr int wide_bytes = WideShape<kD>::lds_bytes(kGather), narrow_bytes = StreamShape<kD>::lds_bytes(kGather);
   constexpr int joint_bytes = wide_bytes > narrow_bytes ? wide_bytes : narrow_bytes;
   static_assert(kWideThreads == kStreamThreads, "one launch serves both kinds");
-  static bool configured = false;  // raising the limits is idempotent; a race only repeats the calls
-  if (!configured) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_mfma_wide_kernel<E, kD, kGather>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, wide_bytes);
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_mfma_joint_kernel<E, kD, kGather>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, joint_bytes);
-    if (e != hipSuccess) return va_fail(VA_ERR_HIP, "raising the LDS limit: %s", hipGetErrorString(e));
-    configured = true;
-  }
   const unsigned wide = (unsigned)n_slots * (unsigned)a.num_kv_heads, narrow = (unsigned)n_narrow * (unsigned)a.num_kv_heads;
+  static std::atomic<unsigned long long> wide_devices{0}, joint_devices{0};
+  const hipError_t allowed =
+      narrow > 0 ? allow_lds(reinterpret_cast<const void*>(&attn_mfma_joint_kernel<E, kD, kGather>), joint_bytes, joint_devices)
+                 : allow_lds(reinterpret_cast<const void*>(&attn_mfma_wide_kernel<E, kD, kGather>), wide_bytes, wide_devices);
+  if (allowed != hipSuccess) return va_fail(VA_ERR_HIP, "raising the LDS limit: %s", hipGetErrorString(allowed));
   if (narrow > 0) {
     hipLaunchKernelGGL((attn_mfma_joint_kernel<E, kD, kGather>), dim3(wide + narrow), dim3(kWideThreads), joint_bytes, stream, a, wide);
   } else {
