@@ -225,29 +225,35 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     }
   }
 
-  // Wide tiles for a group.  n readers in narrow tiles stream their block ceil(n / q_tile) times (once
-  // from memory, then from the die's L2), in wide tiles wide_tile / q_tile times less often -- but wide
-  // tiles run in a launch of their own, whose workgroups each stage a whole tile of queries and write a
-  // whole tile of partial states.  Measured at 16 q / 4 kv heads, head_dim 256, bf16 (q_tile 4, wide_tile
-  // 32 readers): 64 readers of an 8192-token block save 0.47 GB of such re-reads and the launch costs what
-  // they cost (401 -> 403 us); 128 readers of it save 0.94 GB (797 -> 759 us), 64 readers of a 32768-token
-  // block 1.9 GB (494 -> 443 us).  So: on request always; otherwise (plans of free size only) when the
-  // groups that would each save a fair share together save more than 0.64 GB.
+  // Wide tiles for a group.  n readers in narrow tiles stream their block once for every workgroup's tiles (once from
+  // memory, then from the die's L2), in wide tiles half as often or less, but narrow items beside wide ones have a CU
+  // to themselves, and wide tiles write whole tiles of partial states.  At head dims under 256, where a CU otherwise
+  // holds two narrow items, that is never worth it: 128 readers of 8192 tokens beside blocks of 256..2048 tokens, 32 q /
+  // 8 kv heads of 128 dims, us a layer narrow / wide: 208 / 253, 64 q / 16 kv heads of 64 dims 173 / 241.  At 256 dims
+  // (16 q / 4 kv heads, bf16) it is where many re-reads are saved and the rest of the launch is short: 64 readers of
+  // 8192 tokens (0.47 GB saved) beside 0.3 / 0.9 / 1.8 / 5.9 times the tokens that narrow tiles walk for them 72 / 55,
+  // 83 / 73, 99 / 97, 164 / 193; 64 of 32768 (1.9 GB) beside 1.5 / 3.3 times 256 / 206, 359 / 383; 48 of 8192 (0.34 GB)
+  // beside 0.6 times 60 / 52; 128 of 2048 (0.23 GB) beside as many 64 / 68.  Many wide tiles bear more: 256 readers of
+  // 4096 tokens beside 3.5 times 264 / 255, 128 of 8192 beside 5.9 / 13 times 325 / 317, 605 / 615.  So: on request
+  // always; otherwise plans of free size only.
   std::vector<char> group_is_wide(groups.size(), wide_on_request && wide_tile > 0);
-  if (!wide_on_request && wide_tile > 0 && !cap) {
+  if (!wide_on_request && wide_tile > 0 && !cap && shape->head_dim == 256) {
     const int64_t token_bytes = 2ll * shape->num_kv_heads * shape->head_dim * (shape->dtype == VA_F32 ? 4 : 2);
-    constexpr int64_t kWorthALaunch = 640ll << 20, kFairShare = kWorthALaunch / 8;
-    std::vector<int64_t> saved(groups.size(), 0);
-    int64_t total = 0;
+    constexpr int64_t kWorthIt = 300ll << 20, kFairShare = kWorthIt / 8;
+    std::vector<char> many(groups.size(), 0);
+    int64_t saved = 0, walked = 0, rest = 0, most_tiles = 0;  // bytes; tokens that narrow tiles walk; wide tiles of a run
     for (size_t gi = 0; gi < groups.size(); ++gi) {
-      const int64_t n = (int64_t)groups[gi].subrows.size();
-      if (n <= q_tile) continue;
+      const int64_t n = (int64_t)groups[gi].subrows.size(), len = s->seq_lens[groups[gi].rep];
+      const int64_t narrow = (n + q_tile - 1) / q_tile, at_once = tiles_together(kernel, shape->page_size, len);
       cut_tiles(n, tiles, true);
-      saved[gi] = ((n + q_tile - 1) / q_tile - (int64_t)tiles.size()) * s->seq_lens[groups[gi].rep] * token_bytes;
-      if (saved[gi] >= kFairShare) total += saved[gi];
+      const int64_t bytes = (narrow - (int64_t)tiles.size()) * len * token_bytes;
+      many[gi] = n > q_tile && bytes >= kFairShare;
+      (many[gi] ? walked : rest) += (narrow + at_once - 1) / at_once * len;
+      if (!many[gi]) continue;
+      saved += bytes;
+      most_tiles = std::max(most_tiles, (int64_t)tiles.size());
     }
-    if (total >= kWorthALaunch)
-      for (size_t gi = 0; gi < groups.size(); ++gi) group_is_wide[gi] = saved[gi] >= kFairShare;
+    if (saved >= kWorthIt && rest <= (most_tiles >= 4 ? 6 : 2) * walked) group_is_wide = many;
   }
 
   // ---- chains: sub-requests of one prefill request, in table order ----
@@ -359,7 +365,7 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     out.items.push_back(it);
   };
 
-  // Wide decode tiles run in their own launch (one workgroup per CU at a time), so their
+  // Wide decode tiles run one workgroup per CU at a time, so their
   // runs are cut finer: enough chunks for about one workgroup per CU.
   int64_t wide_group_tokens = 0;
   for (auto& gr : groups) {

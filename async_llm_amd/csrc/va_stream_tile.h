@@ -502,68 +502,68 @@ __device__ __forceinline__ void stream_items(const AttnArgs& a, const int (&item
   wave_wait<0>();  // (index entries requested past the end)
 #pragma unroll
   for (int b = 0; b < kB; ++b) {
-  if (b > 0) __syncthreads();  // the block before has been read
-  // row sums live spread over the four contraction groups
-  l_run[b] += __shfl_xor(l_run[b], 16, kWave);
-  l_run[b] += __shfl_xor(l_run[b], 32, kWave);
-  {
-    char* mine = lds + wave * Sh::kWaveRingBytes;
-#pragma unroll
-    for (int q = 0; q < kDimTiles; ++q) *(va_f32x4*)(mine + j * Sh::kFoldRowBytes + 16 * kg + 64 * q) = o[b][q];
-    if (kg == 0) *(float2*)(mine + 16 * Sh::kFoldRowBytes + 8 * j) = make_float2(m_run[b], l_run[b]);
-  }
-  __syncthreads();
-  const int row = tid / 16, seg = tid % 16;
-  const int iq = row / G, part_base = item[b][VA_I_PART_BASE];
-  if (iq >= item[b][VA_I_N_Q]) continue;
-  float weight[kStreamWaves], m = kNegBig, l = 0.f;
-  {
-    float2 state[kStreamWaves];
-#pragma unroll
-    for (int w = 0; w < kStreamWaves; ++w) {
-      state[w] = *(const float2*)(lds + w * Sh::kWaveRingBytes + 16 * Sh::kFoldRowBytes + 8 * row);
-      m = fmaxf(m, state[w].x);
+    if (b > 0) __syncthreads();  // the block before has been read
+    // row sums live spread over the four contraction groups
+    l_run[b] += __shfl_xor(l_run[b], 16, kWave);
+    l_run[b] += __shfl_xor(l_run[b], 32, kWave);
+    {
+      char* mine = lds + wave * Sh::kWaveRingBytes;
+  #pragma unroll
+      for (int q = 0; q < kDimTiles; ++q) *(va_f32x4*)(mine + j * Sh::kFoldRowBytes + 16 * kg + 64 * q) = o[b][q];
+      if (kg == 0) *(float2*)(mine + 16 * Sh::kFoldRowBytes + 8 * j) = make_float2(m_run[b], l_run[b]);
     }
-#pragma unroll
-    for (int w = 0; w < kStreamWaves; ++w) {
-      weight[w] = __builtin_amdgcn_exp2f(state[w].x - m);
-      l += state[w].y * weight[w];
+    __syncthreads();
+    const int row = tid / 16, seg = tid % 16;
+    const int iq = row / G, part_base = item[b][VA_I_PART_BASE];
+    if (iq >= item[b][VA_I_N_Q]) continue;
+    float weight[kStreamWaves], m = kNegBig, l = 0.f;
+    {
+      float2 state[kStreamWaves];
+  #pragma unroll
+      for (int w = 0; w < kStreamWaves; ++w) {
+        state[w] = *(const float2*)(lds + w * Sh::kWaveRingBytes + 16 * Sh::kFoldRowBytes + 8 * row);
+        m = fmaxf(m, state[w].x);
+      }
+  #pragma unroll
+      for (int w = 0; w < kStreamWaves; ++w) {
+        weight[w] = __builtin_amdgcn_exp2f(state[w].x - m);
+        l += state[w].y * weight[w];
+      }
+    }
+    const int hq = hk * G + row - iq * G;
+    va_f32x4 sum[kD / 64];
+  #pragma unroll
+    for (int x = 0; x < kD / 64; ++x) {
+      sum[x] = va_f32x4{0.f, 0.f, 0.f, 0.f};
+  #pragma unroll
+      for (int w = 0; w < kStreamWaves; ++w)
+        sum[x] += *(const va_f32x4*)(lds + w * Sh::kWaveRingBytes + row * Sh::kFoldRowBytes + 16 * (seg + 16 * x)) * weight[w];
+    }
+    if (part_base < 0) {
+      const int qref0 = item[b][VA_I_LINK0 + VA_L_QREF];
+      const long long out_row = (item[b][VA_I_LINK0 + VA_L_FLAGS] & VA_LINK_INDIRECT) ? (long long)a.qref_rows[qref0 + iq]
+                                                                                   : a.sub_worker[qref0 + iq];
+      S* orow = (S*)a.out + (out_row * a.num_q_heads + hq) * (long long)kD;
+      const float inv = l > 0.f ? 1.f / l : 0.f;
+  #pragma unroll
+      for (int x = 0; x < kD / 64; ++x)
+        *(uint2*)(orow + 4 * (seg + 16 * x)) = make_uint2(Mma<E>::pack(sum[x][0] * inv, sum[x][1] * inv),
+                                                         Mma<E>::pack(sum[x][2] * inv, sum[x][3] * inv));
+      if (seg == 0 && a.lse) {
+        const float lse2 = l > 0.f ? m + log2f(l) : -INFINITY;
+        a.lse[out_row * a.num_q_heads + hq] = a.lse_base2 ? lse2 : lse2 * kLn2;
+      }
+    } else {
+      const long long slot = (long long)(part_base + iq) * a.num_q_heads + hq;
+      float* prow = a.part_acc + slot * kD;
+  #pragma unroll
+      for (int x = 0; x < kD / 64; ++x) *(va_f32x4*)(prow + 4 * (seg + 16 * x)) = sum[x];
+      if (seg == 0) {
+        a.part_ml[slot * 2 + 0] = m;
+        a.part_ml[slot * 2 + 1] = l;
+      }
     }
   }
-  const int hq = hk * G + row - iq * G;
-  va_f32x4 sum[kD / 64];
-#pragma unroll
-  for (int x = 0; x < kD / 64; ++x) {
-    sum[x] = va_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int w = 0; w < kStreamWaves; ++w)
-      sum[x] += *(const va_f32x4*)(lds + w * Sh::kWaveRingBytes + row * Sh::kFoldRowBytes + 16 * (seg + 16 * x)) * weight[w];
-  }
-  if (part_base < 0) {
-    const int qref0 = item[b][VA_I_LINK0 + VA_L_QREF];
-    const long long out_row = (item[b][VA_I_LINK0 + VA_L_FLAGS] & VA_LINK_INDIRECT) ? (long long)a.qref_rows[qref0 + iq]
-                                                                                 : a.sub_worker[qref0 + iq];
-    S* orow = (S*)a.out + (out_row * a.num_q_heads + hq) * (long long)kD;
-    const float inv = l > 0.f ? 1.f / l : 0.f;
-#pragma unroll
-    for (int x = 0; x < kD / 64; ++x)
-      *(uint2*)(orow + 4 * (seg + 16 * x)) = make_uint2(Mma<E>::pack(sum[x][0] * inv, sum[x][1] * inv),
-                                                       Mma<E>::pack(sum[x][2] * inv, sum[x][3] * inv));
-    if (seg == 0 && a.lse) {
-      const float lse2 = l > 0.f ? m + log2f(l) : -INFINITY;
-      a.lse[out_row * a.num_q_heads + hq] = a.lse_base2 ? lse2 : lse2 * kLn2;
-    }
-  } else {
-    const long long slot = (long long)(part_base + iq) * a.num_q_heads + hq;
-    float* prow = a.part_acc + slot * kD;
-#pragma unroll
-    for (int x = 0; x < kD / 64; ++x) *(va_f32x4*)(prow + 4 * (seg + 16 * x)) = sum[x];
-    if (seg == 0) {
-      a.part_ml[slot * 2 + 0] = m;
-      a.part_ml[slot * 2 + 1] = l;
-    }
-  }
-  }  // blocks of the tile
 }
 
 // The item (and its partners) of workgroup `block` of the narrow items.
