@@ -66,9 +66,9 @@ inline hipError_t allow_lds(const void* kernel, int bytes, std::atomic<unsigned 
 // `n_wide` leading items are wide tiles (va_mfma_wide.hip: `n_wide_slots` workgroups per kv head, each
 // running the items a.wide_slots gives it), the rest narrow ones: in the same launch behind the wide ones, or in
 // one of their own (va_mfma_stream.hip).
-int launch_mfma(const AttnArgs& a, int dtype, int n_items, int n_wide, int n_wide_slots, int q_tile,
+int launch_mfma(const AttnArgs& a, int dtype, int n_items, int n_wide, int n_wide_slots, int q_tile, bool short_items,
                 hipStream_t stream);
 int launch_mfma_wide(const AttnArgs& a, int dtype, int n_slots, int n_narrow, hipStream_t stream);
-int launch_mfma_stream(const AttnArgs& a, int dtype, int n_items, hipStream_t stream);
+int launch_mfma_stream(const AttnArgs& a, int dtype, int n_items, bool short_items, hipStream_t stream);
 
 }  // namespace va

@@ -27,7 +27,7 @@ int va_mfma_wide_q_tile(int gqa, int head_dim) { return (head_dim == 256 ? 128 :
 
 namespace va {
 
-int launch_mfma(const AttnArgs& a_in, int dtype, int n_items, int n_wide, int n_wide_slots, int q_tile,
+int launch_mfma(const AttnArgs& a_in, int dtype, int n_items, int n_wide, int n_wide_slots, int q_tile, bool short_items,
                 hipStream_t stream) {
   AttnArgs a = a_in;
   const int g = a.num_q_heads / a.num_kv_heads;
@@ -45,7 +45,7 @@ int launch_mfma(const AttnArgs& a_in, int dtype, int n_items, int n_wide, int n_
   if (a.pool_row_stride * 2 * 16 > 0x7fffffffLL) return va_fail(VA_ERR_ARG, "pool rows too far apart");
   a.narrow_items = a.items + (long long)n_wide * VA_ITEM_WORDS;
   if (n_wide > 0 && n_wide_slots > 0) return launch_mfma_wide(a, dtype, n_wide_slots, n_items - n_wide, stream);
-  return launch_mfma_stream(a, dtype, n_items - n_wide, stream);
+  return launch_mfma_stream(a, dtype, n_items - n_wide, short_items, stream);
 }
 
 }  // namespace va

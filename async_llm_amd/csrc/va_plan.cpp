@@ -50,6 +50,7 @@ struct Built {
   std::vector<int32_t> wide_slots;  // indptr over the wide items: the items of each workgroup of the wide launch
   int32_t n_partials = 0;
   int32_t kernel = 0, q_tile = 0, kv_chunk = 0, wide_tile = 0, n_wide = 0;
+  bool short_items = false;  // VA_CHUNK_SHORT_ITEMS
 };
 
 inline int32_t round_up(int64_t x, int32_t m) { return (int32_t)(((x + m - 1) / m) * m); }
@@ -233,15 +234,15 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   // (16 q / 4 kv heads, bf16) it is where many re-reads are saved and the rest of the launch is short: 64 readers of
   // 8192 tokens (0.47 GB saved) beside 0.3 / 0.9 / 1.8 / 5.9 times the tokens that narrow tiles walk for them 72 / 55,
   // 83 / 73, 99 / 97, 164 / 193; 64 of 32768 (1.9 GB) beside 1.5 / 3.3 times 256 / 206, 359 / 383; 48 of 8192 (0.34 GB)
-  // beside 0.6 times 60 / 52; 128 of 2048 (0.23 GB) beside as many 64 / 68.  Many wide tiles bear more: 256 readers of
-  // 4096 tokens beside 3.5 times 264 / 255, 128 of 8192 beside 5.9 / 13 times 325 / 317, 605 / 615.  So: on request
-  // always; otherwise plans of free size only.
+  // beside 0.6 times 60 / 52; 128 of 2048 (0.23 GB) beside as many 64 / 68; 128 of 8192 (0.94 GB) beside 5.9 / 13 times
+  // 325 / 317, 605 / 615; 256 of 4096 beside 3.5 times 264 / 255.  From 0.64 GB on a longer rest is let pass (it costs 64
+  // of 32768 some percent, and gains them with 128 readers).  So: on request always; otherwise plans of free size only.
   std::vector<char> group_is_wide(groups.size(), wide_on_request && wide_tile > 0);
   if (!wide_on_request && wide_tile > 0 && !cap && shape->head_dim == 256) {
     const int64_t token_bytes = 2ll * shape->num_kv_heads * shape->head_dim * (shape->dtype == VA_F32 ? 4 : 2);
-    constexpr int64_t kWorthIt = 300ll << 20, kFairShare = kWorthIt / 8;
+    constexpr int64_t kWorthIt = 300ll << 20, kFairShare = kWorthIt / 8, kWorthMuch = 640ll << 20;
     std::vector<char> many(groups.size(), 0);
-    int64_t saved = 0, walked = 0, rest = 0, most_tiles = 0;  // bytes; tokens that narrow tiles walk; wide tiles of a run
+    int64_t saved = 0, walked = 0, rest = 0;  // bytes; tokens that narrow tiles walk for these groups, for the others
     for (size_t gi = 0; gi < groups.size(); ++gi) {
       const int64_t n = (int64_t)groups[gi].subrows.size(), len = s->seq_lens[groups[gi].rep];
       const int64_t narrow = (n + q_tile - 1) / q_tile, at_once = tiles_together(kernel, shape->page_size, len);
@@ -249,11 +250,9 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
       const int64_t bytes = (narrow - (int64_t)tiles.size()) * len * token_bytes;
       many[gi] = n > q_tile && bytes >= kFairShare;
       (many[gi] ? walked : rest) += (narrow + at_once - 1) / at_once * len;
-      if (!many[gi]) continue;
-      saved += bytes;
-      most_tiles = std::max(most_tiles, (int64_t)tiles.size());
+      if (many[gi]) saved += bytes;
     }
-    if (saved >= kWorthIt && rest <= (most_tiles >= 4 ? 6 : 2) * walked) group_is_wide = many;
+    if (saved >= kWorthIt && rest <= (saved >= kWorthMuch ? 6 : 2) * walked) group_is_wide = many;
   }
 
   // ---- chains: sub-requests of one prefill request, in table order ----
@@ -773,6 +772,23 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   //   * position p of the class holds entry p / 8 of die p % 8; dies with fewer entries are
   //     padded with empty items (n_q = 0, the kernels return at once), which also keeps the
   //     class a multiple of 8 long so the next kv head starts on die 0 again.
+  if (kernel == VA_KERNEL_MFMA && !cap && (int64_t)out.items.size() * shape->num_kv_heads > 256) {
+    int64_t tokens = 0, again = 0;  // of all items; of those that walk together, beyond the first of each workgroup
+    bool only_narrow = true;
+    int32_t in_unit = 0, unit = -1;
+    for (const auto& it : out.items) {  // (the items of a unit stand side by side)
+      only_narrow = only_narrow && it.kind == 0;
+      in_unit = it.unit >= 0 && it.unit == unit ? in_unit + 1 : 0;
+      unit = it.unit;
+      tokens += it.tokens;
+      if (in_unit % it.together) again += it.tokens;
+    }
+    // (a fifth: of 64 requests over 512 shared tokens and blocks of 100..400, 13 % walked again, 35.9 -> 32.5 us apart at
+    // 256 dims, 33 either way at 128, 46.8 -> 36.7 at 64; over 2048, 29 %, at 128 dims 42 together)
+    out.short_items = only_narrow && tokens <= 640 * (int64_t)out.items.size() && again <= tokens / 5;
+    if (out.short_items)
+      for (auto& it : out.items) it.together = 1;
+  }
   std::vector<Item> sorted;
   sorted.reserve(out.items.size() + 2 * kXcds);
   for (int kind = 1; kind >= 0; --kind) {
@@ -1011,7 +1027,7 @@ static int write_plan(const Built& b, const VaSubRequests* subs, const VaShape* 
   h[VA_H_MAGIC] = VA_PLAN_MAGIC;
   h[VA_H_KERNEL] = c.kernel;
   h[VA_H_Q_TILE] = c.q_tile;
-  h[VA_H_KV_CHUNK] = cap ? 0 : c.kv_chunk;  // chosen per plan: not part of a fixed plan's header (see counts)
+  h[VA_H_KV_CHUNK] = cap ? 0 : c.kv_chunk | (b.short_items ? VA_CHUNK_SHORT_ITEMS : 0);  // chosen per plan: not part of a fixed plan's header (see counts)
   h[VA_H_N_WIDE] = cap_wide;
   h[VA_H_WIDE_TILE] = c.wide_tile;
   h[VA_H_N_ITEMS] = cap_wide + cap_narrow;

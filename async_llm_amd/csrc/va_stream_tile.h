@@ -47,7 +47,9 @@ constexpr int kStreamTok = 16;  // tokens per tile
 #endif
 constexpr int kIndexSlots = 8;        // tiles whose index entries a wave's ring of entries holds
 
-template <int kD>
+// kShort: launches of short items (stream_block_short), where an item's set-up and fold count and those of others have to
+// run beside them: one tile a workgroup, and less LDS, for two to four workgroups on a CU.
+template <int kD, bool kShort = false>
 struct StreamShape {
   static constexpr int kChunks = kD / 8;                     // 16-byte pieces of a head row
   static constexpr int kSteps = kD / 32;                     // contraction steps of K.Q^T
@@ -56,21 +58,22 @@ struct StreamShape {
   static constexpr int kRowsPerLoad = kWave / kChunks;       // tile rows one wave-level load covers
   static constexpr int kLoads = kStreamTok / kRowsPerLoad;   // loads of a K (or V) tile
   static constexpr int kTileBytes = kStreamTok * kRowBytes;  // a K (or V) tile
-  static constexpr int kBuffers = kD == 256 ? VA_STREAM_BUFFERS_256 : kD == 128 ? 2 : 4;  // ring depth of a wave, in tiles
-  static constexpr int kMinBlocks = kD == 256 ? VA_STREAM_BLOCKS_256 : 2;                 // workgroups per CU (registers and LDS allow)
-  static constexpr int kWaveRingBytes = kBuffers * 2 * kTileBytes;
-  static constexpr int kRingBytes = kStreamWaves * kWaveRingBytes;
-  // Behind the rings: the rotated query rows of up to four items, or of two and for every wave the index entries of
-  // kIndexSlots tiles.
-  static constexpr int kIndexOffset = kRingBytes + 2 * 16 * kRowBytes;
-  static constexpr int kIndexBytes = kIndexSlots * kStreamTok * 4;
-  static constexpr int lds_bytes(bool gather) {
-    return gather ? kIndexOffset + kStreamWaves * kIndexBytes : kRingBytes + 4 * 16 * kRowBytes;
-  }
+  // ring depth of a wave, in tiles, and workgroups per CU (registers and LDS allow)
+  static constexpr int kBuffers = kShort ? (kD == 64 ? 2 : 1) : kD == 256 ? VA_STREAM_BUFFERS_256 : kD == 128 ? 2 : 4;
+  static constexpr int kMinBlocks = kShort ? (kD == 256 ? 2 : kD == 128 ? 3 : 4) : kD == 256 ? VA_STREAM_BLOCKS_256 : 2;
   // A wave's state at the end, in its own ring: accumulators (rows padded by 16 bytes, so that the sixteen rows of a
   // write spread over the banks), then maxima and sums.
   static constexpr int kFoldRowBytes = kD * 4 + 16;
-  static_assert(16 * (kFoldRowBytes + 8) <= kWaveRingBytes, "room to fold the states");
+  static constexpr int kFoldBytes = (16 * (kFoldRowBytes + 8) + 1023) / 1024 * 1024;
+  static constexpr int kWaveRingBytes = kBuffers * 2 * kTileBytes > kFoldBytes ? kBuffers * 2 * kTileBytes : kFoldBytes;
+  static constexpr int kRingBytes = kStreamWaves * kWaveRingBytes;
+  // Behind the rings: the rotated query rows of up to four items, or of two and for every wave the index entries of
+  // kIndexSlots tiles.
+  static constexpr int kIndexOffset = kRingBytes + (kShort ? 1 : 2) * 16 * kRowBytes;
+  static constexpr int kIndexBytes = kIndexSlots * kStreamTok * 4;
+  static constexpr int lds_bytes(bool gather) {
+    return gather ? kIndexOffset + kStreamWaves * kIndexBytes : kRingBytes + (kShort ? 1 : 4) * 16 * kRowBytes;
+  }
 };
 
 // Piece c of tile row r lies at position c ^ stream_swz(r).  K fragments (16 rows, one piece of each) then hit sixteen
@@ -115,10 +118,11 @@ __device__ __forceinline__ void load_item(const AttnArgs& a, int index, int (&it
 
 // One work item for one kv head, or kB of them that walk the same tokens: a block of up to 16 MFMA rows each.
 // kGather: pages hold less than a tile (1, 2, 4 or 8 tokens; a slot list has pages of one).
-template <typename E, int kD, bool kGather, int kB>
+template <typename E, int kD, bool kGather, int kB, bool kShort = false>
 __device__ __forceinline__ void stream_items(const AttnArgs& a, const int (&item)[kB][VA_ITEM_WORDS], int hk) {
   using S = typename E::storage;
-  using Sh = StreamShape<kD>;
+  using Sh = StreamShape<kD, kShort>;
+  static_assert(!kShort || kB == 1, "room for the query rows of one tile");
   constexpr int kChunks = Sh::kChunks, kSteps = Sh::kSteps, kDimTiles = Sh::kDimTiles, kBuffers = Sh::kBuffers;
   constexpr int kLoads = Sh::kLoads, kRowBytes = Sh::kRowBytes, kTileBytes = Sh::kTileBytes;
   // the entries of tiles i + 1 .. i + 2 kBuffers of a wave are held or on their way at any time
@@ -591,6 +595,23 @@ __device__ __forceinline__ void stream_block(const AttnArgs& a, unsigned block) 
     together(std::integral_constant<int, 2>{});
   } else {
     together(std::integral_constant<int, 4>{});
+  }
+}
+
+// The same where items are short: its workgroups serve a tile each (a plan whose tiles walk together gets them one after
+// the other).
+template <typename E, int kD, bool kGather>
+__device__ __forceinline__ void stream_block_short(const AttnArgs& a, unsigned block) {
+  const ItemHead where = item_and_head(block, a.num_kv_heads);
+  int item[1][VA_ITEM_WORDS];
+  load_item(a, where.item, item[0]);
+  const int partners = item[0][VA_I_PARTNERS];
+  if (item[0][VA_I_N_Q] == 0 || partners < 0) return;
+  for (int b = 0;;) {
+    stream_items<E, kD, kGather, 1, true>(a, item, where.head);
+    if (++b > partners) return;
+    __syncthreads();  // the states of the tile before have been read
+    load_item(a, where.item + 8 * b, item[0]);
   }
 }
 

@@ -65,4 +65,5 @@ def test_partners_walk_the_tokens_of_the_item_before_them(heads, page, fixed):
                     same = [0, 1, 2, 4, 5]  # list, first and last token, causal base, flags: all but the query rows
                     assert [other[LINK0 + w] for w in same] == [item[LINK0 + w] for w in same]
         assert np.array_equal(served, (narrow[:, 2] > 0).astype(int))
-    assert (most > 0) == (heads[0] // heads[1] < 16)  # (16 rows of one request fill a tile)
+    if fixed:  # (packed plans of short items keep their tiles apart; 16 rows of one request fill a tile)
+        assert (most > 0) == (heads[0] // heads[1] < 16)
