@@ -51,8 +51,8 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0
 # carried here together with the digest of the kernel sources they were measured on
 # (csrc_digest()), and are reported only while that digest is the one of the sources in the tree.
 MEASURED_TRAFFIC = {
-    ("batched_decode", "mfma"): {"bytes": 2 * 1024 * (1_129_938 + 8_988) + 1024 * (17_885 + 512), "csrc": "08c375c61b54cd3d"},
-    ("mrope_decode", "mfma"): {"bytes": 2 * 1024 * (2_098_018 + 4_722) + 1024 * (9_297 + 64), "csrc": "08c375c61b54cd3d"},
+    ("batched_decode", "mfma"): {"bytes": 2 * 1024 * (1_112_090 + 4_143) + 1024 * (8_160 + 512), "csrc": "844e07adf982e67e"},
+    ("mrope_decode", "mfma"): {"bytes": 2 * 1024 * (2_097_910 + 1_608) + 1024 * (3_096 + 64), "csrc": "844e07adf982e67e"},
     ("view_prefill", "mfma"): {"bytes": 2 * 1024 * 2_496_982 + 1024 * 131_323, "csrc": "08c375c61b54cd3d"},
     ("mixed_batch", "mfma"): {"bytes": 2 * 1024 * (439_645 + 1_623_108 + 27_058) + 1024 * (47_429 + 12_397 + 10_624),
                               "csrc": "08c375c61b54cd3d"},
