@@ -60,8 +60,9 @@ class LaunchPlan:
     staging: Optional[torch.Tensor] = None
     coarse: Optional["LaunchPlan"] = None
 
-    def __post_init__(self) -> None:
-        self.header_ptr = self.header.ctypes.data
+    @property
+    def header_ptr(self) -> int:
+        return self.header.ctypes.data  # (asked for anew: a copied or reassigned header lies elsewhere)
 
 
 @dataclass

@@ -1,5 +1,7 @@
 """A step's plan and tables go to the device as one staging tensor: what arrives is what was planned."""
 
+import copy
+import pickle
 from types import SimpleNamespace
 
 import numpy as np
@@ -77,3 +79,13 @@ def test_plans_of_one_op_may_overlap():
     assert np.array_equal(launch.header, alone.header)
     assert np.array_equal(launch.blob.numpy()[: native.PLAN_HEADER_WORDS], launch.header)
     assert torch.equal(launch.blob, alone.blob)
+
+
+def test_the_header_handed_to_a_launch_is_the_plans_own():
+    op = _op()
+    launch = op._build_launch(tables=(), refs=[], **_plan_args([(58, 40, [700, 300])], 16))[0]
+    kept = launch.header.ctypes.data
+    copies = [copy.deepcopy(launch), pickle.loads(pickle.dumps(launch))]
+    launch.header = launch.header.copy()
+    for plan in [launch, *copies]:
+        assert plan.header_ptr == plan.header.ctypes.data != kept
