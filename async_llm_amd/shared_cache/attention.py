@@ -807,17 +807,23 @@ class SharedCacheAttention:
         assert isinstance(meta, SharedCacheAttnMetadata)
         return self._forward(q, k, v, layer_id, batch, meta)
 
-    def _forward(self, q, k, v, layer_id: int, batch, meta, *attend_args):
-        if not self.fused_store:
+    def _forward(self, q, k, v, layer_id: int, batch, meta, **wanted):
+        own = type(self)
+        if (not self.fused_store or own.store_new_kv is not _STORE_NEW_KV or own.attend is not _ATTEND
+                or "store_new_kv" in self.__dict__ or "attend" in self.__dict__):
+            # (a subclass or a wrapper puts steps of its own in the place of these two)
             self.store_new_kv(k, v, layer_id, batch)
-            return self.attend(q, layer_id, meta, *attend_args)
+            return self.attend(q, layer_id, meta, **wanted)
         # (the layer's pools and the stream are asked for once: together they cost as much as a launch)
         pools = self.kv_cache.k_cache(layer_id), self.kv_cache.v_cache(layer_id)
         stream = native.current_stream_ptr(self.device)
         self._store(k, v, layer_id, batch, pools, stream)
-        return self._attend(q, meta, pools, stream, *attend_args)
+        return self._attend(q, meta, pools, stream, **wanted)
 
     def forward_with_lse(self, q, k, v, layer_id: int, batch, lse_base2: bool = False):
         """``forward`` that also returns the merged logsumexp ``[W, Hq]``."""
         meta = batch.attn_metadata
-        return self._forward(q, k, v, layer_id, batch, meta, True, lse_base2)
+        return self._forward(q, k, v, layer_id, batch, meta, return_lse=True, lse_base2=lse_base2)
+
+
+_STORE_NEW_KV, _ATTEND = SharedCacheAttention.store_new_kv, SharedCacheAttention.attend
