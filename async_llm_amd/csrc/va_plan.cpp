@@ -524,22 +524,27 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     }
   };
   std::vector<Bundle> bundles;
-  int64_t wide_walk = 0, wide_cost = 0;  // positions of all bundles; with their set-ups
-  int64_t lane_cost = 0;  // over all lanes that have a part of a bundle
+  struct BundleSums {
+    int64_t walk = 0, cost = 0;  // positions of all bundles; with their set-ups
+    int64_t lane_cost = 0;       // over all lanes that have a part of a bundle
+  };
   auto measure_bundles = [&]() {
-    wide_walk = wide_cost = lane_cost = 0;
+    BundleSums sums;
     for (auto& ch : chains) {
       const int32_t nq = s->qo_indptr[ch[0] + 1] - s->qo_indptr[ch[0]];
       cut_tiles(nq, tiles);
       bundles_of(ch, nq, bundles);
       for (auto& bd : bundles) {
-        wide_walk += bd.part;
         const int64_t cost = bd.cost(0, bd.part, seg_cost);
-        wide_cost += cost;
-        lane_cost += cost * bd.m * bd.f;
+        sums.walk += bd.part;
+        sums.cost += cost;
+        sums.lane_cost += cost * bd.m * bd.f;
       }
     }
+    return sums;
   };
+  BundleSums wide_sums;
+  if (pack) wide_sums = measure_bundles();
   if (pack && total_tokens > 0 && wide_chain_tokens > 0) {
     // The launch holds the runs of stand-alone sub-requests as well.  A CU left to those while the wide slots run takes
     // in twice what it gets when all of them stream (52 against 26 bytes a ns: 256 share what the memory gives), so some
@@ -552,33 +557,44 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     const double bytes = 2.0 * (double)total_tokens * shape->num_kv_heads * shape->head_dim * (shape->dtype == VA_F32 ? 4 : 2);
     double best = 0, all_end = 0;
     int32_t best_lanes = all_lanes;
+    const BundleSums all = wide_sums;
     for (; lanes >= 1; lanes -= std::max(1, all_lanes / 8)) {
-      measure_bundles();
-      const double token_ns = 28.0 + 4.0 * lanes / all_lanes, wide_ns = token_ns * (double)wide_cost / groups_wanted;
-      const double idle_ns = std::max(0.0, 256.0 * wide_ns - token_ns * (double)lane_cost * shape->num_kv_heads);
+      const BundleSums sums = lanes == all_lanes ? all : measure_bundles();
+      const double token_ns = 28.0 + 4.0 * lanes / all_lanes, wide_ns = token_ns * (double)sums.cost / groups_wanted;
+      // Fewer lanes walk no less: neither these nor any fewer end before what was found.  (The search is most of the
+      // planner's time where chunks have many blocks: all lanes tried, 8 rows beside 16 chunks of 215 over 20 blocks took
+      // 465 us where 234 are enough.)
+      if (lanes < all_lanes && wide_ns >= best) break;
+      const double idle_ns = std::max(0.0, 256.0 * wide_ns - token_ns * (double)sums.lane_cost * shape->num_kv_heads);
       const double rest_ns = std::max(0.0, bytes - std::min(52.0 * idle_ns, 6560.0 * wide_ns)) / 6560.0;
       const double end = wide_ns + rest_ns + std::min(rest_ns, 40e3);
-      if (lanes == all_lanes) all_end = end;
-      if (lanes == all_lanes || end < 0.98 * best) {
+      if (lanes == all_lanes) {
+        all_end = best = end;
+        if (wide_ns >= 0.92 * all_end) break;  // next to nothing is left behind the wide slots
+      } else if (end < 0.98 * best) {
         best = end;
         best_lanes = lanes;
+        wide_sums = sums;
       }
     }
-    lanes = best < 0.92 * all_end ? best_lanes : all_lanes;  // (an estimate: it has to promise something)
+    lanes = best_lanes;
+    if (best >= 0.92 * all_end) {  // (an estimate: it has to promise something)
+      lanes = all_lanes;
+      wide_sums = all;
+    }
   }
-  if (pack) measure_bundles();
   // The room of a new group is the even share of what is still to be placed over the groups still
   // to be opened, so that a group closed early (less than min_piece of its room left) or run over (a
   // bundle's short remainder kept with the piece before it) is made up for by the groups after it,
   // and their number never exceeds the number wanted.
-  const int64_t group_budget = pack ? std::max<int64_t>((wide_walk + groups_wanted - 1) / groups_wanted, cuts_of_chains.group_floor()) : 0;
+  const int64_t group_budget = pack ? std::max<int64_t>((wide_sums.walk + groups_wanted - 1) / groups_wanted, cuts_of_chains.group_floor()) : 0;
   const int32_t min_piece = cuts_of_chains.least_piece(group_budget);
-  int64_t groups_left = pack ? std::max<int64_t>(1, (wide_walk + group_budget - 1) / group_budget) : 0;
+  int64_t groups_left = pack ? std::max<int64_t>(1, (wide_sums.walk + group_budget - 1) / group_budget) : 0;
   // What is still to be placed, set-ups included: every segment of every bundle, and one more for
   // every group boundary (it falls inside some segment, which is then staged on both sides).  An
   // estimate on the high side leaves the LAST group short, one on the low side would leave it long --
   // and the longest group is the time of the launch.
-  int64_t wide_left = wide_cost + seg_cost * (groups_left - 1);
+  int64_t wide_left = wide_sums.cost + seg_cost * (groups_left - 1);
   auto next_wide_room = [&]() -> int64_t {
     if (groups_left <= 1) return INT32_MAX;  // the last group takes whatever is left
     const int64_t share = std::max<int64_t>((wide_left + groups_left - 1) / groups_left, seg_cost + min_piece);
