@@ -376,6 +376,7 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   const int32_t wide_chunk = std::min<int32_t>(
       kv_chunk, round_up(std::max<int64_t>((wide_group_tokens + wide_items_wanted - 1) / wide_items_wanted, 2 * gran), gran));
 
+  int64_t stream_groups = 0, stream_tokens = 0;  // workgroups per kv head that serve the narrow tiles, what they walk
   for (auto& gr : groups) {
     const int32_t rep = gr.rep;
     const int32_t len = s->seq_lens[rep];
@@ -411,8 +412,14 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     for (size_t ci = 0; ci + 1 < cuts.size(); ++ci) {
       if (cuts[ci] >= cuts[ci + 1]) continue;
       const int32_t unit = next_unit++;  // the narrow tiles of one chunk: same die, side by side
-      for (size_t ti = 0; ti < tiles.size(); ++ti)
-        if (tiles[ti].second - tiles[ti].first <= q_tile) emit_range(ti, cuts[ci], cuts[ci + 1], unit);
+      int32_t in_unit = 0;
+      for (size_t ti = 0; ti < tiles.size(); ++ti) {
+        if (tiles[ti].second - tiles[ti].first > q_tile) continue;
+        emit_range(ti, cuts[ci], cuts[ci + 1], unit);
+        if (in_unit++ % out.items.back().together) continue;
+        ++stream_groups;
+        stream_tokens += out.items.back().tokens;
+      }
     }
     const int32_t per_w = chunk_len(wide_chunk);
     for (size_t ti = 0; ti < tiles.size(); ++ti)
@@ -545,40 +552,48 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   };
   BundleSums wide_sums;
   if (pack) wide_sums = measure_bundles();
-  if (pack && total_tokens > 0 && wide_chain_tokens > 0) {
+  if (pack && stream_groups > 0 && wide_chain_tokens > 0) {
     // The launch holds the runs of stand-alone sub-requests as well.  A CU left to those while the wide slots run takes
     // in twice what it gets when all of them stream (52 against 26 bytes a ns: 256 share what the memory gives), so some
-    // lanes give theirs up: as many as the estimated end of the launch says.  Rates: a wide tile walks a token in 32 ns
-    // where all CUs hold one and in 28 where few do (the clock), what is left to stream behind the wide slots goes out
-    // at 6560 bytes a ns and ends unevenly.  Estimated and measured, us, by lanes (of 8, 16 q / 4 kv heads of 256 dims):
-    // 48 decode rows and 4 chunks of 512, 8 / 7 / 6 / 5 lanes: 1290 / 1160 / 1115 / 1190, 1205 / 1143 / 1093 / 1125
-    // (two launches 1229); 16 rows and 4 chunks of 256: 507 / 471 / 401 / 575, 497 / 472 / 453 / 525 (503);
-    // 40 rows and 3 chunks of 333: 452 / 340 / 342 / 338, 467 / 417 / 396 / 382.
-    const double bytes = 2.0 * (double)total_tokens * shape->num_kv_heads * shape->head_dim * (shape->dtype == VA_F32 ? 4 : 2);
+    // lanes give theirs up: as many as the estimated end of the launch says.  Rates: 24 ns for a token of a wide tile
+    // where all CUs hold one, 21 where few do (the clock), and 10 us for a slot's start and end; a streaming workgroup
+    // costs its CU 5 us of set-up and fold, what is left to stream behind the wide slots goes out at 6560 bytes a ns and
+    // ends unevenly.  One set of rates serves all head sizes: over 80 batches of 2..128 rows and 1..4 chunks of 64..512
+    // tokens, of every number of lanes the one it takes is 1 % behind the best (geometric mean; at most 11 %; with 28..32
+    // ns, no set-up and no start, as measured at 256 dims on long rows alone, 4 % and 19 %).  Estimated and measured, us,
+    // by lanes (of 8, 16 q / 4 kv heads of 256 dims): 48 rows of 1 k..32 k and 4 chunks of 512, 8 / 7 / 6 / 5 / 4 lanes,
+    // 952 / 888 / 757 / 720 / 779 and 1044 / 954 / 900 / 870 / 926 (two launches 1036); 48 rows of 1 k..4 k and a chunk of
+    // 65, 8 / 4 / 2 / 1, 107 / 97 / 92 / 92 and 114 / 105 / 104 / 102 (two launches 124).
+    const double bytes = 2.0 * (double)stream_tokens * shape->num_kv_heads * shape->head_dim * 2;
+    const double cu_ns = 5e3 * (double)stream_groups * shape->num_kv_heads + bytes / 52.0;
+    const double memory_ns = bytes / 6560.0;
+    auto behind = [&](double share) {  // of what is left to stream, with all CUs
+      const double ns = share * std::max(memory_ns, cu_ns / 256.0);
+      return ns + std::min(ns, 20e3);
+    };
+    const BundleSums all = wide_sums;
     double best = 0, all_end = 0;
     int32_t best_lanes = all_lanes;
-    const BundleSums all = wide_sums;
     for (; lanes >= 1; lanes -= std::max(1, all_lanes / 8)) {
       const BundleSums sums = lanes == all_lanes ? all : measure_bundles();
-      const double token_ns = 28.0 + 4.0 * lanes / all_lanes, wide_ns = token_ns * (double)sums.cost / groups_wanted;
-      // Fewer lanes walk no less: neither these nor any fewer end before what was found.  (The search is most of the
-      // planner's time where chunks have many blocks: all lanes tried, 8 rows beside 16 chunks of 215 over 20 blocks took
-      // 465 us where 234 are enough.)
+      const double share = (double)lanes / all_lanes, token_ns = 21.0 + 3.0 * share;
+      const double wide_ns = 10e3 + token_ns * (double)sums.cost / groups_wanted;
+      // (fewer lanes walk no less: neither these nor any fewer end before what was found)
       if (lanes < all_lanes && wide_ns >= best) break;
-      const double idle_ns = std::max(0.0, 256.0 * wide_ns - token_ns * (double)sums.lane_cost * shape->num_kv_heads);
-      const double rest_ns = std::max(0.0, bytes - std::min(52.0 * idle_ns, 6560.0 * wide_ns)) / 6560.0;
-      const double end = wide_ns + rest_ns + std::min(rest_ns, 40e3);
+      const double busy_ns = 256.0 * 10e3 * share + token_ns * (double)sums.lane_cost * shape->num_kv_heads;
+      const double idle_ns = std::max(0.0, 256.0 * wide_ns - busy_ns);
+      const double end = wide_ns + behind(1.0 - std::min({1.0, idle_ns / cu_ns, wide_ns / memory_ns}));
       if (lanes == all_lanes) {
         all_end = best = end;
-        if (wide_ns >= 0.92 * all_end) break;  // next to nothing is left behind the wide slots
-      } else if (end < 0.98 * best) {
+        if (wide_ns >= 0.97 * all_end) break;  // next to nothing is left behind the wide slots
+      } else if (end < 0.97 * best) {
         best = end;
         best_lanes = lanes;
         wide_sums = sums;
       }
     }
     lanes = best_lanes;
-    if (best >= 0.92 * all_end) {  // (an estimate: it has to promise something)
+    if (best >= 0.97 * all_end) {  // (an estimate: it has to promise something)
       lanes = all_lanes;
       wide_sums = all;
     }

@@ -162,3 +162,14 @@ def test_sharing_out_the_cus_costs_little_planning(heads, rows, requests):
             assert rc == 0
         best.append(min(times))
     assert best[1] <= 1.3 * best[0], best
+
+
+@pytest.mark.parametrize("heads", [(16, 4, 256), (32, 8, 128), (8, 2, 128)])
+def test_rows_that_outlast_a_small_chunk_get_the_cus_at_once(heads):
+    # 48 rows of 2500 tokens beside a chunk of 65: the chunk's walk in as many slots as there are CUs would keep the rows
+    # waiting for 25 us (measured at 1 k..4 k, all lanes / the fewest: 114 / 102, 132 / 123, 43 / 36 us)
+    tables = _with_decode_rows(_tables([(65, 700, [64, 900])], 16), 48, 2500, 16)
+    rc, blob, counts = build_plan(*tables, heads=heads, page=16, dtype=native.VA_BF16, kernel=native.VA_KERNEL_MFMA)
+    qo, kvp, _, lens, flags, _, sw, n_rows = tables
+    assert rc == 0 and 0 < counts.n_wide_slots <= 256 // heads[1] // 2
+    check_coverage(blob, qo, kvp, lens, flags, sw, n_rows)
