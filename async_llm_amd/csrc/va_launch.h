@@ -67,7 +67,7 @@ inline hipError_t allow_lds(const void* kernel, int bytes, std::atomic<unsigned 
 // running the items a.wide_slots gives it), the rest narrow ones: in the same launch behind the wide ones, or in
 // one of their own (va_mfma_stream.hip).
 int launch_mfma(const AttnArgs& a, int dtype, int n_items, int n_wide, int n_wide_slots, int q_tile, bool short_items,
-                hipStream_t stream);
+                bool apart, hipStream_t stream);
 int launch_mfma_wide(const AttnArgs& a, int dtype, int n_slots, int n_narrow, hipStream_t stream);
 int launch_mfma_stream(const AttnArgs& a, int dtype, int n_items, bool short_items, hipStream_t stream);
 

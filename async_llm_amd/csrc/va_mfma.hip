@@ -6,8 +6,9 @@
 //     read the same KV run (up to four such tiles a workgroup), and short prefill tiles.  Bound by HBM.
 //   * wide kernel (va_mfma_wide.hip): query tiles of up to 128 MFMA rows for view-conditioned
 //     prefill.  Bound by the matrix pipe.
-// A plan lists its wide items first.  Where it has both kinds one launch serves them: the streaming workgroups take
-// the CUs that the wide ones leave and, when those are done, all of them.
+// A plan lists its wide items first.  Where it has both kinds one launch serves them as a rule: the streaming workgroups
+// take the CUs that the wide ones leave and, when those are done, all of them.  Many short streaming items at head dims
+// under 256, which want to share CUs, get a launch of their own (VA_CHUNK_APART).
 #include <hip/hip_runtime.h>
 
 #include "va_internal.h"
@@ -28,7 +29,7 @@ int va_mfma_wide_q_tile(int gqa, int head_dim) { return (head_dim == 256 ? 128 :
 namespace va {
 
 int launch_mfma(const AttnArgs& a_in, int dtype, int n_items, int n_wide, int n_wide_slots, int q_tile, bool short_items,
-                hipStream_t stream) {
+                bool apart, hipStream_t stream) {
   AttnArgs a = a_in;
   const int g = a.num_q_heads / a.num_kv_heads;
   if (!va_mfma_supported(dtype, a.head_dim, g))
@@ -44,7 +45,10 @@ int launch_mfma(const AttnArgs& a_in, int dtype, int n_items, int n_wide, int n_
   // the streaming kernel addresses a tile's rows with 32-bit byte offsets from its first row
   if (a.pool_row_stride * 2 * 16 > 0x7fffffffLL) return va_fail(VA_ERR_ARG, "pool rows too far apart");
   a.narrow_items = a.items + (long long)n_wide * VA_ITEM_WORDS;
-  if (n_wide > 0 && n_wide_slots > 0) return launch_mfma_wide(a, dtype, n_wide_slots, n_items - n_wide, stream);
+  if (n_wide > 0 && n_wide_slots > 0) {
+    const int rc = launch_mfma_wide(a, dtype, n_wide_slots, apart ? 0 : n_items - n_wide, stream);
+    if (rc || !apart) return rc;
+  }
   return launch_mfma_stream(a, dtype, n_items - n_wide, short_items, stream);
 }
 

@@ -1052,8 +1052,8 @@ __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_wide_kernel(AttnArg
 // of a layer, two launches and this one: 48 decode rows and 4 chunks of 512 tokens, contexts of 1 k..32 k, 16 q / 4 kv
 // heads of 256 dims 1229 -> 1090 us, 16 rows and 4 chunks of 256 503 -> 457, 24 rows and 4 chunks of 400, 32 q / 8 kv
 // heads of 128 dims 441 -> 373; where the streaming items are a few tail rows it saves their launch (plain prefill of 6
-// requests 0.7 %).  At head dims under 256 a streaming workgroup has a CU to itself here (registers of the wide
-// kind), beside another where no wide items are: all of 48 rows and 3 chunks at 64 dims 1222 -> 1232.
+// requests 0.7 %).  A streaming workgroup has a CU to itself here (registers of the wide kind): where many short ones
+// want to share, at head dims under 256, the planner gives them a launch of their own.
 template <typename E, int kD, bool kGather>
 __global__ __launch_bounds__(kWideThreads, 1) void attn_mfma_joint_kernel(AttnArgs a, unsigned wide) {
   if (blockIdx.x < wide) {

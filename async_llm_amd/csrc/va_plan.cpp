@@ -50,7 +50,7 @@ struct Built {
   std::vector<int32_t> wide_slots;  // indptr over the wide items: the items of each workgroup of the wide launch
   int32_t n_partials = 0;
   int32_t kernel = 0, q_tile = 0, kv_chunk = 0, wide_tile = 0, n_wide = 0;
-  bool short_items = false;  // VA_CHUNK_SHORT_ITEMS
+  bool short_items = false, apart = false;  // VA_CHUNK_SHORT_ITEMS, VA_CHUNK_APART
 };
 
 inline int32_t round_up(int64_t x, int32_t m) { return (int32_t)(((x + m - 1) / m) * m); }
@@ -116,6 +116,16 @@ int tiles_together(int kernel, int page_size, int64_t tokens) {
 int default_target(int kernel, int num_kv_heads) {
   return kernel == VA_KERNEL_MFMA ? std::max(512 / num_kv_heads, num_kv_heads > 8 ? 64 : 128) : std::max(64, 2048 / num_kv_heads);
 }
+
+// Whether wide and narrow items of a recorded plan get a launch each.  The capacity does not say how long the items are:
+// where it has both decode rows and chunks, apart wins at 64 dims (64 rows of 200..900 tokens and a chunk of 65, us, one
+// launch / two 122 / 87, 48 of 1 k..32 k and 4 chunks of 512 1281 / 1261), together at 256 (76 / 101, 872 / 1186), and at 128
+// by more than it loses (111 / 103, 950 / 1440).
+bool fixed_apart(const VaShape* shape, const VaPlanCapacity& cap) {
+  return shape->head_dim == 64 && cap.max_wide_items > 0 && cap.max_qrefs > 0;
+}
+
+constexpr int64_t kShortItem = 640;  // tokens of a narrow item, on average, up to which several workgroups share a CU
 
 // How finely the walks of chains may be cut (tokens; `gran` below is 64).  The cost of a wide tile's set-up in
 // walked tokens decides what a cut is worth; the floors keep the pieces of small launches worth their
@@ -552,7 +562,8 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   };
   BundleSums wide_sums;
   if (pack) wide_sums = measure_bundles();
-  if (pack && stream_groups > 0 && wide_chain_tokens > 0) {
+  out.apart = cap && fixed_apart(shape, *cap);
+  if (!out.apart && stream_groups > 0 && wide_chain_tokens + wide_group_tokens > 0) {
     // The launch holds the runs of stand-alone sub-requests as well.  A CU left to those while the wide slots run takes
     // in twice what it gets when all of them stream (52 against 26 bytes a ns: 256 share what the memory gives), so some
     // lanes give theirs up: as many as the estimated end of the launch says.  Rates: 24 ns for a token of a wide tile
@@ -572,19 +583,23 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
       return ns + std::min(ns, 20e3);
     };
     const BundleSums all = wide_sums;
-    double best = 0, all_end = 0;
+    // (wide tiles of decode rows, and the chunks' where they fill the machine several times over, are left out of both sides)
+    double best = std::max(memory_ns, cu_ns / 256.0), all_end = best, all_wide_ns = 0;
     int32_t best_lanes = all_lanes;
-    for (; lanes >= 1; lanes -= std::max(1, all_lanes / 8)) {
+    for (; pack && wide_chain_tokens > 0 && lanes >= 1; lanes -= std::max(1, all_lanes / 8)) {
       const BundleSums sums = lanes == all_lanes ? all : measure_bundles();
       const double share = (double)lanes / all_lanes, token_ns = 21.0 + 3.0 * share;
       const double wide_ns = 10e3 + token_ns * (double)sums.cost / groups_wanted;
-      // (fewer lanes walk no less: neither these nor any fewer end before what was found)
+      // Fewer lanes walk no less: neither these nor any fewer end before what was found.  (The search is most of the
+      // planner's time where chunks have many blocks: all lanes tried, 8 rows beside 16 chunks of 215 over 20 blocks took
+      // 465 us where 234 are enough.)
       if (lanes < all_lanes && wide_ns >= best) break;
       const double busy_ns = 256.0 * 10e3 * share + token_ns * (double)sums.lane_cost * shape->num_kv_heads;
       const double idle_ns = std::max(0.0, 256.0 * wide_ns - busy_ns);
       const double end = wide_ns + behind(1.0 - std::min({1.0, idle_ns / cu_ns, wide_ns / memory_ns}));
       if (lanes == all_lanes) {
         all_end = best = end;
+        all_wide_ns = wide_ns;
         if (wide_ns >= 0.97 * all_end) break;  // next to nothing is left behind the wide slots
       } else if (end < 0.97 * best) {
         best = end;
@@ -594,6 +609,21 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     }
     lanes = best_lanes;
     if (best >= 0.97 * all_end) {  // (an estimate: it has to promise something)
+      lanes = all_lanes;
+      best = all_end;
+      wide_sums = all;
+    }
+    // Beside wide slots a streaming workgroup has a CU to itself.  In a launch of its own, 15 us behind the wide one's
+    // start, two of them share a CU at head dims under 256, three or four where items are short (two at 256): that wins
+    // where their set-ups and folds outweigh what the wide slots leave idle.  64 rows of 300..900 tokens and a chunk of
+    // 300, us, one launch / two: 63 / 74 at 256 dims (16 q / 4 kv heads), 76 / 78 at 128 (32 / 8), 111 / 78 at 64 (64 / 16);
+    // 128 of 136..436 and a chunk of 100 66 / 72, 90 / 74, 133 / 74; 48 of 1 k..4 k and 2 chunks of 512 136 / 164,
+    // 153 / 161, 187 / 174; 32 of 4 k..9 k and one 188 / 228, 212 / 234, 249 / 266.
+    const bool are_short = stream_tokens <= kShortItem * stream_groups;
+    const double beside = shape->head_dim == 256 ? (are_short ? 1.3 : 1.0) : shape->head_dim == 128 ? (are_short ? 1.6 : 1.4)
+                                                                                                   : (are_short ? 2.2 : 1.6);
+    if (!cap && all_wide_ns + 15e3 + std::max(memory_ns, cu_ns / 256.0 / beside) < 0.97 * best) {
+      out.apart = true;
       lanes = all_lanes;
       wide_sums = all;
     }
@@ -793,7 +823,7 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     }
   }
 
-  // Launch order.  Wide items first (their own launch), then narrow ones.  The hardware hands
+  // Launch order.  Wide items first, then narrow ones (behind them in one launch, or in one of their own).  The hardware hands
   // workgroup b of a launch to die b % 8, and each die has its own L2, so within a class:
   //   * units (the tiles that stream one K/V chunk) are dealt to the 8 dies, heaviest first, each
   //     to the least loaded die, and stay together there: the chunk is fetched from HBM by one
@@ -803,20 +833,25 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   //   * position p of the class holds entry p / 8 of die p % 8; dies with fewer entries are
   //     padded with empty items (n_q = 0, the kernels return at once), which also keeps the
   //     class a multiple of 8 long so the next kv head starts on die 0 again.
-  if (kernel == VA_KERNEL_MFMA && !cap && (int64_t)out.items.size() * shape->num_kv_heads > 256) {
-    int64_t tokens = 0, again = 0;  // of all items; of those that walk together, beyond the first of each workgroup
-    bool only_narrow = true;
+  if (kernel == VA_KERNEL_MFMA && !cap) {
+    // of the narrow items; of those that walk together, beyond the first of each workgroup
+    int64_t n = 0, tokens = 0, again = 0;
+    bool by_themselves = true;
     int32_t in_unit = 0, unit = -1;
     for (const auto& it : out.items) {  // (the items of a unit stand side by side)
-      only_narrow = only_narrow && it.kind == 0;
+      if (it.kind != 0) {
+        by_themselves = out.apart;
+        continue;
+      }
       in_unit = it.unit >= 0 && it.unit == unit ? in_unit + 1 : 0;
       unit = it.unit;
+      ++n;
       tokens += it.tokens;
       if (in_unit % it.together) again += it.tokens;
     }
     // (a fifth: of 64 requests over 512 shared tokens and blocks of 100..400, 13 % walked again, 35.9 -> 32.5 us apart at
     // 256 dims, 33 either way at 128, 46.8 -> 36.7 at 64; over 2048, 29 %, at 128 dims 42 together)
-    out.short_items = only_narrow && tokens <= 640 * (int64_t)out.items.size() && again <= tokens / 5;
+    out.short_items = by_themselves && n * shape->num_kv_heads > 256 && tokens <= kShortItem * n && again <= tokens / 5;
     if (out.short_items)
       for (auto& it : out.items) it.together = 1;
   }
@@ -1058,7 +1093,8 @@ static int write_plan(const Built& b, const VaSubRequests* subs, const VaShape* 
   h[VA_H_MAGIC] = VA_PLAN_MAGIC;
   h[VA_H_KERNEL] = c.kernel;
   h[VA_H_Q_TILE] = c.q_tile;
-  h[VA_H_KV_CHUNK] = cap ? 0 : c.kv_chunk | (b.short_items ? VA_CHUNK_SHORT_ITEMS : 0);  // chosen per plan: not part of a fixed plan's header (see counts)
+  // (the chunk is chosen per plan: not part of a fixed plan's header, see counts)
+  h[VA_H_KV_CHUNK] = (cap ? 0 : c.kv_chunk) | (b.short_items ? VA_CHUNK_SHORT_ITEMS : 0) | (b.apart ? VA_CHUNK_APART : 0);
   h[VA_H_N_WIDE] = cap_wide;
   h[VA_H_WIDE_TILE] = c.wide_tile;
   h[VA_H_N_ITEMS] = cap_wide + cap_narrow;

@@ -61,15 +61,18 @@ enum {
 #define VA_TOGETHER 4
 #define VA_TOGETHER_SCATTERED 2
 
-// Beside the chunk in its header word (a multiple of 64; the word is 0 in plans of fixed capacity, so that a recorded
-// launch keeps its kernel): narrow items by themselves that are short, more than one for every CU, and that walk next to
-// no tokens together.  An item's set-up and fold take as long as its walk there, so several workgroups share a CU
+// Flags beside the chunk in its header word (a multiple of 64; 0 in plans of fixed capacity).
+// Narrow items of a launch of their own that are short, more than one for every CU, and that walk next to
+// no tokens together (packed plans only: a recorded launch keeps its kernel).  An item's set-up and fold take as long as its walk there, so several workgroups share a CU
 // (attn_stream_short_kernel).
 // 64 requests over a shared block and one or two private ones, us a layer, one workgroup a CU (two under 256 dims) and
 // now: 64 shared tokens and blocks of 300..900, 16 q / 4 kv heads of 256 dims 59.0 -> 51.4, 32 / 8 of 128 54.5 -> 51.0,
 // 64 / 16 of 64 70.1 -> 53.6; blocks of 100..400 34.5 -> 29.7, 30.6 -> 29.7, 44.7 -> 33.3.  Where the tiles of 8192 shared
 // tokens make up the launch they stay together: at 128 dims 55 us, and 84 apart.
 #define VA_CHUNK_SHORT_ITEMS 1
+// Wide and narrow items get a launch each (one launch serves both otherwise).  In a plan of fixed capacity a matter of the
+// capacity and the shape alone.
+#define VA_CHUNK_APART 2
 
 // link word indices
 enum {

@@ -870,7 +870,8 @@ static int attention_launches(const void* q_dev, int64_t q_row_stride, const voi
   if (n_items > 0) {
     if (h[VA_H_KERNEL] == VA_KERNEL_MFMA) {
       rc = va::launch_mfma(a, shape->dtype, n_items, h[VA_H_N_WIDE], h[VA_H_N_WIDE_SLOTS], h[VA_H_Q_TILE],
-                           (h[VA_H_KV_CHUNK] & VA_CHUNK_SHORT_ITEMS) != 0, s);
+                           (h[VA_H_KV_CHUNK] & VA_CHUNK_SHORT_ITEMS) != 0, (h[VA_H_KV_CHUNK] & VA_CHUNK_APART) != 0,
+                           s);
     } else {
       VA_DISPATCH_DTYPE(shape->dtype, rc = va::launch_generic<E>(a, n_items, s));
     }

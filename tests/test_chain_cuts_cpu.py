@@ -8,6 +8,7 @@ import pytest
 
 from async_llm_amd import native
 
+from .test_fixed_plan_cpu import fixed_plan
 from .test_native_abi_cpu import H, build_plan, check_coverage, decode_plan
 
 
@@ -148,19 +149,20 @@ def test_sharing_out_the_cus_costs_little_planning(heads, rows, requests):
     # (measured: 1.04 to 1.13 times the chunks' own planning; every number of lanes tried, 1.4 to 2.2 times)
     chunks = _tables(requests, 16)
     shape, params = native.VaShape(*heads, 16, native.VA_BF16), native.VaPlanParams(native.VA_KERNEL_MFMA, 0, 0, 0, 0)
-    blob, counts, best = np.empty(1 << 20, dtype=np.int32), native.VaPlanCounts(), []
-    for tables in (chunks, _with_decode_rows(chunks, rows, 2000, 16)):
-        qo, kvp, kvi, lens, flags, chain, sw, n_rows = tables
+    blob, counts, plans, best = np.empty(1 << 20, dtype=np.int32), native.VaPlanCounts(), [], [np.inf, np.inf]
+    for qo, kvp, kvi, lens, flags, chain, sw, n_rows in (chunks, _with_decode_rows(chunks, rows, 2000, 16)):
         i32 = [np.asarray(a, dtype=np.int32) for a in (qo, kvp, kvi, lens, flags, chain)]
         sub_worker = np.asarray(sw, dtype=np.int64)
-        subs = native.VaSubRequests(len(lens), len(sw), n_rows, *(a.ctypes.data for a in i32), sub_worker.ctypes.data)
-        times = []
-        for _ in range(30):
+        plans.append((i32, sub_worker, native.VaSubRequests(len(lens), len(sw), n_rows, *(a.ctypes.data for a in i32),
+                                                            sub_worker.ctypes.data)))
+    for k in range(300):  # (in turn, and longer where the machine is busy with something else)
+        for i, (*_, subs) in enumerate(plans):
             start = time.perf_counter()
             rc = native.lib.va_plan_build_within(subs, shape, params, -1, blob.ctypes.data, blob.size, counts)
-            times.append(time.perf_counter() - start)
+            best[i] = min(best[i], time.perf_counter() - start)
             assert rc == 0
-        best.append(min(times))
+        if k >= 20 and best[1] <= 1.3 * best[0]:
+            break
     assert best[1] <= 1.3 * best[0], best
 
 
@@ -173,3 +175,24 @@ def test_rows_that_outlast_a_small_chunk_get_the_cus_at_once(heads):
     qo, kvp, _, lens, flags, _, sw, n_rows = tables
     assert rc == 0 and 0 < counts.n_wide_slots <= 256 // heads[1] // 2
     check_coverage(blob, qo, kvp, lens, flags, sw, n_rows)
+
+
+@pytest.mark.parametrize("heads,apart", [((16, 4, 256), 0), ((8, 2, 128), 0), ((32, 8, 128), 1), ((64, 16, 64), 1)])
+def test_many_short_rows_get_a_launch_of_their_own(heads, apart):
+    # (128 rows of 136..436 tokens beside a chunk of 100, us, one launch / two: 66 / 72, 31 / 44, 90 / 74, 133 / 74)
+    chunk = _tables([(100, 64, [250])], 16)
+    tables = _with_decode_rows(chunk, 128, 250, 16)
+    rc, blob, counts = build_plan(*tables, heads=heads, page=16, dtype=native.VA_BF16, kernel=native.VA_KERNEL_MFMA)
+    qo, kvp, _, lens, flags, _, sw, n_rows = tables
+    assert rc == 0 and counts.n_wide_items > 0
+    assert blob[H["KV_CHUNK"]] == counts.kv_chunk + 3 * apart  # VA_CHUNK_SHORT_ITEMS, VA_CHUNK_APART
+    check_coverage(blob, qo, kvp, lens, flags, sw, n_rows)
+    # a long row beside the chunk: together
+    rc, blob, counts = build_plan(*_with_decode_rows(chunk, 1, 9000, 16), heads=heads, page=16, dtype=native.VA_BF16,
+                                  kernel=native.VA_KERNEL_MFMA)
+    assert rc == 0 and blob[H["KV_CHUNK"]] == counts.kv_chunk
+    # recorded: by the capacity and the shape alone, whatever the plan holds
+    for rows, held in [(128, tables), (128, _with_decode_rows(chunk, 1, 9000, 16)), (0, chunk)]:
+        limits = native.VaPlanLimits(rows, rows, 1, 2, 100, 100 + rows)
+        rc, blob, *_ = fixed_plan(held, limits, heads=heads, page=16, kernel=native.VA_KERNEL_MFMA)
+        assert rc == 0 and blob[H["KV_CHUNK"]] == (2 if heads[2] == 64 and rows else 0)

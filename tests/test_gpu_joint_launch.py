@@ -31,3 +31,19 @@ def test_wide_and_streaming_items_share_a_launch(dtype, heads, page, rows, chunk
     # planned again, the same bits: nothing hangs on which workgroup a CU gets first
     again, again_lse = wl.op.attend(wl.q, 0, wl.meta, return_lse=True)
     assert torch.equal(out, again) and torch.equal(lse, again_lse)
+
+
+@pytest.mark.parametrize("dtype,heads,page,apart", [(torch.bfloat16, (64, 16, 64), 16, 3), (torch.float16, (32, 8, 128), 16, 3),
+                                                    (torch.bfloat16, (32, 16, 128), 1, 3), (torch.float16, (64, 16, 64), 24, 3),
+                                                    (torch.bfloat16, (16, 4, 256), 16, 0)])
+def test_short_rows_beside_a_chunk_get_a_launch_of_their_own(dtype, heads, page, apart):
+    print(f"heads {heads} page {page}", flush=True)
+    wl = workloads.mixed_batch(DEV, decode_rows=128, chunks=1, chunk_len=100, ctx_lo=200, ctx_hi=500, shared_len=64,
+                               heads=heads, dtype=dtype, page_size=page, kernel="mfma")
+    assert wl.meta.launch.counts.n_wide_items > 0 and wl.meta.launch.header[3] % 64 == apart
+    out, lse = wl.op.forward_with_lse(wl.q, wl.k, wl.v, 0, wl.batch)
+    wl.op.plan_params.kernel = native.VA_KERNEL_GENERIC
+    expected, expected_lse = wl.op.attend(wl.q, 0, wl.op.prepare_mixed(wl.group, wl.pending, wl.new_token_slots, wl.specs),
+                                          return_lse=True)
+    assert_close(out.cpu(), expected.cpu().view_as(out.cpu()), dtype, "out")
+    assert_close(lse.cpu(), expected_lse.cpu(), dtype, "lse")
