@@ -125,6 +125,7 @@ bool fixed_apart(const VaShape* shape, const VaPlanCapacity& cap) {
   return shape->head_dim == 64 && cap.max_wide_items > 0 && cap.max_qrefs > 0;
 }
 
+constexpr int32_t kLongestShort = 1024;  // tokens: a run up to this is short
 constexpr int64_t kShortItem = 640;  // tokens of a narrow item, on average, up to which several workgroups share a CU
 
 // How finely the walks of chains may be cut (tokens; `gran` below is 64).  The cost of a wide tile's set-up in
@@ -414,10 +415,15 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     // narrow tiles: chunk-major; wide tiles: their own (finer) chunking
     const int32_t per = chunk_len(kv_chunk);
     // The last chunk of a run is cut in two: every run then contributes short items, which the
-    // launch order puts last, so the launch does not end on a round of full-length items (not where all run at once).
+    // launch order puts last, so the launch does not end on a round of full-length items.  Not where all run at once, and
+    // not a run of one short chunk: two set-ups and folds cost more than the shorter walks give (64 requests over 512 shared
+    // tokens and blocks of 100..400, us, cut / whole: 32.5 / 26.0 at 256 dims, 33.0 / 26.8 at 128, 36.9 / 28.1 at 64; over
+    // 8192 and blocks of 256..8192, 296 / 307 if the long ones are left whole as well).
     std::vector<int32_t> cuts{0};
     for (int32_t t0 = per; t0 < len; t0 += per) cuts.push_back(t0);
-    if (len - cuts.back() >= 4 * gran && !one_round) cuts.push_back(cuts.back() + round_up((len - cuts.back()) / 2, gran));
+    const bool whole = kernel == VA_KERNEL_MFMA && cuts.size() == 1 && len <= kLongestShort;
+    if (len - cuts.back() >= 4 * gran && !one_round && !whole)
+      cuts.push_back(cuts.back() + round_up((len - cuts.back()) / 2, gran));
     cuts.push_back(len);
     for (size_t ci = 0; ci + 1 < cuts.size(); ++ci) {
       if (cuts[ci] >= cuts[ci + 1]) continue;

@@ -196,3 +196,17 @@ def test_many_short_rows_get_a_launch_of_their_own(heads, apart):
         limits = native.VaPlanLimits(rows, rows, 1, 2, 100, 100 + rows)
         rc, blob, *_ = fixed_plan(held, limits, heads=heads, page=16, kernel=native.VA_KERNEL_MFMA)
         assert rc == 0 and blob[H["KV_CHUNK"]] == (2 if heads[2] == 64 and rows else 0)
+
+
+@pytest.mark.parametrize("heads", [(16, 4, 256), (32, 8, 128), (64, 16, 64)])
+def test_runs_of_one_short_chunk_stay_whole(heads):
+    # 64 rows of 300..400 tokens: a second set-up and fold cost more than half the walk (64 over 512 shared tokens and blocks
+    # of 100..400, us, cut in two / whole: 32.5 / 26.0, 33.0 / 26.8, 36.9 / 28.1); longer ones are cut, for the end of the launch
+    rows = [300 + 7 * (i % 15) for i in range(64)] + [1500] * 9
+    kvp = np.cumsum([0] + [-(-n // 16) for n in rows]).tolist()
+    tables = (list(range(len(rows) + 1)), kvp, list(range(kvp[-1])), rows, [0] * len(rows), [-1] * len(rows),
+              list(range(len(rows))), len(rows))
+    rc, blob, _ = build_plan(*tables, heads=heads, page=16, dtype=native.VA_BF16, kernel=native.VA_KERNEL_MFMA, kv_chunk=1536)
+    assert rc == 0
+    walked = sorted(int(it[4]) for it in decode_plan(blob)[1] if it[2] > 0)
+    assert walked == sorted(rows[:64] + [768] * 9 + [732] * 9)
