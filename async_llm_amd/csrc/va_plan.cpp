@@ -101,7 +101,7 @@ inline int32_t visible_end(int32_t len, int32_t nq, bool causal, int32_t b) {
   return causal ? std::min(len, len - nq + b) : len;
 }
 
-// Narrow tiles of a run of `tokens` that a workgroup serves together.  Four where the run is long: 64 readers of
+// Narrow tiles of a run of `tokens` that a workgroup serves together at most.  Four where the run is long: 64 readers of
 // 8192 tokens beside private blocks (16 q / 4 kv heads of 256 dims) 353 us a layer alone, 322 in pairs, 313 in fours.
 // Four tiles walk at two thirds of the pace of two when memory does not bound them, which a short run beside long ones
 // shows: 48 readers of 512 tokens, 483 us in pairs, 494 in fours.
@@ -125,8 +125,8 @@ bool fixed_apart(const VaShape* shape, const VaPlanCapacity& cap) {
   return shape->head_dim == 64 && cap.max_wide_items > 0 && cap.max_qrefs > 0;
 }
 
-constexpr int32_t kLongestShort = 1024;  // tokens: a run up to this is short
-constexpr int64_t kShortItem = 640;  // tokens of a narrow item, on average, up to which several workgroups share a CU
+constexpr int32_t kLongestShort = 1024;  // tokens of a short run or item
+constexpr int64_t kReadAgain = 256ll << 20;  // bytes that tiles of one run, apart, may read again from the dies' L2
 
 // How finely the walks of chains may be cut (tokens; `gran` below is 64).  The cost of a wide tile's set-up in
 // walked tokens decides what a cut is worth; the floors keep the pieces of small launches worth their
@@ -249,8 +249,8 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   // 325 / 317, 605 / 615; 256 of 4096 beside 3.5 times 264 / 255.  From 0.64 GB on a longer rest is let pass (it costs 64
   // of 32768 some percent, and gains them with 128 readers).  So: on request always; otherwise plans of free size only.
   std::vector<char> group_is_wide(groups.size(), wide_on_request && wide_tile > 0);
+  const int64_t token_bytes = 2ll * shape->num_kv_heads * shape->head_dim * (shape->dtype == VA_F32 ? 4 : 2);
   if (!wide_on_request && wide_tile > 0 && !cap && shape->head_dim == 256) {
-    const int64_t token_bytes = 2ll * shape->num_kv_heads * shape->head_dim * (shape->dtype == VA_F32 ? 4 : 2);
     constexpr int64_t kWorthIt = 300ll << 20, kFairShare = kWorthIt / 8, kWorthMuch = 640ll << 20;
     std::vector<char> many(groups.size(), 0);
     int64_t saved = 0, walked = 0, rest = 0;  // bytes; tokens that narrow tiles walk for these groups, for the others
@@ -293,18 +293,6 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   }
 
   // ---- total tokens -> chunk size for split-KV ----
-  // (walks of a run of `gr`, whose tiles cut_tiles left in `tiles`: narrow tiles walk it together.  A recorded plan
-  // counts every tile: its capacity, and with it the workgroups that find nothing to do, hangs on the items.)
-  auto walks_of = [&](const Group& gr, bool may_be_wide) {
-    const int64_t n = (int64_t)tiles.size(), at_once = tiles_together(kernel, shape->page_size, s->seq_lens[gr.rep]);
-    return may_be_wide || cap ? n : (n + at_once - 1) / at_once;
-  };
-  int64_t total_tokens = 0;
-  for (auto& gr : groups) {
-    const bool may_be_wide = group_is_wide[&gr - &groups[0]];
-    cut_tiles((int64_t)gr.subrows.size(), tiles, may_be_wide);
-    total_tokens += walks_of(gr, may_be_wide) * s->seq_lens[gr.rep];
-  }
   int64_t chain_tiles = 0, chain_tokens = 0, wide_chain_tokens = 0;
   for (auto& ch : chains) {
     const int32_t nq = s->qo_indptr[ch[0] + 1] - s->qo_indptr[ch[0]];
@@ -322,34 +310,62 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   // would otherwise triple it, and the decode items would run in two long rounds instead of four short ones)
   int32_t kv_chunk = params && params->kv_chunk > 0 ? round_up(params->kv_chunk, gran) : 0;
   bool one_round = false;  // the narrow items of the launch all start at once
-  if (kv_chunk == 0) {
-    const int64_t per_item = (total_tokens + target - 1) / target;
+  // Walks of a group's run, and tokens of all walks: by every tile ([1]), or by the workgroups, whose narrow tiles walk it
+  // together ([0]).
+  std::vector<int64_t> walks[2];
+  int64_t walked[2] = {0, 0};
+  for (size_t gi = 0; gi < groups.size(); ++gi) {
+    const int64_t len = s->seq_lens[groups[gi].rep], at_once = group_is_wide[gi] ? 1 : tiles_together(kernel, shape->page_size, len);
+    cut_tiles((int64_t)groups[gi].subrows.size(), tiles, group_is_wide[gi]);
+    for (int each = 0; each < 2; ++each) {
+      walks[each].push_back(each ? (int64_t)tiles.size() : ((int64_t)tiles.size() + at_once - 1) / at_once);
+      walked[each] += walks[each].back() * len;
+    }
+  }
+  const bool any_wide = wide_chain_tokens > 0 || std::find(group_is_wide.begin(), group_is_wide.end(), 1) != group_is_wide.end();
+  auto size_chunk = [&](bool each) {
+    if (params && params->kv_chunk > 0) return;
+    const int64_t per_item = (walked[each] + target - 1) / target;
     // No chunk under four granules as a rule (an item's set-up is worth a few hundred tokens) -- unless the
     // launch holds so few tokens that such chunks would leave most of the machine idle: then the time of
     // the launch is the walk of ONE item, a chain of dependent trips to memory, and shorter walks side by
     // side (down to one granule) are what shortens it.
     int64_t least = 4 * gran;
-    if (kernel == VA_KERNEL_MFMA && per_item < 8 * gran) {
-      // The shortest chunks of up to eight granules whose items all run at once and leave a quarter of the room: chunks
+    one_round = false;
+    const int64_t most = (shape->head_dim == 128 ? 16 : 8) * gran;
+    if (kernel == VA_KERNEL_MFMA && per_item < most) {
+      // The shortest chunks of up to eight granules whose items all run at once and leave a fifth to a quarter of the room: chunks
       // of 128 / 192 / 256 / 320 tokens, attention and merge of a layer, 4 requests of 2100..4000 tokens (4 kv heads of
       // 256 dims, 60 / 43 / 35 / 29 items for 64 at once) 18.2 / 15.8 / 16.1 / 17.0 us; 256 / 320 / 384 / 512, 8 of
-      // 1400..4000 (8 of 128 dims, 69 / 60 / 53 / 42 for 64) 21.4 / 19.6 / 20.1 / 19.6.
-      const int64_t at_once = std::max(1, (shape->head_dim == 256 ? 192 : 384) / shape->num_kv_heads);
-      for (least = gran; least < 8 * gran; least += gran) {
+      // 1400..4000 (8 of 128 dims, 69 / 60 / 53 / 42 for 64) 21.4 / 19.6 / 20.1 / 19.6.  At 128 dims up to sixteen: 16
+      // requests of 64..2048 behind 1500 shared tokens (8 kv heads), chunks of 512 / 896, 30.9 / 28.6 us.
+      const int64_t at_once = std::max(1, (shape->head_dim != 256 ? 384 : any_wide ? 192 : 208) / shape->num_kv_heads);
+      for (least = gran; least < most; least += gran) {
         int64_t n = 0;
-        for (size_t gi = 0; gi < groups.size(); ++gi) {
-          cut_tiles((int64_t)groups[gi].subrows.size(), tiles, group_is_wide[gi]);
-          n += walks_of(groups[gi], group_is_wide[gi]) * ((s->seq_lens[groups[gi].rep] + least - 1) / least);
-        }
+        for (size_t gi = 0; gi < groups.size(); ++gi) n += walks[each][gi] * ((s->seq_lens[groups[gi].rep] + least - 1) / least);
         one_round = n <= at_once;
         if (one_round) break;
       }
+      if (!one_round) least = 8 * gran;
     } else if (kernel != VA_KERNEL_MFMA) {
-      const int64_t spread = (total_tokens + (256 / shape->num_kv_heads) - 1) / std::max(1, 256 / shape->num_kv_heads);
+      const int64_t spread = (walked[each] + (256 / shape->num_kv_heads) - 1) / std::max(1, 256 / shape->num_kv_heads);
       least = std::min<int64_t>(least, std::max<int64_t>(gran, round_up(spread, gran)));
     }
     kv_chunk = round_up(std::max<int64_t>(per_item, least), gran);
-  }
+  };
+  // Short items want to share CUs (VA_CHUNK_SHORT_ITEMS), a tile a workgroup: the set-ups and folds of fours and pairs are
+  // serial.  Attention and merge of a layer, us, fours / pairs / apart in the kernel for short items: 16 readers of 4096 tokens
+  // and blocks of 64..200 29.5 / 23.3 / 16.9 at 256 dims (16 q / 4 kv heads), 23.6 / 20.6 / 15.6 at 128 (32 / 8),
+  // 20.2 / 20.3 / 17.7 at 64 (64 / 16); 64 of 2048 and 100..400, pairs / apart, 43 / 40, 38 / 38, 51 / 39; 128 of 2048 and
+  // 64..256 68 / 52, 62 / 54, 75 / 73.  Not where what the tiles read again from the dies' L2 is the launch: 128 of 4096
+  // (0.4 GB) and 100..400 at 128 dims, fours 74, apart 105; nor in longer chunks: 64 of 2048 and 1000..2000 (1344) 112 / 121,
+  // 116 / 122.  (A recorded plan, whose kernel may not change, counts every tile: its capacity, and with it the workgroups
+  // that find nothing to do, hangs on the items.)
+  bool each = kernel != VA_KERNEL_MFMA || cap || !any_wide;
+  size_chunk(each);
+  const bool tiles_short = kernel == VA_KERNEL_MFMA && !cap && !any_wide && kv_chunk <= kLongestShort &&
+                           (walked[1] - walked[0]) * token_bytes <= kReadAgain;
+  if (kernel == VA_KERNEL_MFMA && !cap && each && !tiles_short) size_chunk(each = false);
 
   out.kernel = kernel;
   out.q_tile = q_tile;
@@ -387,7 +403,6 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   const int32_t wide_chunk = std::min<int32_t>(
       kv_chunk, round_up(std::max<int64_t>((wide_group_tokens + wide_items_wanted - 1) / wide_items_wanted, 2 * gran), gran));
 
-  int64_t stream_groups = 0, stream_tokens = 0;  // workgroups per kv head that serve the narrow tiles, what they walk
   for (auto& gr : groups) {
     const int32_t rep = gr.rep;
     const int32_t len = s->seq_lens[rep];
@@ -428,19 +443,36 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     for (size_t ci = 0; ci + 1 < cuts.size(); ++ci) {
       if (cuts[ci] >= cuts[ci + 1]) continue;
       const int32_t unit = next_unit++;  // the narrow tiles of one chunk: same die, side by side
-      int32_t in_unit = 0;
-      for (size_t ti = 0; ti < tiles.size(); ++ti) {
-        if (tiles[ti].second - tiles[ti].first > q_tile) continue;
-        emit_range(ti, cuts[ci], cuts[ci + 1], unit);
-        if (in_unit++ % out.items.back().together) continue;
-        ++stream_groups;
-        stream_tokens += out.items.back().tokens;
-      }
+      for (size_t ti = 0; ti < tiles.size(); ++ti)
+        if (tiles[ti].second - tiles[ti].first <= q_tile) emit_range(ti, cuts[ci], cuts[ci + 1], unit);
     }
     const int32_t per_w = chunk_len(wide_chunk);
     for (size_t ti = 0; ti < tiles.size(); ++ti)
       if (tiles[ti].second - tiles[ti].first > q_tile)
         for (int32_t t0 = 0; t0 < len; t0 += per_w) emit_range(ti, t0, std::min(len, t0 + per_w));
+  }
+
+  // Tiles that walk together: not where all start at once apart, and no more to a workgroup than leave every CU one (16
+  // readers of 4096 tokens and blocks of 64..200, 256 dims, recorded: in fours 41 us, in pairs 23; 8 readers of 64 tokens and
+  // blocks of 64..200, 32 items to each head: in pairs 12.7, apart 10.1).
+  const int64_t room = shape->head_dim == 256 ? 320 : 512;  // workgroups that start at once (at 256 dims and a few)
+  int64_t stream_groups = 0, stream_tokens = 0;  // workgroups per kv head that serve the narrow tiles, what they walk
+  if (kernel == VA_KERNEL_MFMA) {
+    int32_t most = tiles_short || (int64_t)out.items.size() * shape->num_kv_heads <= room ? 1 : VA_TOGETHER;
+    for (;; most /= 2) {
+      stream_groups = stream_tokens = 0;
+      int32_t in_unit = 0, unit = -1;
+      for (auto& it : out.items) {  // (the items of a unit stand side by side)
+        if (it.kind != 0) continue;
+        in_unit = it.unit == unit ? in_unit + 1 : 0;
+        unit = it.unit;
+        it.together = std::min(it.together, most);
+        if (in_unit % it.together) continue;
+        ++stream_groups;
+        stream_tokens += it.tokens;
+      }
+      if (most == 1 || stream_groups * shape->num_kv_heads >= 256) break;
+    }
   }
 
   // Chains.  When the tiles of all chains are many (several rounds of one workgroup per CU) every
@@ -625,7 +657,7 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     // 300, us, one launch / two: 63 / 74 at 256 dims (16 q / 4 kv heads), 76 / 78 at 128 (32 / 8), 111 / 78 at 64 (64 / 16);
     // 128 of 136..436 and a chunk of 100 66 / 72, 90 / 74, 133 / 74; 48 of 1 k..4 k and 2 chunks of 512 136 / 164,
     // 153 / 161, 187 / 174; 32 of 4 k..9 k and one 188 / 228, 212 / 234, 249 / 266.
-    const bool are_short = stream_tokens <= kShortItem * stream_groups;
+    const bool are_short = kv_chunk <= kLongestShort;
     const double beside = shape->head_dim == 256 ? (are_short ? 1.3 : 1.0) : shape->head_dim == 128 ? (are_short ? 1.6 : 1.4)
                                                                                                    : (are_short ? 2.2 : 1.6);
     if (!cap && all_wide_ns + 15e3 + std::max(memory_ns, cu_ns / 256.0 / beside) < 0.97 * best) {
@@ -840,24 +872,25 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   //     padded with empty items (n_q = 0, the kernels return at once), which also keeps the
   //     class a multiple of 8 long so the next kv head starts on die 0 again.
   if (kernel == VA_KERNEL_MFMA && !cap) {
-    // of the narrow items; of those that walk together, beyond the first of each workgroup
-    int64_t n = 0, tokens = 0, again = 0;
+    int64_t n = 0, tokens = 0;
+    int32_t longest = 0;
     bool by_themselves = true;
-    int32_t in_unit = 0, unit = -1;
-    for (const auto& it : out.items) {  // (the items of a unit stand side by side)
+    for (const auto& it : out.items) {
       if (it.kind != 0) {
         by_themselves = out.apart;
         continue;
       }
-      in_unit = it.unit >= 0 && it.unit == unit ? in_unit + 1 : 0;
-      unit = it.unit;
       ++n;
       tokens += it.tokens;
-      if (in_unit % it.together) again += it.tokens;
+      longest = std::max(longest, it.tokens);
     }
-    // (a fifth: of 64 requests over 512 shared tokens and blocks of 100..400, 13 % walked again, 35.9 -> 32.5 us apart at
-    // 256 dims, 33 either way at 128, 46.8 -> 36.7 at 64; over 2048, 29 %, at 128 dims 42 together)
-    out.short_items = by_themselves && n * shape->num_kv_heads > 256 && tokens <= kShortItem * n && again <= tokens / 5;
+    // Where CUs have one item each the other kernel's deeper rings are the better ones (12 requests of 300..2000 behind 128
+    // shared tokens, 300 workgroups at 256 dims, 22.6 / 24.6 us; at 64 dims they never are) unless readers of one run walk it
+    // apart: their tiles in flight, 128 KB a CU, push each other out of the die's L2 (16 readers of 4096 tokens, 224
+    // workgroups at 256 dims, 22.5 / 16.9).
+    const int64_t one_each = shape->head_dim == 256 ? room : shape->head_dim == 128 ? 256 : 0, again = walked[1] - walked[0];
+    out.short_items = by_themselves && longest <= kLongestShort && again * token_bytes <= kReadAgain &&
+                      (n * shape->num_kv_heads > one_each || again > tokens / 8);
     if (out.short_items)
       for (auto& it : out.items) it.together = 1;
   }

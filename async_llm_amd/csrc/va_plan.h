@@ -62,13 +62,11 @@ enum {
 #define VA_TOGETHER_SCATTERED 2
 
 // Flags beside the chunk in its header word (a multiple of 64; 0 in plans of fixed capacity).
-// Narrow items of a launch of their own that are short, more than one for every CU, and that walk next to
-// no tokens together (packed plans only: a recorded launch keeps its kernel).  An item's set-up and fold take as long as its walk there, so several workgroups share a CU
-// (attn_stream_short_kernel).
-// 64 requests over a shared block and one or two private ones, us a layer, one workgroup a CU (two under 256 dims) and
-// now: 64 shared tokens and blocks of 300..900, 16 q / 4 kv heads of 256 dims 59.0 -> 51.4, 32 / 8 of 128 54.5 -> 51.0,
-// 64 / 16 of 64 70.1 -> 53.6; blocks of 100..400 34.5 -> 29.7, 30.6 -> 29.7, 44.7 -> 33.3.  Where the tiles of 8192 shared
-// tokens make up the launch they stay together: at 128 dims 55 us, and 84 apart.
+// Narrow items of a launch of their own that are short: their set-up and fold take as long as their walk, so several
+// workgroups share a CU and serve a tile each (attn_stream_short_kernel, whose workgroups take no notice of VA_I_PARTNERS).
+// 64 requests over 64 shared tokens and one or two private blocks, us a layer, in the kernel before independent waves / in
+// the ordinary kernel / now: blocks of 300..900, 16 q / 4 kv heads of 256 dims 48.9 / 60.3 / 50.3, 32 / 8 of 128
+// 51.7 / 53.6 / 49.9, 64 / 16 of 64 61.3 / 61.9 / 50.9; of 100..400 26.9 / 31.6 / 24.8, 28.4 / 29.4 / 26.2, 36.5 / 40.1 / 28.0.
 #define VA_CHUNK_SHORT_ITEMS 1
 // Wide and narrow items get a launch each (one launch serves both otherwise).  In a plan of fixed capacity a matter of the
 // capacity and the shape alone.

@@ -598,21 +598,14 @@ __device__ __forceinline__ void stream_block(const AttnArgs& a, unsigned block) 
   }
 }
 
-// The same where items are short: its workgroups serve a tile each (a plan whose tiles walk together gets them one after
-// the other).
+// The same where items are short: its workgroups serve a tile each, also one that a plan would have walk with others.
 template <typename E, int kD, bool kGather>
 __device__ __forceinline__ void stream_block_short(const AttnArgs& a, unsigned block) {
   const ItemHead where = item_and_head(block, a.num_kv_heads);
   int item[1][VA_ITEM_WORDS];
   load_item(a, where.item, item[0]);
-  const int partners = item[0][VA_I_PARTNERS];
-  if (item[0][VA_I_N_Q] == 0 || partners < 0) return;
-  for (int b = 0;;) {
-    stream_items<E, kD, kGather, 1, true>(a, item, where.head);
-    if (++b > partners) return;
-    __syncthreads();  // the states of the tile before have been read
-    load_item(a, where.item + 8 * b, item[0]);
-  }
+  if (item[0][VA_I_N_Q] == 0) return;
+  stream_items<E, kD, kGather, 1, true>(a, item, where.head);
 }
 
 }  // namespace va

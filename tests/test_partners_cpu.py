@@ -37,7 +37,7 @@ def _tables(rng, page):
 def test_partners_walk_the_tokens_of_the_item_before_them(heads, page, fixed):
     rng = random.Random(f"{heads}{page}")
     most = 0
-    for _ in range(2):
+    for _ in range(3):
         tables = _tables(rng, page)
         qo, kvp, kvi, lens, flags, chain, sw, n_rows = tables
         if fixed:
@@ -67,3 +67,34 @@ def test_partners_walk_the_tokens_of_the_item_before_them(heads, page, fixed):
         assert np.array_equal(served, (narrow[:, 2] > 0).astype(int))
     if fixed:  # (packed plans of short items keep their tiles apart; 16 rows of one request fill a tile)
         assert (most > 0) == (heads[0] // heads[1] < 16)
+
+
+def _readers(readers, shared, own, page=16):
+    kvi, kvp, lens, sw = [], [0], [], []
+    fresh = -(-shared // page)
+    for r in range(readers):
+        for pages, length in ((list(range(-(-shared // page))), shared), (list(range(fresh, fresh - (-own // page))), own)):
+            kvi += pages
+            kvp.append(len(kvi)), lens.append(length), sw.append(r)
+        fresh += -(-own // page)
+    return list(range(len(lens) + 1)), kvp, kvi, lens, [0] * len(lens), [-1] * len(lens), sw, readers
+
+
+@pytest.mark.parametrize("heads,readers,shared,own,short,packed,recorded", [
+    # all start at once apart (pairs 12.7 us, apart 10.1)
+    ((16, 4, 256), 8, 64, 130, False, 0, 0), ((16, 4, 256), 16, 64, 40, True, 0, 0), ((32, 8, 128), 8, 64, 130, False, 0, 0),
+    # pairs or fours would leave CUs without a workgroup (fours 29.5 us, apart 16.9; recorded fours 41, pairs 23)
+    ((16, 4, 256), 16, 4096, 130, True, 0, 0), ((32, 8, 128), 16, 4096, 130, True, 0, 0),
+    ((16, 4, 256), 30, 4096, 130, True, 0, 1),
+    # short items with few tokens read again; many read again; long items
+    ((32, 8, 128), 64, 2048, 250, True, 0, 1), ((32, 8, 128), 128, 4096, 250, False, 3, 3), ((16, 4, 256), 64, 8192, 5000, False, 3, 3),
+])
+def test_tiles_walk_together_where_the_launch_is_long(heads, readers, shared, own, short, packed, recorded):
+    tables = _readers(readers, shared, own)
+    rc, blob, _ = build_plan(*tables, heads=heads, page=16, dtype=native.VA_BF16, kernel=native.VA_KERNEL_MFMA, wide_tile=-1)
+    assert rc == 0
+    header, items, *_ = decode_plan(blob)
+    assert (header[H["KV_CHUNK"]] & 1 == 1) == short and max(items[:, PARTNERS]) == packed
+    limits = native.VaPlanLimits(2 * readers, 2 * readers, 0, 0, 0, readers)
+    rc, blob, *_ = fixed_plan(tables, limits, heads=heads, page=16, kernel=native.VA_KERNEL_MFMA)
+    assert rc == 0 and max(decode_plan(blob)[1][:, PARTNERS]) == recorded
