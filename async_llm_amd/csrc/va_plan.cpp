@@ -889,7 +889,7 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     // apart: their tiles in flight, 128 KB a CU, push each other out of the die's L2 (16 readers of 4096 tokens, 224
     // workgroups at 256 dims, 22.5 / 16.9).
     const int64_t one_each = shape->head_dim == 256 ? room : shape->head_dim == 128 ? 256 : 0, again = walked[1] - walked[0];
-    out.short_items = by_themselves && longest <= kLongestShort && again * token_bytes <= kReadAgain &&
+    out.short_items = by_themselves && (tiles_short || any_wide) && longest <= kLongestShort && again * token_bytes <= kReadAgain &&
                       (n * shape->num_kv_heads > one_each || again > tokens / 8);
     if (out.short_items)
       for (auto& it : out.items) it.together = 1;
