@@ -239,21 +239,23 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
 
   // Wide tiles for a group.  n readers in narrow tiles stream their block once for every workgroup's tiles (once from
   // memory, then from the die's L2), in wide tiles half as often or less, but narrow items beside wide ones have a CU
-  // to themselves, and wide tiles write whole tiles of partial states.  At head dims under 256, where a CU otherwise
-  // holds two narrow items, that is never worth it: 128 readers of 8192 tokens beside blocks of 256..2048 tokens, 32 q /
-  // 8 kv heads of 128 dims, us a layer narrow / wide: 208 / 253, 64 q / 16 kv heads of 64 dims 173 / 241.  At 256 dims
-  // (16 q / 4 kv heads, bf16) it is where many re-reads are saved and the rest of the launch is short: 64 readers of
-  // 8192 tokens (0.47 GB saved) beside 0.3 / 0.9 / 1.8 / 5.9 times the tokens that narrow tiles walk for them 72 / 55,
-  // 83 / 73, 99 / 97, 164 / 193; 64 of 32768 (1.9 GB) beside 1.5 / 3.3 times 256 / 206, 359 / 383; 48 of 8192 (0.34 GB)
-  // beside 0.6 times 60 / 52; 128 of 2048 (0.23 GB) beside as many 64 / 68; 128 of 8192 (0.94 GB) beside 5.9 / 13 times
-  // 325 / 317, 605 / 615; 256 of 4096 beside 3.5 times 264 / 255.  From 0.64 GB on a longer rest is let pass (it costs 64
-  // of 32768 some percent, and gains them with 128 readers).  So: on request always; otherwise plans of free size only.
+  // to themselves or wait for them, and wide tiles write whole tiles of partial states.  It is worth it where many re-reads
+  // are saved and the rest of the launch is short.  256 dims (16 q / 4 kv heads, bf16), us a layer narrow / wide: 64
+  // readers of 8192 tokens (0.47 GB saved) beside 0.2 / 0.9 / 3.1 times the tokens that narrow tiles walk for them 68 / 52,
+  // 78 / 68, 107 / 122; 64 of 16384 (0.94 GB) beside 0.1 / 0.5 / 1.5 times 113 / 59, 112 / 75, 139 / 128; 128 of 2048
+  // (0.23 GB) beside as many 52 / 68; 128 of 8192 beside 5.9 / 13 times 325 / 317, 605 / 615.  At 128 dims (32 / 8) the rest
+  // has to be under half: 128 of 8192 (0.94 GB) beside 0.2 / 0.9 / 3.0 times 91 / 85, 104 / 109, 183 / 212, 256 of 4096 0.4 / 1.7
+  // 157 / 105, 144 / 154; from 128 narrow tiles on twice: 512 of 4096 0.4 / 1.7 / 5.9 237 / 161, 315 / 228, 593 / 694.  At 64
+  // dims (64 / 16) it is hardly felt from 64 tiles on: 256 of 4096 beside 0.4 / 1.7 / 6.0 times 158 / 107, 199 / 134, 343 / 311;
+  // with 32, 128 of 16384, 0.4 / 1.5 / 5.9 177 / 164, 239 / 224, 561 / 633; with 16, 64 of 16384, 0.1 / 0.5 / 1.5 107 / 77,
+  // 90 / 94, 129 / 151.  So: on request always; otherwise plans of free size only.
   std::vector<char> group_is_wide(groups.size(), wide_on_request && wide_tile > 0);
   const int64_t token_bytes = 2ll * shape->num_kv_heads * shape->head_dim * (shape->dtype == VA_F32 ? 4 : 2);
-  if (!wide_on_request && wide_tile > 0 && !cap && shape->head_dim == 256) {
+  if (!wide_on_request && wide_tile > 0 && !cap) {
     constexpr int64_t kWorthIt = 300ll << 20, kFairShare = kWorthIt / 8, kWorthMuch = 640ll << 20;
     std::vector<char> many(groups.size(), 0);
     int64_t saved = 0, walked = 0, rest = 0;  // bytes; tokens that narrow tiles walk for these groups, for the others
+    int64_t most_tiles = 0;                   // narrow ones of one of these groups
     for (size_t gi = 0; gi < groups.size(); ++gi) {
       const int64_t n = (int64_t)groups[gi].subrows.size(), len = s->seq_lens[groups[gi].rep];
       const int64_t narrow = (n + q_tile - 1) / q_tile, at_once = tiles_together(kernel, shape->page_size, len);
@@ -261,9 +263,16 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
       const int64_t bytes = (narrow - (int64_t)tiles.size()) * len * token_bytes;
       many[gi] = n > q_tile && bytes >= kFairShare;
       (many[gi] ? walked : rest) += (narrow + at_once - 1) / at_once * len;
-      if (many[gi]) saved += bytes;
+      if (!many[gi]) continue;
+      saved += bytes;
+      most_tiles = std::max(most_tiles, narrow);
     }
-    if (saved >= kWorthIt && rest <= (saved >= kWorthMuch ? 6 : 2) * walked) group_is_wide = many;
+    double times = -1;  // what is walked for them that the rest may be
+    if (saved >= kWorthMuch && shape->head_dim == 256) times = 6;
+    else if (saved >= kWorthIt && shape->head_dim == 256) times = 2;
+    else if (saved >= kWorthMuch && shape->head_dim == 128) times = most_tiles >= 128 ? 2 : 0.5;
+    else if (saved >= kWorthMuch) times = most_tiles >= 64 ? 6 : most_tiles >= 32 ? 2 : 0.25;
+    if ((double)rest <= times * (double)walked) group_is_wide = many;
   }
 
   // ---- chains: sub-requests of one prefill request, in table order ----

@@ -148,7 +148,7 @@ typedef struct VaPlanParams {
   int32_t kv_chunk;      /* 0 = derive from the launch's total KV tokens      */
   int32_t target_items;  /* 0 = default (work items wanted per kv head)       */
   int32_t wide_tile;     /* rows of a wide query tile: 0 = default (prefill tiles; decode readers of one
-                            block only where the re-reads saved outweigh a second launch), >0 = this many
+                            block only where the re-reads saved outweigh what the others lose), >0 = this many
                             rows, decode readers included, <0 = never */
 } VaPlanParams;
 

@@ -98,3 +98,15 @@ def test_tiles_walk_together_where_the_launch_is_long(heads, readers, shared, ow
     limits = native.VaPlanLimits(2 * readers, 2 * readers, 0, 0, 0, readers)
     rc, blob, *_ = fixed_plan(tables, limits, heads=heads, page=16, kernel=native.VA_KERNEL_MFMA)
     assert rc == 0 and max(decode_plan(blob)[1][:, PARTNERS]) == recorded
+
+
+@pytest.mark.parametrize("heads,readers,shared,own,wide", [
+    ((64, 16, 64), 256, 4096, 250, True), ((64, 16, 64), 128, 8192, 200, True), ((64, 16, 64), 64, 8192, 200, False),
+    ((64, 16, 64), 64, 16384, 800, False), ((32, 8, 128), 256, 4096, 64, True), ((32, 8, 128), 256, 4096, 250, False),
+    ((32, 8, 128), 512, 4096, 250, True), ((16, 4, 256), 64, 16384, 250, True), ((16, 4, 256), 64, 4096, 250, False)])
+def test_many_readers_get_wide_tiles_where_the_rest_is_short(heads, readers, shared, own, wide):
+    # us, narrow / wide: 199 / 134, 120 / 114, 70 / 61 (but 106 / 140 beside longer blocks), 129 / 151, 157 / 105, 144 / 154,
+    # 315 / 228, 112 / 75, 59 / 64
+    rc, _, counts = build_plan(*_readers(readers, shared, own), heads=heads, page=16, dtype=native.VA_BF16,
+                               kernel=native.VA_KERNEL_MFMA)
+    assert rc == 0 and (counts.n_wide_items > 0) == wide
