@@ -21,6 +21,8 @@ VA_ROPE_TABLE, VA_ROPE_MROPE = 0, 1
 VA_KERNEL_AUTO, VA_KERNEL_GENERIC, VA_KERNEL_MFMA = 0, 1, 2
 VA_SUB_CAUSAL, VA_SUB_SLOTS = 1, 2
 PLAN_HEADER_WORDS = 24
+PLAN_FLAGS_WORD = 3  # of a header: the chunk, with flags in its low bits
+PLAN_SHORT_ITEMS = 1  # narrow items are short: several workgroups share a CU
 VA_ERR_ARG, VA_ERR_CAPACITY = -1, -2
 STATIC_SCRATCH_BYTES = 32 << 20  # VA_STATIC_SCRATCH_BYTES: the array va_attention_static keeps on every GPU
 

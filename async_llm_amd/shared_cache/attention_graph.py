@@ -45,6 +45,7 @@ class _FixedPlanBuffers:
         self.plan_words = int(native.lib.va_plan_fixed_words(self.capacity))
         self.n_subrows = n_subrows
         self.kv_entries = kv_entries
+        self.launch_flags = 0  # of the recorded launch, the same for every plan
 
         def pair(shape, dtype):
             host = torch.zeros(shape, dtype=dtype, pin_memory=self._cuda)
@@ -93,6 +94,7 @@ class _FixedPlanBuffers:
             raise ValueError(f"Shared attention exceeds graph plan capacity: {native.lib.va_last_error().decode()}")
         native.check(rc)
         header = self._blob_host[: native.PLAN_HEADER_WORDS].numpy().copy()
+        header[native.PLAN_FLAGS_WORD] |= self.launch_flags
         if self.header is None:
             self.header = header
         elif not np.array_equal(header, self.header):
@@ -131,6 +133,13 @@ class SharedDecodeAttentionBuffers(_FixedPlanBuffers):
         total = self.main_count + workers
         limits = native.VaPlanLimits(total, total, 0, 0, 0, workers)
         super().__init__(attention, limits, total, max_pages + workers, use_3d=False)
+        # A recorded launch keeps its kernel.  Where there is no room for more than 1024 tokens a view block, its items are
+        # short and want to share CUs: 64 workers over 64 shared tokens and blocks of 100..400, us a layer, apart / sharing,
+        # 35.0 / 25.8 (16 q / 4 kv heads of 256 dims), 30.9 / 29.8 (32 / 8 of 128), 44.7 / 34.5 (64 / 16 of 64); 128 of 2048
+        # and 64..256 64 / 49, 62 / 51, 83 / 73.  With more room a long run may come: 64 of 8192 and 256..8192 302 / 327,
+        # 299 / 327, 307 / 377.
+        if max_pages * attention.page_size <= 1024 * self.main_count:
+            self.launch_flags = native.PLAN_SHORT_ITEMS
         self.dummy_slots = dummy_slots
         self.dummy_cpu = [0] * workers if dummy_slots is None else dummy_slots.cpu().tolist()
         assert len(self.dummy_cpu) == workers, "one dummy slot per worker"

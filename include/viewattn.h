@@ -220,8 +220,10 @@ VA_API int va_plan_build_within(const VaSubRequests* subs, const VaShape* shape,
  * same buffers; only the contents of the plan blob (and of kv_indices,
  * sub_worker, sub_loc) change.  (Three informational header words differ from a packed
  * plan's: the sub-row and empty-row counts hold max_qrefs and max_rows, and the
- * KV chunk, which is chosen per plan, reads 0, but for the flags beside it; counts->kv_chunk has it.)  Rows beyond subs->n_rows, up to max_rows, get
- * out = 0 and lse = -inf.  A plan that does not fit returns VA_ERR_CAPACITY and
+ * KV chunk, which is chosen per plan, reads 0, but for the flags beside it; counts->kv_chunk has it.  Of the flags
+ * a caller may set bit 0 in the header that it passes to va_attention, for all plans of a recorded launch alike: the
+ * narrow items are served by the kernel for short ones then, whatever they are.)  Rows beyond subs->n_rows, up to
+ * max_rows, get out = 0 and lse = -inf.  A plan that does not fit returns VA_ERR_CAPACITY and
  * names the section.
  */
 typedef struct VaPlanCapacity {

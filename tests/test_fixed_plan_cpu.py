@@ -422,3 +422,18 @@ def test_empty_catalogue_and_foreign_owner(monkeypatch):
     assert not att._workspace_prepared
     with pytest.raises(ValueError, match="belong"):
         att.prepare_workspace([SimpleNamespace(attention=object())])
+
+
+@pytest.mark.parametrize("page,max_pages,short", [(16, 384, True), (16, 385, False), (4, 1536, True), (1, 6145, False)])
+def test_recorded_decode_goes_by_the_room_for_pages(page, max_pages, short):
+    # 2 workers x 3 blocks of 1024 tokens: the flag of the launch hangs on the capacity, not on what a plan holds
+    att, pages = make_attention(page), Pages(page)
+    buffers = SharedDecodeAttentionBuffers(att, workers=2, depth=3, max_pages=max_pages)
+    flag = native.PLAN_SHORT_ITEMS if short else 0
+    assert buffers.header[native.PLAN_FLAGS_WORD] == flag and buffers.meta.launch.header is buffers.header
+    own = [pages.block(2000 if w else 5) for w in range(2)]
+    group = WorkerGroup(cache_structure=[[b] for b in own], write_to=own)
+    pending, slots, _ = plan_decode_writes(group, page, pages, CPU)
+    meta = att.prepare(group, pending, slots, graph_buffers=buffers)
+    assert meta.launch.header[native.PLAN_FLAGS_WORD] == flag
+    assert np.array_equal(meta.launch.blob[: native.PLAN_HEADER_WORDS].numpy()[4:], meta.launch.header[4:])

@@ -61,13 +61,14 @@ def record(op, statics, meta):
     return graph, out, lse
 
 
-@pytest.mark.parametrize("page,dtype,rotary", [(16, torch.bfloat16, 64), (4, torch.float32, 32)])
-def test_decode_graph_follows_each_new_plan(page, dtype, rotary):
+@pytest.mark.parametrize("page,dtype,rotary,max_pages", [(16, torch.bfloat16, 64, 256), (4, torch.float32, 32, 256),
+                                                         (16, torch.float16, 64, 1024), (4, torch.bfloat16, 64, 256)])
+def test_decode_graph_follows_each_new_plan(page, dtype, rotary, max_pages):
     W, depth, theta = 4, 3, 1e4
     Hq, Hkv, D = 8, 2, 64
     op, cpu_pool, dev_pool, gen = make_op_and_pool(DEV, dtype, (Hq, Hkv, D), page, 512, theta, rotary_dim=rotary,
                                                    seed=11, max_pos=2048)
-    buffers = SharedDecodeAttentionBuffers(op, W, depth, max_pages=256, dummy_slots=torch.zeros(W, dtype=torch.int64))
+    buffers = SharedDecodeAttentionBuffers(op, W, depth, max_pages=max_pages, dummy_slots=torch.zeros(W, dtype=torch.int64))
     op.prepare_workspace([buffers])
     workspace = op._workspace.data_ptr()
     q_s = torch.zeros(W, Hq * D, dtype=dtype, device=DEV)
