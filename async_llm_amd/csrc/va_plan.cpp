@@ -463,24 +463,39 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
 
   // Tiles that walk together: not where all start at once apart, and no more to a workgroup than leave every CU one (16
   // readers of 4096 tokens and blocks of 64..200, 256 dims, recorded: in fours 41 us, in pairs 23; 8 readers of 64 tokens and
-  // blocks of 64..200, 32 items to each head: in pairs 12.7, apart 10.1).
+  // blocks of 64..200, 32 items to each head: in pairs 12.7, apart 10.1), nor fours whose longest
+  // takes four fifths of the launch: a four walks a token in 57 ns at 256 dims, a pair in 26, a tile in 17.  Recorded, us,
+  // fours / pairs, and what the longest takes: 256 readers of 4096 in items of 2048 beside blocks of 64..512 235 / 198 (0.87),
+  // 128 of them in 1408 98 / 83 (1.2), 64 of 8192 in 4096 beside 256..8192 301 / 307 (0.79); not recorded, in 2752, 297 / 318
+  // (0.53), and 128 of 4096 in 585 at 128 dims 75 / 90 (0.16).
   const int64_t room = shape->head_dim == 256 ? 320 : 512;  // workgroups that start at once (at 256 dims and a few)
   int64_t stream_groups = 0, stream_tokens = 0;  // workgroups per kv head that serve the narrow tiles, what they walk
   if (kernel == VA_KERNEL_MFMA) {
+    const double wide = shape->head_dim / 256.0;
     int32_t most = tiles_short || (int64_t)out.items.size() * shape->num_kv_heads <= room ? 1 : VA_TOGETHER;
     for (;; most /= 2) {
       stream_groups = stream_tokens = 0;
+      double cu_ns = 0, longest_four = 0;  // per kv head
       int32_t in_unit = 0, unit = -1;
       for (auto& it : out.items) {  // (the items of a unit stand side by side)
         if (it.kind != 0) continue;
         in_unit = it.unit == unit ? in_unit + 1 : 0;
         unit = it.unit;
         it.together = std::min(it.together, most);
-        if (in_unit % it.together) continue;
+        const int32_t place = in_unit % it.together;
+        cu_ns += 5e3;
+        if (place == 2) {
+          cu_ns += (57.0 - 26.0) * wide * it.tokens;
+          longest_four = std::max(longest_four, 57.0 * wide * it.tokens);
+        } else if (place < 2) {
+          cu_ns += (place == 1 ? 26.0 - 17.0 : 17.0) * wide * it.tokens;
+        }
+        if (place) continue;
         ++stream_groups;
         stream_tokens += it.tokens;
       }
-      if (most == 1 || stream_groups * shape->num_kv_heads >= 256) break;
+      const double launch_ns = shape->num_kv_heads * std::max(cu_ns / 256.0, 2.0 * (double)stream_tokens * shape->head_dim * 2 / 6560.0);
+      if (most == 1 || (stream_groups * shape->num_kv_heads >= 256 && longest_four <= 0.8 * launch_ns)) break;
     }
   }
 

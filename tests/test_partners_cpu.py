@@ -87,7 +87,10 @@ def _readers(readers, shared, own, page=16):
     ((16, 4, 256), 16, 4096, 130, True, 0, 0), ((32, 8, 128), 16, 4096, 130, True, 0, 0),
     ((16, 4, 256), 30, 4096, 130, True, 0, 1),
     # short items with few tokens read again; many read again; long items
-    ((32, 8, 128), 64, 2048, 250, True, 0, 1), ((32, 8, 128), 128, 4096, 250, False, 3, 3), ((16, 4, 256), 64, 8192, 5000, False, 3, 3),
+    ((32, 8, 128), 64, 2048, 250, True, 0, 1),
+    # fours would take most of a recorded launch, whose chunks are longer (235 us, in pairs 198)
+    ((16, 4, 256), 256, 4096, 430, False, 3, 1),
+    ((32, 8, 128), 128, 4096, 250, False, 3, 3), ((16, 4, 256), 64, 8192, 5000, False, 3, 3),
 ])
 def test_tiles_walk_together_where_the_launch_is_long(heads, readers, shared, own, short, packed, recorded):
     tables = _readers(readers, shared, own)
