@@ -22,8 +22,10 @@ DEV = torch.device("cuda")
                                          (1, 1), (1, 129), (1, 513), (1, 1000), (8, 257), (8, 961)])
 def test_tiles_that_walk_together(dtype, heads, readers, page, length):
     print(f"heads {heads} readers {readers} length {length} page {page}", flush=True)
-    # one run of 2100 tokens, cut in two and more: the launch's items are not short; many of a token or two fill the CUs
-    lengths = [2100] + [1 + i % 2 for i in range(560 // heads[1])]
+    # a run of 2100 tokens, cut in two and more: the launch's items are not short; more where fours are due, which the
+    # launch has to outlast (at 57 ns a token of 256 dims); many of a token or two fill the CUs
+    together = 4 if length >= 4096 and page == 16 else 2
+    lengths = [2100] * (112 if together == 4 else 1) + [1 + i % 2 for i in range(560 // heads[1])]
     total = -(-length // page) + readers * -(-24 // page) + sum(-(-(n + 1) // page) for n in lengths)
     op, cpu_pool, dev_pool, gen = make_op_and_pool(DEV, dtype, heads, page, total, 1e6, seed=length + readers, scale=0.5,
                                                    kernel="mfma", max_pos=8192)
@@ -49,7 +51,6 @@ def test_tiles_that_walk_together(dtype, heads, readers, page, length):
     items = _items(meta)
     partners = [int(it[6]) for it in items]
     tiles = -(-readers // (16 // (heads[0] // heads[1])))
-    together = 4 if length >= 4096 and page == 16 else 2
     assert max(partners) == min(together, tiles) - 1
     assert sum(1 + p for p in partners if p >= 0) == len(partners)  # every tile is served once
     if tiles > 1:  # the longest of them walks the run, or a third of the long one
