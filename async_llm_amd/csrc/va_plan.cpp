@@ -895,9 +895,11 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   //   * position p of the class holds entry p / 8 of die p % 8; dies with fewer entries are
   //     padded with empty items (n_q = 0, the kernels return at once), which also keeps the
   //     class a multiple of 8 long so the next kv head starts on die 0 again.
+  int32_t longest = 0;  // narrow item
+  for (const auto& it : out.items)
+    if (it.kind == 0) longest = std::max(longest, it.tokens);
   if (kernel == VA_KERNEL_MFMA && !cap) {
     int64_t n = 0, tokens = 0;
-    int32_t longest = 0;
     bool by_themselves = true;
     for (const auto& it : out.items) {
       if (it.kind != 0) {
@@ -906,7 +908,6 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
       }
       ++n;
       tokens += it.tokens;
-      longest = std::max(longest, it.tokens);
     }
     // Where CUs have one item each the other kernel's deeper rings are the better ones (12 requests of 300..2000 behind 128
     // shared tokens, 300 workgroups at 256 dims, 22.6 / 24.6 us; at 64 dims they never are) unless readers of one run walk it
@@ -923,6 +924,7 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
   for (int kind = 1; kind >= 0; --kind) {
     struct Unit {
       int64_t cost = 0, item_cost = 0;
+      int64_t groups = 0;  // workgroups per kv head
       std::vector<int32_t> members;
     };
     std::vector<Unit> units;
@@ -937,7 +939,10 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
       }
       Unit& u = units[at->second];
       const int64_t cost = it.tokens;  // a tile streams its tokens once whatever its row count, and so do partners
-      if (u.members.size() % it.together == 0) u.cost += cost;
+      if (u.members.size() % it.together == 0) {
+        u.cost += cost;
+        ++u.groups;
+      }
       u.item_cost = std::max(u.item_cost, cost);
       u.members.push_back(i);
     }
@@ -1015,6 +1020,7 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
       for (int32_t m : members) {
         Unit single;
         single.cost = single.item_cost = out.items[m].tokens;
+        single.groups = 1;
         single.members.push_back(m);
         units.push_back(single);
         die = pick_die(1);
@@ -1024,16 +1030,25 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     }
     std::vector<int32_t> die_items[kXcds];
     size_t depth = 0;
+    // Workgroups that start together and stream the same number of tokens also finish together, and while they all write
+    // results and set up their next item the memory system idles.  So the first round of a die -- one workgroup for each of
+    // its 32 CUs, two of short items at 256 dims -- is a spread sample of all its sizes where more than two rounds follow:
+    // their staggered ends keep the later ones out of step.  Sixty-four blocks a die over the kv heads, whatever serves
+    // them, is not as good there: 256 requests of 100..800 tokens behind 2048 shared ones at 256 dims 173 us against 164,
+    // 32 of 3000..6000 behind 4096 with 2 heads of 128 57 against 53, 64 of 300..900 behind 64 at 256 dims 50 against 47.
+    // For short items under 256 dims and for launches with tiles of prefill it is the better one: 128 requests of 100..400
+    // tokens behind 64, at 128 dims 45 us against 47, at 64 dims 51 against 53; 48 and two prompts of 512 50 against 54.
+    const bool brief = longest <= kLongestShort && (out.short_items || cap);  // (a caller may give a fixed plan the kernel for short items)
+    const bool by_groups = kind == 0 && (out.n_wide == 0 || out.apart) && (!brief || shape->head_dim == 256);
+    const int64_t slots = out.short_items ? 64 : 32;
     for (int d = 0; d < kXcds; ++d) {
       std::stable_sort(die_units[d].begin(), die_units[d].end(),
                        [&](int32_t x, int32_t y) { return units[x].item_cost > units[y].item_cost; });
-      // Workgroups that start together and stream the same number of tokens also finish together,
-      // and while they all write results and set up their next item the memory system idles.  So
-      // the first round of a die (the items that start at once: 64 workgroup slots) is a spread
-      // sample of all its sizes; their staggered ends keep the later rounds out of step.
       const size_t n_u = die_units[d].size();
-      const size_t first_round = std::min<size_t>(n_u, std::max(1, 64 / shape->num_kv_heads));
-      if (first_round > 1 && n_u > first_round) {
+      int64_t serving = 0;
+      for (int32_t u : die_units[d]) serving += units[u].groups * shape->num_kv_heads;
+      const size_t first_round = by_groups ? slots * n_u / std::max<int64_t>(1, serving) : 64 / shape->num_kv_heads;
+      if (first_round > 1 && (by_groups ? serving > 2 * slots : n_u > first_round)) {
         std::vector<int32_t> head, rest;
         std::vector<char> picked(n_u, 0);
         for (size_t k = 0; k < first_round; ++k) picked[k * (n_u - 1) / (first_round - 1)] = 1;

@@ -210,3 +210,21 @@ def test_runs_of_one_short_chunk_stay_whole(heads):
     assert rc == 0
     walked = sorted(int(it[4]) for it in decode_plan(blob)[1] if it[2] > 0)
     assert walked == sorted(rows[:64] + [768] * 9 + [732] * 9)
+
+
+@pytest.mark.parametrize("heads,each,first", [((16, 4, 256), 1040, 8), ((8, 2, 128), 1040, 16), ((64, 16, 64), 1040, 2),
+                                              ((16, 4, 256), 300, 16)])
+def test_a_die_starts_with_a_spread_of_sizes_for_its_cus(heads, each, first):
+    # one workgroup for each of the 32 CUs of a die (two of short items at 256 dims): its longest, its shortest and those
+    # between, and the rest by size; in turn over the dies
+    rows = [each + i for i in range(400)]
+    kvp = np.cumsum([0] + [-(-n // 16) for n in rows]).tolist()
+    tables = (list(range(len(rows) + 1)), kvp, list(range(kvp[-1])), rows, [0] * len(rows), [-1] * len(rows),
+              list(range(len(rows))), len(rows))
+    rc, blob, counts = build_plan(*tables, heads=heads, page=16, dtype=native.VA_BF16, kernel=native.VA_KERNEL_MFMA,
+                                  kv_chunk=4096 if each > 1000 else 1024)
+    assert rc == 0 and blob[H["KV_CHUNK"]] % 64 == (each < 1000)
+    for die in range(8):
+        walked = [int(it[4]) for it in decode_plan(blob)[1][die::8] if it[2] > 0]
+        assert walked == sorted(walked[:first], reverse=True) + sorted(walked[first:], reverse=True)
+        assert (walked[0], walked[first - 1]) == (max(walked), min(walked))
