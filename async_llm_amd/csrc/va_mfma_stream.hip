@@ -39,12 +39,10 @@ template <typename E, int kD>
 static int launch_stream_dim(const AttnArgs& a, int n_items, bool short_items, hipStream_t stream) {
   // Pages of at least 16 tokens take one scalar lookup per tile, smaller ones an entry per token.  The choice hangs
   // on the page size alone, so that a recorded launch keeps its kernel; in one kernel, the registers of the second
-  // kind spilled into the first at head_dim 256.  (Other page sizes, slot lists beside larger pages, and rings
-  // built deeper than the index entries allow go through the first kernel's per-lane lookups.)
-  if constexpr (StreamShape<kD>::kBuffers <= 4) {
-    if (a.page_size < kStreamTok && (a.page_size & (a.page_size - 1)) == 0)
-      return launch_stream_one<E, kD, true>(a, n_items, short_items, stream);
-  }
+  // kind spilled into the first at head_dim 256.  (Other page sizes and slot lists beside larger
+  // pages go through the first kernel's per-lane lookups.)
+  if (a.page_size < kStreamTok && (a.page_size & (a.page_size - 1)) == 0)
+    return launch_stream_one<E, kD, true>(a, n_items, short_items, stream);
   return launch_stream_one<E, kD, false>(a, n_items, short_items, stream);
 }
 

@@ -1089,7 +1089,7 @@ static int launch_wide_dim(const AttnArgs& a, int n_slots, int n_narrow, hipStre
   // entry per token; the choice hangs on the page size alone, so that a recorded launch keeps its kernel.
   // (Other page sizes, slot lists beside larger pages, and rings built deeper than the index entries allow go
   // through the first kernel's per-lane lookups.)
-  if constexpr (kWideAhead <= 2 && StreamShape<kD>::kBuffers <= 4) {
+  if constexpr (kWideAhead <= 2) {
     if (a.page_size < 16 && (a.page_size & (a.page_size - 1)) == 0)
       return launch_wide_one<E, kD, true>(a, n_slots, n_narrow, stream);
   }

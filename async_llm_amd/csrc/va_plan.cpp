@@ -106,7 +106,7 @@ inline int32_t visible_end(int32_t len, int32_t nq, bool causal, int32_t b) {
 // Four tiles walk at two thirds of the pace of two when memory does not bound them, which a short run beside long ones
 // shows: 48 readers of 512 tokens, 483 us in pairs, 494 in fours.
 int tiles_together(int kernel, int page_size, int64_t tokens) {
-  return kernel != VA_KERNEL_MFMA ? 1 : page_size < 16 || tokens < 4096 ? 2 : VA_TOGETHER;
+  return kernel != VA_KERNEL_MFMA ? 1 : page_size < 16 ? VA_TOGETHER_SCATTERED : tokens < 4096 ? 2 : VA_TOGETHER;
 }
 
 // Work items wanted per kv head.  The streaming kernel: 512 workgroups, but not so few items that their ends leave the

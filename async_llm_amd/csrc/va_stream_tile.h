@@ -39,13 +39,7 @@ constexpr int kStreamThreads = 256;
 constexpr int kStreamWaves = 4;
 constexpr int kStreamTok = 16;  // tokens per tile
 
-#ifndef VA_STREAM_BUFFERS_256
-#define VA_STREAM_BUFFERS_256 2
-#endif
-#ifndef VA_STREAM_BLOCKS_256
-#define VA_STREAM_BLOCKS_256 1
-#endif
-constexpr int kIndexSlots = 8;        // tiles whose index entries a wave's ring of entries holds
+constexpr int kIndexSlots = 8;  // tiles whose index entries a wave's ring of entries holds
 
 // kShort: launches of short items (stream_block_short), where an item's set-up and fold count and those of others have to
 // run beside them: one tile a workgroup, and less LDS, for two to four workgroups on a CU.
@@ -58,21 +52,21 @@ struct StreamShape {
   static constexpr int kRowsPerLoad = kWave / kChunks;       // tile rows one wave-level load covers
   static constexpr int kLoads = kStreamTok / kRowsPerLoad;   // loads of a K (or V) tile
   static constexpr int kTileBytes = kStreamTok * kRowBytes;  // a K (or V) tile
-  // ring depth of a wave, in tiles, and workgroups per CU (registers and LDS allow)
-  static constexpr int kBuffers = kShort ? (kD == 64 ? 2 : 1) : kD == 256 ? VA_STREAM_BUFFERS_256 : kD == 128 ? 2 : 4;
-  static constexpr int kMinBlocks = kShort ? (kD == 256 ? 2 : kD == 128 ? 3 : 4) : kD == 256 ? VA_STREAM_BLOCKS_256 : 2;
+  // ring depth of a wave, in tiles, and workgroups per CU (as registers and LDS allow)
+  static constexpr int kBuffers = kShort ? (kD == 64 ? 2 : 1) : kD == 64 ? 4 : 2;
+  static constexpr int kMinBlocks = kShort ? (kD == 256 ? 2 : kD == 128 ? 3 : 4) : kD == 256 ? 1 : 2;
   // A wave's state at the end, in its own ring: accumulators (rows padded by 16 bytes, so that the sixteen rows of a
   // write spread over the banks), then maxima and sums.
   static constexpr int kFoldRowBytes = kD * 4 + 16;
   static constexpr int kFoldBytes = (16 * (kFoldRowBytes + 8) + 1023) / 1024 * 1024;
   static constexpr int kWaveRingBytes = kBuffers * 2 * kTileBytes > kFoldBytes ? kBuffers * 2 * kTileBytes : kFoldBytes;
   static constexpr int kRingBytes = kStreamWaves * kWaveRingBytes;
-  // Behind the rings: the rotated query rows of up to four items, or of two and for every wave the index entries of
-  // kIndexSlots tiles.
-  static constexpr int kIndexOffset = kRingBytes + (kShort ? 1 : 2) * 16 * kRowBytes;
+  // Behind the rings: the rotated query rows of the items that walk together, over scattered rows of fewer and for every
+  // wave the index entries of kIndexSlots tiles.
+  static constexpr int kIndexOffset = kRingBytes + (kShort ? 1 : VA_TOGETHER_SCATTERED) * 16 * kRowBytes;
   static constexpr int kIndexBytes = kIndexSlots * kStreamTok * 4;
   static constexpr int lds_bytes(bool gather) {
-    return gather ? kIndexOffset + kStreamWaves * kIndexBytes : kRingBytes + (kShort ? 1 : 4) * 16 * kRowBytes;
+    return gather ? kIndexOffset + kStreamWaves * kIndexBytes : kRingBytes + (kShort ? 1 : VA_TOGETHER) * 16 * kRowBytes;
   }
 };
 
@@ -122,7 +116,8 @@ template <typename E, int kD, bool kGather, int kB, bool kShort = false>
 __device__ __forceinline__ void stream_items(const AttnArgs& a, const int (&item)[kB][VA_ITEM_WORDS], int hk) {
   using S = typename E::storage;
   using Sh = StreamShape<kD, kShort>;
-  static_assert(!kShort || kB == 1, "room for the query rows of one tile");
+  static_assert(kB <= (kShort ? 1 : kGather ? VA_TOGETHER_SCATTERED : VA_TOGETHER), "room for the query rows of so many tiles");
+  static_assert(Sh::kMinBlocks * Sh::lds_bytes(kGather) <= 160 * 1024, "the LDS of a CU");
   constexpr int kChunks = Sh::kChunks, kSteps = Sh::kSteps, kDimTiles = Sh::kDimTiles, kBuffers = Sh::kBuffers;
   constexpr int kLoads = Sh::kLoads, kRowBytes = Sh::kRowBytes, kTileBytes = Sh::kTileBytes;
   // the entries of tiles i + 1 .. i + 2 kBuffers of a wave are held or on their way at any time
@@ -589,13 +584,18 @@ __device__ __forceinline__ void stream_block(const AttnArgs& a, unsigned block) 
       if (b > partners) items[b][VA_I_N_Q] = 0;
     stream_items<E, kD, kGather, kB>(a, items, where.head);
   };
+  static_assert(VA_TOGETHER == 4 && VA_TOGETHER_SCATTERED == 2, "the tiles served together below");
   if (partners == 0) {
     stream_items<E, kD, kGather, 1>(a, item, where.head);
-  } else if (kGather || partners == 1) {
-    together(std::integral_constant<int, 2>{});
-  } else {
-    together(std::integral_constant<int, 4>{});
+    return;
   }
+  if constexpr (!kGather) {
+    if (partners > 1) {
+      together(std::integral_constant<int, 4>{});
+      return;
+    }
+  }
+  together(std::integral_constant<int, 2>{});
 }
 
 // The same where items are short: its workgroups serve a tile each, also one that a plan would have walk with others.
