@@ -29,8 +29,12 @@ def test_wide_and_streaming_items_share_a_launch(dtype, heads, page, rows, chunk
     assert_close(out.cpu(), expected.cpu().view_as(out.cpu()), dtype, "out")
     assert_close(lse.cpu(), expected_lse.cpu(), dtype, "lse")
     # planned again, the same bits: nothing hangs on which workgroup a CU gets first
-    again, again_lse = wl.op.attend(wl.q, 0, wl.meta, return_lse=True)
-    assert torch.equal(out, again) and torch.equal(lse, again_lse)
+    wl.op.plan_params.kernel = native.VA_KERNEL_MFMA
+    fresh = wl.op.prepare_mixed(wl.group, wl.pending, wl.new_token_slots, wl.specs)
+    assert fresh.launch.counts.kernel == native.VA_KERNEL_MFMA
+    for meta in (wl.meta, fresh):
+        again, again_lse = wl.op.attend(wl.q, 0, meta, return_lse=True)
+        assert torch.equal(out, again) and torch.equal(lse, again_lse)
 
 
 @pytest.mark.parametrize("dtype,heads,page,apart", [(torch.bfloat16, (64, 16, 64), 16, 3), (torch.float16, (32, 8, 128), 16, 3),

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from async_llm_amd.shared_cache import CacheBlock, WorkerGroup
-from tests.util import make_op_and_pool, run_decode_parity
+from tests.util import make_op_and_pool, narrow_items, run_decode_parity
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda")
@@ -48,7 +48,7 @@ def test_tiles_that_walk_together(dtype, heads, readers, page, length):
     *_, meta = run_decode_parity(op, cpu_pool, dev_pool, group, allocator, 1e6, gen)
     counts = meta.launch.counts
     assert counts.n_wide_items == 0 < counts.n_items and not meta.launch.header[3] & 1  # not the kernel for short items
-    items = _items(meta)
+    items = narrow_items(meta)
     partners = [int(it[6]) for it in items]
     tiles = -(-readers // (16 // (heads[0] // heads[1])))
     assert max(partners) == min(together, tiles) - 1
@@ -59,10 +59,3 @@ def test_tiles_that_walk_together(dtype, heads, readers, page, length):
         rings = 4 if heads[2] == 64 else 2
         assert length < 700 or longest > 64 * rings  # its waves refill their rings
         assert length not in (513, 1000, 961) or page == 16 or longest > 64 * 8  # and come round in their index entries
-
-
-def _items(meta):
-    header = meta.launch.header
-    words = meta.launch.blob.cpu().numpy()
-    items = words[header[10]: header[10] + 16 * meta.launch.counts.n_items].reshape(-1, 16)
-    return [it for it in items if it[2] > 0]

@@ -100,6 +100,13 @@ def fused_rows(dev, *parts):
     return views
 
 
+def narrow_items(meta):
+    """The item words of a decode plan, without the padding."""
+    words, header = meta.launch.blob.cpu().numpy(), meta.launch.header
+    items = words[header[10]: header[10] + 16 * meta.launch.counts.n_items].reshape(-1, 16)
+    return [it for it in items if it[2] > 0]
+
+
 def run_decode_parity(op, cpu_pool, dev_pool, group, page_alloc, theta, gen, scale=None, check_pool_exact=True,
                       lse_base2=False, fused_qkv=False):
     """One decode step through the product op and through the oracle; returns
