@@ -587,15 +587,11 @@ __device__ __forceinline__ void stream_block(const AttnArgs& a, unsigned block) 
   static_assert(VA_TOGETHER == 4 && VA_TOGETHER_SCATTERED == 2, "the tiles served together below");
   if (partners == 0) {
     stream_items<E, kD, kGather, 1>(a, item, where.head);
-    return;
+  } else if (kGather || partners == 1) {
+    together(std::integral_constant<int, 2>{});
+  } else if constexpr (!kGather) {
+    together(std::integral_constant<int, 4>{});
   }
-  if constexpr (!kGather) {
-    if (partners > 1) {
-      together(std::integral_constant<int, 4>{});
-      return;
-    }
-  }
-  together(std::integral_constant<int, 2>{});
 }
 
 // The same where items are short: its workgroups serve a tile each, also one that a plan would have walk with others.
