@@ -34,7 +34,8 @@ HOST_FLAGS = ["--offload-arch=gfx950", "--cuda-host-only"]
 # score products are read by the vector ALU at once and want ordinary registers (the long-lived
 # output accumulators are pinned in accumulation registers by hand).
 # The streaming kernel rescales its accumulators now and then: in accumulation registers it would copy all of them
-# back and forth in every tile.
+# back and forth in every tile.  At 256 dims the flag spares that where a workgroup serves one tile; with two, 76 of the 748
+# instructions of a tile's loop still move accumulators, with four 399 of 1421: they do not fit 256 registers.
 SOURCE_DEVICE_FLAGS = {"va_mfma_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
                        "va_mfma_stream.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 

@@ -104,7 +104,9 @@ inline int32_t visible_end(int32_t len, int32_t nq, bool causal, int32_t b) {
 // Narrow tiles of a run of `tokens` that a workgroup serves together at most.  Four where the run is long: 64 readers of
 // 8192 tokens beside private blocks (16 q / 4 kv heads of 256 dims) 353 us a layer alone, 322 in pairs, 313 in fours.
 // Four tiles walk at two thirds of the pace of two when memory does not bound them, which a short run beside long ones
-// shows: 48 readers of 512 tokens, 483 us in pairs, 494 in fours.
+// shows: 48 readers of 512 tokens, 483 us in pairs, 494 in fours.  Where the line lies, us in pairs / in fours, 256 dims and
+// 2 kv heads of 128: 128 readers of 2048 tokens 270 / 281, 73 / 78; 48 of 3000 139 / 139, 45 / 45; 64 of 4096 166 / 163,
+// 49 / 46; 64 of 12000 349 / 308, 90 / 90 (at 64 dims 48 of 3000 142 / 139, 64 of 4096 170 / 166, 64 of 12000 330 / 307).
 int tiles_together(int kernel, int page_size, int64_t tokens) {
   return kernel != VA_KERNEL_MFMA ? 1 : page_size < 16 ? VA_TOGETHER_SCATTERED : tokens < 4096 ? 2 : VA_TOGETHER;
 }
@@ -418,7 +420,8 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     cut_tiles((int64_t)gr.subrows.size(), tiles, group_is_wide[&gr - &groups[0]]);
     // A run that a single query tile reads is fetched once per kv head and never again: its rows are
     // requested as lines to evict first, so that they stream through the die's L2 without pushing
-    // out the rows that several tiles read side by side (a block shared by many views).
+    // out the rows that several tiles read side by side (a block shared by many views).  (Runs whose few tiles all share
+    // one workgroup are fetched once too, but asked for as the shared ones are.)
     const int32_t lflags = VA_LINK_INDIRECT | ((s->flags[rep] & VA_SUB_SLOTS) ? VA_LINK_SLOTS : 0) |
                            (tiles.size() == 1 ? VA_LINK_ONCE : 0);
     std::vector<int32_t> tile_qref;

@@ -65,7 +65,7 @@ enum {
 // Narrow items of a launch of their own that are short: their set-up and fold take as long as their walk, so several
 // workgroups share a CU and serve a tile each (attn_stream_short_kernel, whose workgroups take no notice of VA_I_PARTNERS).
 // 64 requests over 64 shared tokens and one or two private blocks, us a layer, in the kernel before independent waves / in
-// the ordinary kernel / now: blocks of 300..900, 16 q / 4 kv heads of 256 dims 48.9 / 60.3 / 50.3, 32 / 8 of 128
+// the ordinary kernel / now: blocks of 300..900, 16 q / 4 kv heads of 256 dims 48.9 / 60.3 / 47.1, 32 / 8 of 128
 // 51.7 / 53.6 / 49.9, 64 / 16 of 64 61.3 / 61.9 / 50.9; of 100..400 26.9 / 31.6 / 24.8, 28.4 / 29.4 / 26.2, 36.5 / 40.1 / 28.0.
 #define VA_CHUNK_SHORT_ITEMS 1
 // Wide and narrow items get a launch each (one launch serves both otherwise).  In a plan of fixed capacity a matter of the

@@ -13,9 +13,9 @@
 //   * a wave keeps its own softmax state; the four are folded through LDS at the end of the item;
 //   * up to four items that walk the same tokens (the tiles of one run's many readers) share a workgroup: the tokens
 //     are read once for all of them, where each used to read them from the die's L2.
-// Launches of 16 q / 4 kv heads of 256 dims, bf16, us before and now: 64 requests over a shared prompt 353 -> 313
-// (1.96 GB = 6.3 TB/s), eight of 131072 tokens 678 -> 636 (4.3 GB = 6.8), 48 of 1 k..32 k 508 -> 487; 32 requests over
-// token slots, 32 q / 8 kv heads of 128 dims, 92 -> 90.  An item costs about 5 us of set-up and fold, hence the few
+// Launches of 16 q / 4 kv heads of 256 dims, bf16, us with one ring and with four: 64 requests over a shared prompt
+// 353 -> 313 to 323 (1.96 GB = 6.1 to 6.3 TB/s), eight of 131072 tokens 678 -> 636 to 662 (4.3 GB = 6.5 to 6.8), 48 of
+// 1 k..32 k 508 -> 487; 32 requests over token slots, 32 q / 8 kv heads of 128 dims, 92 -> 90 to 93.  An item costs about 5 us of set-up and fold, hence the few
 // long items the planner makes (default_target).
 //
 //   S^T[16 tokens, 16 rows] = K . Q^T    v_mfma_f32_16x16x32, K from LDS as the A operand, the rotated query
