@@ -1034,16 +1034,18 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     std::vector<int32_t> die_items[kXcds];
     size_t depth = 0;
     // Workgroups that start together and stream the same number of tokens also finish together, and while they all write
-    // results and set up their next item the memory system idles.  So the first round of a die -- one workgroup for each of
-    // its 32 CUs, two of short items at 256 dims -- is a spread sample of all its sizes where more than two rounds follow:
-    // their staggered ends keep the later ones out of step.  Sixty-four blocks a die over the kv heads, whatever serves
-    // them, is not as good there: 256 requests of 100..800 tokens behind 2048 shared ones at 256 dims 173 us against 164,
-    // 32 of 3000..6000 behind 4096 with 2 heads of 128 57 against 53, 64 of 300..900 behind 64 at 256 dims 50 against 47.
-    // For short items under 256 dims and for launches with tiles of prefill it is the better one: 128 requests of 100..400
-    // tokens behind 64, at 128 dims 45 us against 47, at 64 dims 51 against 53; 48 and two prompts of 512 50 against 54.
+    // results and set up their next item the memory system idles.  So the first round of a die -- what its 32 CUs start of
+    // the ordinary kernel, one workgroup each at 256 dims (two of short items) and two under that -- is a spread sample of
+    // all its sizes where more than two rounds follow: their staggered ends keep the later ones out of step.  Sixty-four
+    // blocks a die over the kv heads, whatever serves them, are not as good there: 256 requests of 100..800 tokens behind
+    // 2048 shared ones at 256 dims 173 us against 164, 32 of 600..6000 over token slots 97 against 89, 32 of 3000..6000
+    // behind 4096 with 2 heads of 128 57 against 53.  Nor is one workgroup a CU under 256 dims (64 of 1000..8000 over slots
+    // at 128 dims 191 against 201).  For short items under 256 dims and for launches with tiles of prefill the blocks are
+    // the better ones: 128 requests of 100..400 tokens behind 64, at 128 dims 45 us against 47, at 64 dims 51 against 53; 48
+    // and two prompts of 512 50 against 54.
     const bool brief = longest <= kLongestShort && (out.short_items || cap);  // (a caller may give a fixed plan the kernel for short items)
     const bool by_groups = kind == 0 && (out.n_wide == 0 || out.apart) && (!brief || shape->head_dim == 256);
-    const int64_t slots = out.short_items ? 64 : 32;
+    const int64_t slots = shape->head_dim == 256 && !out.short_items ? 32 : 64;
     for (int d = 0; d < kXcds; ++d) {
       std::stable_sort(die_units[d].begin(), die_units[d].end(),
                        [&](int32_t x, int32_t y) { return units[x].item_cost > units[y].item_cost; });

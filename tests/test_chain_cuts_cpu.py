@@ -212,11 +212,11 @@ def test_runs_of_one_short_chunk_stay_whole(heads):
     assert walked == sorted(rows[:64] + [768] * 9 + [732] * 9)
 
 
-@pytest.mark.parametrize("heads,each,first", [((16, 4, 256), 1040, 8), ((8, 2, 128), 1040, 16), ((64, 16, 64), 1040, 2),
+@pytest.mark.parametrize("heads,each,first", [((16, 4, 256), 2100, 8), ((8, 2, 128), 2100, 32), ((64, 16, 64), 2100, 4),
                                               ((16, 4, 256), 300, 16)])
 def test_a_die_starts_with_a_spread_of_sizes_for_its_cus(heads, each, first):
-    # one workgroup for each of the 32 CUs of a die (two of short items at 256 dims): its longest, its shortest and those
-    # between, and the rest by size; in turn over the dies
+    # what the 32 CUs of a die start, one workgroup each at 256 dims (two of short items), two under that: its longest, its
+    # shortest and those between, and the rest by size
     rows = [each + i for i in range(400)]
     kvp = np.cumsum([0] + [-(-n // 16) for n in rows]).tolist()
     tables = (list(range(len(rows) + 1)), kvp, list(range(kvp[-1])), rows, [0] * len(rows), [-1] * len(rows),
