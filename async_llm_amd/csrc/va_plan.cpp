@@ -917,7 +917,13 @@ int build(const VaSubRequests* s, const VaShape* shape, const VaPlanParams* para
     // apart: their tiles in flight, 128 KB a CU, push each other out of the die's L2 (16 readers of 4096 tokens, 224
     // workgroups at 256 dims, 22.5 / 16.9).
     const int64_t one_each = shape->head_dim == 256 ? room : shape->head_dim == 128 ? 256 : 0, again = walked[1] - walked[0];
-    out.short_items = by_themselves && (tiles_short || any_wide) && longest <= kLongestShort && again * token_bytes <= kReadAgain &&
+    // At 128 dims the ordinary kernel, with two workgroups on a CU, is also the better one for items of more than 704 tokens
+    // (32 requests of 600..6000 over token slots, 960 a walk, short / ordinary 90.4 / 89.8 us; 2 kv heads, 32 of 3000..8000 in
+    // 768 45.0 / 42.6, 64 of 2048 shared tokens and 1000..2000 39.0 / 35.8; of 704 66.6 / 67.3 and 68.1 / 71.0) unless all
+    // start at once (24 of 300..2000 over token slots, 360 workgroups, 31.1 / 31.7; the 16 readers of 4096 apart 16.0 / 16.8).
+    const bool rounds = n * shape->num_kv_heads > (again > tokens / 8 ? 768 : 512);
+    const int32_t longest_short = shape->head_dim == 128 && rounds ? 704 : kLongestShort;
+    out.short_items = by_themselves && (tiles_short || any_wide || again == 0) && longest <= longest_short && again * token_bytes <= kReadAgain &&
                       (n * shape->num_kv_heads > one_each || again > tokens / 8);
     if (out.short_items)
       for (auto& it : out.items) it.together = 1;

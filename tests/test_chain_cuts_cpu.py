@@ -228,3 +228,17 @@ def test_a_die_starts_with_a_spread_of_sizes_for_its_cus(heads, each, first):
         walked = [int(it[4]) for it in decode_plan(blob)[1][die::8] if it[2] > 0]
         assert walked == sorted(walked[:first], reverse=True) + sorted(walked[first:], reverse=True)
         assert (walked[0], walked[first - 1]) == (max(walked), min(walked))
+
+
+@pytest.mark.parametrize("heads,rows,short", [
+    ((64, 16, 64), [800 + 3 * i for i in range(64)], 1),  # runs that one tile reads: as long as its items are, whatever the chunk
+    ((32, 8, 128), [600 + 174 * i for i in range(32)], 0),  # 128 dims, more than start at once: up to 704 tokens an item
+    ((32, 8, 128), [300 + 4 * i for i in range(100)], 1),
+    ((32, 8, 128), [300 + 70 * i for i in range(24)], 1),  # all at once
+])
+def test_short_items_by_their_length(heads, rows, short):
+    kvp = np.cumsum([0] + [-(-n // 16) for n in rows]).tolist()
+    tables = (list(range(len(rows) + 1)), kvp, list(range(kvp[-1])), rows, [0] * len(rows), [-1] * len(rows),
+              list(range(len(rows))), len(rows))
+    rc, blob, counts = build_plan(*tables, heads=heads, page=16, dtype=native.VA_BF16, kernel=native.VA_KERNEL_MFMA)
+    assert rc == 0 and blob[H["KV_CHUNK"]] - counts.kv_chunk == short
