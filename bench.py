@@ -51,11 +51,10 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0
 # carried here together with the digest of the kernel sources they were measured on
 # (csrc_digest()), and are reported only while that digest is the one of the sources in the tree.
 MEASURED_TRAFFIC = {
-    ("batched_decode", "mfma"): {"bytes": 2 * 1024 * (1_112_090 + 4_143) + 1024 * (8_160 + 512), "csrc": "844e07adf982e67e"},
-    ("mrope_decode", "mfma"): {"bytes": 2 * 1024 * (2_097_910 + 1_608) + 1024 * (3_096 + 64), "csrc": "844e07adf982e67e"},
-    ("view_prefill", "mfma"): {"bytes": 2 * 1024 * 2_496_982 + 1024 * 131_323, "csrc": "08c375c61b54cd3d"},
-    ("mixed_batch", "mfma"): {"bytes": 2 * 1024 * (439_645 + 1_623_108 + 27_058) + 1024 * (47_429 + 12_397 + 10_624),
-                              "csrc": "08c375c61b54cd3d"},
+    ("batched_decode", "mfma"): {"bytes": 2 * 1024 * (1_120_577 + 4_022) + 1024 * (7_918 + 512), "csrc": "cb1697e5b50cbbc4"},
+    ("mrope_decode", "mfma"): {"bytes": 2 * 1024 * (2_097_913 + 1_608) + 1024 * (3_096 + 64), "csrc": "cb1697e5b50cbbc4"},
+    ("view_prefill", "mfma"): {"bytes": 2 * 1024 * 2_515_933 + 1024 * 131_129, "csrc": "cb1697e5b50cbbc4"},
+    ("mixed_batch", "mfma"): {"bytes": 2 * 1024 * (2_330_836 + 20_575) + 1024 * (48_209 + 9_088), "csrc": "cb1697e5b50cbbc4"},
 }
 
 
