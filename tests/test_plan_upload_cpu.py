@@ -89,3 +89,5 @@ def test_the_header_handed_to_a_launch_is_the_plans_own():
     launch.header = launch.header.copy()
     for plan in [launch, *copies]:
         assert plan.header_ptr == plan.header.ctypes.data != kept
+        plan.header.flags.writeable = False
+        assert plan.header_ptr == plan.header.ctypes.data
